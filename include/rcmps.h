@@ -107,11 +107,11 @@ typedef struct {
     double trajectory_ms, pullback_ms, boundary_ms, total_ms;
     int krylov_matvecs;
     double krylov_residual;
-    /* per system, workgroup 0 of the trajectory kernel, microseconds spent in: wait for stage
-       inputs, load inputs, level-1 products, level-2 products before the neighbour tiles, wait for
-       neighbour tiles, load them, remaining products and epilogue, integrator bookkeeping,
-       step end (error norm, record, all-gather), whole kernel, publishing the next stage input,
-       stage entry.  The excitation action: [0][0..3] its kinetic phases; [4][0..3] workgroup 0 of
+    /* per system, workgroup 0 of the trajectory kernel, microseconds spent in: wait for the stage
+       input (its loads included), split precision: slicing it, level-1 products and their publish,
+       level-2 products before the neighbour tiles, wait for the neighbour tiles, split: slicing them,
+       remaining products and epilogue, integrator bookkeeping, step end (error norm, record,
+       all-gather), whole kernel, publishing the next stage input, unused.  The excitation action: [0][0..3] its kinetic phases; [4][0..3] workgroup 0 of
        the persistent action ODE launch in the right-hand-side products, the exchanges between
        stages, the step controller and the whole launch */
     double phase_us[6][12];

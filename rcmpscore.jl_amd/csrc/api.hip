@@ -27,8 +27,9 @@
 #include "trajectory.h"
 
 int rc_trajectory_smem_bytes(int nb, int split);
-hipError_t rc_trajectory_capacity(int nb, int split, int* blocks);
-hipError_t rc_launch_trajectory(int nb, int split, int nblocks, const TrajParams* dparams, hipStream_t stream);
+hipError_t rc_trajectory_capacity(int nb, int split, int z2, int timed, int* blocks);
+hipError_t rc_launch_fill_empty(void* dst, size_t bytes, hipStream_t stream);
+hipError_t rc_launch_trajectory(int nb, int split, int z2, int timed, int nblocks, const TrajParams* dparams, hipStream_t stream);
 
 using rc::cd;
 using rc::Mat;
@@ -87,13 +88,10 @@ struct KineticWork {
 };
 
 struct TrajBufs {
-    DevBuf Y[RC_NSYS], P[RC_NSYS], rec[RC_NSYS], samples[RC_NSYS], E, fixed, flags, out;
-    size_t flag_bytes = 0;
+    DevBuf samples[RC_NSYS], fixed;
     void release() {
-        for (int s = 0; s < RC_NSYS; ++s) {
-            Y[s].release(); P[s].release(); rec[s].release(); samples[s].release();
-        }
-        E.release(); fixed.release(); flags.release(); out.release();
+        for (int s = 0; s < RC_NSYS; ++s) samples[s].release();
+        fixed.release();
     }
 };
 
@@ -181,6 +179,7 @@ struct rcmps_context {
     // trajectory workspaces: per evaluation of a launch, and the launch description
     std::vector<std::unique_ptr<TrajBufs>> tb;
     DevBuf traj_params, traj_tasks, traj_sys, traj_sched, traj_points, abort_word;
+    DevBuf traj_exch, traj_out;   // exchange rings and system results of one launch's evaluations
     // pullback / misc workspaces
     DevBuf nodes_w, nodes_j, tmpM, partial, scratch, small;
     // krylov workspaces
@@ -857,7 +856,7 @@ void rcmps_context_destroy(rcmps_context* ctx) {
     ctx->workers.clear();
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-    DevBuf* all[] = {&ctx->traj_params, &ctx->traj_tasks, &ctx->traj_sys, &ctx->traj_sched,
+    DevBuf* all[] = {&ctx->traj_params, &ctx->traj_tasks, &ctx->traj_sys, &ctx->traj_sched, &ctx->traj_exch, &ctx->traj_out,
                      &ctx->traj_points, &ctx->abort_word, &ctx->nodes_w, &ctx->nodes_j,
                      &ctx->tmpM, &ctx->partial, &ctx->scratch, &ctx->small, &ctx->kry_V, &ctx->kry_w,
                      &ctx->kry_t1, &ctx->kry_t2, &ctx->kry_x, &ctx->kry_b, &ctx->kry_z, &ctx->kry_h,
@@ -1119,8 +1118,29 @@ void ensure_quadrature(rcmps_context* ctx, const rcmps_integrator* ip) {
 
 // Fixed insertion sources, the six systems and their tasks for one state (src/observables.jl:7-29:
 // kinetic edges sqrt2 with op R or [Q,R], :phi^4: edges k -> k+1 with coefficient k).
-void build_state(rcmps_context* ctx, TrajBufs& tb, const rcmps_state* st, bool adjoint, bool quartic_only, bool z2,
-                 int npts, std::vector<TrajSys>& sys, std::vector<TrajTask>& tasks) {
+int system_tasks(int s, int NT, bool adjoint, bool quartic_only) {
+    // the commutator adjoint system (s = 3) forms channel 1's E = X C in NT tasks of its own,
+    // ranked after the channels' tasks, so channel 1 has one level-1 product like every other
+    // channel and channel 0's insertion does not wait for a second one
+    return (!adjoint && s % 2) || (quartic_only && s < 4) ? 0 : kLive[s] * NT + (s == 3 ? NT : 0);
+}
+
+// bytes of a system's exchange rings (stage inputs twice, level-1 tiles, E, error records) and of one
+// evaluation's
+size_t system_exchange_bytes(int Dp, int s, int ntasks) {
+    const size_t mb = (size_t)Dp * Dp * 16;
+    return ntasks == 0 ? 0 : RC_RING * (3 * kLive[s] + (s == 3 ? 1 : 0)) * mb + (size_t)RC_REC_RING * ntasks * RC_REC * 8;
+}
+size_t exchange_bytes(int Dp, bool adjoint, bool quartic_only) {
+    const int NT = (Dp / 16) * (Dp / 16);
+    size_t bytes = 0;
+    for (int s = 0; s < RC_NSYS; ++s)
+        bytes += system_exchange_bytes(Dp, s, system_tasks(s, NT, adjoint, quartic_only));
+    return bytes;
+}
+
+void build_state(rcmps_context* ctx, TrajBufs& tb, char* exch, double* out, const rcmps_state* st, bool adjoint,
+                 bool quartic_only, bool z2, int npts, std::vector<TrajSys>& sys, std::vector<TrajTask>& tasks) {
     const int D = st->D, Dp = st->Dp, NB = Dp / 16, NT = NB * NB;
     // parity of every live channel's stage input for a Z2 state (rho0 and I even; R, R^+, [Q,R] odd;
     // the insertions and the fixed sources flip it once per operator factor)
@@ -1146,13 +1166,6 @@ void build_state(rcmps_context* ctx, TrajBufs& tb, const rcmps_state* st, bool a
     dv.gemm(0, st->rho.d(), 0, st->Rh.d(), fQF, 1.0, 1.0);
     dv.axpby(cd(4, 0), st->R.d(), cd(4, 0), st->Rh.d(), fQA);         // 4 (R + R^+)
 
-    size_t flag_words = 0;
-    for (int s = 0; s < RC_NSYS; ++s) flag_words += (size_t)2 * kLive[s] * NT + NT + 64;
-    ck(tb.flags.ensure(flag_words * 4));
-    tb.flag_bytes = flag_words * 4;
-    ck(tb.out.ensure(RC_NSYS * RC_OUT_STRIDE * 8));
-    ck(tb.E.ensure((size_t)RC_NSTAGE_BUF * mb));
-    uint32_t* fl = static_cast<uint32_t*>(tb.flags.p);
     const int sys_base = (int)sys.size();
     for (int s = 0; s < RC_NSYS; ++s) {
         TrajSys Sy{};
@@ -1160,29 +1173,19 @@ void build_state(rcmps_context* ctx, TrajBufs& tb, const rcmps_state* st, bool a
         Sy.has_scalar = kHasScalar[s];
         Sy.adj = s % 2;
         Sy.first_task = (int)tasks.size();
-        // the commutator adjoint system (s = 3) forms channel 1's E = X C in NT tasks of its own,
-        // ranked after the channels' tasks, so channel 1 has one level-1 product like every other
-        // channel and channel 0's insertion does not wait for a second one
-        Sy.ntasks = (!adjoint && s % 2) || (quartic_only && s < 4) ? 0 : kLive[s] * NT + (s == 3 ? NT : 0);
+        Sy.ntasks = system_tasks(s, NT, adjoint, quartic_only);
         Sy.D = D;
         Sy.n_elems = (double)kLive[s] * D * D + kHasScalar[s];
         Sy.Q = st->Q.d(); Sy.Qh = st->Qh.d(); Sy.R = st->R.d(); Sy.Rh = st->Rh.d(); Sy.C = st->C.d();
-        Sy.flagY = fl; fl += kLive[s] * NT;
-        Sy.flagP = fl; fl += kLive[s] * NT;
-        Sy.flagE = fl; fl += NT;
-        Sy.flagR = fl; fl += 64;
-        Sy.out = tb.out.d() + s * RC_OUT_STRIDE;
+        Sy.out = out + s * RC_OUT_STRIDE;
         if (Sy.ntasks > 64) throw Fail{RCMPS_ERR_UNSUPPORTED};
         if (Sy.ntasks > 0) {
             if ((size_t)npts * kLive[s] * mb >= (size_t)1 << 31) throw Fail{RCMPS_ERR_UNSUPPORTED};
-            ck(tb.Y[s].ensure((size_t)RC_NSTAGE_BUF * kLive[s] * mb));
-            ck(tb.P[s].ensure((size_t)RC_NSTAGE_BUF * kLive[s] * mb));
-            ck(tb.rec[s].ensure((size_t)2 * Sy.ntasks * RC_REC * 8));
             ck(tb.samples[s].ensure((size_t)npts * kLive[s] * mb));
-            Sy.Y = tb.Y[s].d();
-            Sy.P = tb.P[s].d();
-            Sy.E = s == 3 ? tb.E.d() : nullptr;
-            Sy.rec = tb.rec[s].d();
+            Sy.has_E = s == 3;
+            Sy.exch_bytes = (uint32_t)system_exchange_bytes(Dp, s, Sy.ntasks);
+            Sy.exch = reinterpret_cast<double*>(exch);
+            exch += Sy.exch_bytes;
             Sy.samples = tb.samples[s].d();
         }
         const int term = s / 2, adj = s % 2;
@@ -1192,6 +1195,10 @@ void build_state(rcmps_context* ctx, TrajBufs& tb, const rcmps_state* st, bool a
                     TrajTask t{};
                     t.sys = sys_base + s; t.ch = ch; t.b = b; t.c = c; t.adj = adj;
                     t.edge_src = -1;
+                    // what another channel's insertion or the E tasks read: the level-1 tiles of :phi^4:'s
+                    // channels and of the kinetic adjoint's channel 1, the commutator adjoint's channel 1
+                    t.pub_p = term == 2 || (s == 1 && ch == 1);
+                    t.pub_y = s == 3 && ch == 1;
                     {
                         const int px = kParity[s][ch];
                         const int m1 = adj ? z2_kmask(NB, zt, b, c, px, 1) : z2_kmask(NB, zt, b, c, 1, px);
@@ -1229,7 +1236,6 @@ void build_state(rcmps_context* ctx, TrajBufs& tb, const rcmps_state* st, bool a
                     TrajTask t{};
                     t.sys = sys_base + s; t.ch = 1; t.b = b; t.c = c; t.adj = 1;
                     t.edge_src = -1;
-                    t.has_E = 1;
                     t.e_only = 1;
                     t.kmask = z2_kmask(NB, zt, b, c, kParity[3][1], 1) << 16;   // E = X C of channel 1
                     tasks.push_back(t);
@@ -1247,16 +1253,28 @@ void run_class(rcmps_context* ctx, int Dp, bool split, bool quartic_only, bool t
     std::vector<TrajSys> sys;
     std::vector<TrajTask> tasks;
     while (ctx->tb.size() < tb0 + idx.size()) ctx->tb.emplace_back(new TrajBufs());
+    // the parity blocks are skipped when every state of the launch has them (a mixed launch runs every
+    // k-tile: the same bits)
+    bool all_z2 = z2;
+    for (int i : idx) all_z2 = all_z2 && reqs[i].st->z2_tiles > 0;
     std::vector<int> state_first, state_ntasks;
+    size_t exch_bytes = 0;
+    for (int i : idx) exch_bytes += exchange_bytes(Dp, reqs[i].adjoint(), quartic_only);
+    const size_t out_bytes = idx.size() * RC_NSYS * RC_OUT_STRIDE * 8;
+    ck(ctx->traj_exch.ensure(exch_bytes));
+    ck(ctx->traj_out.ensure(out_bytes));
+    char* exch = static_cast<char*>(ctx->traj_exch.p);
     for (size_t j = 0; j < idx.size(); ++j) {
         const int first = (int)tasks.size();
-        build_state(ctx, *ctx->tb[tb0 + j], reqs[idx[j]].st, reqs[idx[j]].adjoint(), quartic_only, z2, npts, sys,
-                    tasks);
+        const EvalReq& r = reqs[idx[j]];
+        build_state(ctx, *ctx->tb[tb0 + j], exch, ctx->traj_out.d() + j * RC_NSYS * RC_OUT_STRIDE, r.st, r.adjoint(),
+                    quartic_only, all_z2, npts, sys, tasks);
+        exch += exchange_bytes(Dp, r.adjoint(), quartic_only);
         state_first.push_back(first);
         state_ntasks.push_back((int)tasks.size() - first);
     }
     int capacity = 0;
-    ck(rc_trajectory_capacity(NB, split ? 1 : 0, &capacity));
+    ck(rc_trajectory_capacity(NB, split ? 1 : 0, all_z2 ? 1 : 0, timers ? 1 : 0, &capacity));
     // gang schedule: a state's tasks share one round
     std::vector<std::vector<int>> rounds;
     int nblocks = 0;
@@ -1274,7 +1292,6 @@ void run_class(rcmps_context* ctx, int Dp, bool split, bool quartic_only, bool t
     P.Dp = Dp;
     P.npoints = npts;
     P.nrounds = (int)rounds.size();
-    P.timers = timers ? 1 : 0;
     P.a = std::sqrt(ip->max_point);
     P.atol = ip->atol;
     P.rtol = ip->rtol;
@@ -1299,19 +1316,15 @@ void run_class(rcmps_context* ctx, int Dp, bool split, bool quartic_only, bool t
     ck(hipMemcpyAsync(ctx->traj_sys.p, sys.data(), sys.size() * sizeof(TrajSys), hipMemcpyHostToDevice, ctx->stream));
     ck(hipMemcpyAsync(ctx->traj_sched.p, sched.data(), sched.size() * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
     ck(hipMemcpyAsync(ctx->traj_params.p, &P, sizeof(TrajParams), hipMemcpyHostToDevice, ctx->stream));
-    for (size_t j = 0; j < idx.size(); ++j) {
-        ck(hipMemsetAsync(ctx->tb[tb0 + j]->flags.p, 0, ctx->tb[tb0 + j]->flag_bytes, ctx->stream));
-        ck(hipMemsetAsync(ctx->tb[tb0 + j]->out.p, 0, RC_NSYS * RC_OUT_STRIDE * 8, ctx->stream));
-    }
+    ck(rc_launch_fill_empty(ctx->traj_exch.p, exch_bytes, ctx->stream));
+    ck(hipMemsetAsync(ctx->traj_out.p, 0, out_bytes, ctx->stream));
     ck(hipMemsetAsync(ctx->abort_word.p, 0, 256, ctx->stream));
     ck(hipEventRecord(ctx->ev[0], ctx->stream));
-    ck(rc_launch_trajectory(NB, split ? 1 : 0, nblocks, static_cast<const TrajParams*>(ctx->traj_params.p),
+    ck(rc_launch_trajectory(NB, split ? 1 : 0, all_z2 ? 1 : 0, timers ? 1 : 0, nblocks, static_cast<const TrajParams*>(ctx->traj_params.p),
                             ctx->stream));
     ck(hipEventRecord(ctx->ev[1], ctx->stream));
     std::vector<double> outs(idx.size() * RC_NSYS * RC_OUT_STRIDE);
-    for (size_t j = 0; j < idx.size(); ++j)
-        ck(hipMemcpyAsync(outs.data() + j * RC_NSYS * RC_OUT_STRIDE, ctx->tb[tb0 + j]->out.d(),
-                          RC_NSYS * RC_OUT_STRIDE * 8, hipMemcpyDeviceToHost, ctx->stream));
+    ck(hipMemcpyAsync(outs.data(), ctx->traj_out.p, out_bytes, hipMemcpyDeviceToHost, ctx->stream));
     ck(hipStreamSynchronize(ctx->stream));
     float tms = 0;
     ck(hipEventElapsedTime(&tms, ctx->ev[0], ctx->ev[1]));

@@ -62,6 +62,21 @@ __device__ __forceinline__ void st_coh(__amdgpu_buffer_rsrc_t r, uint32_t byte_o
     __builtin_amdgcn_raw_buffer_store_b128(v, r, byte_offset, 0, RC_COHERENT_POLICY);
 }
 
+// the same at voff + soff, soff wave-uniform (both within the buffer together)
+__device__ __forceinline__ cplx ld_coh_s(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    v4u v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, RC_COHERENT_POLICY);
+    cplx z;
+    z.re = __builtin_bit_cast(double, (uint64_t)v.x | ((uint64_t)v.y << 32));
+    z.im = __builtin_bit_cast(double, (uint64_t)v.z | ((uint64_t)v.w << 32));
+    return z;
+}
+__device__ __forceinline__ void st_coh_s(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, cplx z) {
+    uint64_t a = __builtin_bit_cast(uint64_t, z.re), b = __builtin_bit_cast(uint64_t, z.im);
+    v4u v;
+    v.x = (uint32_t)a; v.y = (uint32_t)(a >> 32); v.z = (uint32_t)b; v.w = (uint32_t)(b >> 32);
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, voff, soff, RC_COHERENT_POLICY);
+}
+
 __device__ __forceinline__ double ld_coh_f64(const double* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

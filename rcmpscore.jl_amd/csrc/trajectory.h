@@ -4,7 +4,11 @@
 
 #define RC_NSYS 6           // (kinetic, kinetic commutator, phi^4) x (forward, adjoint)
 #define RC_MAX_LIVE 4
-#define RC_NSTAGE_BUF 16    // one buffer per stage slot of a step
+#define RC_RING 32          // exchange slots: one per stage event, emptied again 16 events later
+#define RC_REC_RING 4       // slots of the error records: one per attempt
+// word of an empty exchange slot (in all four dwords of a complex): as the high half of a double a
+// quiet NaN with a payload of its own
+#define RC_EMPTY_WORD 0xfffac0deu
 #define RC_REC 16           // doubles per workgroup record: e5, e3, 12 trace partials, spare
 
 // status codes (shared with the C-ABI): 1-5 as the DOP853 controller of the reference GPU
@@ -21,10 +25,10 @@ struct TrajTask {
     int adj;
     int edge_src;       // live channel (same system) whose level-1 tile feeds the insertion, -1 none
     int edge_from_E;    // 1: the insertion reads the E buffer (X * [Q,R]) of edge_src
-    int has_E;          // load the C = [Q, R] column block of E = X C (the E tasks of the kinetic commutator)
     int trace_kind;     // 0 none; 1: Re sum X conj(O) over the tile; 2: Re diag of the level-1 tile
     int e_only;         // 1: only form and publish channel ch's E tile each stage (no stage input,
                         // no samples, an empty error record)
+    int pub_y, pub_p;   // Dp = 16: another workgroup reads this channel's stage input / level-1 tile
     // k-tiles that contribute to each tile product, four bits per product: level 1 [0, 4), the two
     // level-2a products [4, 8) and [8, 12), level 2b [12, 16), the E product [16, 20).  All ones
     // for a general state; for a Z2-symmetric state only the k-tiles of the one parity block that
@@ -41,14 +45,11 @@ struct TrajSys {
     int nlive, has_scalar, adj, first_task, ntasks, D;
     double n_elems;          // nlive * D^2 + has_scalar: denominator of the RMS norm
     const double *Q, *Qh, *R, *Rh, *C;   // the state's matrices, Dp x Dp
-    double* Y;               // [16][nlive][Dp*Dp] complex
-    double* P;               // [16][nlive][Dp*Dp] complex
-    double* E;               // [16][Dp*Dp] complex or null
-    double* rec;             // [2][ntasks][RC_REC]
-    uint32_t* flagY;         // [nlive][NB*NB]
-    uint32_t* flagP;         // [nlive][NB*NB]
-    uint32_t* flagE;         // [NB*NB]
-    uint32_t* flagR;         // [ntasks]
+    // exchange buffers: Y in two orders and P, each [RC_RING][nlive][Dp*Dp] complex, with has_E
+    // E [RC_RING][Dp*Dp], error records [RC_REC_RING][ntasks][RC_REC] doubles
+    double* exch;
+    uint32_t exch_bytes;
+    int has_E;
     double* samples;         // [npoints][nlive][Dp*Dp] complex
     double* out;             // [32]: status/counters, then phase timers of workgroup 0
 };
@@ -57,7 +58,7 @@ struct TrajSys {
 // are gang-scheduled in rounds: workgroup w runs task schedule[r * nblocks + w] (or idles, -1)
 // in round r, and all tasks of a system share a round, so every wait is on a running partner.
 struct TrajParams {
-    int Dp, npoints, nrounds, timers;   // timers: fill the per-phase timers of workgroup 0
+    int Dp, npoints, nrounds, pad;
     double a, atol, rtol, h0;
     long long max_steps, wait_ticks;   // wait_ticks: time budget of one wait (constant-rate clock ticks)
     const double* points;

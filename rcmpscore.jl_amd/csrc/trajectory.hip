@@ -8,18 +8,41 @@
 // error norm h e5 / sqrt((e5 + 0.01 e3) N), factor min(10, 0.9 err^-1/8), rejection factor
 // max(0.2, .), no step across t = 0, 7th-order dense output at the Gauss nodes, as the reference
 // GPU package (gpu/src/rcmps_gpu/optimizer/runtime/ode_backend.py:500-586,
-// device_control_backend.py:30-47).  The FSAL stage is evaluated only after acceptance.
+// device_control_backend.py:30-47).  The FSAL stage counts as evaluated only after acceptance.
 //
 // Work decomposition: one workgroup per (system, live channel, 16x16 output tile), plus, for the
 // kinetic commutator's adjoint system, one E task per tile forming E = X [Q,R] of channel 1, which
 // channel 0's insertion reads (so no channel forms two level-1 products).  A stage is
 // two levels: level 1 forms the tile of P = R X (forward) or X R (adjoint) and publishes it;
 // level 2 forms Q X + X Q^+ (resp. Q^+ X + X Q) while neighbours' P tiles arrive, then adds
-// P R^+ (resp. R^+ P), the insertion terms and the next stage input.  Workgroups never meet at
-// a grid barrier: each waits on per-tile event flags of the tiles it reads; data written for
-// other workgroups uses agent-coherent stores and loads.  The step-end error norm is a
-// deterministic all-gather of per-workgroup records, so every workgroup of a system takes the
-// same controller decision.  Every wait is bounded by a time budget and watches an abort word.
+// P R^+ (resp. R^+ P), the insertion terms and the next stage input.
+//
+// Exchange between workgroups: the data are their own arrival flags.  Every stage input Y, level-1
+// tile P, E tile and error record goes into a ring of slots whose words hold a NaN pattern no
+// computation produces (rc_empty) until the value is stored; a consumer loads the elements it needs
+// with device-coherent loads straight into its MFMA fragments and repeats those that are still
+// empty.  An exchange is then one store and one load of device scope, with no wait for the store's
+// completion, no flag and no barrier of the workgroup; the products were a third of a stage and
+// these round trips most of the rest.  Ring of RC_RING events: the step-end all-gather of error
+// records meets at least every 15 events (slots 12..15 and 1..11 of a step), so at event e every
+// reader is done with event e - 16, whose slot the producer empties again; the slot is used next at
+// event e + 16, and a gather lies between, before which the producer waited for its stores.
+// The gather is deterministic (every workgroup adds the same records in the same order), so every
+// workgroup of a system takes the same controller decision.  Every wait is bounded by a time
+// budget and watches an abort word.
+//
+// FP64 products read no LDS: each wave runs one k-step of every k-tile, so the operands of its
+// products are fragments it alone needs, loaded from the exchange buffers into registers (the
+// constant panels R, Q, .. once per task).  LDS holds only the four waves' partial tiles, in one
+// buffer per level, which leaves two barriers per stage.  Split precision stages digit planes in
+// LDS (every wave needs every row of a panel's digits).  With one tile per channel (Dp = 16) the
+// stage input and P stay in LDS and only what another channel reads is exchanged.
+//
+// What bounds it: two exchanges of about 1.7 us and 2 us of products (64 MFMAs a wave) per stage at
+// D = 64.  Measured on MI355X, per right-hand side of the slowest system, against one flag per
+// tile, a wait for the store and LDS panels: D = 8 5.8 -> 3.0 us, D = 32 with Z2 blocks 7.3 -> 3.7,
+// D = 40 9.1 -> 4.7, D = 64 9.4 -> 5.4 (split 9.5 -> 6.6); six trajectories at D = 64, window 30,
+// 1e-13/1e-12: 62 -> 36 ms.
 #include "device_common.h"
 #include "split.h"
 #include "trajectory.h"
@@ -29,101 +52,117 @@ namespace {
 template <int NB>
 struct Lay {
     static constexpr int Dp = 16 * NB;
-    static constexpr int RS = Dp + 1;                  // padded row stride of row blocks
-    static constexpr int ROWBLK = 16 * RS;
-    static constexpr int COLBLK = Dp * 16;
-    static constexpr int BLK = ROWBLK > COLBLK ? ROWBLK : COLBLK;
-    static constexpr int XR = 0, XC = BLK, PB = 2 * BLK, K0 = 3 * BLK, K1 = 4 * BLK, K2 = 5 * BLK,
-                         K3 = 6 * BLK, K4 = 7 * BLK, RED = 8 * BLK;
-    static constexpr int NCPLX = 8 * BLK + 1024;
+    // partial tiles of the two levels, then (Dp = 16 only) the stage input and P tiles, rows of 17
+    static constexpr int RED1 = 0, RED2 = 1024, YT = 2048, PT = YT + 16 * 17;
+    static constexpr int NCPLX = NB == 1 ? PT + 16 * 17 : 2048;
     static constexpr int NDOUBLE_SCRATCH = 64;
     static constexpr int BYTES = NCPLX * 16 + NDOUBLE_SCRATCH * 8;
 };
+
+// c k + a, each part one fused multiply-add: the instantiations of the kernel (Z2 blocks or every
+// k-tile, timed or not) round alike whatever the compiler would contract
+__device__ __forceinline__ cplx cfma(double c, cplx k, cplx a) { return cmake(fma(c, k.re, a.re), fma(c, k.im, a.im)); }
 
 struct Ctl {
     uint32_t* abort_flag;
     long long wait_ticks;   // longest single wait, in ticks of the constant-rate clock (s_memrealtime)
 };
 
-// Wave 0 polls up to 64 flags (lane l: flags[l] >= target); all waves then meet.  Returns false
-// when the abort word is set or the wait outlasts its time budget (then the abort word is set).
-// The budget is wall-clock time, not a poll count: a workgroup that starts a later round of a
-// batched launch early may wait a whole round for partners that are still running.
-__device__ bool wait_flags(const Ctl& ctl, uint32_t* const* addr_lane, int n, uint32_t target,
-                           int* s_abort) {
-    const int tid = threadIdx.x, lane = tid & 63;
-    if (tid < 64) {
-        uint32_t* a = lane < n ? addr_lane[lane] : nullptr;
-        const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
-        int bad = 0;
-        for (uint32_t polls = 1;; ++polls) {
-            // the flag and the abort word are loaded together: one round trip per poll
-            const uint32_t fv = a ? ld_flag(a) : 0u;
-            const uint32_t ab = ld_flag(ctl.abort_flag);
-            const bool ok = a ? (fv >= target) : true;
-            if (__all(ok)) break;
-            if (ab) { bad = 1; break; }
-            // the clock is read every 64th poll only
-            if ((polls & 63) == 0 && (long long)(__builtin_amdgcn_s_memrealtime() - t0) > ctl.wait_ticks) {
-                bad = 1;
+// Barrier of the workgroup that orders LDS accesses only: device-coherent stores and polling loads
+// in flight stay in flight (__syncthreads would wait for them).
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// the empty slot's word: a quiet NaN whose payload no arithmetic here produces (the hardware's own
+// NaN has payload zero, the state's matrices are finite)
+__device__ __forceinline__ bool rc_arrived(cplx v) {
+    return (uint32_t)__double2hiint(v.re) != RC_EMPTY_WORD && (uint32_t)__double2hiint(v.im) != RC_EMPTY_WORD;
+}
+__device__ __forceinline__ double rc_not_empty(double x) {
+    return (uint32_t)__double2hiint(x) == RC_EMPTY_WORD ? __longlong_as_double(0x7ff8000000000000LL) : x;
+}
+// publish a value / empty a slot again (device-coherent stores; every aligned 8-byte half is
+// written whole, and a reader checks both)
+__device__ __forceinline__ void rc_put(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, cplx z) {
+    st_coh_s(r, voff, soff, cmake(rc_not_empty(z.re), rc_not_empty(z.im)));
+}
+__device__ __forceinline__ void rc_reset(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
+    const double e = __hiloint2double((int)RC_EMPTY_WORD, (int)RC_EMPTY_WORD);
+    st_coh_s(r, voff, soff, cmake(e, e));
+}
+
+// Elements voff + soff + t stride, t < N, of the lanes that `use` them: the loads alone; rc_await then
+// repeats them until every element of the wave has arrived.  False when the abort word is set or
+// the wait outlasts its time budget (then the abort word is set).  The budget is wall-clock time: a
+// workgroup that starts a later round of a batched launch early may wait a whole round for
+// partners that are still running.
+template <int N>
+__device__ __forceinline__ void rc_fetch(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, uint32_t stride,
+                                         cplx* v, bool use = true) {
+    if (use) {
+#pragma unroll
+        for (int t = 0; t < N; ++t) v[t] = ld_coh_s(r, voff, soff + t * stride);
+    } else {
+#pragma unroll
+        for (int t = 0; t < N; ++t) v[t] = cmake(0, 0);
+    }
+}
+template <int N>
+__device__ __forceinline__ bool rc_all_arrived(const cplx* v) {
+    bool ok = true;
+#pragma unroll
+    for (int t = 0; t < N; ++t) ok &= rc_arrived(v[t]);
+    return __all(ok);
+}
+// Hide the values from the compiler's count of outstanding loads: they have arrived, and their later
+// uses must not wait for whatever store or load was issued since.
+template <int N>
+__device__ __forceinline__ void rc_settle(cplx* v) {
+#pragma unroll
+    for (int t = 0; t < N; ++t) asm volatile("" : "+v"(v[t].re), "+v"(v[t].im));
+}
+template <int N>
+__device__ __forceinline__ bool rc_await(const Ctl& ctl, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff,
+                                         uint32_t stride, cplx* v, bool use = true) {
+    uint64_t t0 = 0;
+    bool ok = true;
+    for (uint32_t polls = 1; !rc_all_arrived<N>(v); ++polls) {
+        asm volatile("" ::: "memory");
+        rc_fetch<N>(r, voff, soff, stride, v, use);
+        if ((polls & 63) == 0) {   // the clock and the abort word are read every 64th poll only
+            const uint64_t now = __builtin_amdgcn_s_memrealtime();
+            if (t0 == 0) t0 = now;
+            const bool over = (long long)(now - t0) > ctl.wait_ticks;
+            if (over) st_flag(ctl.abort_flag, 1u);
+            if (over || uni((int)ld_flag(ctl.abort_flag))) {
+                ok = false;
                 break;
             }
-            __builtin_amdgcn_s_sleep(1);
-        }
-        if (lane == 0) {
-            if (bad) st_flag(ctl.abort_flag, 1u);
-            *s_abort = bad;
         }
     }
-    __syncthreads();
-    return uni(*s_abort) == 0;
+    rc_settle<N>(v);
+    return ok;
 }
 
-// Every store another workgroup reads is a device-scope (sc1) store, which completes only once
-// it is coherent at device scope; waiting for all of them (vmcnt 0) before the flag store is
-// therefore a release for that data, and no L2 writeback is needed (nothing read across
-// workgroups is ever written with a non-coherent store).
-__device__ __forceinline__ void publish(uint32_t* flag, uint32_t value) {
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (threadIdx.x == 0) st_flag(flag, value);
-}
-
-// A fragment from a row block M[16][RS]: lane l, k-step ks -> M[l%16][4ks + l/16]
-template <int NB>
-__device__ __forceinline__ cplx fragA(const cplx* M, int ks, int lane) {
-    return M[(lane & 15) * Lay<NB>::RS + 4 * ks + (lane >> 4)];
-}
-// B fragment from a column block N[Dp][16]: N[4ks + l/16][l%16]
-__device__ __forceinline__ cplx fragB(const cplx* N, int ks, int lane) {
-    return N[(4 * ks + (lane >> 4)) * 16 + (lane & 15)];
-}
-
-// acc += A(row block) * B(col block) over this wave's share of the k-steps, k-tiles in `kmask`
-// only (uniform; bit t: k-tile t).  Each wave runs one k-step of every k-tile.
-template <int NB>
-__device__ __forceinline__ void tile_product(cacc& acc, const cplx* A, const cplx* B, int wave, int lane,
-                                             int kmask) {
+// acc += A B over this wave's k-steps (fragment t: its k-step of the t-th k-tile)
+template <int KT>
+__device__ __forceinline__ void frag_product(cacc& acc, const cplx* A, const cplx* B) {
 #pragma unroll
-    for (int ks = wave; ks < 4 * NB; ks += 4)
-        if ((kmask >> (ks >> 2)) & 1) cmfma(acc, fragA<NB>(A, ks, lane), fragB(B, ks, lane));
+    for (int t = 0; t < KT; ++t) cmfma(acc, A[t], B[t]);
 }
 
-// Sum the four waves' partial tiles; thread t receives element (t/16, t%16).
-__device__ __forceinline__ cplx reduce_tile(const cacc& acc, cplx* red, int wave, int lane) {
+// Sum of the four waves' partial tiles; thread t receives element (t/16, t%16).  The barrier also
+// orders the other level's buffer: its readers pass here before anyone writes it again.
+__device__ __forceinline__ void put_partial(const cacc& acc, cplx* red, int wave, int lane) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) red[wave * 256 + (4 * q + (lane >> 4)) * 16 + (lane & 15)] = cacc_get(acc, q);
-    __syncthreads();
+}
+__device__ __forceinline__ cplx sum_partial(const cplx* red) {
     const int t = threadIdx.x;
-    cplx s = red[t];
-    s = cadd(s, red[256 + t]);
-    s = cadd(s, red[512 + t]);
-    s = cadd(s, red[768 + t]);
-    __syncthreads();
-    return s;
+    return cadd(cadd(cadd(red[t], red[256 + t]), red[512 + t]), red[768 + t]);
 }
 
-// Deterministic block sum (same inputs give the same bits in every workgroup).
 // a DPP move of a double within each row of 16 lanes (CTRL a compile-time DPP control)
 template <int CTRL>
 __device__ __forceinline__ double dpp_move(double x) {
@@ -146,110 +185,6 @@ __device__ __forceinline__ double wave_sum(double v) {
     return ((read_lane(v, 0) + read_lane(v, 16)) + read_lane(v, 32)) + read_lane(v, 48);
 }
 
-__device__ __forceinline__ double block_sum(double v, double* scratch) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    v = wave_sum(v);
-    if (lane == 0) scratch[wave] = v;
-    __syncthreads();
-    double s = ((scratch[0] + scratch[1]) + scratch[2]) + scratch[3];
-    __syncthreads();
-    return s;
-}
-// two block sums with one exchange
-__device__ __forceinline__ void block_sum2(double& a, double& b, double* scratch) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    a = wave_sum(a);
-    b = wave_sum(b);
-    if (lane == 0) {
-        scratch[wave] = a;
-        scratch[4 + wave] = b;
-    }
-    __syncthreads();
-    a = ((scratch[0] + scratch[1]) + scratch[2]) + scratch[3];
-    b = ((scratch[4] + scratch[5]) + scratch[6]) + scratch[7];
-    __syncthreads();
-}
-
-// Load a row block (rows 16b.., all Dp columns) of a global Dp x Dp matrix into M[16][RS].
-template <int NB, bool COH>
-__device__ __forceinline__ void load_rowblk(cplx* M, const double* g, uint32_t gbytes, int b) {
-    constexpr int Dp = Lay<NB>::Dp;
-    const int t = threadIdx.x;
-    cplx v[NB];
-    if (COH) {
-        __amdgpu_buffer_rsrc_t r = rc_rsrc(g, gbytes);
-#pragma unroll
-        for (int it = 0; it < NB; ++it) {
-            int idx = it * 256 + t, i = idx / Dp, k = idx % Dp;
-            v[it] = ld_coh(r, (uint32_t)(((16 * b + i) * Dp + k) * 16));
-        }
-    } else {
-        const cplx* gc = reinterpret_cast<const cplx*>(g);
-#pragma unroll
-        for (int it = 0; it < NB; ++it) {
-            int idx = it * 256 + t, i = idx / Dp, k = idx % Dp;
-            v[it] = gc[(16 * b + i) * Dp + k];
-        }
-    }
-#pragma unroll
-    for (int it = 0; it < NB; ++it) {
-        int idx = it * 256 + t, i = idx / Dp, k = idx % Dp;
-        M[i * Lay<NB>::RS + k] = v[it];
-    }
-}
-
-// Load a column block (all rows, columns 16c..) into N[Dp][16].
-template <int NB, bool COH>
-__device__ __forceinline__ void load_colblk(cplx* N, const double* g, uint32_t gbytes, int c) {
-    constexpr int Dp = Lay<NB>::Dp;
-    const int t = threadIdx.x;
-    cplx v[NB];
-    if (COH) {
-        __amdgpu_buffer_rsrc_t r = rc_rsrc(g, gbytes);
-#pragma unroll
-        for (int it = 0; it < NB; ++it) {
-            int idx = it * 256 + t, k = idx / 16, j = idx % 16;
-            v[it] = ld_coh(r, (uint32_t)((k * Dp + 16 * c + j) * 16));
-        }
-    } else {
-        const cplx* gc = reinterpret_cast<const cplx*>(g);
-#pragma unroll
-        for (int it = 0; it < NB; ++it) {
-            int idx = it * 256 + t, k = idx / 16, j = idx % 16;
-            v[it] = gc[k * Dp + 16 * c + j];
-        }
-    }
-#pragma unroll
-    for (int it = 0; it < NB; ++it) {
-        int idx = it * 256 + t, k = idx / 16, j = idx % 16;
-        N[k * 16 + j] = v[it];
-    }
-}
-
-// Row block b and column block c of the same matrix, all loads in flight together.
-template <int NB>
-__device__ __forceinline__ void load_row_col_coh(cplx* M, cplx* N, const double* g, uint32_t gbytes, int b, int c) {
-    constexpr int Dp = Lay<NB>::Dp;
-    const int t = threadIdx.x;
-    __amdgpu_buffer_rsrc_t r = rc_rsrc(g, gbytes);
-    cplx vr[NB], vc[NB];
-#pragma unroll
-    for (int it = 0; it < NB; ++it) {
-        int idx = it * 256 + t, i = idx / Dp, k = idx % Dp;
-        vr[it] = ld_coh(r, (uint32_t)(((16 * b + i) * Dp + k) * 16));
-        int kk = idx / 16, j = idx % 16;
-        vc[it] = ld_coh(r, (uint32_t)((kk * Dp + 16 * c + j) * 16));
-    }
-#pragma unroll
-    for (int it = 0; it < NB; ++it) {
-        int idx = it * 256 + t, i = idx / Dp, k = idx % Dp;
-        M[i * Lay<NB>::RS + k] = vr[it];
-        int kk = idx / 16, j = idx % 16;
-        N[kk * 16 + j] = vc[it];
-    }
-}
-
-
 // Record i of a read-only array through scalar loads, so that every field is known wave-uniform.
 template <typename T>
 __device__ __forceinline__ T load_scalar(const T* arr, int i) {
@@ -268,10 +203,9 @@ __device__ __forceinline__ T load_scalar(const T* arr, int i) {
 // ---------------------------------------------------------------------------------------
 struct LaySplit {
     static constexpr int P = RC_PANEL_BYTES;
-    static constexpr int XR = 0, XC = P, PB = 2 * P, K0 = 3 * P, K1 = 4 * P, K2 = 5 * P, K3 = 6 * P,
-                         K4 = 7 * P;
-    static constexpr int RED = 8 * P;                  // 4 x 256 doubles
-    static constexpr int SCR = RED + 4 * 256 * 8;      // 64 doubles
+    static constexpr int XR = 0, XC = P, PB = 2 * P, K0 = 3 * P, K1 = 4 * P, K2 = 5 * P, K3 = 6 * P;
+    static constexpr int RED = 7 * P;                  // two levels of 4 x 256 doubles
+    static constexpr int SCR = RED + 2 * 4 * 256 * 8;  // 64 doubles
     static constexpr int BYTES = SCR + 64 * 8;
 };
 
@@ -308,35 +242,21 @@ __device__ __forceinline__ void block_scales(const double* m, int* S, double* sc
 // Thread t holds four consecutive k of one row (row t / 16, k = 4 (t % 16) + q) of a row block,
 // or of one column (column t / 16, k = 4 (t % 16) + q) of a column block; zero beyond Dp.  The 16
 // lanes of one row or column are consecutive, so its largest entry is a 16-lane reduction.
-template <int NB, bool COH>
-__device__ __forceinline__ void fetch_row4(cplx* v, const double* g, uint32_t gbytes, int b) {
+template <int NB>
+__device__ __forceinline__ void fetch_row4(cplx* v, const double* g, int b) {
     constexpr int Dp = 16 * NB;
     const int t = threadIdx.x, i = t >> 4, k0 = 4 * (t & 15);
-    if (COH) {
-        const __amdgpu_buffer_rsrc_t r = rc_rsrc(g, gbytes);
+    const cplx* gc = reinterpret_cast<const cplx*>(g);
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            v[q] = k0 < Dp ? ld_coh(r, (uint32_t)(((16 * b + i) * Dp + k0 + q) * 16)) : cmake(0, 0);
-    } else {
-        const cplx* gc = reinterpret_cast<const cplx*>(g);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = k0 < Dp ? gc[(16 * b + i) * Dp + k0 + q] : cmake(0, 0);
-    }
+    for (int q = 0; q < 4; ++q) v[q] = k0 < Dp ? gc[(16 * b + i) * Dp + k0 + q] : cmake(0, 0);
 }
-template <int NB, bool COH>
-__device__ __forceinline__ void fetch_col4(cplx* v, const double* g, uint32_t gbytes, int c) {
+template <int NB>
+__device__ __forceinline__ void fetch_col4(cplx* v, const double* g, int c) {
     constexpr int Dp = 16 * NB;
     const int t = threadIdx.x, j = t >> 4, k0 = 4 * (t & 15);
-    if (COH) {
-        const __amdgpu_buffer_rsrc_t r = rc_rsrc(g, gbytes);
+    const cplx* gc = reinterpret_cast<const cplx*>(g);
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            v[q] = k0 < Dp ? ld_coh(r, (uint32_t)(((k0 + q) * Dp + 16 * c + j) * 16)) : cmake(0, 0);
-    } else {
-        const cplx* gc = reinterpret_cast<const cplx*>(g);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) v[q] = k0 < Dp ? gc[(k0 + q) * Dp + 16 * c + j] : cmake(0, 0);
-    }
+    for (int q = 0; q < 4; ++q) v[q] = k0 < Dp ? gc[(k0 + q) * Dp + 16 * c + j] : cmake(0, 0);
 }
 template <int NB>
 __device__ __forceinline__ void store_row4(unsigned char* panel, const cplx* v, int S) {
@@ -378,8 +298,8 @@ __device__ __forceinline__ int line_scale(const cplx* v, int* sg) {
 template <int NB>
 __device__ __forceinline__ int const_panel(unsigned char* panel, const double* g, bool row, int blk, double* scr) {
     cplx v[4];
-    if (row) fetch_row4<NB, false>(v, g, 0, blk);
-    else fetch_col4<NB, false>(v, g, 0, blk);
+    if (row) fetch_row4<NB>(v, g, blk);
+    else fetch_col4<NB>(v, g, blk);
     const double m = max4(v);
     int S;
     block_scales<1>(&m, &S, scr);
@@ -391,431 +311,534 @@ __device__ __forceinline__ int const_panel(unsigned char* panel, const double* g
 
 // Waves 0..3 hold the real products re.re, im.im, re.im, im.re of the same complex tile product;
 // thread t receives element (t/16, t%16) of the complex result.
-__device__ __forceinline__ cplx reduce_split(const double* part, double* red, int wave, int lane) {
+__device__ __forceinline__ void put_partial_split(const double* part, double* red, int wave, int lane) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) red[wave * 256 + (4 * (lane >> 4) + q) * 16 + (lane & 15)] = part[q];
-    __syncthreads();
+}
+__device__ __forceinline__ cplx sum_partial_split(const double* red) {
     const int t = threadIdx.x;
-    const cplx s = cmake(red[t] - red[256 + t], red[512 + t] + red[768 + t]);
-    __syncthreads();
+    return cmake(red[t] - red[256 + t], red[512 + t] + red[768 + t]);
+}
+
+// Combinations that follow stage s, without their last term: rows of coefficients for the window of
+// stage derivatives before k_s enters it (k_j at position 16 - s + j, zero elsewhere).  Row s, s in
+// 1..14: the next stage input, A[s + 1]; row 11: the solution, B; 16 and 17: the error estimators E5
+// and E3 (after stage 11); 18..21: the dense output D (after stage 15).
+#define RC_NROWS 22
+struct RcRows {
+    double c[RC_NROWS][16];
+};
+constexpr RcRows rc_make_rows() {
+    RcRows r{};
+    for (int s = 1; s < RC_NSTAGES_EXT - 1; ++s)
+        for (int j = 0; j < s; ++j) r.c[s][16 - s + j] = s == RC_NSTAGES - 1 ? RC_B[j] : RC_A[s + 1][j];
+    for (int j = 0; j < RC_NSTAGES - 1; ++j) {
+        r.c[16][16 - (RC_NSTAGES - 1) + j] = RC_E5[j];
+        r.c[17][16 - (RC_NSTAGES - 1) + j] = RC_E3[j];
+    }
+    for (int q = 0; q < 4; ++q)
+        for (int j = 0; j < RC_NSTAGES_EXT - 1; ++j) r.c[18 + q][1 + j] = RC_D[q][j];
+    return r;
+}
+__constant__ const RcRows rc_rows = rc_make_rows();
+
+// sum_q c[row][q] k[q], q increasing (row uniform: the coefficients come through the scalar cache).
+// One loop-free sum for every stage: the zero coefficients cost a few multiply-adds in the shadow of
+// an exchange and spare a branch tree over stages with its own code and constants for each.
+__device__ __forceinline__ cplx rc_row_sum(int row, const cplx* k) {
+    const __attribute__((address_space(4))) double* c =
+        (const __attribute__((address_space(4))) double*)&rc_rows.c[row][0];
+    cplx s = cmake(0, 0);
+#pragma unroll
+    for (int q = 0; q < RC_NSTAGES_EXT; ++q) s = cfma(c[q], k[q], s);
     return s;
-}
-
-// DOP853 combinations sum_j c_j k_j with the tableau as compile-time constants: zero terms
-// vanish and every index of the stage-derivative window k is static, so k stays in registers.
-// k_j sits at k[OFF + j].  The sum runs over j in increasing order from zero, as a running
-// accumulation would.
-enum RcRow { RC_ROW_A, RC_ROW_B, RC_ROW_E5, RC_ROW_E3, RC_ROW_D };
-
-template <RcRow W, int S>
-__device__ __forceinline__ constexpr double rc_coef(int j) {
-    if constexpr (W == RC_ROW_A) return RC_A[S][j];
-    if constexpr (W == RC_ROW_B) return j < RC_NSTAGES ? RC_B[j] : 0.0;
-    if constexpr (W == RC_ROW_E5) return j < RC_NSTAGES ? RC_E5[j] : 0.0;
-    if constexpr (W == RC_ROW_E3) return j < RC_NSTAGES ? RC_E3[j] : 0.0;
-    return RC_D[S][j];
-}
-
-template <RcRow W, int S, int N, int OFF, int J = 0>
-__device__ __forceinline__ cplx rc_comb(const cplx* k, cplx acc) {
-    if constexpr (J == N) {
-        return acc;
-    } else {
-        constexpr double c = rc_coef<W, S>(J);
-        if constexpr (c != 0.0) acc = cadd(acc, cscale(c, k[OFF + J]));
-        return rc_comb<W, S, N, OFF, J + 1>(k, acc);
-    }
-}
-
-// sum_{j < s} A[s][j] k_j for a uniform stage index s in 1..15, taken right after k_{s-1}
-// entered the window (k_j at k[16 - s + j])
-template <int S = 1>
-__device__ __forceinline__ cplx rc_stage_comb(int s, const cplx* k) {
-    if constexpr (S == RC_NSTAGES_EXT - 1) {
-        return rc_comb<RC_ROW_A, S, S, RC_NSTAGES_EXT - S>(k, cmake(0, 0));
-    } else {
-        if (s == S) return rc_comb<RC_ROW_A, S, S, RC_NSTAGES_EXT - S>(k, cmake(0, 0));
-        return rc_stage_comb<S + 1>(s, k);
-    }
 }
 
 }  // namespace
 
-template <int NB, bool SPLIT>
+template <int NB, int KT, bool SPLIT, bool TIMED>
 __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw) {
     using L = Lay<NB>;
-    constexpr int Dp = L::Dp, NT = NB * NB;
+    constexpr int Dp = L::Dp;
+    constexpr bool LOCAL = NB == 1 && !SPLIT;   // one tile per channel: its stage input and P stay in LDS
     cplx* sm = reinterpret_cast<cplx*>(smem_raw);
-    cplx* Xr = sm + L::XR;
-    cplx* Xc = sm + L::XC;
-    cplx* Pb = sm + L::PB;
-    cplx* Kl1 = sm + L::K0;   // level-1 constant: R row block (fwd) / R col block (adj)
-    cplx* Kq = sm + L::K1;    // Q row block (fwd) / Q^+ row block (adj)
-    cplx* Kx = sm + L::K2;    // Q^+ col block (fwd) / Q col block (adj)
-    cplx* Kp = sm + L::K3;    // R^+ col block (fwd) / R^+ row block (adj)
-    cplx* Kc = sm + L::K4;    // C col block (adj channel with E)
-    cplx* red = sm + L::RED;
-    // split precision: digit planes of the same operands (FP64 blocks above unused)
+    cplx* red1 = sm + L::RED1;
+    cplx* red2 = sm + L::RED2;
+    cplx* Yt = sm + L::YT;
+    cplx* Pt = sm + L::PT;
+    // split precision: digit planes of the stage input's row and column block, of the P block and of
+    // the constant panels, and the partial real products
     unsigned char* pXr = smem_raw + LaySplit::XR;
     unsigned char* pXc = smem_raw + LaySplit::XC;
     unsigned char* pPb = smem_raw + LaySplit::PB;
-    unsigned char* pK0 = smem_raw + LaySplit::K0;
-    unsigned char* pK1 = smem_raw + LaySplit::K1;
-    unsigned char* pK2 = smem_raw + LaySplit::K2;
-    unsigned char* pK3 = smem_raw + LaySplit::K3;
-    unsigned char* pK4 = smem_raw + LaySplit::K4;
-    double* redd = reinterpret_cast<double*>(smem_raw + LaySplit::RED);
+    unsigned char* pK1 = smem_raw + LaySplit::K0;
+    unsigned char* pKq = smem_raw + LaySplit::K1;
+    unsigned char* pKx = smem_raw + LaySplit::K2;
+    unsigned char* pKp = smem_raw + LaySplit::K3;
+    double* redd1 = reinterpret_cast<double*>(smem_raw + LaySplit::RED);
+    double* redd2 = redd1 + 4 * 256;
     double* scratch = SPLIT ? reinterpret_cast<double*>(smem_raw + LaySplit::SCR)
                             : reinterpret_cast<double*>(sm + L::NCPLX);
-    __shared__ int s_abort;
-    __shared__ uint32_t* s_addr[64];
-    __shared__ double s_tot[16];
+    __shared__ int s_bad;   // a wait of this attempt failed (read at the step's end only)
+    __shared__ double s_tot[17];
+    __shared__ double s_err[8];
+    __shared__ double s_trp[RC_NSTAGES_EXT][4], s_trs[RC_NSTAGES_EXT];   // trace: wave sums, coefficient
+    __shared__ double s_src[2][RC_NSTAGES_EXT];                         // source values, by attempt parity
+    __shared__ double s_cheb[RC_SOURCE_SEGMENTS * (RC_SOURCE_DEGREE + 1)];
+    __shared__ double s_cnode[RC_NSTAGES_EXT], s_alast[RC_NSTAGES_EXT];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
     const int spa = (wave == 1 || wave == 3), spb = (wave == 1 || wave == 2);   // this wave's real product
     const int ei = tid >> 4, ej = tid & 15;
     const TrajTask tk = load_scalar<TrajTask>(p.tasks, task);
     const TrajSys S = load_scalar<TrajSys>(p.sys, tk.sys);
     const int b = tk.b, c = tk.c, ch = tk.ch, adj = tk.adj;
-    // k-tile masks of the tile products (uniform)
+    // k-tile masks of the tile products (uniform): level 1, the two of level 2a, level 2b, E.  KT = NB:
+    // every k-tile of every product.  KT = NB / 2 (Z2 states, FP64): a product has the k-tiles of one
+    // parity block or none, and a tile either forms level 1 (do1) or level 2 (do2), since the
+    // stage input and P = R X have opposite parities.  Split precision skips whole products.
     const int m1 = tk.kmask & 15, m2a = (tk.kmask >> 4) & 15, m2b = (tk.kmask >> 8) & 15,
               m3 = (tk.kmask >> 12) & 15, mE = (tk.kmask >> 16) & 15;
+    const bool do1 = (KT == NB && !SPLIT) || m1 != 0, do2 = (KT == NB && !SPLIT) || m2a != 0;
+    const bool doE = (KT == NB && !SPLIT) || mE != 0;
+    auto first = [](int m) { return KT == NB || m == 0 ? 0 : __builtin_ctz(m); };
+    // first k-tile of the column block's and the row block's fragments, and of P's
+    const int tc = first(m2a ? m2a : adj ? 0 : m1), tr = first(tk.e_only ? mE : m2b ? m2b : adj ? m1 : 0), tp = first(m3);
     const int row = 16 * b + ei, col = 16 * c + ej;
     const bool e_only = tk.e_only != 0;                  // uniform over the workgroup
     const bool real_el = !e_only && row < S.D && col < S.D;
     const Ctl ctl{p.abort_flag, p.wait_ticks};
     const uint32_t mat_bytes = (uint32_t)(Dp * Dp * 16);
     const uint32_t stage_stride = (uint32_t)S.nlive * mat_bytes;
-    const uint32_t ybytes = RC_NSTAGE_BUF * stage_stride;
-    const __amdgpu_buffer_rsrc_t rY = rc_rsrc(S.Y, ybytes);
-    const __amdgpu_buffer_rsrc_t rP = rc_rsrc(S.P, ybytes);
-    const __amdgpu_buffer_rsrc_t rE = rc_rsrc(S.E, S.E ? RC_NSTAGE_BUF * mat_bytes : 0);
+    // the system's exchange buffers: rings of stage inputs Y (copies A and B), of level-1 tiles P and of
+    // E tiles, then the error records
+    const __amdgpu_buffer_rsrc_t rX = rc_rsrc(S.exch, S.exch_bytes);
+    const uint32_t oB = RC_RING * stage_stride, oP = 2 * oB, oE = 3 * oB, oR = oE + (S.has_E ? RC_RING * mat_bytes : 0);
     const uint32_t el_off = (uint32_t)((row * Dp + col) * 16);
-    const uint32_t el_off_t = (uint32_t)((col * Dp + row) * 16);   // transposed position
+    // The exchange buffers hold whole tiles (tile (r, c) at (r NB + c) TB), each in the order in which
+    // its readers' waves take it, so that one load instruction of a wave reads one contiguous 1 KB
+    // (split: four of 256 B): copy A for the readers of row blocks (FP64: column by column), copy B
+    // for those of column blocks (row by row).  A stage input has both, P the one its readers need.
+    // Element (r, c) of a tile at byte at_a / at_b.
+    constexpr uint32_t TB = 4096;
+    auto at_a = [](int r, int c) { return (uint32_t)((SPLIT ? (c & 3) * 64 + r * 4 + (c >> 2) : c * 16 + r) * 16); };
+    auto at_b = [](int r, int c) { return (uint32_t)((SPLIT ? (r & 3) * 64 + c * 4 + (r >> 2) : r * 16 + c) * 16); };
+    const uint32_t my_tile = (uint32_t)(b * NB + c) * TB, mirror_tile = (uint32_t)(c * NB + b) * TB;
+    const uint32_t ya_off = my_tile + at_a(ei, ej), yb_off = my_tile + at_b(ei, ej);   // own element of Y
+    const uint32_t pub_off = adj ? yb_off : ya_off;                                   // and of P
+    // own and mirrored element of the insertion source (E is held as copy B)
+    const bool ins_b = adj || tk.edge_from_E;
+    const uint32_t ins_off = ins_b ? yb_off : ya_off;
+    const uint32_t ins_off_t = mirror_tile + (ins_b ? at_b(ej, ei) : at_a(ej, ei));
+    // this lane's element of k-tile 0's fragment in row block b and in column block c, and the
+    // distance to the next k-tile's; split: this thread's four consecutive k of a row or column
+    const int fi = lane & 15, fk = 4 * wave + (lane >> 4);
+    const uint32_t in_tile = (uint32_t)(SPLIT ? (ei * 4 + (ej & 3)) * 16 : tid * 16);
+    constexpr uint32_t row_step = SPLIT ? 1024 : TB, col_step = SPLIT ? 1024 : NB * TB;
+    const uint32_t row_off0 = (uint32_t)(b * NB + (SPLIT ? ej >> 2 : 0)) * TB + in_tile;
+    const uint32_t col_off0 = (uint32_t)((SPLIT ? (ej >> 2) * NB : 0) + c) * TB + in_tile;
+    const uint32_t row_off = row_off0 + (SPLIT ? 0 : tr * row_step), col_off = col_off0 + (SPLIT ? 0 : tc * col_step);
+    const uint32_t p_off = (adj ? col_off0 : row_off0) + (SPLIT ? 0 : tp * (adj ? col_step : row_step));
+    const uint32_t p_step = adj ? col_step : row_step;
+    constexpr int NF = SPLIT ? 4 : KT;
+    // split: the lanes whose k lies in a k-tile that can be nonzero (the others' tiles are never written)
+    auto lanes = [&](int m) { return !SPLIT || (((m >> (ej >> 2)) & 1) && 4 * ej < Dp); };
+    const bool use_r = lanes(tk.e_only ? mE : m2b | (adj ? m1 : 0)), use_c = lanes(m2a | (adj ? 0 : m1)), use_p = lanes(m3);
 
-    // constant blocks
-    int sK0 = 0, sK1 = 0, sK2 = 0, sK3 = 0, sK4 = 0;   // split-precision panel scales
+    // constant panels: fragments in registers (split: digit planes).  K1 level 1 (R; an E task's C),
+    // Kq and Kx the one-sided products, Kp level 2
+    cplx K1[KT], Kq[KT], Kx[KT], Kp[KT];
+    int sK1 = 0, sKq = 0, sKx = 0, sKp = 0;   // split-precision panel scales
     // per-row / per-column scales of the stage input's row block [0, 16) and column block
     // [16, 32), and of the P block (split precision)
     int* sgX = reinterpret_cast<int*>(scratch + 16);
     int* sgP = sgX + 32;
     if constexpr (SPLIT) {
         // zero every digit plane once: k beyond Dp stays zero
-        for (int i = tid; i < 8 * RC_PANEL_BYTES / 16; i += 256) reinterpret_cast<v4i*>(smem_raw)[i] = v4i{0, 0, 0, 0};
+        for (int i = tid; i < 7 * RC_PANEL_BYTES / 16; i += 256) reinterpret_cast<v4i*>(smem_raw)[i] = v4i{0, 0, 0, 0};
         __syncthreads();
-        if (!adj) {
-            sK0 = const_panel<NB>(pK0, S.R, true, b, scratch);
-            sK1 = const_panel<NB>(pK1, S.Q, true, b, scratch);
-            sK2 = const_panel<NB>(pK2, S.Qh, false, c, scratch);
-            sK3 = const_panel<NB>(pK3, S.Rh, false, c, scratch);
+        if (e_only) {
+            sK1 = const_panel<NB>(pK1, S.C, false, c, scratch);
+        } else if (!adj) {
+            sK1 = const_panel<NB>(pK1, S.R, true, b, scratch);
+            sKq = const_panel<NB>(pKq, S.Q, true, b, scratch);
+            sKx = const_panel<NB>(pKx, S.Qh, false, c, scratch);
+            sKp = const_panel<NB>(pKp, S.Rh, false, c, scratch);
         } else {
-            sK0 = const_panel<NB>(pK0, S.R, false, c, scratch);
-            sK1 = const_panel<NB>(pK1, S.Qh, true, b, scratch);
-            sK2 = const_panel<NB>(pK2, S.Q, false, c, scratch);
-            sK3 = const_panel<NB>(pK3, S.Rh, true, b, scratch);
-            if (tk.has_E) sK4 = const_panel<NB>(pK4, S.C, false, c, scratch);
+            sK1 = const_panel<NB>(pK1, S.R, false, c, scratch);
+            sKq = const_panel<NB>(pKq, S.Qh, true, b, scratch);
+            sKx = const_panel<NB>(pKx, S.Q, false, c, scratch);
+            sKp = const_panel<NB>(pKp, S.Rh, true, b, scratch);
         }
-    } else if (!adj) {
-        load_rowblk<NB, false>(Kl1, S.R, 0, b);
-        load_rowblk<NB, false>(Kq, S.Q, 0, b);
-        load_colblk<NB, false>(Kx, S.Qh, 0, c);
-        load_colblk<NB, false>(Kp, S.Rh, 0, c);
     } else {
-        load_colblk<NB, false>(Kl1, S.R, 0, c);
-        load_rowblk<NB, false>(Kq, S.Qh, 0, b);
-        load_colblk<NB, false>(Kx, S.Q, 0, c);
-        load_rowblk<NB, false>(Kp, S.Rh, 0, b);
-        if (tk.has_E) load_colblk<NB, false>(Kc, S.C, 0, c);
+        auto rows = [&](cplx* K, const double* g, int m) {
+            const cplx* gc = reinterpret_cast<const cplx*>(g);
+#pragma unroll
+            for (int t = 0; t < KT; ++t) K[t] = gc[(16 * b + fi) * Dp + 16 * (first(m) + t) + fk];
+        };
+        auto cols = [&](cplx* K, const double* g, int m) {
+            const cplx* gc = reinterpret_cast<const cplx*>(g);
+#pragma unroll
+            for (int t = 0; t < KT; ++t) K[t] = gc[(16 * (first(m) + t) + fk) * Dp + 16 * c + fi];
+        };
+        if (!adj) {
+            rows(K1, S.R, m1); rows(Kq, S.Q, m2a); cols(Kx, S.Qh, m2b); cols(Kp, S.Rh, m3);
+        } else {
+            cols(K1, e_only ? S.C : S.R, e_only ? mE : m1); rows(Kq, S.Qh, m2a); cols(Kx, S.Q, m2b); rows(Kp, S.Rh, m3);
+        }
     }
     cplx fixed_e = cmake(0, 0), trop_e = cmake(0, 0);
     if (tk.fixed) fixed_e = reinterpret_cast<const cplx*>(tk.fixed)[row * Dp + col];
     if (tk.trace_kind == 1) trop_e = reinterpret_cast<const cplx*>(tk.trace_op)[row * Dp + col];
+    for (int i = tid; i < RC_SOURCE_SEGMENTS * (RC_SOURCE_DEGREE + 1); i += 256) s_cheb[i] = p.cheb[i];
+    if (tid < RC_NSTAGES_EXT) {
+        s_cnode[tid] = RC_C[tid];
+        // coefficient of the newest derivative k_s in the stage input after stage s
+        s_alast[tid] = tid == RC_NSTAGES - 1 ? RC_B[tid] : tid + 1 < RC_NSTAGES_EXT ? RC_A[tid + 1][tid] : 0.0;
+    }
+    if (tid == 0) s_bad = 0;
     __syncthreads();
 
-    uint32_t* flagY = S.flagY + ch * NT;
-    uint32_t* flagP = S.flagP + ch * NT;
-    const int my_tile = b * NB + c;
-
-    // ------------------------------------------------------------------------------------
-    // one right-hand-side evaluation on the stage input published in slot si with event ev
-    // ------------------------------------------------------------------------------------
-    // phase timers (constant-rate clock ticks): wait Y, load X, level 1 + publish P, level 2a,
-    // wait P, load P/insertions, level 2b + epilogue, integrator bookkeeping, step end (error
-    // norm, record, all-gather), total, publish Y, stage entry
-    // The timers run only when the caller asks for them: each reading of the clock waits for the
-    // scalar memory counter, which the untimed kernel does not pay.
-    const bool timed = uni(p.timers) != 0;
+    // phase timers (constant-rate clock ticks): wait for the stage input, (split) slice it, level 1 +
+    // publish P, level 2a, wait for P, (split) slice it, level 2b + epilogue, integrator bookkeeping,
+    // step end (error norm, record, all-gather), total, publish Y.
+    // The timers are an instantiation of their own (TIMED): each reading of the clock waits for the
+    // scalar memory counter and the sums take registers, which the untimed kernel does not pay.
     uint64_t tacc[RC_NTIMERS];
 #pragma unroll
     for (int q = 0; q < RC_NTIMERS; ++q) tacc[q] = 0;
-    uint64_t tmark = timed ? __builtin_amdgcn_s_memrealtime() : 0;
+    uint64_t tmark = TIMED ? __builtin_amdgcn_s_memrealtime() : 0;
     const uint64_t tstart = tmark;
     auto lap = [&](int q) {
-        if (timed) {
+        if constexpr (TIMED) {
             uint64_t now = __builtin_amdgcn_s_memrealtime();
             tacc[q] += now - tmark;
             tmark = now;
         }
     };
-    auto stage = [&](int si, uint32_t ev, double ts, double src, cplx& k_out, double& tr_out) -> bool {
-        const double jac = 2.0 * fabs(ts);
-        // wait for own channel's column block c and row block b
-        if (tid < 64) {
-            int n = 0;
-            if (lane < NB) s_addr[lane] = flagY + lane * NB + c;                    // (lane, c)
-            if (lane < NB) s_addr[NB + lane] = flagY + b * NB + lane;               // (b, lane)
-            (void)n;
-        }
-        __syncthreads();
-        lap(11);
-        if (!wait_flags(ctl, s_addr, 2 * NB, ev, &s_abort)) return false;
-        lap(0);
-        const double* Ych = S.Y + ((size_t)si * S.nlive + ch) * Dp * Dp * 2;
-        cplx xel = cmake(0, 0);   // own element of the stage input (split path)
-        if constexpr (SPLIT) {
-            cplx vr[4], vc[4];
-            fetch_row4<NB, true>(vr, Ych, mat_bytes, b);
-            fetch_col4<NB, true>(vc, Ych, mat_bytes, c);
-            if (tk.trace_kind == 1) xel = ld_coh(rY, (uint32_t)si * stage_stride + (uint32_t)ch * mat_bytes + el_off);
-            store_row4<NB>(pXr, vr, line_scale(vr, sgX));
-            store_col4<NB>(pXc, vc, line_scale(vc, sgX + 16));
-        } else {
-            load_row_col_coh<NB>(Xr, Xc, Ych, mat_bytes, b, c);
-        }
-        __syncthreads();
-        // per-element product scales: this lane's output rows 4 (lane/16) + q and column lane%16
-        int sXr[4], sXc = 0;
-        if constexpr (SPLIT) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) sXr[q] = sgX[4 * (lane >> 4) + q];
-            sXc = sgX[16 + (lane & 15)];
-        }
-        lap(1);
-        if (e_only) {
-            // E = X C of channel ch: its row block b times C's column block c
-            cplx Ee;
-            if constexpr (SPLIT) {
-                double pe[4] = {0.0, 0.0, 0.0, 0.0};
-                const int s2[4] = {-(sXr[0] + sK4), -(sXr[1] + sK4), -(sXr[2] + sK4), -(sXr[3] + sK4)};
-                if (mE) rc_split_product(pe, pXr, spa, pK4, spb, s2, lane);
-                Ee = reduce_split(pe, redd, wave, lane);
-            } else {
-                cacc ae;
-                cacc_zero(ae);
-                tile_product<NB>(ae, Xr, Kc, wave, lane, mE);
-                Ee = reduce_tile(ae, red, wave, lane);
-            }
-            st_coh(rE, (uint32_t)si * mat_bytes + el_off, Ee);
-            publish(S.flagE + my_tile, ev);
-            k_out = cmake(0, 0);
-            tr_out = 0.0;
-            return true;
-        }
-        // level 1
-        cacc acc;
-        double part[4] = {0.0, 0.0, 0.0, 0.0};
-        cplx Pe;
-        if constexpr (SPLIT) {
-            if (!adj) {
-                const int s2[4] = {-(sK0 + sXc), -(sK0 + sXc), -(sK0 + sXc), -(sK0 + sXc)};
-                if (m1) rc_split_product(part, pK0, spa, pXc, spb, s2, lane);
-            } else {
-                const int s2[4] = {-(sXr[0] + sK0), -(sXr[1] + sK0), -(sXr[2] + sK0), -(sXr[3] + sK0)};
-                if (m1) rc_split_product(part, pXr, spa, pK0, spb, s2, lane);
-            }
-            Pe = reduce_split(part, redd, wave, lane);
-        } else {
-            cacc_zero(acc);
-            if (!adj) tile_product<NB>(acc, Kl1, Xc, wave, lane, m1);
-            else tile_product<NB>(acc, Xr, Kl1, wave, lane, m1);
-            Pe = reduce_tile(acc, red, wave, lane);
-        }
-        const uint32_t poff = (uint32_t)si * stage_stride + (uint32_t)ch * mat_bytes;
-        st_coh(rP, poff + el_off, Pe);
-        double trv = 0.0;
-        if (tk.trace_kind == 2 && b == c && ei == ej && real_el) trv = Pe.re;
-        if (tk.trace_kind == 1 && real_el) {
-            const cplx x = SPLIT ? xel : Xr[ei * L::RS + col];
-            trv = x.re * trop_e.re + x.im * trop_e.im;   // Re(x conj(o))
-        }
-        publish(flagP + my_tile, ev);
-        lap(2);
-        // level 2a
-        if constexpr (SPLIT) {
-            part[0] = part[1] = part[2] = part[3] = 0.0;
-            const int s2a[4] = {-(sK1 + sXc), -(sK1 + sXc), -(sK1 + sXc), -(sK1 + sXc)};
-            const int s2b[4] = {-(sXr[0] + sK2), -(sXr[1] + sK2), -(sXr[2] + sK2), -(sXr[3] + sK2)};
-            if (m2a) rc_split_product(part, pK1, spa, pXc, spb, s2a, lane);
-            if (m2b) rc_split_product(part, pXr, spa, pK2, spb, s2b, lane);
-        } else {
-            cacc_zero(acc);
-            tile_product<NB>(acc, Kq, Xc, wave, lane, m2a);
-            tile_product<NB>(acc, Xr, Kx, wave, lane, m2b);
-        }
-        __syncthreads();
-        lap(3);
-        // wait for the P tiles of this channel and the insertion source tiles
-        if (tid < 64) {
-            if (lane < NB) s_addr[lane] = adj ? (flagP + lane * NB + c) : (flagP + b * NB + lane);
-            if (lane == 0 && tk.edge_src >= 0) {
-                uint32_t* fs = tk.edge_from_E ? S.flagE : (S.flagP + tk.edge_src * NT);
-                s_addr[NB] = fs + b * NB + c;
-                s_addr[NB + 1] = fs + c * NB + b;
-            }
-        }
-        __syncthreads();
-        const int nw = NB + (tk.edge_src >= 0 ? 2 : 0);
-        if (!wait_flags(ctl, s_addr, nw, ev, &s_abort)) return false;
-        lap(4);
-        const double* Pch = S.P + ((size_t)si * S.nlive + ch) * Dp * Dp * 2;
-        cplx vp[4];
-        if constexpr (SPLIT) {
-            if (!adj) fetch_row4<NB, true>(vp, Pch, mat_bytes, b);
-            else fetch_col4<NB, true>(vp, Pch, mat_bytes, c);
-        } else {
-            if (!adj) load_rowblk<NB, true>(Pb, Pch, mat_bytes, b);
-            else load_colblk<NB, true>(Pb, Pch, mat_bytes, c);
-        }
-        cplx ins = cmake(0, 0);
-        if (tk.edge_src >= 0) {
-            cplx s1, s2;
-            if (tk.edge_from_E) {
-                s1 = ld_coh(rE, (uint32_t)si * mat_bytes + el_off);
-                s2 = ld_coh(rE, (uint32_t)si * mat_bytes + el_off_t);
-            } else {
-                uint32_t so = (uint32_t)si * stage_stride + (uint32_t)tk.edge_src * mat_bytes;
-                s1 = ld_coh(rP, so + el_off);
-                s2 = ld_coh(rP, so + el_off_t);
-            }
-            ins = cscale(tk.edge_coef, cadd(s1, cconj(s2)));
-        }
-        if constexpr (SPLIT) {
-            if (!adj) store_row4<NB>(pPb, vp, line_scale(vp, sgP));
-            else store_col4<NB>(pPb, vp, line_scale(vp, sgP));
-        }
-        __syncthreads();
-        lap(5);
-        cplx Le;
-        if constexpr (SPLIT) {
-            if (!adj) {
-                const int s2[4] = {-(sgP[4 * (lane >> 4)] + sK3), -(sgP[4 * (lane >> 4) + 1] + sK3),
-                                   -(sgP[4 * (lane >> 4) + 2] + sK3), -(sgP[4 * (lane >> 4) + 3] + sK3)};
-                if (m3) rc_split_product(part, pPb, spa, pK3, spb, s2, lane);
-            } else {
-                const int sc = -(sK3 + sgP[lane & 15]);
-                const int s2[4] = {sc, sc, sc, sc};
-                if (m3) rc_split_product(part, pK3, spa, pPb, spb, s2, lane);
-            }
-            Le = reduce_split(part, redd, wave, lane);
-        } else {
-            if (!adj) tile_product<NB>(acc, Pb, Kp, wave, lane, m3);
-            else tile_product<NB>(acc, Kp, Pb, wave, lane, m3);
-            Le = reduce_tile(acc, red, wave, lane);
-        }
-        cplx k = cadd(cscale(jac, Le), cscale(src, cadd(ins, fixed_e)));
-        if (!real_el) k = cmake(0, 0);
-        k_out = k;
-        if (tk.trace_kind) tr_out = tk.trace_coef * src * block_sum(trv, scratch);
-        else tr_out = 0.0;
-        lap(6);
-        return true;
-    };
-
-    auto publish_Y = [&](int si, uint32_t ev, cplx v) {
-        lap(7);
-        if (!e_only) {   // an E task reads channel ch's stage input; the channel's own task writes it
-            st_coh(rY, (uint32_t)si * stage_stride + (uint32_t)ch * mat_bytes + el_off, v);
-            publish(flagY + my_tile, ev);
-        }
-        lap(10);
-    };
 
     // ------------------------------------------------------------------------------------
-    // integrator: a state machine over stage slots with a single stage call site.  The stage
-    // derivatives of the attempt are kept per element in a window kst that shifts by one as each
-    // arrives (the newest at kst[15]); every combination (next stage input, solution, error
-    // estimators, dense output) is a sum with the tableau's constant coefficients, selected by
-    // the uniform slot, so no array is indexed at run time.
+    // integrator state.  The stage derivatives of the attempt are kept per element in a window kst
+    // that shifts by one as each arrives (the newest at kst[15]), so no register array is indexed at
+    // run time.  All of a combination (next stage input, solution, error estimators) but its last term
+    // is summed while the stage waits for its neighbours' P tiles, so one multiply-add stands between
+    // a stage's derivative and the next stage input.
     // ------------------------------------------------------------------------------------
     const double a = p.a;
     cplx kst[RC_NSTAGES_EXT];
 #pragma unroll
     for (int q = 0; q < RC_NSTAGES_EXT; ++q) kst[q] = cmake(0, 0);
     cplx y = cmake(0, 0), ynew = cmake(0, 0), k0 = cmake(0, 0), k12 = cmake(0, 0);
-    __shared__ double s_trp[RC_NSTAGES_EXT];
-    __shared__ double s_src[RC_NSTAGES_EXT];
-    __shared__ double s_cheb[RC_SOURCE_SEGMENTS * (RC_SOURCE_DEGREE + 1)];
-    for (int i = tid; i < RC_SOURCE_SEGMENTS * (RC_SOURCE_DEGREE + 1); i += 256) s_cheb[i] = p.cheb[i];
-    __shared__ double s_cnode[RC_NSTAGES_EXT];
-    if (tid < RC_NSTAGES_EXT) s_cnode[tid] = RC_C[tid];
-    __syncthreads();
-
+    cplx pre5 = cmake(0, 0), pre3 = cmake(0, 0);   // prefix sums of the error estimators
     double ysc = 0.0, ysc_new = 0.0;
     double t = -a, h = fmin(p.h0, 2.0 * a), t_new = t, endpoint = 0.0, factor = 1.0;
     uint32_t ev = 0;
-    long long attempts = 0, accepted = 0, rejected = 0, dense = 0;
+    uint32_t attempts = 0, accepted = 0, rejected = 0, dense = 0, rhs = 0;
     int next_point = 0, rej = 0, status = RC_ST_OK;
     bool alive = true;
     const __amdgpu_buffer_rsrc_t rS = rc_rsrc(S.samples, (uint32_t)((size_t)p.npoints * S.nlive * mat_bytes));
     const int my_rank = task - S.first_task;
 
+    // stage input of the next event
+    auto publish_Y = [&](cplx v) {
+        ++ev;
+        if (e_only) return;   // an E task reads channel ch's stage input; the channel's own task writes it
+        if constexpr (LOCAL) Yt[ei * 17 + ej] = v;
+        const uint32_t so = (ev & (RC_RING - 1)) * stage_stride + (uint32_t)ch * mat_bytes;
+        if (LOCAL ? tk.pub_y : do2) {
+            rc_put(rX, ya_off, so, v);
+            if constexpr (!LOCAL) rc_put(rX, yb_off, oB + so, v);
+        }
+    };
+
+    // empty this workgroup's slots of event ev - 16 (once for every event, also one that is skipped)
+    auto empty_old = [&] {
+        if (ev <= RC_RING / 2) return;
+        const uint32_t old = (ev - RC_RING / 2) & (RC_RING - 1), so = old * stage_stride + (uint32_t)ch * mat_bytes;
+        if (e_only) {
+            rc_reset(rX, yb_off, oE + old * mat_bytes);
+            return;
+        }
+        if (LOCAL ? tk.pub_y : do2) {
+            rc_reset(rX, ya_off, so);
+            if constexpr (!LOCAL) rc_reset(rX, yb_off, oB + so);
+        }
+        if (LOCAL ? tk.pub_p : do1) rc_reset(rX, pub_off, oP + so);
+    };
+
+    // ------------------------------------------------------------------------------------
+    // one right-hand-side evaluation on the stage input of event ev (own element `own`); al: the
+    // coefficient of its derivative in the combination that follows, which is the next stage input
+    // and published at once when `chain`
+    // ------------------------------------------------------------------------------------
+    auto stage = [&](int slot, double ts, cplx own, double al, bool chain, cplx& k_out, cplx& comb_out) {
+        const double jac = 2.0 * fabs(ts);
+        const uint32_t ring = ev & (RC_RING - 1);
+        const uint32_t so = ring * stage_stride + (uint32_t)ch * mat_bytes;
+        cplx xr[NF], xc[NF];
+        if (e_only) {
+            // E = X C of channel ch: its row block b times C's column block c
+            if (doE) {
+                cplx Ee;
+                rc_fetch<NF>(rX, row_off, so, row_step, xr, use_r);
+                if (!rc_await<NF>(ctl, rX, row_off, so, row_step, xr, use_r)) s_bad = 1;
+                lap(0);
+                // the two partial buffers alternate: one barrier a stage
+                if constexpr (SPLIT) {
+                    store_row4<NB>(pXr, xr, line_scale(xr, sgX));
+                    lds_barrier();
+                    lap(1);
+                    int s2[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) s2[q] = -(sgX[4 * (lane >> 4) + q] + sK1);
+                    double pe[4] = {0.0, 0.0, 0.0, 0.0};
+                    rc_split_product(pe, pXr, spa, pK1, spb, s2, lane);
+                    double* redd = (rhs & 1) ? redd2 : redd1;
+                    put_partial_split(pe, redd, wave, lane);
+                    lds_barrier();
+                    Ee = sum_partial_split(redd);
+                } else {
+                    cacc ae;
+                    cacc_zero(ae);
+                    frag_product<KT>(ae, xr, K1);
+                    cplx* red = (rhs & 1) ? red2 : red1;
+                    put_partial(ae, red, wave, lane);
+                    lds_barrier();
+                    Ee = sum_partial(red);
+                }
+                rc_put(rX, yb_off, oE + ring * mat_bytes, Ee);
+            }
+            empty_old();
+            k_out = comb_out = cmake(0, 0);
+            if (chain) publish_Y(comb_out);
+            lap(2);
+            return;
+        }
+        // stage input
+        bool ok = true;
+        const bool get_c = do2 || !adj, get_r = do2 || adj;   // what the tile's products read
+        if constexpr (LOCAL) {
+            lds_barrier();
+            xr[0] = Yt[fi * 17 + fk];
+            xc[0] = Yt[fk * 17 + fi];
+        } else {
+            if (get_c) rc_fetch<NF>(rX, col_off, oB + so, col_step, xc, use_c);
+            if (get_r) rc_fetch<NF>(rX, row_off, so, row_step, xr, use_r);
+            if (get_c) ok = rc_await<NF>(ctl, rX, col_off, oB + so, col_step, xc, use_c);
+            if (get_r) ok = rc_await<NF>(ctl, rX, row_off, so, row_step, xr, use_r) && ok;
+        }
+        lap(0);
+        cacc acc;
+        double part[4] = {0.0, 0.0, 0.0, 0.0};
+        int sXr[4], sXc = 0;
+        cplx Pe = cmake(0, 0);
+        if constexpr (SPLIT) {
+            if (get_r) store_row4<NB>(pXr, xr, line_scale(xr, sgX));
+            if (get_c) store_col4<NB>(pXc, xc, line_scale(xc, sgX + 16));
+            lds_barrier();
+            lap(1);
+            // per-element product scales: this lane's output rows 4 (lane/16) + q and column lane%16
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sXr[q] = sgX[4 * (lane >> 4) + q];
+            sXc = sgX[16 + (lane & 15)];
+        }
+        if (do1) {
+            if constexpr (SPLIT) {
+                if (!adj) {
+                    const int s2[4] = {-(sK1 + sXc), -(sK1 + sXc), -(sK1 + sXc), -(sK1 + sXc)};
+                    rc_split_product(part, pK1, spa, pXc, spb, s2, lane);
+                } else {
+                    const int s2[4] = {-(sXr[0] + sK1), -(sXr[1] + sK1), -(sXr[2] + sK1), -(sXr[3] + sK1)};
+                    rc_split_product(part, pXr, spa, pK1, spb, s2, lane);
+                }
+                put_partial_split(part, redd1, wave, lane);
+            } else {
+                cacc_zero(acc);
+                if (!adj) frag_product<KT>(acc, K1, xc);
+                else frag_product<KT>(acc, xr, K1);
+                put_partial(acc, red1, wave, lane);
+            }
+            lds_barrier();
+            Pe = SPLIT ? sum_partial_split(redd1) : sum_partial(red1);
+            if constexpr (LOCAL) Pt[ei * 17 + ej] = Pe;
+            if (!LOCAL || tk.pub_p) rc_put(rX, pub_off, oP + so, Pe);
+        } else {
+            lds_barrier();   // two level-2 sums in a row need a barrier between them
+        }
+        lap(2);
+        // the slots of event ev - 16 (ahead of the P loads: a wait for those does not include a younger store)
+        empty_old();
+        // level 2a
+        if (do2) {
+            if constexpr (SPLIT) {
+                part[0] = part[1] = part[2] = part[3] = 0.0;
+                const int s2a[4] = {-(sKq + sXc), -(sKq + sXc), -(sKq + sXc), -(sKq + sXc)};
+                const int s2b[4] = {-(sXr[0] + sKx), -(sXr[1] + sKx), -(sXr[2] + sKx), -(sXr[3] + sKx)};
+                rc_split_product(part, pKq, spa, pXc, spb, s2a, lane);
+                rc_split_product(part, pXr, spa, pKx, spb, s2b, lane);
+            } else {
+                cacc_zero(acc);
+                frag_product<KT>(acc, Kq, xc);
+                frag_product<KT>(acc, xr, Kx);
+            }
+        }
+        // the P tiles of this channel (row block forward, column block adjoint) and the insertion source
+        cplx vp[NF], s1 = cmake(0, 0), s2 = cmake(0, 0);
+        const bool insert = do2 && tk.edge_src >= 0;
+        const uint32_t so_i = tk.edge_from_E ? oE + ring * mat_bytes
+                                             : oP + ring * stage_stride + (uint32_t)tk.edge_src * mat_bytes;
+        if (!LOCAL && do2) rc_fetch<NF>(rX, p_off, oP + so, p_step, vp, use_p);
+        if (insert) {
+            s1 = ld_coh_s(rX, ins_off, so_i);
+            s2 = ld_coh_s(rX, ins_off_t, so_i);
+        }
+        // while they arrive: the trace of this stage and the prefix sums
+        if (tk.trace_kind) {
+            double trv = 0.0;
+            if (tk.trace_kind == 2 && b == c && ei == ej && real_el) trv = Pe.re;
+            if (tk.trace_kind == 1 && real_el) trv = fma(own.re, trop_e.re, own.im * trop_e.im);   // Re(x conj(o))
+            trv = wave_sum(trv);
+            if (lane == 0) s_trp[slot][wave] = trv;
+        }
+        const cplx pre = rc_row_sum(slot, kst);
+        if (slot == RC_NSTAGES - 1) {
+            pre5 = rc_row_sum(16, kst);
+            pre3 = rc_row_sum(17, kst);
+        }
+        const double src = slot == 0 ? rc_source(ts, s_cheb) : unid(s_src[attempts & 1][slot]);
+        if (tk.trace_kind && tid == 0) s_trs[slot] = tk.trace_coef * src;
+        lap(3);
+        cplx Le = cmake(0, 0);
+        if (do2) {
+            if constexpr (LOCAL) {
+                lds_barrier();
+                vp[0] = adj ? Pt[fk * 17 + fi] : Pt[fi * 17 + fk];
+            } else {
+                ok = rc_await<NF>(ctl, rX, p_off, oP + so, p_step, vp, use_p) && ok;
+            }
+            lap(4);
+            if constexpr (SPLIT) {
+                if (!adj) store_row4<NB>(pPb, vp, line_scale(vp, sgP));
+                else store_col4<NB>(pPb, vp, line_scale(vp, sgP));
+                lds_barrier();
+                lap(5);
+                if (!adj) {
+                    const int s2[4] = {-(sgP[4 * (lane >> 4)] + sKp), -(sgP[4 * (lane >> 4) + 1] + sKp),
+                                       -(sgP[4 * (lane >> 4) + 2] + sKp), -(sgP[4 * (lane >> 4) + 3] + sKp)};
+                    rc_split_product(part, pPb, spa, pKp, spb, s2, lane);
+                } else {
+                    const int sc = -(sKp + sgP[lane & 15]);
+                    const int s2[4] = {sc, sc, sc, sc};
+                    rc_split_product(part, pKp, spa, pPb, spb, s2, lane);
+                }
+                put_partial_split(part, redd2, wave, lane);
+            } else {
+                if (!adj) frag_product<KT>(acc, vp, Kp);
+                else frag_product<KT>(acc, Kp, vp);
+                put_partial(acc, red2, wave, lane);
+            }
+            if (insert) {
+                ok = rc_await<1>(ctl, rX, ins_off, so_i, 0, &s1) && ok;
+                ok = rc_await<1>(ctl, rX, ins_off_t, so_i, 0, &s2) && ok;
+            }
+            lds_barrier();
+            Le = SPLIT ? sum_partial_split(redd2) : sum_partial(red2);
+        } else {
+            lds_barrier();   // two level-1 sums in a row likewise
+        }
+        if (!ok) s_bad = 1;
+        const cplx ins = cfma(insert ? tk.edge_coef : 0.0, cadd(s1, cconj(s2)), fixed_e);
+        cplx k = cfma(jac, Le, cscale(src, ins));
+        if (!real_el) k = cmake(0, 0);
+        k_out = k;
+        comb_out = cfma(h, cfma(al, k, pre), y);
+        lap(6);
+        if (chain) publish_Y(comb_out);
+        lap(10);
+    };
+
+    // ------------------------------------------------------------------------------------
+    // a state machine over stage slots with a single stage call site; the stage input of the event
+    // at hand is published before the stage is entered
+    // ------------------------------------------------------------------------------------
     int slot = 0;
     cplx Yin = y;
     double ts = t;
+    publish_Y(Yin);
     while (true) {
-        ++ev;
-        publish_Y(slot, ev, Yin);
-        cplx kn;
-        double trn;
-        const double src = slot == 0 ? rc_source(ts, s_cheb) : unid(s_src[slot]);
-        if (!(alive = stage(slot, ev, ts, src, kn, trn))) break;
-        if (tid == 0) s_trp[slot] = trn;
-        int next = -1;   // -1: start a new step attempt
-#pragma unroll
-        for (int q = 0; q < RC_NSTAGES_EXT - 1; ++q) kst[q] = kst[q + 1];
-        kst[RC_NSTAGES_EXT - 1] = kn;
+        cplx kn, comb;
+        ++rhs;
+        // stages 1..10 and, when a quadrature node lies in the step, 12..14 chain to the next one
+        const bool node_due = slot >= RC_NSTAGES && next_point < p.npoints && ld_const(p.points, next_point) <= t_new;
+        const bool chain = slot < RC_NSTAGES - 1 ? slot > 0 : node_due && slot < RC_NSTAGES_EXT - 1;
+        stage(slot, ts, Yin, s_alast[slot], chain, kn, comb);
+        int next = -1;       // -1: start a new step attempt
+        bool published = chain, interpolate = false;
+        const double t_old = t, h_old = h;
+        const cplx y_old = y, k0_old = k0;
         if (slot == 0) {
             k0 = kn;
         } else if (slot < RC_NSTAGES - 1) {
             next = slot + 1;
         } else if (slot == RC_NSTAGES - 1) {
             lap(7);
-            // k_j at kst[4 + j] after k_11
-            const cplx accB = rc_comb<RC_ROW_B, 0, RC_NSTAGES, 4>(kst, cmake(0, 0));
-            const cplx acc5 = rc_comb<RC_ROW_E5, 0, RC_NSTAGES, 4>(kst, cmake(0, 0));
-            const cplx acc3 = rc_comb<RC_ROW_E3, 0, RC_NSTAGES, 4>(kst, cmake(0, 0));
-            ynew = cadd(y, cscale(h, accB));
+            ynew = comb;
+            const cplx acc5 = cfma(RC_E5[RC_NSTAGES - 1], kn, pre5);
+            const cplx acc3 = cfma(RC_E3[RC_NSTAGES - 1], kn, pre3);
             double e5p = 0.0, e3p = 0.0;
             if (real_el) {
                 double sc = p.atol + p.rtol * fmax(cabsd(y), cabsd(ynew));
-                e5p = cabs2(cmake(acc5.re / sc, acc5.im / sc));
-                e3p = cabs2(cmake(acc3.re / sc, acc3.im / sc));
+                const cplx r5 = cmake(acc5.re / sc, acc5.im / sc), r3 = cmake(acc3.re / sc, acc3.im / sc);
+                e5p = fma(r5.re, r5.re, r5.im * r5.im);
+                e3p = fma(r3.re, r3.re, r3.im * r3.im);
             }
-            block_sum2(e5p, e3p, scratch);
-            // record for the all-gather: e5, e3, trace partials of k_0..k_11
-            const uint32_t par = (uint32_t)(attempts & 1);
-            if (tid < RC_REC) {
-                double v = 0.0;
-                if (tid == 0) v = e5p;
-                else if (tid == 1) v = e3p;
-                else if (tid < 2 + RC_NSTAGES) v = s_trp[tid - 2];
-                st_coh_f64(S.rec + ((size_t)par * S.ntasks + my_rank) * RC_REC + tid, v);
+            e5p = wave_sum(e5p);
+            e3p = wave_sum(e3p);
+            if (lane == 0) {
+                s_err[wave] = e5p;
+                s_err[4 + wave] = e3p;
             }
-            lap(8);
-            publish(S.flagR + my_rank, (uint32_t)attempts);
-            if (tid < 64) s_addr[lane] = S.flagR + (lane < S.ntasks ? lane : 0);
-            __syncthreads();
-            if (!(alive = wait_flags(ctl, s_addr, S.ntasks, (uint32_t)attempts, &s_abort))) break;
-            if (tid < 64) {
+            // every emptied slot is empty at device scope before the record can be seen
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            lds_barrier();
+            // record for the all-gather: (e5, e3), then the trace partials of k_0..k_11 in pairs
+            const uint32_t rec_bytes = (uint32_t)(S.ntasks * RC_REC * 8);
+            const uint32_t so_rec = oR + (attempts & (RC_REC_RING - 1)) * rec_bytes;
+            constexpr int NREC = (2 + RC_NSTAGES) / 2;
+            if (wave == 0 && lane < (S.has_scalar ? NREC : 1)) {
+                cplx v;
+                if (lane == 0) {
+                    v = cmake(((s_err[0] + s_err[1]) + s_err[2]) + s_err[3], ((s_err[4] + s_err[5]) + s_err[6]) + s_err[7]);
+                } else {
+                    const int q = 2 * lane - 2;
+                    v = tk.trace_kind ? cmake(s_trs[q] * (((s_trp[q][0] + s_trp[q][1]) + s_trp[q][2]) + s_trp[q][3]),
+                                              s_trs[q + 1] * (((s_trp[q + 1][0] + s_trp[q + 1][1]) + s_trp[q + 1][2]) +
+                                                              s_trp[q + 1][3]))
+                                      : cmake(0, 0);
+                }
+                const uint32_t off = (uint32_t)(my_rank * RC_REC * 8 + 16 * lane);
+                rc_put(rX, off, so_rec, v);
+                // the record of attempt - 2: every workgroup published that of attempt - 1, so all read it
+                rc_reset(rX, off, oR + ((attempts + 2) & (RC_REC_RING - 1)) * rec_bytes);
+            }
+            // the FSAL stage's input, published ahead of the verdict (a rejected step's is never read)
+            publish_Y(ynew);
+            if (wave == 0) {
                 // every record in flight at once, then one deterministic reduction per entry
-                const __amdgpu_buffer_rsrc_t rR = rc_rsrc(S.rec, (uint32_t)(2 * S.ntasks * RC_REC * 8));
-                const uint32_t base = (uint32_t)(((size_t)par * S.ntasks + lane) * RC_REC * 8);
-                cplx v[(2 + RC_NSTAGES) / 2];
+                cplx v[NREC];
+                const uint32_t off = (uint32_t)(lane * RC_REC * 8);
+                bool ok;
+                if (S.has_scalar) {
+                    rc_fetch<NREC>(rX, off, so_rec, 16, v, lane < S.ntasks);
+                    ok = rc_await<NREC>(ctl, rX, off, so_rec, 16, v, lane < S.ntasks);
+                } else {
+                    rc_fetch<1>(rX, off, so_rec, 16, v, lane < S.ntasks);
+                    ok = rc_await<1>(ctl, rX, off, so_rec, 16, v, lane < S.ntasks);
+                }
+                if (lane == 0) s_tot[16] = ok && !s_bad ? 0.0 : 1.0;
 #pragma unroll
-                for (int q = 0; q < (2 + RC_NSTAGES) / 2; ++q)
-                    v[q] = lane < S.ntasks ? ld_coh(rR, base + 16 * q) : cmake(0, 0);
-#pragma unroll
-                for (int q = 0; q < (2 + RC_NSTAGES) / 2; ++q) {
+                for (int q = 0; q < NREC; ++q) {
+                    if (q > 0 && !S.has_scalar) break;
                     double x = v[q].re, z = v[q].im;
 #pragma unroll
                     for (int off = 32; off > 0; off >>= 1) {
@@ -828,8 +851,8 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
                     }
                 }
             }
-            __syncthreads();
-            lap(8);
+            lds_barrier();
+            if (!(alive = unid(s_tot[16]) == 0.0)) break;
             double e5 = unid(s_tot[0]), e3 = unid(s_tot[1]);
             ysc_new = ysc;
             if (S.has_scalar) {
@@ -846,24 +869,26 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
                 e5 += (s5 / sc) * (s5 / sc);
                 e3 += (s3 / sc) * (s3 / sc);
             }
-            __syncthreads();
             const double den = e5 + 0.01 * e3;
             const double error = den > 0.0 ? h * e5 / sqrt(den * S.n_elems) : 0.0;
+            lap(8);
             if (!isfinite(error)) { status = RC_ST_NONFINITE; break; }
             factor = error > 0.0 ? fmin(10.0, 0.9 * pow(error, -1.0 / 8.0)) : 10.0;
             if (error > 1.0) {
                 ++rejected;
                 rej = 1;
                 h *= fmax(0.2, factor);
+                empty_old();   // the FSAL event published above is skipped
                 next = -1;
             } else {
                 ++accepted;
                 t_new = (h == endpoint - t) ? endpoint : t + h;
                 next = RC_NSTAGES;   // FSAL stage
+                published = true;
             }
         } else if (slot == RC_NSTAGES) {
             k12 = kn;
-            if (next_point < p.npoints && ld_const(p.points, next_point) <= t_new) {
+            if (node_due) {
                 ++dense;
                 next = RC_NSTAGES + 1;
             } else {
@@ -872,74 +897,97 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
         } else if (slot < RC_NSTAGES_EXT - 1) {
             next = slot + 1;
         } else {
-            const cplx d0 = csub(ynew, y);
-            const cplx d1 = csub(cscale(h, k0), d0);
-            const cplx d2 = csub(cscale(2.0, d0), cscale(h, cadd(k12, k0)));
-            // k_j at kst[j] after k_15
-            cplx dd[4];
-            dd[0] = cscale(h, rc_comb<RC_ROW_D, 0, RC_NSTAGES_EXT, 0>(kst, cmake(0, 0)));
-            dd[1] = cscale(h, rc_comb<RC_ROW_D, 1, RC_NSTAGES_EXT, 0>(kst, cmake(0, 0)));
-            dd[2] = cscale(h, rc_comb<RC_ROW_D, 2, RC_NSTAGES_EXT, 0>(kst, cmake(0, 0)));
-            dd[3] = cscale(h, rc_comb<RC_ROW_D, 3, RC_NSTAGES_EXT, 0>(kst, cmake(0, 0)));
-            while (next_point < p.npoints && ld_const(p.points, next_point) <= t_new) {
-                const double pt = ld_const(p.points, next_point);
-                cplx v;
-                if (pt == t_new) {
-                    v = ynew;
-                } else {
-                    const double x = (pt - t) / h, xm = 1.0 - x;
-                    cplx r = cscale(x, dd[3]);
-                    r = cscale(xm, cadd(r, dd[2]));
-                    r = cscale(x, cadd(r, dd[1]));
-                    r = cscale(xm, cadd(r, dd[0]));
-                    r = cscale(x, cadd(r, d2));
-                    r = cscale(xm, cadd(r, d1));
-                    r = cscale(x, cadd(r, d0));
-                    v = cadd(r, y);
-                }
-                if (!e_only) st_coh(rS, (uint32_t)next_point * stage_stride + (uint32_t)ch * mat_bytes + el_off, v);
-                ++next_point;
-            }
+            interpolate = true;
             next = -2;
         }
         if (next == -2) {
             // accepted step complete: FSAL and state update
             y = ynew;
             k0 = k12;
-            if (tid == 0) s_trp[0] = s_trp[RC_NSTAGES];
+            if (tk.trace_kind && tid == 0) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) s_trp[0][q] = s_trp[RC_NSTAGES][q];
+                s_trs[0] = s_trs[RC_NSTAGES];
+            }
             t = t_new;
             ysc = ysc_new;
             h *= rej ? fmin(1.0, factor) : factor;
             rej = 0;
             next = -1;
         }
+        bool done = false;
         if (next == -1) {
             // start an attempt from (t, y, k0) with step h
-            if (!(t < a)) break;
-            endpoint = t < 0.0 ? 0.0 : a;
-            h = fmin(h, endpoint - t);
-            if (!(h > 10.0 * fabs(nextafter(t, INFINITY) - t))) { status = RC_ST_STEP_UNDERFLOW; break; }
-            if (attempts >= p.max_steps) { status = RC_ST_MAX_STEPS; break; }
-            ++attempts;
-            kst[RC_NSTAGES_EXT - 1] = k0;   // k_0 of the attempt enters the window
-            // source values at every stage time of this attempt (stages 1..15), one lane each
-            if (tid >= 1 && tid < RC_NSTAGES_EXT) s_src[tid] = rc_source(t + s_cnode[tid] * h, s_cheb);
-            __syncthreads();
+            if (!(t < a)) {
+                done = true;
+            } else {
+                endpoint = t < 0.0 ? 0.0 : a;
+                h = fmin(h, endpoint - t);
+                if (!(h > 10.0 * fabs(nextafter(t, INFINITY) - t))) { status = RC_ST_STEP_UNDERFLOW; done = true; }
+                else if ((long long)attempts >= p.max_steps) { status = RC_ST_MAX_STEPS; done = true; }
+                else ++attempts;
+            }
             next = 1;
         }
-        slot = uni(next);
-        next_point = uni(next_point);
         t = unid(t);
         h = unid(h);
-        if (slot == RC_NSTAGES) {
-            Yin = ynew;
-            ts = t + h;
-        } else {
-            Yin = cadd(y, cscale(h, rc_stage_comb(slot, kst)));
-            ts = t + RC_C[slot] * h;
+        if (!done) {
+            if (next == 1) {
+                Yin = cfma(h, cscale(RC_A[1][0], k0), y);
+                ts = t + RC_C[1] * h;
+            } else {
+                Yin = comb;   // also the solution, the FSAL stage's input
+                ts = t + s_cnode[next] * h;
+            }
+            lap(7);
+            if (!published) publish_Y(Yin);
         }
+        // behind the publish: the source values of the attempt's stages (one lane each), the dense
+        // output, the window
+        if (next == 1 && !done && tid >= 1 && tid < RC_NSTAGES_EXT)
+            s_src[attempts & 1][tid] = rc_source(t + s_cnode[tid] * h, s_cheb);
+        if (interpolate) {
+            cplx dd[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                dd[q] = cscale(h_old, cfma(RC_D[q][RC_NSTAGES_EXT - 1], kn, rc_row_sum(18 + q, kst)));
+            const cplx d0 = csub(ynew, y_old);
+            const cplx d1 = cfma(h_old, k0_old, cmake(-d0.re, -d0.im));
+            const cplx d2 = cfma(-h_old, cadd(k12, k0_old), cscale(2.0, d0));
+            while (next_point < p.npoints && ld_const(p.points, next_point) <= t_new) {
+                const double pt = ld_const(p.points, next_point);
+                cplx v;
+                if (pt == t_new) {
+                    v = ynew;
+                } else {
+                    const double x = (pt - t_old) / h_old, xm = 1.0 - x;
+                    cplx r = cfma(x, dd[3], dd[2]);
+                    r = cfma(xm, r, dd[1]);
+                    r = cfma(x, r, dd[0]);
+                    r = cfma(xm, r, d2);
+                    r = cfma(x, r, d1);
+                    r = cfma(xm, r, d0);
+                    v = cfma(x, r, y_old);
+                }
+                if (!e_only) st_coh(rS, (uint32_t)next_point * stage_stride + (uint32_t)ch * mat_bytes + el_off, v);
+                ++next_point;
+            }
+            next_point = uni(next_point);
+        }
+        if (done) break;
+        if (next == 1) {   // k_0 of a new attempt enters an empty window
+#pragma unroll
+            for (int q = 0; q < RC_NSTAGES_EXT - 1; ++q) kst[q] = cmake(0, 0);
+            kst[RC_NSTAGES_EXT - 1] = k0;
+        } else {
+#pragma unroll
+            for (int q = 0; q < RC_NSTAGES_EXT - 1; ++q) kst[q] = kst[q + 1];
+            kst[RC_NSTAGES_EXT - 1] = kn;
+        }
+        slot = uni(next);
     }
-    if (!alive) status = RC_ST_WAIT_LIMIT;
+    // an attempt cut short by a wait that failed anywhere may end in a nonfinite error norm first
+    if (!alive || (status == RC_ST_NONFINITE && uni((int)ld_flag(ctl.abort_flag)))) status = RC_ST_WAIT_LIMIT;
     if (status == RC_ST_OK && next_point != p.npoints) status = RC_ST_MISSING_SAMPLES;
     __builtin_amdgcn_s_waitcnt(0);
     if (my_rank == 0 && tid == 0) {
@@ -948,18 +996,18 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
         S.out[RC_OUT_ACCEPTED] = (double)accepted;
         S.out[RC_OUT_REJECTED] = (double)rejected;
         S.out[RC_OUT_DENSE] = (double)dense;
-        S.out[RC_OUT_RHS] = (double)ev;
+        S.out[RC_OUT_RHS] = (double)rhs;
         S.out[RC_OUT_SCALAR] = ysc;
         S.out[RC_OUT_T] = t;
         S.out[RC_OUT_NEXTPOINT] = next_point;
         lap(7);
-        if (timed) tacc[9] = __builtin_amdgcn_s_memrealtime() - tstart;
+        if constexpr (TIMED) tacc[9] = __builtin_amdgcn_s_memrealtime() - tstart;
 #pragma unroll
         for (int q = 0; q < RC_NTIMERS; ++q) S.out[RC_OUT_TIMERS + q] = (double)tacc[q];
     }
 }
 
-template <int NB, bool SPLIT>
+template <int NB, int KT, bool SPLIT, bool TIMED>
 __global__ void __launch_bounds__(256, 1) rc_trajectory(const TrajParams* __restrict__ pp) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const TrajParams& p = *pp;
@@ -967,9 +1015,15 @@ __global__ void __launch_bounds__(256, 1) rc_trajectory(const TrajParams* __rest
     for (int r = 0; r < p.nrounds; ++r) {
         const int task = __builtin_amdgcn_readfirstlane(sched[r * (int)gridDim.x + (int)blockIdx.x]);
         if (task < 0) continue;
-        run_task<NB, SPLIT>(p, task, smem_raw);
+        run_task<NB, KT, SPLIT, TIMED>(p, task, smem_raw);
         __syncthreads();
     }
+}
+
+// Empty every slot of a launch's exchange buffers (n 16-byte words).
+__global__ void __launch_bounds__(256) rc_fill_empty(v4u* w, long long n) {
+    const v4u e = {RC_EMPTY_WORD, RC_EMPTY_WORD, RC_EMPTY_WORD, RC_EMPTY_WORD};
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) w[i] = e;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -986,23 +1040,30 @@ int rc_trajectory_smem_bytes(int nb, int split) {
     }
 }
 
-static const void* trajectory_fn(int nb, int split) {
+template <bool TIMED>
+static const void* trajectory_fn(int nb, int split, int z2) {
+    if (z2 && !split && nb == 2) return (const void*)rc_trajectory<2, 1, false, TIMED>;
+    if (z2 && !split && nb == 4) return (const void*)rc_trajectory<4, 2, false, TIMED>;
     switch (nb * 2 + (split ? 1 : 0)) {
-        case 2: return (const void*)rc_trajectory<1, false>;
-        case 3: return (const void*)rc_trajectory<1, true>;
-        case 4: return (const void*)rc_trajectory<2, false>;
-        case 5: return (const void*)rc_trajectory<2, true>;
-        case 6: return (const void*)rc_trajectory<3, false>;
-        case 7: return (const void*)rc_trajectory<3, true>;
-        case 8: return (const void*)rc_trajectory<4, false>;
-        case 9: return (const void*)rc_trajectory<4, true>;
+        case 2: return (const void*)rc_trajectory<1, 1, false, TIMED>;
+        case 3: return (const void*)rc_trajectory<1, 1, true, TIMED>;
+        case 4: return (const void*)rc_trajectory<2, 2, false, TIMED>;
+        case 5: return (const void*)rc_trajectory<2, 2, true, TIMED>;
+        case 6: return (const void*)rc_trajectory<3, 3, false, TIMED>;
+        case 7: return (const void*)rc_trajectory<3, 3, true, TIMED>;
+        case 8: return (const void*)rc_trajectory<4, 4, false, TIMED>;
+        case 9: return (const void*)rc_trajectory<4, 4, true, TIMED>;
         default: return nullptr;
     }
 }
+// z2: every state of the launch is Z2-symmetric with whole-tile parity blocks
+static const void* trajectory_fn(int nb, int split, int z2, int timed) {
+    return timed ? trajectory_fn<true>(nb, split, z2) : trajectory_fn<false>(nb, split, z2);
+}
 
 // workgroups of the trajectory kernel that can be resident at once on the current device
-hipError_t rc_trajectory_capacity(int nb, int split, int* blocks) {
-    const void* fn = trajectory_fn(nb, split);
+hipError_t rc_trajectory_capacity(int nb, int split, int z2, int timed, int* blocks) {
+    const void* fn = trajectory_fn(nb, split, z2, timed);
     if (!fn) return hipErrorInvalidValue;
     const int bytes = rc_trajectory_smem_bytes(nb, split);
     hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
@@ -1015,12 +1076,20 @@ hipError_t rc_trajectory_capacity(int nb, int split, int* blocks) {
     return hipSuccess;
 }
 
-hipError_t rc_launch_trajectory(int nb, int split, int nblocks, const TrajParams* dparams, hipStream_t stream) {
+hipError_t rc_launch_trajectory(int nb, int split, int z2, int timed, int nblocks, const TrajParams* dparams, hipStream_t stream) {
     void* args[] = {(void*)&dparams};
-    const void* fn = trajectory_fn(nb, split);
+    const void* fn = trajectory_fn(nb, split, z2, timed);
     const int bytes = rc_trajectory_smem_bytes(nb, split);
     if (!fn) return hipErrorInvalidValue;
     hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (e != hipSuccess) return e;
     return hipLaunchCooperativeKernel(fn, dim3(nblocks), dim3(256), args, (unsigned)bytes, stream);
+}
+
+hipError_t rc_launch_fill_empty(void* dst, size_t bytes, hipStream_t stream) {
+    const long long n = (long long)(bytes / 16);
+    const long long blocks = (n + 1023) / 1024;
+    hipLaunchKernelGGL(rc_fill_empty, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(256), 0, stream,
+                       static_cast<v4u*>(dst), n);
+    return hipGetLastError();
 }
