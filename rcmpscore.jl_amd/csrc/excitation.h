@@ -29,6 +29,7 @@ __host__ __device__ inline int rc_qmats(int nb) { return 2 * RC_QCH + 2 * nb; }
 struct RcQuarticArgs {
     int Dp, na;
     const double* U;
+    double* P;            // level-1 matrices, in the layout of U
     double* F;
     const double *Q, *Qh, *Qs, *Qhs, *R, *Rh, *Vrep, *Wrep;
     long long qstride;    // complex stride between the tangents' Qs (and Qhs); 0 when shared
@@ -50,6 +51,7 @@ struct RcQuarticArgs {
     const int* active;    // device flag: the launch does nothing when it reads 0 (null: always runs)
 };
 
+__global__ void rc_quartic_p(RcQuarticArgs g);
 __global__ void rc_quartic_rhs(RcQuarticArgs g);
 
 // arguments of rc_pair_rhs: pair p's state at U + p ustride (matrix (channel c, block k) at (4 c + k)
@@ -125,14 +127,15 @@ struct RcOdeCtl {
 struct RcOdeRun {
     RcQuarticArgs g;           // the right-hand side's operands (U, F, epilogue fields unused)
     double* ybuf;              // [N] the state at entry, the end state on exit
-    double* u0;                // [N] stage inputs exchanged between workgroups (two buffers)
-    double* u1;
-    double* slots;             // [nwg][2] per-tile error sums
-    uint32_t* flags;           // [nwg] per-workgroup event counters, zero at entry
+    // exchange rings, every slot empty at entry: stage inputs in two orders and P tiles, each
+    // [RC_RING][matrices][Dp*Dp] complex, then error sums [RC_REC_RING][nslots] pairs
+    double* exch;
+    uint32_t exch_bytes;
+    int nslots;                // tiles of every matrix
     double* Sf;                // samples, as OdeWork
     double* Sa;
     long long N, half;
-    int nwg, ntrack, nranges, pad;
+    int ntrack, nranges;
     const int* ranges;
     const double* stops;
     const int* stop_node;
@@ -144,10 +147,10 @@ struct RcOdeRun {
     double* out;               // [8] status, attempts, accepted, rejected; workgroup 0's clock ticks in
                                // the products, the exchanges, the controller and the whole launch
 };
-__global__ void rc_quartic_ode(const RcOdeRun* pp);
-#define RC_QUARTIC_ODE_MAX_WG 256   // workgroups one exchange round of rc_quartic_ode polls
-hipError_t rc_quartic_ode_capacity(int* blocks);
-hipError_t rc_launch_quartic_ode(dim3 grid, const RcOdeRun* dparams, hipStream_t stream);
+// z2: only the tiles of the parity blocks that can be nonzero have a workgroup (g.zt > 0)
+hipError_t rc_quartic_ode_capacity(int nb, int z2, int nslots, int ntrack, int* blocks);
+hipError_t rc_launch_quartic_ode(int nb, int z2, int nwg, int nslots, int ntrack, const RcOdeRun* dparams,
+                                 hipStream_t stream);
 __global__ void rc_ode_step(RcOdeCtl* c, int finish, const double* partial, const int* ranges, int nranges,
                             int ntrack, double cnt, const double* stops, const int* stop_node, const double* cheb,
                             double* cf);

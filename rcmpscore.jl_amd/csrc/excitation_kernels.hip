@@ -1,7 +1,10 @@
 // Device kernels of the tangent-space excitation action: the momentum-shifted no-jump
 // preconditioner, Gram-Schmidt over sets of Arnoldi bases, the fused right-hand side of the :phi^4:
 // action ODEs, DOP853 stage combinations and error norms, and batched trace products.
+#include <algorithm>
+
 #include "device_common.h"
+#include "exchange.h"
 #include "excitation.h"
 #include "trajectory.h"
 
@@ -111,8 +114,9 @@ __global__ void rc_stage(long long N, const double* y, const double* K, long lon
 // worst over trajectories; accept or reject and the next step size.  Then, unless done, set up the
 // next attempt: the step clipped at the next stop (a quadrature node, 0 or the window's end) and the
 // source coefficients [2|t_s|, s(t_s)] of stages 1..12 (one thread each) with the step at cf[26].
-// The controller step shared by rc_ode_step and the persistent launch (c in device or LDS memory; C:
-// the error partials are read with device-coherent loads).  No barrier after the cf writes.
+// The controller step shared by rc_ode_step and the persistent launch (C: c and every operand in LDS,
+// barriers that order LDS only; stops[0], stops[1] and stop_node[0] are the stop c->si, the one after
+// it and its node).  No barrier after the cf writes.
 template <bool C>
 __device__ __forceinline__ void ode_step_body(RcOdeCtl* c, int finish, const double* partial, const int* ranges,
                                               int nranges, int ntrack, double cnt, const double* stops,
@@ -132,14 +136,8 @@ __device__ __forceinline__ void ode_step_body(RcOdeCtl* c, int finish, const dou
             for (int r = 0; r < nranges; ++r) {
                 const int first = ranges[2 * (tr * nranges + r)], count = ranges[2 * (tr * nranges + r) + 1];
                 for (int q = lane; q < count; q += 64) {
-                    if constexpr (C) {
-                        e5 += __hip_atomic_load(partial + 2 * (first + q), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        e3 += __hip_atomic_load(partial + 2 * (first + q) + 1, __ATOMIC_RELAXED,
-                                                __HIP_MEMORY_SCOPE_AGENT);
-                    } else {
-                        e5 += partial[2 * (first + q)];
-                        e3 += partial[2 * (first + q) + 1];
-                    }
+                    e5 += partial[2 * (first + q)];
+                    e3 += partial[2 * (first + q) + 1];
                 }
             }
 #pragma unroll
@@ -157,9 +155,11 @@ __device__ __forceinline__ void ode_step_body(RcOdeCtl* c, int finish, const dou
             sbad[wave] = bad;
         }
     }
-    __syncthreads();
+    if constexpr (C) lds_barrier();
+    else __syncthreads();
     if (tid == 0) {
         s_go = 0;
+        int moved = 0;   // the step reached its stop
         if (judge) {
             const double err = fmax(fmax(smax[0], smax[1]), fmax(smax[2], smax[3]));
             const int bad = sbad[0] | sbad[1] | sbad[2] | sbad[3];
@@ -173,13 +173,14 @@ __device__ __forceinline__ void ode_step_body(RcOdeCtl* c, int finish, const dou
                 c->accepted += 1;
                 c->commit = 1;
                 c->t = c->tn;
-                if (c->t == stops[c->si]) {
-                    const int nd = stop_node[c->si];
+                if (c->t == stops[C ? 0 : c->si]) {
+                    const int nd = stop_node[C ? 0 : c->si];
                     if (nd >= 0) {
                         c->sample = nd;
                         c->node = nd + 1;
                     }
                     c->si += 1;
+                    moved = 1;
                 }
                 double factor = err == 0 ? 10.0 : fmin(10.0, 0.9 * pow(err, -1.0 / 8));
                 if (c->last_rejected) factor = fmin(1.0, factor);
@@ -198,7 +199,7 @@ __device__ __forceinline__ void ode_step_body(RcOdeCtl* c, int finish, const dou
         }
         c->active = 0;
         if (!c->done) {
-            const double t = c->t, h = c->h, stop = stops[c->si];
+            const double t = c->t, h = c->h, stop = stops[C ? moved : c->si];
             double he = fmin(h, stop - t);
             const int clipped = he < h;
             if (stop - t - he <= 1e-14 * fmax(1.0, fabs(stop))) he = stop - t;
@@ -221,7 +222,8 @@ __device__ __forceinline__ void ode_step_body(RcOdeCtl* c, int finish, const dou
             }
         }
     }
-    __syncthreads();
+    if constexpr (C) lds_barrier();
+    else __syncthreads();
     if (s_go && tid >= 1 && tid < 13) {
         const double ts = tid < 12 ? s_t + RC_C[tid] * s_he : s_tn;
         cf[2 * tid] = 2 * fabs(ts);
@@ -262,7 +264,7 @@ __global__ void rc_ode_stage(const RcOdeCtl* c, long long N, long long half, dou
         yi = reinterpret_cast<const cplx*>(y)[i];
         ki = reinterpret_cast<const cplx*>(K0)[i];
     }
-    if (active) reinterpret_cast<cplx*>(U1)[i] = cadd(yi, cscale(hp[0], cscale(a10, ki)));
+    if (active) reinterpret_cast<cplx*>(U1)[i] = cfma(hp[0], cscale(a10, ki), yi);
 }
 
 // Resolvent step in the transfer's eigenbasis: out[v][k] = Y[src(v)][k] / (1 - z_i (mu_k + i s_b)) for
@@ -450,10 +452,11 @@ __global__ void rc_trace_axpy_n(int n, int nj, int nodes, const double* tr, cons
 }
 
 // ---------------------------------------------------------------------------------------------
-// One right-hand side of the :phi^4: action ODEs (forward and adjoint, every tangent and channel)
-// in a single launch.  Workgroup = one 16 x 16 output tile of one derivative matrix; all products
-// of that tile accumulate in one MFMA accumulator (k split across the 4 waves), the two-sided
-// products A X B through a Dp x 16 column block X B[:, tile] staged in LDS.
+// One right-hand side of the :phi^4: action ODEs (forward and adjoint, every tangent and channel) in
+// two launches, the graph route's (rc_quartic_ode has both levels in one persistent launch).
+// Workgroup = one 16 x 16 tile of one matrix; the products of a tile accumulate in one MFMA accumulator
+// (k split across the 4 waves).  rc_quartic_p forms P, the inner factor of the two-sided products and
+// the neighbour channel's one-sided insertion; rc_quartic_rhs the rest.
 //   forward  dx_k = jac (Q x + x Q^+ + R x R^+) + k jt (R x_{k-1} + x_{k-1} R^+)
 //            dy_k = jac (Qs y + y Q^+ + R y R^+ + v x + w x R^+) + k jt (R y_{k-1} + y_{k-1} R^+ + w x_{k-1})
 //   adjoint  da0_k = jac (Qhs a0 + a0 Q + R^+ (a0 R + a1 w) + a1 v) + (k+1) jt (a0 R + a1 w + R^+ a0)_{k+1}
@@ -465,35 +468,16 @@ namespace {
 // Every fragment of this wave's k-steps (Dp / 16 of them, at most 4) is loaded before the first MFMA,
 // so a product pays one load round trip instead of one per k-step; the MFMAs run in the same k order.
 // Wave w runs k-step w + 4 i of k-tile i.  kmask (uniform) selects the k-tiles: bit i for k-tile i.
-// The stage input as a buffer resource (device-coherent 16-byte loads of the elements another
-// workgroup of the same launch wrote; offsets outside it read zero).
-struct QCoh {
-    __amdgpu_buffer_rsrc_t r;
-    const cplx* base;
-};
-
-// An operand element; C: a device-coherent load from the stage input q.
-template <bool C>
-__device__ __forceinline__ cplx qld(const QCoh* q, const cplx* p) {
-    if constexpr (C) {
-        return ld_coh(q->r, (uint32_t)((p - q->base) * (long long)sizeof(cplx)));
-    } else {
-        (void)q;
-        return *p;
-    }
-}
-
-template <bool CA = false, bool CB = false>
 __device__ __forceinline__ void qprod(cacc& acc, const cplx* A, const cplx* B, int Dp, int bi, int bj, int wave,
-                                      int lane, double scale, int kmask = 15, const QCoh* q = nullptr) {
+                                      int lane, double scale, int kmask = 15) {
     const int nk = Dp / 16;
     cplx a[4], b[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
         if (i < nk && ((kmask >> i) & 1)) {
             const int kk = 4 * (wave + 4 * i) + (lane >> 4);
-            a[i] = qld<CA>(q, &A[(16 * bi + (lane & 15)) * Dp + kk]);
-            b[i] = qld<CB>(q, &B[kk * Dp + 16 * bj + (lane & 15)]);
+            a[i] = A[(16 * bi + (lane & 15)) * Dp + kk];
+            b[i] = B[kk * Dp + 16 * bj + (lane & 15)];
         }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -540,18 +524,15 @@ __device__ __forceinline__ cplx qreduce(const cacc& acc, cplx* red, int wave, in
 }
 
 // One wave's whole product A(bi, :) B(:, bj) over every k-step (no cross-wave reduction), one k-tile of
-// fragments loaded ahead of its four MFMAs; kmask selects the k-tiles (bit t: k-steps 4t .. 4t + 3).
-template <bool CA = false>
-__device__ __forceinline__ void qprod_rows(cacc& acc, const cplx* A, const cplx* B, int Dp, int bi, int bj, int lane,
-                                           int kmask, const QCoh* q = nullptr) {
+// fragments loaded ahead of its four MFMAs.
+__device__ __forceinline__ void qprod_rows(cacc& acc, const cplx* A, const cplx* B, int Dp, int bi, int bj, int lane) {
     const int nk = Dp / 16;
     for (int t = 0; t < nk; ++t) {
-        if (!((kmask >> t) & 1)) continue;
         cplx a[4], b[4];
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             const int kk = 16 * t + 4 * s + (lane >> 4);
-            a[s] = qld<CA>(q, &A[(16 * bi + (lane & 15)) * Dp + kk]);
+            a[s] = A[(16 * bi + (lane & 15)) * Dp + kk];
             b[s] = B[kk * Dp + 16 * bj + (lane & 15)];
         }
 #pragma unroll
@@ -559,19 +540,17 @@ __device__ __forceinline__ void qprod_rows(cacc& acc, const cplx* A, const cplx*
     }
 }
 
-// one term X B[:, bj] of an LDS column block, with the operands' Z2 parities (X null: no term)
+// one term X B[:, bj] of an LDS column block (X null: no term)
 struct QTerm {
     const cplx* X;
     const cplx* B;
-    int pa, pb;
 };
 
 // Column blocks (Dp x 16, in LDS) T0 = a0 + a1 and, when T1 is given, T1 = b0 + b1.  The row tiles of
 // both blocks are spread over the waves, each wave running every k-step of its row tiles and writing
-// them straight to LDS; one barrier at the end.  zt: Z2 parity blocks (0: every k-tile).
-template <bool CX = false>
+// them straight to LDS; one barrier at the end.
 __device__ __forceinline__ void qcolumns(cplx* T0, QTerm a0, QTerm a1, cplx* T1, QTerm b0, QTerm b1, int Dp, int bj,
-                                         int wave, int lane, int zt, const QCoh* qc = nullptr) {
+                                         int wave, int lane) {
     const int nbt = Dp / 16, ntask = (T1 ? 2 : 1) * nbt;
     for (int i = wave; i < ntask; i += 4) {
         const int col = i / nbt, rt = i % nbt;
@@ -579,8 +558,8 @@ __device__ __forceinline__ void qcolumns(cplx* T0, QTerm a0, QTerm a1, cplx* T1,
         cplx* T = col ? T1 : T0;
         cacc acc;
         cacc_zero(acc);
-        qprod_rows<CX>(acc, p.X, p.B, Dp, rt, bj, lane, zmask(zt, nbt, rt, bj, p.pa, p.pb), qc);
-        if (q.X) qprod_rows<CX>(acc, q.X, q.B, Dp, rt, bj, lane, zmask(zt, nbt, rt, bj, q.pa, q.pb), qc);
+        qprod_rows(acc, p.X, p.B, Dp, rt, bj, lane);
+        if (q.X) qprod_rows(acc, q.X, q.B, Dp, rt, bj, lane);
 #pragma unroll
         for (int e = 0; e < 4; ++e) T[(16 * rt + 4 * e + (lane >> 4)) * 16 + (lane & 15)] = cacc_get(acc, e);
     }
@@ -589,225 +568,388 @@ __device__ __forceinline__ void qcolumns(cplx* T0, QTerm a0, QTerm a1, cplx* T1,
 
 }  // namespace
 
-// One right-hand-side tile of the :phi^4: action ODE (the products of rc_quartic_rhs for output tile
-// (bi, bj) of matrix mi = blockIdx.y, reduced over the waves): thread t receives element (t/16, t%16).
-// U: the stage input; C: its elements are read with device-coherent loads (another workgroup of the
-// same launch wrote them).
-template <bool C>
-__device__ __forceinline__ cplx quartic_tile(const RcQuarticArgs& g, const cplx* U, double jac, double jt, int bi,
-                                             int bj, int mi, cplx* red, cplx* T1, cplx* T2) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int Dp = g.Dp;
-    const int nb = g.na * RC_QCH;
-    // block, tangent and channel of matrix mi (rc_qmat's inverse; the shared blocks 0 and 3 take a = 0)
-    int blk, a, k;
+// block, tangent and channel of matrix mi (rc_qmat's inverse; the shared blocks 0 and 3 take a = 0)
+__device__ __forceinline__ void qmat_of(int mi, int nb, int& blk, int& a, int& k) {
     if (mi < RC_QCH) { blk = 0; a = 0; k = mi; }
     else if (mi < RC_QCH + nb) { blk = 1; a = (mi - RC_QCH) / RC_QCH; k = (mi - RC_QCH) % RC_QCH; }
     else if (mi < RC_QCH + 2 * nb) { blk = 2; a = (mi - RC_QCH - nb) / RC_QCH; k = (mi - RC_QCH - nb) % RC_QCH; }
     else { blk = 3; a = 0; k = mi - RC_QCH - 2 * nb; }
-    const long long m = (long long)Dp * Dp;
-    auto mat = [&](int b, int ch) { return U + (long long)rc_qmat(b, a, ch, nb) * m; };
-    const cplx* Q = reinterpret_cast<const cplx*>(g.Q);
-    const cplx* Qh = reinterpret_cast<const cplx*>(g.Qh);
-    const cplx* Qs = reinterpret_cast<const cplx*>(g.Qs) + (long long)a * g.qstride;     // tangent's momentum
-    const cplx* Qhs = reinterpret_cast<const cplx*>(g.Qhs) + (long long)a * g.qstride;
-    const cplx* R = reinterpret_cast<const cplx*>(g.R);
-    const cplx* Rh = reinterpret_cast<const cplx*>(g.Rh);
-    const cplx* v = reinterpret_cast<const cplx*>(g.Vrep) + (long long)a * 5 * m;
-    const cplx* w = reinterpret_cast<const cplx*>(g.Wrep) + (long long)a * 5 * m;
-    // Z2 parities (g.zt > 0): Q, Q^+ and the shifted ones even, R, R^+ odd, w = W of parity pw,
-    // v = -R^+ W of parity pw ^ 1; channels x_k and a1_k of parity k & 1 (x_0 = rho, a1 of the last
-    // channel = I), y_k and a0_k of parity (k + 1 + pw) & 1 (y_0 = R W, a0 driven by a1 w and a1 v)
-    const int zt = g.zt, nk = Dp / 16, pw = g.wpar;
-    const int px = k & 1, py = (k + 1 + pw) & 1;
-    auto zm = [&](int pa, int pb) { return zmask(zt, nk, bi, bj, pa, pb); };
-    const QCoh qc{rc_rsrc(U, (uint32_t)((long long)rc_qmats(nb) * m * (long long)sizeof(cplx))), U};
+}
+
+// Operands of tile (bi, bj) of matrix mi: the constant matrices, the tangent's, the stage input's and the
+// level-1 matrices' of this channel and of its neighbour, whose insertion it takes; Z2 parities and
+// k-tile masks (see RcQuarticArgs).  Parities for g.zt > 0: Q, Q^+ and the shifted ones even, R, R^+
+// odd, w = W of parity pw, v = -R^+ W of parity pw ^ 1; channels x_k and a1_k of parity k & 1 (x_0 =
+// rho, a1 of the last channel = I), y_k and a0_k of parity (k + 1 + pw) & 1 (y_0 = R W, a0 driven by
+// a1 w and a1 v).
+struct QTile {
+    int Dp, bi, bj, blk, a, k, nb, zt, nk, pw, px, py, lane, wave;
+    long long m;
+    const cplx *Q, *Qh, *Qs, *Qhs, *R, *Rh, *v, *w;
+    __device__ __forceinline__ QTile(const RcQuarticArgs& g) {
+        lane = threadIdx.x & 63;
+        wave = threadIdx.x >> 6;
+        Dp = g.Dp;
+        nk = Dp / 16;
+        bi = blockIdx.x / nk;
+        bj = blockIdx.x % nk;
+        nb = g.na * RC_QCH;
+        qmat_of(blockIdx.y, nb, blk, a, k);
+        m = (long long)Dp * Dp;
+        Q = reinterpret_cast<const cplx*>(g.Q);
+        Qh = reinterpret_cast<const cplx*>(g.Qh);
+        Qs = reinterpret_cast<const cplx*>(g.Qs) + (long long)a * g.qstride;
+        Qhs = reinterpret_cast<const cplx*>(g.Qhs) + (long long)a * g.qstride;
+        R = reinterpret_cast<const cplx*>(g.R);
+        Rh = reinterpret_cast<const cplx*>(g.Rh);
+        v = reinterpret_cast<const cplx*>(g.Vrep) + (long long)a * 5 * m;
+        w = reinterpret_cast<const cplx*>(g.Wrep) + (long long)a * 5 * m;
+        zt = g.zt;
+        pw = g.wpar;
+        px = k & 1;
+        py = (k + 1 + pw) & 1;
+    }
+    __device__ __forceinline__ const cplx* mat(const cplx* U, int b, int ch) const {
+        return U + (long long)rc_qmat(b, a, ch, nb) * m;
+    }
+    // acc += scale A(bi, :) B(:, bj), operands of parities pa, pb
+    __device__ __forceinline__ void add(cacc& acc, double scale, const cplx* A, int pa, const cplx* B, int pb) const {
+        qprod(acc, A, B, Dp, bi, bj, wave, lane, scale, zmask(zt, nk, bi, bj, pa, pb));
+    }
+    __device__ __forceinline__ long long element() const {
+        return (long long)blockIdx.y * m + (16 * bi + (threadIdx.x >> 4)) * Dp + 16 * bj + (threadIdx.x & 15);
+    }
+};
+
+// Level 1 of a right-hand side: the tiles of P (x R^+, y R^+, a0 R + a1 w, a1 R).
+__global__ void __launch_bounds__(256) rc_quartic_p(RcQuarticArgs g) {
+    __shared__ cplx red[1024];
+    if (g.active && !*g.active) return;
+    const QTile q(g);
+    const cplx* U = reinterpret_cast<const cplx*>(g.U);
+    cacc acc;
+    cacc_zero(acc);
+    if (q.blk == 0) q.add(acc, 1.0, q.mat(U, 0, q.k), q.px, q.Rh, 1);
+    else if (q.blk == 1) q.add(acc, 1.0, q.mat(U, 1, q.k), q.py, q.Rh, 1);
+    else if (q.blk == 2) {
+        q.add(acc, 1.0, q.mat(U, 2, q.k), q.py, q.R, 1);
+        q.add(acc, 1.0, q.mat(U, 3, q.k), q.px, q.w, q.pw);
+    } else q.add(acc, 1.0, q.mat(U, 3, q.k), q.px, q.R, 1);
+    reinterpret_cast<cplx*>(g.P)[q.element()] = qreduce(acc, red, q.wave, q.lane);
+}
+
+// Level 2: the one-sided products, then R P (and w P^x), then the insertion's P tile; thread t receives
+// element (t/16, t%16).  The order of the sums is rc_quartic_ode's.
+__device__ __forceinline__ cplx quartic_tile(const RcQuarticArgs& g, const QTile& q, double jac, double jt, cplx* red) {
+    const cplx* U = reinterpret_cast<const cplx*>(g.U);
+    const cplx* P = reinterpret_cast<const cplx*>(g.P);
+    const int blk = q.blk, k = q.k, px = q.px, py = q.py, pw = q.pw;
+    const double c = (blk < 2 ? k : k + 1) * jt;
+    const bool nbr = blk < 2 ? k >= 1 : k <= 3;   // the channel has an insertion
+    const int kn = blk < 2 ? k - 1 : k + 1;
     cacc acc;
     cacc_zero(acc);
     if (blk == 0) {
-        const cplx* x = mat(0, k);
-        if (jac != 0.0) {
-            qprod<false, C>(acc, Q, x, Dp, bi, bj, wave, lane, jac, zm(0, px), &qc);
-            qprod<C, false>(acc, x, Qh, Dp, bi, bj, wave, lane, jac, zm(px, 0), &qc);
-            qcolumns<C>(T1, QTerm{x, Rh, px, 1}, QTerm{}, nullptr, QTerm{}, QTerm{}, Dp, bj, wave, lane, zt, &qc);
-            qprod_t(acc, R, T1, Dp, bi, wave, lane, jac, zm(1, px ^ 1));
-        }
-        if (k >= 1) {
-            const cplx* xp = mat(0, k - 1);
-            qprod<false, C>(acc, R, xp, Dp, bi, bj, wave, lane, k * jt, zm(1, px ^ 1), &qc);
-            qprod<C, false>(acc, xp, Rh, Dp, bi, bj, wave, lane, k * jt, zm(px ^ 1, 1), &qc);
-        }
+        const cplx* x = q.mat(U, 0, k);
+        q.add(acc, jac, q.Q, 0, x, px);
+        q.add(acc, jac, x, px, q.Qh, 0);
+        if (nbr) q.add(acc, c, q.R, 1, q.mat(U, 0, kn), px ^ 1);
+        q.add(acc, jac, q.R, 1, q.mat(P, 0, k), px ^ 1);
     } else if (blk == 1) {
-        const cplx* y = mat(1, k);
-        const cplx* x = mat(0, k);
-        if (jac != 0.0) {
-            qprod<false, C>(acc, Qs, y, Dp, bi, bj, wave, lane, jac, zm(0, py), &qc);
-            qprod<C, false>(acc, y, Qh, Dp, bi, bj, wave, lane, jac, zm(py, 0), &qc);
-            qprod<false, C>(acc, v, x, Dp, bi, bj, wave, lane, jac, zm(pw ^ 1, px), &qc);
-            qcolumns<C>(T1, QTerm{y, Rh, py, 1}, QTerm{}, T2, QTerm{x, Rh, px, 1}, QTerm{}, Dp, bj, wave, lane, zt, &qc);
-            qprod_t(acc, R, T1, Dp, bi, wave, lane, jac, zm(1, py ^ 1));
-            qprod_t(acc, w, T2, Dp, bi, wave, lane, jac, zm(pw, px ^ 1));
+        const cplx* y = q.mat(U, 1, k);
+        q.add(acc, jac, q.Qs, 0, y, py);
+        q.add(acc, jac, y, py, q.Qh, 0);
+        q.add(acc, jac, q.v, pw ^ 1, q.mat(U, 0, k), px);
+        if (nbr) {
+            q.add(acc, c, q.R, 1, q.mat(U, 1, kn), py ^ 1);
+            q.add(acc, c, q.w, pw, q.mat(U, 0, kn), px ^ 1);
         }
-        if (k >= 1) {
-            const cplx* yp = mat(1, k - 1);
-            const cplx* xp = mat(0, k - 1);
-            qprod<false, C>(acc, R, yp, Dp, bi, bj, wave, lane, k * jt, zm(1, py ^ 1), &qc);
-            qprod<C, false>(acc, yp, Rh, Dp, bi, bj, wave, lane, k * jt, zm(py ^ 1, 1), &qc);
-            qprod<false, C>(acc, w, xp, Dp, bi, bj, wave, lane, k * jt, zm(pw, px ^ 1), &qc);
-        }
+        q.add(acc, jac, q.R, 1, q.mat(P, 1, k), py ^ 1);
+        q.add(acc, jac, q.w, pw, q.mat(P, 0, k), px ^ 1);
     } else if (blk == 2) {
-        const cplx* a0 = mat(2, k);
-        const cplx* a1 = mat(3, k);
-        if (jac != 0.0) {
-            qprod<false, C>(acc, Qhs, a0, Dp, bi, bj, wave, lane, jac, zm(0, py), &qc);
-            qprod<C, false>(acc, a0, Q, Dp, bi, bj, wave, lane, jac, zm(py, 0), &qc);
-            qprod<C, false>(acc, a1, v, Dp, bi, bj, wave, lane, jac, zm(px, pw ^ 1), &qc);
-            qcolumns<C>(T1, QTerm{a0, R, py, 1}, QTerm{a1, w, px, pw}, nullptr, QTerm{}, QTerm{}, Dp, bj, wave, lane, zt, &qc);
-            qprod_t(acc, Rh, T1, Dp, bi, wave, lane, jac, zm(1, py ^ 1));
-        }
-        if (k <= 3) {
-            const double c = (k + 1) * jt;
-            const cplx* a0n = mat(2, k + 1);
-            const cplx* a1n = mat(3, k + 1);
-            qprod<C, false>(acc, a0n, R, Dp, bi, bj, wave, lane, c, zm(py ^ 1, 1), &qc);
-            qprod<C, false>(acc, a1n, w, Dp, bi, bj, wave, lane, c, zm(px ^ 1, pw), &qc);
-            qprod<false, C>(acc, Rh, a0n, Dp, bi, bj, wave, lane, c, zm(1, py ^ 1), &qc);
-        }
+        const cplx* a0 = q.mat(U, 2, k);
+        q.add(acc, jac, q.Qhs, 0, a0, py);
+        q.add(acc, jac, a0, py, q.Q, 0);
+        q.add(acc, jac, q.mat(U, 3, k), px, q.v, pw ^ 1);
+        if (nbr) q.add(acc, c, q.Rh, 1, q.mat(U, 2, kn), py ^ 1);
+        q.add(acc, jac, q.Rh, 1, q.mat(P, 2, k), py ^ 1);
     } else {
-        const cplx* a1 = mat(3, k);
-        if (jac != 0.0) {
-            qprod<false, C>(acc, Qh, a1, Dp, bi, bj, wave, lane, jac, zm(0, px), &qc);
-            qprod<C, false>(acc, a1, Q, Dp, bi, bj, wave, lane, jac, zm(px, 0), &qc);
-            qcolumns<C>(T1, QTerm{a1, R, px, 1}, QTerm{}, nullptr, QTerm{}, QTerm{}, Dp, bj, wave, lane, zt, &qc);
-            qprod_t(acc, Rh, T1, Dp, bi, wave, lane, jac, zm(1, px ^ 1));
-        }
-        if (k <= 3) {
-            const double c = (k + 1) * jt;
-            const cplx* a1n = mat(3, k + 1);
-            qprod<C, false>(acc, a1n, R, Dp, bi, bj, wave, lane, c, zm(px ^ 1, 1), &qc);
-            qprod<false, C>(acc, Rh, a1n, Dp, bi, bj, wave, lane, c, zm(1, px ^ 1), &qc);
-        }
+        const cplx* a1 = q.mat(U, 3, k);
+        q.add(acc, jac, q.Qh, 0, a1, px);
+        q.add(acc, jac, a1, px, q.Q, 0);
+        if (nbr) q.add(acc, c, q.Rh, 1, q.mat(U, 3, kn), px ^ 1);
+        q.add(acc, jac, q.Rh, 1, q.mat(P, 3, k), px ^ 1);
     }
-    (void)tid;
-    return qreduce(acc, red, wave, lane);
+    cplx ins = cmake(0, 0);
+    if (nbr) ins = q.mat(P, blk, kn)[q.element() - (long long)blockIdx.y * q.m];
+    const cplx val = qreduce(acc, red, q.wave, q.lane);
+    return nbr ? cfma(c, ins, val) : val;
+}
+
+// This tile's part of the error sums, |r|^2 / sc^2 of the thread's element summed over the workgroup:
+// the waves' sums in order (thread 0 holds them); s: 8 doubles of LDS, `sync` a workgroup barrier
+__device__ __forceinline__ void tile_error_put(cplx r5, cplx r3, double sc, double* s, int wave, int lane) {
+    const double e5 = wave_sum(fma(r5.re, r5.re, r5.im * r5.im) / (sc * sc));
+    const double e3 = wave_sum(fma(r3.re, r3.re, r3.im * r3.im) / (sc * sc));
+    if (lane == 0) {
+        s[wave] = e5;
+        s[4 + wave] = e3;
+    }
+}
+__device__ __forceinline__ cplx tile_error_sum(const double* s) {
+    return cmake(((s[0] + s[1]) + s[2]) + s[3], ((s[4] + s[5]) + s[6]) + s[7]);
 }
 
 __global__ void __launch_bounds__(256) rc_quartic_rhs(RcQuarticArgs g) {
     __shared__ cplx red[1024];
-    __shared__ cplx T1[64 * 16];
-    __shared__ cplx T2[64 * 16];
     if (g.active && !*g.active) return;
     const int tid = threadIdx.x;
-    const int Dp = g.Dp, nbt = Dp / 16, bi = blockIdx.x / nbt, bj = blockIdx.x % nbt;
-    const int mi = blockIdx.y;
-    const long long m = (long long)Dp * Dp;
+    const QTile q(g);
+    const int nbt = q.nk, mi = blockIdx.y;
     const cplx* U = reinterpret_cast<const cplx*>(g.U);
     const double jac = g.coef ? g.coef[0] : g.jac;
     const double jt = g.coef ? g.coef[1] : g.jt;
-    const cplx val = quartic_tile<false>(g, U, jac, jt, bi, bj, mi, red, T1, T2);
-    const long long e = (long long)mi * m + (16 * bi + (tid >> 4)) * Dp + 16 * bj + (tid & 15);
+    const cplx val = quartic_tile(g, q, jac, jt, red);
+    const long long e = q.element();
     reinterpret_cast<cplx*>(g.F)[e] = val;
     if (g.epi == 0) return;
     const cplx* Kc = reinterpret_cast<const cplx*>(g.K);
     const cplx y0 = reinterpret_cast<const cplx*>(g.y)[e];
     if (g.epi == 1) {
         const double h = g.hp ? g.hp[0] : g.h;
-        cplx sum = cscale(g.comb.a[g.stage], val);
+        cplx sum = cmake(0, 0);
         for (int j = 0; j < g.stage; ++j)
-            if (g.comb.a[j] != 0.0) sum = cadd(sum, cscale(g.comb.a[j], Kc[(long long)j * g.sk + e]));
-        reinterpret_cast<cplx*>(g.Unext)[e] = cadd(y0, cscale(h, sum));
+            if (g.comb.a[j] != 0.0) sum = cfma(g.comb.a[j], Kc[(long long)j * g.sk + e], sum);
+        reinterpret_cast<cplx*>(g.Unext)[e] = cfma(h, cfma(g.comb.a[g.stage], val, sum), y0);
         return;
     }
-    cplx r5 = cscale(g.comb.a[g.stage], val), r3 = cscale(g.comb3.a[g.stage], val);
+    cplx r5 = cmake(0, 0), r3 = cmake(0, 0);
     for (int j = 0; j < g.stage; ++j) {
         const cplx kj = Kc[(long long)j * g.sk + e];
-        if (g.comb.a[j] != 0.0) r5 = cadd(r5, cscale(g.comb.a[j], kj));
-        if (g.comb3.a[j] != 0.0) r3 = cadd(r3, cscale(g.comb3.a[j], kj));
+        if (g.comb.a[j] != 0.0) r5 = cfma(g.comb.a[j], kj, r5);
+        if (g.comb3.a[j] != 0.0) r3 = cfma(g.comb3.a[j], kj, r3);
     }
-    const double sc = g.atol + g.rtol * fmax(cabsd(y0), cabsd(U[e]));
-    double* s5 = reinterpret_cast<double*>(red);
-    double* s3 = s5 + 256;
-    s5[tid] = cabs2(r5) / (sc * sc);
-    s3[tid] = cabs2(r3) / (sc * sc);
+    r5 = cfma(g.comb.a[g.stage], val, r5);
+    r3 = cfma(g.comb3.a[g.stage], val, r3);
+    double* se = reinterpret_cast<double*>(red);
+    tile_error_put(r5, r3, g.atol + g.rtol * fmax(cabsd(y0), cabsd(U[e])), se, tid >> 6, tid & 63);
     __syncthreads();
-    for (int hh = 128; hh > 0; hh >>= 1) {
-        if (tid < hh) { s5[tid] += s5[tid + hh]; s3[tid] += s3[tid + hh]; }
-        __syncthreads();
-    }
     if (tid == 0) {
         const long long slot = (long long)mi * nbt * nbt + blockIdx.x;
-        g.partial[2 * slot] = s5[0];
-        g.partial[2 * slot + 1] = s3[0];
+        const cplx es = tile_error_sum(se);
+        g.partial[2 * slot] = es.re;
+        g.partial[2 * slot + 1] = es.im;
     }
 }
 
 // ---------------------------------------------------------------------------------------------
 // The whole :phi^4: action ODE integration in one persistent launch (cooperative: every workgroup
-// resident).  Workgroup (bi, bj, mi) owns the same 16 x 16 tile as in rc_quartic_rhs and keeps its
-// elements of y, of the stage derivatives K_0..K_12 (LDS) and of the step end in registers.  Each
-// stage input is exchanged through `ubuf` (two buffers, device-coherent stores and loads) with one
-// all-workgroup event per stage: every workgroup publishes its counter and waits for all others.  The
-// step controller runs redundantly in every workgroup on the same error partials (exchanged the same
-// way), so every workgroup takes the same decisions; the arithmetic is the graph path's, so the
-// results are the same bits.  Waits are bounded in wall time: a workgroup that outlasts the budget
-// sets the abort word and every workgroup leaves with RC_ST_WAIT_LIMIT.
+// resident), tiles exchanged between workgroups as in rc_trajectory (exchange.h): ring slots that are
+// empty until the value is stored, polling loads straight into MFMA fragments, constants in
+// registers, two barriers of the workgroup per right-hand side.
+//
+// Workgroup = one 16 x 16 tile of one matrix.  A right-hand side has two levels: level 1 forms the
+// tile of P (x R^+, y R^+, a0 R + a1 w, a1 R) and publishes it; the one-sided products of the stage
+// input and of the neighbour channel's follow while the P tiles travel; level 2 adds R P (and
+// w P^x) and the neighbour's P tile, which is its insertion.  The order of every sum is that of
+// rc_quartic_p and rc_quartic_rhs, so the two routes give the same bits.
+//
+// Z2 states (KT = NB / 2): the tiles that are exactly zero have no workgroup; the workgroup of tile
+// (bi, bj) also forms the P tile (bi, bj') of the other parity block, and products run half the
+// k-tiles.
+//
+// Step controller: every workgroup reads all tiles' error sums and runs ode_step_body on them, so
+// all take the same decision.  Ring: 12 events between two gathers, so at event e every reader is
+// done with event e - 16, which is emptied then and next used at e + 16.  Waits are bounded in wall
+// time: a workgroup that outlasts the budget sets the abort word and every workgroup leaves with
+// RC_ST_WAIT_LIMIT.
+//
+// What bounds it: the two exchanges (about 1.2 us each) around up to eight products of a tile.
 // ---------------------------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) rc_quartic_ode(const RcOdeRun* __restrict__ pp) {
-    __shared__ cplx red[1024];
-    __shared__ cplx T1[64 * 16];
-    __shared__ cplx T2[64 * 16];
-    __shared__ cplx sK[13][256];
-    __shared__ RcOdeCtl sc;
-    __shared__ double s_cf[32];
-    __shared__ int s_abort;
-    const RcOdeRun& p = *pp;
-    const RcQuarticArgs& g = p.g;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int Dp = g.Dp, nbt = Dp / 16, bi = blockIdx.x / nbt, bj = blockIdx.x % nbt, mi = blockIdx.y;
-    const int wg = mi * nbt * nbt + (int)blockIdx.x;   // also the tile's error slot
-    const long long m = (long long)Dp * Dp;
-    const long long e = (long long)mi * m + (16 * bi + (tid >> 4)) * Dp + 16 * bj + (tid & 15);
-    cplx* const u0 = reinterpret_cast<cplx*>(p.u0);
-    cplx* const u1 = reinterpret_cast<cplx*>(p.u1);
-    uint32_t ev = 0;
-    auto put = [&](int buf, cplx v) {
-        double* d = reinterpret_cast<double*>((buf ? u1 : u0) + e);
-        __hip_atomic_store(d, v.re, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(d + 1, v.im, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    };
-    // publish this workgroup's next event once its stores are complete, then wait until every
-    // workgroup has published it (wave 0 polls every counter in each round: lane l those of
-    // workgroups l, l + 64, l + 128, l + 192; at most 256 workgroups)
-    auto sync_all = [&]() -> bool {
-        ++ev;
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        if (tid == 0) st_flag(p.flags + wg, ev);
-        if (tid < 64) {
-            const uint64_t t0 = __builtin_amdgcn_s_memrealtime();
-            int bad = 0;
-            for (uint32_t polls = 1;; ++polls) {
-                uint32_t fv[4];
+// Combinations after stage s of the action ODE without their last term, over a window of 13 (k_j at
+// 13 - s + j before k_s enters): rows 1..10 the next stage input, 11 the step end, 12 and 13 the
+// error estimators after stage 12.
+struct RcOdeRows {
+    double c[14][13];
+};
+constexpr RcOdeRows rc_make_ode_rows() {
+    RcOdeRows r{};
+    for (int s = 1; s < 12; ++s)
+        for (int j = 0; j < s; ++j) r.c[s][13 - s + j] = s == 11 ? RC_B[j] : RC_A[s + 1][j];
+    for (int j = 0; j < 12; ++j) {
+        r.c[12][1 + j] = RC_E5[j];
+        r.c[13][1 + j] = RC_E3[j];
+    }
+    return r;
+}
+__constant__ const RcOdeRows rc_ode_rows = rc_make_ode_rows();
+
+__device__ __forceinline__ cplx ode_row_sum(int row, const cplx* k) {
+    const __attribute__((address_space(4))) double* c =
+        (const __attribute__((address_space(4))) double*)&rc_ode_rows.c[row][0];
+    cplx s = cmake(0, 0);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) fv[q] = lane + 64 * q < p.nwg ? ld_flag(p.flags + lane + 64 * q) : ev;
-                const uint32_t ab = ld_flag(p.abort_flag);
-                if (__all(fv[0] >= ev && fv[1] >= ev && fv[2] >= ev && fv[3] >= ev)) break;
-                if (ab) { bad = 1; break; }
-                if ((polls & 63) == 0 && (long long)(__builtin_amdgcn_s_memrealtime() - t0) > p.wait_ticks) {
-                    bad = 1;
-                    break;
-                }
-                __builtin_amdgcn_s_sleep(1);
-            }
-            if (lane == 0) {
-                if (bad) st_flag(p.abort_flag, 1u);
-                s_abort = bad;
-            }
+    for (int q = 0; q < 13; ++q) s = cfma(c[q], k[q], s);
+    return s;
+}
+
+// dynamic LDS: two levels of partial tiles, every tile's error sums, the trajectories' slot ranges (two
+// of two ints each)
+#define RC_ODE_LDS(nslots, ntrack) (2048 * 16 + (nslots) * 16 + (ntrack) * 16)
+
+#define RC_ODE_LDS_ALONE (84 * 1024)
+
+template <int NB, int KT>
+__global__ void __launch_bounds__(256, KT <= 2 ? 2 : 1) rc_quartic_ode(const RcOdeRun* __restrict__ pp) {
+    extern __shared__ __align__(16) unsigned char ode_lds[];
+    cplx* red1 = reinterpret_cast<cplx*>(ode_lds);
+    cplx* red2 = red1 + 1024;
+    double* s_slots = reinterpret_cast<double*>(red2 + 1024);
+    __shared__ RcOdeCtl sc;
+    __shared__ double s_cf[32], s_err[8], s_al[13], s_stops[2];
+    __shared__ double s_cheb[RC_SOURCE_SEGMENTS * (RC_SOURCE_DEGREE + 1)];
+    __shared__ int s_bad, s_stop, s_node;
+    const RcOdeRun& p = *pp;
+    // the slot ranges of the tracked trajectories, behind the error sums
+    int* s_ranges = reinterpret_cast<int*>(s_slots + 2 * p.nslots);
+    const RcQuarticArgs& g = p.g;
+    constexpr int Dp = 16 * NB, NT = NB * NB;
+    constexpr uint32_t TB = 4096;
+    const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
+    const int ei = tid >> 4, ej = tid & 15, fi = lane & 15, fk = 4 * wave + (lane >> 4);
+    const int nb = g.na * RC_QCH, nmat = rc_qmats(nb);
+    const int wg = blockIdx.x, mi = wg / (NB * KT), bi = wg / KT % NB, jj = wg % KT;
+    int blk, a, k;
+    qmat_of(mi, nb, blk, a, k);
+    // parities (all k-tiles when KT = NB): as quartic_tile
+    const int pw = g.wpar, px = k & 1, py = (k + 1 + pw) & 1, po = blk == 0 || blk == 3 ? px : py;
+    const int hb = KT < NB ? bi / KT : 0;                     // parity block of the row tile
+    auto kt0 = [&](int pa) { return KT < NB ? KT * (hb ^ pa) : 0; };   // first k-tile of A(bi, :) of parity pa
+    const int bj = kt0(po) + jj, bjp = kt0(po ^ 1) + jj;      // own tile's column and its P tile's
+    const long long m = (long long)Dp * Dp;
+    const double c_nbr = blk < 2 ? k : k + 1;
+    const bool nbr = blk < 2 ? k >= 1 : k <= 3;
+    // matrices read besides the own one: the neighbour channel's, x_k and x_{k-1} (y), a1_k (a0)
+    const int mn = blk < 2 ? mi - 1 : mi + 1;
+    const int mx = blk == 1 ? rc_qmat(0, 0, k, nb) : rc_qmat(3, 0, k, nb), mxn = blk == 1 ? mx - 1 : mx + 1;
+    // constant panels
+    cplx cQ[KT], cB[KT], cR[KT], cL[KT], cV[KT], cW[KT];
+    {
+        auto rows = [&](cplx* K, const double* gm, int t0) {
+            const cplx* q = reinterpret_cast<const cplx*>(gm);
+#pragma unroll
+            for (int t = 0; t < KT; ++t) K[t] = q[(16 * bi + fi) * Dp + 16 * (t0 + t) + fk];
+        };
+        auto cols = [&](cplx* K, const double* gm, int t0, int col) {
+            const cplx* q = reinterpret_cast<const cplx*>(gm);
+#pragma unroll
+            for (int t = 0; t < KT; ++t) K[t] = q[(16 * (t0 + t) + fk) * Dp + 16 * col + fi];
+        };
+        const double *Qs = g.Qs + 2 * (long long)a * g.qstride, *Qhs = g.Qhs + 2 * (long long)a * g.qstride;
+        const double *v = g.Vrep + 2 * (long long)a * 5 * m, *w = g.Wrep + 2 * (long long)a * 5 * m;
+        rows(cQ, blk == 0 ? g.Q : blk == 1 ? Qs : blk == 2 ? Qhs : g.Qh, kt0(0));
+        cols(cB, blk < 2 ? g.Qh : g.Q, kt0(po), bj);
+        rows(cR, blk < 2 ? g.R : g.Rh, kt0(1));
+        cols(cL, blk < 2 ? g.Rh : g.R, kt0(po), bjp);
+        if (blk == 1) {
+            rows(cV, v, kt0(pw ^ 1));
+            rows(cW, w, kt0(pw));
+        } else {   // unused by x and a1
+            cols(cV, v, kt0(px), bj);
+            cols(cW, w, kt0(px), bjp);
         }
-        __syncthreads();
-        return s_abort == 0;
+    }
+    // exchange buffers: tile (r, c) of a matrix at (r NB + c) TB, copy A (read as row blocks) column by
+    // column, copy B (read as column blocks) row by row; P as copy B
+    const __amdgpu_buffer_rsrc_t rX = rc_rsrc(p.exch, p.exch_bytes);
+    const uint32_t mat_bytes = NT * TB, ring_bytes = (uint32_t)nmat * mat_bytes;
+    const uint32_t oB = RC_RING * ring_bytes, oP = 2 * oB, oR = 3 * oB, rec_bytes = (uint32_t)p.nslots * 16;
+    const uint32_t tile = (uint32_t)(bi * NB + bj) * TB, ptile = (uint32_t)(bi * NB + bjp) * TB;
+    const uint32_t a_el = tile + (uint32_t)(ej * 16 + ei) * 16, b_el = tile + (uint32_t)tid * 16;
+    const uint32_t p_el = ptile + (uint32_t)tid * 16;
+    // fragment offsets: row block bi from k-tile t0, column block col from k-tile t0
+    auto row_at = [&](int t0) { return (uint32_t)(bi * NB + t0) * TB + (uint32_t)tid * 16; };
+    auto col_at = [&](int t0) { return (uint32_t)(t0 * NB + bj) * TB + (uint32_t)tid * 16; };
+    constexpr uint32_t rs = TB, cs = NB * TB;
+    const uint32_t f_r1 = row_at(kt0(po)), f_r2 = row_at(kt0(px));
+    const uint32_t f_c1 = col_at(kt0(0)), f_c2 = col_at(kt0(pw ^ 1)), f_c3 = col_at(kt0(1)), f_c4 = col_at(kt0(pw));
+    const uint32_t sx = (uint32_t)mi * mat_bytes, sn = (uint32_t)mn * mat_bytes, sxx = (uint32_t)mx * mat_bytes,
+                   sxn = (uint32_t)mxn * mat_bytes;
+    const Ctl ctl{p.abort_flag, p.wait_ticks};
+    const long long e = (long long)mi * m + (16 * bi + ei) * Dp + 16 * bj + ej;
+
+    uint32_t ev = 0;
+    auto put = [&](cplx v) {
+        ++ev;
+        const uint32_t so = (ev & (RC_RING - 1)) * ring_bytes + sx;
+        rc_put(rX, a_el, so, v);
+        rc_put(rX, b_el, oB + so, v);
     };
-    // workgroup 0's time (constant-rate clock) in the products, the exchanges and the controller
+    cplx kst[13];   // window of stage derivatives, the newest last
+#pragma unroll
+    for (int q = 0; q < 13; ++q) kst[q] = cmake(0, 0);
+    cplx pre = cmake(0, 0), pre3 = cmake(0, 0);
+    // right-hand side on the stage input of event ev; row: the combinations to sum meanwhile (after
+    // stage `row`), -1 none
+    auto rhs = [&](double jac, double jt, int row) -> cplx {
+        const uint32_t ring = (ev & (RC_RING - 1)) * ring_bytes;
+        const double c = c_nbr * jt;
+        cplx r1[KT], r2[KT], c1[KT], c2[KT], c3[KT], c4[KT], q1[KT], q2[KT], ins = cmake(0, 0);
+        const RcWant<KT> w1{f_r1, ring + sx, rs, r1, true, true}, w2{f_r2, ring + sxx, rs, r2, blk == 2, true},
+            w3{f_c1, oB + ring + sx, cs, c1, true, true}, w4{f_c2, oB + ring + sxx, cs, c2, blk == 1, true},
+            w5{f_c3, oB + ring + sn, cs, c3, nbr, true}, w6{f_c4, oB + ring + sxn, cs, c4, nbr && blk == 1, true};
+        w1.fetch(rX);
+        w2.fetch(rX);
+        w3.fetch(rX);
+        w4.fetch(rX);
+        w5.fetch(rX);
+        w6.fetch(rX);
+        bool ok = rc_await_all(ctl, rX, w1, w2, w3, w4, w5, w6);
+        // level 1
+        cacc acc;
+        cacc_zero(acc);
+        frag_product<KT>(acc, r1, cL);
+        if (blk == 2) frag_product<KT>(acc, r2, cW);
+        put_partial(acc, red1, wave, lane);
+        lds_barrier();
+        rc_put(rX, p_el, oP + ring + sx, sum_partial(red1));
+        if (ev > RC_RING / 2) {   // empty the slots of event ev - 16
+            const uint32_t old = ((ev - RC_RING / 2) & (RC_RING - 1)) * ring_bytes + sx;
+            rc_reset(rX, a_el, old);
+            rc_reset(rX, b_el, oB + old);
+            rc_reset(rX, p_el, oP + old);
+        }
+        // one-sided products
+        cacc_zero(acc);
+        auto scaled = [&](double f, const cplx* A, const cplx* B) {
+#pragma unroll
+            for (int t = 0; t < KT; ++t) cmfma(acc, cscale(f, A[t]), B[t]);
+        };
+        scaled(jac, cQ, c1);
+        scaled(jac, r1, cB);
+        if (blk == 1) scaled(jac, cV, c2);
+        if (blk == 2) scaled(jac, r2, cV);
+        if (nbr) scaled(c, cR, c3);
+        if (nbr && blk == 1) scaled(c, cW, c4);
+        // level 2
+        const RcWant<KT> p1{f_c3, oP + ring + sx, cs, q1, true, true}, p2{f_c4, oP + ring + sxx, cs, q2, blk == 1, true};
+        const RcWant<1> p3{b_el, oP + ring + sn, 0, &ins, nbr, true};
+        p1.fetch(rX);
+        p2.fetch(rX);
+        p3.fetch(rX);
+        if (row >= 0) pre = ode_row_sum(row, kst);
+        if (row == 12) pre3 = ode_row_sum(13, kst);
+        ok = rc_await_all(ctl, rX, p1, p2, p3) && ok;
+        scaled(jac, cR, q1);
+        if (blk == 1) scaled(jac, cW, q2);
+        put_partial(acc, red2, wave, lane);
+        if (!ok) s_bad = 1;
+        lds_barrier();
+        const cplx val = sum_partial(red2);
+        return nbr ? cfma(c, ins, val) : val;
+    };
+    // workgroup 0's time (constant-rate clock) in the right-hand sides (exchanges included), the step
+    // end's exchange and the controller
     uint64_t t_rhs = 0, t_sync = 0, t_ctl = 0, tk = __builtin_amdgcn_s_memrealtime();
     const uint64_t t_start = tk;
     auto lap = [&](uint64_t& acc) {
@@ -815,71 +957,77 @@ __global__ void __launch_bounds__(256) rc_quartic_ode(const RcOdeRun* __restrict
         acc += now - tk;
         tk = now;
     };
-    cplx yv = reinterpret_cast<const cplx*>(p.ybuf)[e];
-    if (tid == 0) sc = p.c0;
-    bool ok = true;
-    // the first right-hand side (first same as last) on y, exchanged through buffer 1 (the first
-    // attempt writes buffer 0 before its event, buffer 1 only after the next)
-    put(1, yv);
-    if (!(ok = sync_all())) goto done;
-    sK[0][tid] = quartic_tile<true>(g, u1, p.jac0, p.jt0, bi, bj, mi, red, T1, T2);
-    ode_step_body<true>(&sc, 0, p.slots, p.ranges, p.nranges, p.ntrack, p.cnt, p.stops, p.stop_node, p.cheb, s_cf);
+    cplx yv = reinterpret_cast<const cplx*>(p.ybuf)[e], k0 = cmake(0, 0);
+    if (tid == 0) {
+        sc = p.c0;
+        s_bad = s_stop = 0;
+    }
+    // what the controller reads, in LDS: each of its device loads would stand in the step's chain
+    for (int i = tid; i < RC_SOURCE_SEGMENTS * (RC_SOURCE_DEGREE + 1); i += 256) s_cheb[i] = p.cheb[i];
+    for (int i = tid; i < 2 * p.ntrack * p.nranges; i += 256) s_ranges[i] = p.ranges[i];
+    if (tid < 2) s_stops[tid] = p.c0.si + tid < p.c0.nstops ? p.stops[p.c0.si + tid] : 0.0;
+    if (tid == 0) s_node = p.stop_node[p.c0.si];
+    if (tid < 13) s_al[tid] = tid == 11 ? RC_B[11] : tid < 11 ? RC_A[tid + 1][tid] : 0.0;
     __syncthreads();
-    while (sc.active) {
+    put(yv);
+    k0 = rhs(p.jac0, p.jt0, -1);   // the first right-hand side (first same as last)
+    ode_step_body<true>(&sc, 0, s_slots, s_ranges, p.nranges, p.ntrack, p.cnt, s_stops, &s_node, s_cheb, s_cf);
+    lds_barrier();
+    while (sc.active && !s_stop) {
         const double he = s_cf[26];
-        put(0, cadd(yv, cscale(he, cscale(RC_A[1][0], sK[0][tid]))));
+        put(cfma(he, cscale(RC_A[1][0], k0), yv));
+#pragma unroll
+        for (int q = 0; q < 12; ++q) kst[q] = cmake(0, 0);
+        kst[12] = k0;
+        cplx ynew = cmake(0, 0), F = cmake(0, 0);
         lap(t_ctl);
-        if (!(ok = sync_all())) break;
-        lap(t_sync);
-        cplx ynew = cmake(0, 0);
+        // the stops the verdict of this attempt may need, behind its first publish
+        if (tid < 2) s_stops[tid] = sc.si + tid < sc.nstops ? p.stops[sc.si + tid] : 0.0;
+        if (tid == 2) s_node = p.stop_node[sc.si];
         for (int st = 1; st < 13; ++st) {
-            const cplx F = quartic_tile<true>(g, ((st - 1) & 1) ? u1 : u0, s_cf[2 * st], s_cf[2 * st + 1], bi, bj,
-                                              mi, red, T1, T2);
-            lap(t_rhs);
-            sK[st][tid] = F;
-            if (st < 12) {   // the next stage input (stage 12's is the step end, B weights)
-                cplx sum = cscale(st < 11 ? RC_A[st + 1][st] : RC_B[st], F);
-                for (int j = 0; j < st; ++j) {
-                    const double aj = st < 11 ? RC_A[st + 1][j] : RC_B[j];
-                    if (aj != 0.0) sum = cadd(sum, cscale(aj, sK[j][tid]));
-                }
-                const cplx u = cadd(yv, cscale(he, sum));
-                if (st == 11) ynew = u;
-                put(st & 1, u);
-                if (!(ok = sync_all())) break;
-                lap(t_sync);
-            } else {         // error sums of this tile
-                cplx r5 = cscale(RC_E5[12], F), r3 = cscale(RC_E3[12], F);
-                for (int j = 0; j < 12; ++j) {
-                    const cplx kj = sK[j][tid];
-                    if (RC_E5[j] != 0.0) r5 = cadd(r5, cscale(RC_E5[j], kj));
-                    if (RC_E3[j] != 0.0) r3 = cadd(r3, cscale(RC_E3[j], kj));
-                }
-                const double scl = p.atol + p.rtol * fmax(cabsd(yv), cabsd(ynew));
-                double* s5 = reinterpret_cast<double*>(red);
-                double* s3 = s5 + 256;
-                s5[tid] = cabs2(r5) / (scl * scl);
-                s3[tid] = cabs2(r3) / (scl * scl);
-                __syncthreads();
-                for (int hh = 128; hh > 0; hh >>= 1) {
-                    if (tid < hh) { s5[tid] += s5[tid + hh]; s3[tid] += s3[tid + hh]; }
-                    __syncthreads();
-                }
-                if (tid == 0) {
-                    __hip_atomic_store(p.slots + 2 * wg, s5[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_store(p.slots + 2 * wg + 1, s3[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-                if (!(ok = sync_all())) break;
-                lap(t_sync);
+            F = rhs(s_cf[2 * st], s_cf[2 * st + 1], st);
+            if (st == 12) break;
+            const cplx u = cfma(he, cfma(s_al[st], F, pre), yv);
+            put(u);
+            ynew = u;   // stage 11's is the step end
+#pragma unroll
+            for (int q = 0; q < 12; ++q) kst[q] = kst[q + 1];
+            kst[12] = F;
+        }
+        lap(t_rhs);
+        // error sums of this tile, and of every other
+        tile_error_put(cfma(RC_E5[12], F, pre), cfma(RC_E3[12], F, pre3), p.atol + p.rtol * fmax(cabsd(yv), cabsd(ynew)),
+                       s_err, wave, lane);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every emptied slot is empty before the record is seen
+        lds_barrier();
+        const uint32_t att = (uint32_t)sc.attempts;
+        const uint32_t so_rec = oR + (att & (RC_REC_RING - 1)) * rec_bytes;
+        const uint32_t so_old = oR + ((att + 2) & (RC_REC_RING - 1)) * rec_bytes;
+        if (tid < (KT < NB ? 2 : 1)) {   // Z2: the tile of the other parity block, exactly zero, has no workgroup
+            const uint32_t off = (uint32_t)(mi * NT + bi * NB + (tid ? bjp : bj)) * 16;
+            rc_put(rX, off, so_rec, tid ? cmake(0, 0) : tile_error_sum(s_err));
+            rc_reset(rX, off, so_old);   // attempt - 2: all published attempt - 1 after reading it
+        }
+        bool ok = true;
+        for (int q0 = 0; q0 < p.nslots; q0 += 256) {
+            const bool use = q0 + tid < p.nslots;
+            cplx v;
+            rc_fetch<1>(rX, (uint32_t)(q0 + tid) * 16, so_rec, 0, &v, use);
+            ok = rc_await<1>(ctl, rX, (uint32_t)(q0 + tid) * 16, so_rec, 0, &v, use) && ok;
+            if (use) {
+                s_slots[2 * (q0 + tid)] = v.re;
+                s_slots[2 * (q0 + tid) + 1] = v.im;
             }
         }
-        if (!ok) break;
-        ode_step_body<true>(&sc, 1, p.slots, p.ranges, p.nranges, p.ntrack, p.cnt, p.stops, p.stop_node, p.cheb,
-                            s_cf);
-        __syncthreads();
+        if (!ok) s_bad = 1;
+        lds_barrier();
+        if (tid == 0) s_stop = s_bad;
+        lap(t_sync);
+        ode_step_body<true>(&sc, 1, s_slots, s_ranges, p.nranges, p.ntrack, p.cnt, s_stops, &s_node, s_cheb, s_cf);
+        lds_barrier();
         if (sc.commit) {
             yv = ynew;
-            sK[0][tid] = sK[12][tid];
+            k0 = F;
             const int smp = sc.sample;
             if (smp >= 0) {
                 if (e < p.half) reinterpret_cast<cplx*>(p.Sf)[(long long)smp * p.half + e] = ynew;
@@ -887,10 +1035,10 @@ __global__ void __launch_bounds__(256) rc_quartic_ode(const RcOdeRun* __restrict
             }
         }
     }
-done:
     reinterpret_cast<cplx*>(p.ybuf)[e] = yv;
     if (wg == 0 && tid == 0) {
-        p.out[0] = ok ? (double)sc.status : (double)RC_ST_WAIT_LIMIT;
+        const bool cut = s_stop || (sc.status == RC_ST_NONFINITE && ld_flag(p.abort_flag));
+        p.out[0] = cut ? (double)RC_ST_WAIT_LIMIT : (double)sc.status;
         p.out[1] = (double)sc.attempts;
         p.out[2] = (double)sc.accepted;
         p.out[3] = (double)sc.rejected;
@@ -901,22 +1049,49 @@ done:
     }
 }
 
-// workgroups of rc_quartic_ode that can be resident at once on the current device
-hipError_t rc_quartic_ode_capacity(int* blocks) {
+static const void* quartic_ode_fn(int nb, int z2) {
+    switch (nb) {
+        case 1: return (const void*)rc_quartic_ode<1, 1>;
+        case 2: return z2 ? (const void*)rc_quartic_ode<2, 1> : (const void*)rc_quartic_ode<2, 2>;
+        case 3: return (const void*)rc_quartic_ode<3, 3>;
+        case 4: return z2 ? (const void*)rc_quartic_ode<4, 2> : (const void*)rc_quartic_ode<4, 4>;
+        default: return nullptr;
+    }
+}
+
+// workgroups of rc_quartic_ode that can be resident at once on the current device (0: not launchable)
+hipError_t rc_quartic_ode_capacity(int nb, int z2, int nslots, int ntrack, int* blocks) {
     int per_cu = 0, dev = 0, cus = 0, coop = 0;
     hipError_t e;
+    const void* fn = quartic_ode_fn(nb, z2);
+    const int lds = RC_ODE_LDS(nslots, ntrack);
+    *blocks = 0;
+    if (!fn || nslots > 4096) return hipSuccess;
     if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
     if ((e = hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev)) != hipSuccess) return e;
-    if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)rc_quartic_ode, 256, 0)) != hipSuccess)
+    if ((e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, std::max(lds, RC_ODE_LDS_ALONE))) !=
+        hipSuccess)
         return e;
+    if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 256, lds)) != hipSuccess) return e;
     if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
     *blocks = coop ? per_cu * cus : 0;
     return hipSuccess;
 }
 
-hipError_t rc_launch_quartic_ode(dim3 grid, const RcOdeRun* dparams, hipStream_t stream) {
+hipError_t rc_launch_quartic_ode(int nb, int z2, int nwg, int nslots, int ntrack, const RcOdeRun* dparams,
+                                 hipStream_t stream) {
     void* args[] = {(void*)&dparams};
-    return hipLaunchCooperativeKernel((const void*)rc_quartic_ode, grid, dim3(256), args, 0, stream);
+    const void* fn = quartic_ode_fn(nb, z2);
+    if (!fn) return hipErrorInvalidValue;
+    int dev = 0, cus = 0;
+    hipError_t e;
+    if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
+    if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
+    // a workgroup per CU where there are CUs for all: more LDS than half a CU's keeps two from sharing one
+    // (and its matrix cores) while others idle
+    const int lds = RC_ODE_LDS(nslots, ntrack);
+    return hipLaunchCooperativeKernel(fn, dim3(nwg), dim3(256), args, nwg <= cus ? std::max(lds, RC_ODE_LDS_ALONE) : lds,
+                                      stream);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -934,7 +1109,7 @@ __device__ __forceinline__ void lindblad_tile(int Dp, int adjoint, const double*
     const cplx* b2 = reinterpret_cast<const cplx*>(adjoint ? Q : Qh);    // X b2
     const cplx* c = reinterpret_cast<const cplx*>(adjoint ? R : Rh);     // T = X c[:, bj]
     const cplx* l = reinterpret_cast<const cplx*>(adjoint ? Rh : R);     // l T
-    qcolumns(T, QTerm{x, c, 0, 0}, QTerm{}, nullptr, QTerm{}, QTerm{}, Dp, bj, wave, lane, 0);
+    qcolumns(T, QTerm{x, c}, QTerm{}, nullptr, QTerm{}, QTerm{}, Dp, bj, wave, lane);
     cacc acc;
     cacc_zero(acc);
     qprod(acc, a1, x, Dp, bi, bj, wave, lane, 1.0);
@@ -984,8 +1159,8 @@ __global__ void __launch_bounds__(256) rc_two_sided(int Dp, int D, const double*
     __shared__ cplx T[64 * 16];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nbt = Dp / 16, bi = blockIdx.x / nbt, bj = blockIdx.x % nbt;
-    qcolumns(T, QTerm{reinterpret_cast<const cplx*>(X), reinterpret_cast<const cplx*>(B), 0, 0}, QTerm{}, nullptr,
-             QTerm{}, QTerm{}, Dp, bj, wave, lane, 0);
+    qcolumns(T, QTerm{reinterpret_cast<const cplx*>(X), reinterpret_cast<const cplx*>(B)}, QTerm{}, nullptr,
+             QTerm{}, QTerm{}, Dp, bj, wave, lane);
     cacc acc;
     cacc_zero(acc);
     qprod_t(acc, reinterpret_cast<const cplx*>(A), T, Dp, bi, wave, lane, 1.0);
@@ -1049,22 +1224,22 @@ __global__ void __launch_bounds__(256) rc_pair_rhs(RcPairArgs g) {
         qprod(acc, k == 1 ? Qs : k == 2 ? Qb : Q, xk, Dp, bi, bj, wave, lane, jac);
         qprod(acc, xk, Qh, Dp, bi, bj, wave, lane, jac);
         if (k == 0) {
-            qcolumns(T1, QTerm{xk, Rh, 0, 0}, QTerm{}, nullptr, QTerm{}, QTerm{}, Dp, bj, wave, lane, 0);
+            qcolumns(T1, QTerm{xk, Rh}, QTerm{}, nullptr, QTerm{}, QTerm{}, Dp, bj, wave, lane);
             qprod_t(acc, R, T1, Dp, bi, wave, lane, jac);
         } else if (k == 1) {
             qprod(acc, v, x(c, 0), Dp, bi, bj, wave, lane, jac);
-            qcolumns(T1, QTerm{xk, Rh, 0, 0}, QTerm{}, T2, QTerm{x(c, 0), Rh, 0, 0}, QTerm{}, Dp, bj, wave, lane, 0);
+            qcolumns(T1, QTerm{xk, Rh}, QTerm{}, T2, QTerm{x(c, 0), Rh}, QTerm{}, Dp, bj, wave, lane);
             qprod_t(acc, R, T1, Dp, bi, wave, lane, jac);
             qprod_t(acc, w, T2, Dp, bi, wave, lane, jac);
         } else if (k == 2) {
             qprod(acc, x(c, 0), vbh, Dp, bi, bj, wave, lane, jac);
-            qcolumns(T1, QTerm{xk, Rh, 0, 0}, QTerm{x(c, 0), uh, 0, 0}, nullptr, QTerm{}, QTerm{}, Dp, bj, wave, lane, 0);
+            qcolumns(T1, QTerm{xk, Rh}, QTerm{x(c, 0), uh}, nullptr, QTerm{}, QTerm{}, Dp, bj, wave, lane);
             qprod_t(acc, R, T1, Dp, bi, wave, lane, jac);
         } else {
             qprod(acc, v, x(c, 2), Dp, bi, bj, wave, lane, jac);
             qprod(acc, x(c, 1), vbh, Dp, bi, bj, wave, lane, jac);
-            qcolumns(T1, QTerm{xk, Rh, 0, 0}, QTerm{x(c, 1), uh, 0, 0}, T2, QTerm{x(c, 2), Rh, 0, 0},
-                     QTerm{x(c, 0), uh, 0, 0}, Dp, bj, wave, lane, 0);
+            qcolumns(T1, QTerm{xk, Rh}, QTerm{x(c, 1), uh}, T2, QTerm{x(c, 2), Rh},
+                     QTerm{x(c, 0), uh}, Dp, bj, wave, lane);
             qprod_t(acc, R, T1, Dp, bi, wave, lane, jac);
             qprod_t(acc, w, T2, Dp, bi, wave, lane, jac);
         }

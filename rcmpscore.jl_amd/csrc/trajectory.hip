@@ -44,6 +44,7 @@
 // D = 40 9.1 -> 4.7, D = 64 9.4 -> 5.4 (split 9.5 -> 6.6); six trajectories at D = 64, window 30,
 // 1e-13/1e-12: 62 -> 36 ms.
 #include "device_common.h"
+#include "exchange.h"
 #include "split.h"
 #include "trajectory.h"
 
@@ -58,132 +59,6 @@ struct Lay {
     static constexpr int NDOUBLE_SCRATCH = 64;
     static constexpr int BYTES = NCPLX * 16 + NDOUBLE_SCRATCH * 8;
 };
-
-// c k + a, each part one fused multiply-add: the instantiations of the kernel (Z2 blocks or every
-// k-tile, timed or not) round alike whatever the compiler would contract
-__device__ __forceinline__ cplx cfma(double c, cplx k, cplx a) { return cmake(fma(c, k.re, a.re), fma(c, k.im, a.im)); }
-
-struct Ctl {
-    uint32_t* abort_flag;
-    long long wait_ticks;   // longest single wait, in ticks of the constant-rate clock (s_memrealtime)
-};
-
-// Barrier of the workgroup that orders LDS accesses only: device-coherent stores and polling loads
-// in flight stay in flight (__syncthreads would wait for them).
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-// the empty slot's word: a quiet NaN whose payload no arithmetic here produces (the hardware's own
-// NaN has payload zero, the state's matrices are finite)
-__device__ __forceinline__ bool rc_arrived(cplx v) {
-    return (uint32_t)__double2hiint(v.re) != RC_EMPTY_WORD && (uint32_t)__double2hiint(v.im) != RC_EMPTY_WORD;
-}
-__device__ __forceinline__ double rc_not_empty(double x) {
-    return (uint32_t)__double2hiint(x) == RC_EMPTY_WORD ? __longlong_as_double(0x7ff8000000000000LL) : x;
-}
-// publish a value / empty a slot again (device-coherent stores; every aligned 8-byte half is
-// written whole, and a reader checks both)
-__device__ __forceinline__ void rc_put(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, cplx z) {
-    st_coh_s(r, voff, soff, cmake(rc_not_empty(z.re), rc_not_empty(z.im)));
-}
-__device__ __forceinline__ void rc_reset(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-    const double e = __hiloint2double((int)RC_EMPTY_WORD, (int)RC_EMPTY_WORD);
-    st_coh_s(r, voff, soff, cmake(e, e));
-}
-
-// Elements voff + soff + t stride, t < N, of the lanes that `use` them: the loads alone; rc_await then
-// repeats them until every element of the wave has arrived.  False when the abort word is set or
-// the wait outlasts its time budget (then the abort word is set).  The budget is wall-clock time: a
-// workgroup that starts a later round of a batched launch early may wait a whole round for
-// partners that are still running.
-template <int N>
-__device__ __forceinline__ void rc_fetch(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, uint32_t stride,
-                                         cplx* v, bool use = true) {
-    if (use) {
-#pragma unroll
-        for (int t = 0; t < N; ++t) v[t] = ld_coh_s(r, voff, soff + t * stride);
-    } else {
-#pragma unroll
-        for (int t = 0; t < N; ++t) v[t] = cmake(0, 0);
-    }
-}
-template <int N>
-__device__ __forceinline__ bool rc_all_arrived(const cplx* v) {
-    bool ok = true;
-#pragma unroll
-    for (int t = 0; t < N; ++t) ok &= rc_arrived(v[t]);
-    return __all(ok);
-}
-// Hide the values from the compiler's count of outstanding loads: they have arrived, and their later
-// uses must not wait for whatever store or load was issued since.
-template <int N>
-__device__ __forceinline__ void rc_settle(cplx* v) {
-#pragma unroll
-    for (int t = 0; t < N; ++t) asm volatile("" : "+v"(v[t].re), "+v"(v[t].im));
-}
-template <int N>
-__device__ __forceinline__ bool rc_await(const Ctl& ctl, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff,
-                                         uint32_t stride, cplx* v, bool use = true) {
-    uint64_t t0 = 0;
-    bool ok = true;
-    for (uint32_t polls = 1; !rc_all_arrived<N>(v); ++polls) {
-        asm volatile("" ::: "memory");
-        rc_fetch<N>(r, voff, soff, stride, v, use);
-        if ((polls & 63) == 0) {   // the clock and the abort word are read every 64th poll only
-            const uint64_t now = __builtin_amdgcn_s_memrealtime();
-            if (t0 == 0) t0 = now;
-            const bool over = (long long)(now - t0) > ctl.wait_ticks;
-            if (over) st_flag(ctl.abort_flag, 1u);
-            if (over || uni((int)ld_flag(ctl.abort_flag))) {
-                ok = false;
-                break;
-            }
-        }
-    }
-    rc_settle<N>(v);
-    return ok;
-}
-
-// acc += A B over this wave's k-steps (fragment t: its k-step of the t-th k-tile)
-template <int KT>
-__device__ __forceinline__ void frag_product(cacc& acc, const cplx* A, const cplx* B) {
-#pragma unroll
-    for (int t = 0; t < KT; ++t) cmfma(acc, A[t], B[t]);
-}
-
-// Sum of the four waves' partial tiles; thread t receives element (t/16, t%16).  The barrier also
-// orders the other level's buffer: its readers pass here before anyone writes it again.
-__device__ __forceinline__ void put_partial(const cacc& acc, cplx* red, int wave, int lane) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) red[wave * 256 + (4 * q + (lane >> 4)) * 16 + (lane & 15)] = cacc_get(acc, q);
-}
-__device__ __forceinline__ cplx sum_partial(const cplx* red) {
-    const int t = threadIdx.x;
-    return cadd(cadd(cadd(red[t], red[256 + t]), red[512 + t]), red[768 + t]);
-}
-
-// a DPP move of a double within each row of 16 lanes (CTRL a compile-time DPP control)
-template <int CTRL>
-__device__ __forceinline__ double dpp_move(double x) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xF, 0xF, false);
-    return __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double read_lane(double x, int l) {
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), l),
-                            __builtin_amdgcn_readlane(__double2loint(x), l));
-}
-// Wave sum in a fixed order: pairs, quads (quad_perm), halves (row_half_mirror) and rows
-// (row_mirror) by DPP moves, every lane of a row holding the same row sum (addition commutes),
-// then the four row sums in order.
-__device__ __forceinline__ double wave_sum(double v) {
-    v += dpp_move<0xB1>(v);
-    v += dpp_move<0x4E>(v);
-    v += dpp_move<0x141>(v);
-    v += dpp_move<0x140>(v);
-    return ((read_lane(v, 0) + read_lane(v, 16)) + read_lane(v, 32)) + read_lane(v, 48);
-}
 
 // Record i of a read-only array through scalar loads, so that every field is known wave-uniform.
 template <typename T>
@@ -622,10 +497,11 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
             xr[0] = Yt[fi * 17 + fk];
             xc[0] = Yt[fk * 17 + fi];
         } else {
-            if (get_c) rc_fetch<NF>(rX, col_off, oB + so, col_step, xc, use_c);
-            if (get_r) rc_fetch<NF>(rX, row_off, so, row_step, xr, use_r);
-            if (get_c) ok = rc_await<NF>(ctl, rX, col_off, oB + so, col_step, xc, use_c);
-            if (get_r) ok = rc_await<NF>(ctl, rX, row_off, so, row_step, xr, use_r) && ok;
+            const RcWant<NF> wc{col_off, oB + so, col_step, xc, get_c, use_c};
+            const RcWant<NF> wr{row_off, so, row_step, xr, get_r, use_r};
+            wc.fetch(rX);
+            wr.fetch(rX);
+            ok = rc_await_all(ctl, rX, wc, wr);
         }
         lap(0);
         cacc acc;
@@ -738,8 +614,8 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
                 put_partial(acc, red2, wave, lane);
             }
             if (insert) {
-                ok = rc_await<1>(ctl, rX, ins_off, so_i, 0, &s1) && ok;
-                ok = rc_await<1>(ctl, rX, ins_off_t, so_i, 0, &s2) && ok;
+                ok = rc_await_all(ctl, rX, RcWant<1>{ins_off, so_i, 0, &s1, true, true},
+                                  RcWant<1>{ins_off_t, so_i, 0, &s2, true, true}) && ok;
             }
             lds_barrier();
             Le = SPLIT ? sum_partial_split(redd2) : sum_partial(red2);
