@@ -28,6 +28,8 @@
 
 int rc_trajectory_smem_bytes(int nb, int split);
 hipError_t rc_trajectory_capacity(int nb, int split, int z2, int timed, int* blocks);
+#include "gmres.h"
+
 hipError_t rc_launch_fill_empty(void* dst, size_t bytes, hipStream_t stream);
 hipError_t rc_launch_trajectory(int nb, int split, int z2, int timed, int nblocks, const TrajParams* dparams, hipStream_t stream);
 
@@ -89,9 +91,11 @@ struct KineticWork {
 
 struct TrajBufs {
     DevBuf samples[RC_NSYS], fixed;
+    DevBuf fin;   // the pullback's XR, XQ, environment and covector, the boundary solve's solution
     void release() {
         for (int s = 0; s < RC_NSYS; ++s) samples[s].release();
         fixed.release();
+        fin.release();
     }
 };
 
@@ -184,6 +188,10 @@ struct rcmps_context {
     DevBuf nodes_w, nodes_j, tmpM, partial, scratch, small;
     // krylov workspaces
     DevBuf kry_V, kry_w, kry_t1, kry_t2, kry_x, kry_b, kry_z, kry_h, kry_tmp;
+    // fused solves (rc_gmres): exchange areas, descriptors, results and the abort word; equations
+    // per launch by tiles per side (-1: not asked yet)
+    DevBuf gm_exch, gm_prob, gm_out;
+    int gm_cap[5] = {-1, -1, -1, -1, -1};
     // GMRES read-back: two pinned slots of one Hessenberg column each, and their completion events
     double* kry_pinned = nullptr;
     size_t kry_pinned_doubles = 0;
@@ -676,6 +684,92 @@ bool gmres(Dev& dv, const std::function<void(const double*, double*)>& A, const 
     return converged;
 }
 
+// ------------------------------------------------------------------------------------------
+// Fused solves: one launch of rc_gmres for a whole solve.  States whose no-jump inverse is in the
+// eigenbasis and Dp <= 64; the others run gmres() above.  A launch of more than one tile per side is
+// cooperative, so it does not share the device with a running trajectory launch.
+// ------------------------------------------------------------------------------------------
+int fused_capacity(rcmps_context* ctx, const rcmps_state* st) {
+    const int nb = st->Dp / 16;
+    if (nb > 4 || st->nojump_schur) return 0;
+    if (ctx->gm_cap[nb] < 0) ck(rc_gmres_capacity(nb, &ctx->gm_cap[nb]));
+    return ctx->gm_cap[nb];
+}
+
+struct FusedResult {
+    bool converged;
+    int matvecs;
+    double resid, nb, true_res;
+};
+
+// the operator's part of an equation: direction, momentum shift and the rank-one pin phi, psi
+RcGmresProb fused_problem(const rcmps_state* st, bool adj, double sigma) {
+    RcGmresProb p{};
+    p.D = st->D;
+    p.adjoint = adj ? 1 : 0;
+    p.m = std::min(st->D * st->D, RC_GMRES_MAX_M);
+    p.maxiter = 200;
+    p.A1 = adj ? st->VH.d() : st->Vinv.d();
+    p.B1 = adj ? st->V.d() : st->VinvH.d();
+    p.A2 = adj ? st->VinvH.d() : st->V.d();
+    p.B2 = adj ? st->Vinv.d() : st->VH.d();
+    p.lam = st->lam.d();
+    p.s_re = st->shift;
+    p.s_im = p.sig = adj ? -sigma : sigma;
+    p.C1 = adj ? st->Qh.d() : st->Q.d();
+    p.C2 = adj ? st->Q.d() : st->Qh.d();
+    p.C3 = adj ? st->R.d() : st->Rh.d();
+    p.C4 = adj ? st->Rh.d() : st->R.d();
+    p.phi = adj ? st->rho.d() : st->ident.d();
+    p.psi = adj ? st->ident.d() : st->rho.d();
+    p.c2 = p.ds = 1.0;
+    return p;
+}
+
+// Solve the equations (one padded size, at most fused_capacity of them) and read the results.  The
+// workspaces are given (per equation exch and 8 doubles of out, and an abort word behind those), so
+// that a caller with fixed memory allocates nothing.
+void fused_run(rcmps_context* ctx, int nb, std::vector<RcGmresProb>& ps, double* exch, double* out,
+               RcGmresProb* many, std::vector<FusedResult>& res) {
+    const int n = (int)ps.size();
+    const size_t eb = rc_gmres_exch_bytes(nb);
+    for (int i = 0; i < n; ++i) {
+        ps[i].exch = exch + (size_t)i * eb / 8;
+        ps[i].out = out + 8 * i;
+    }
+    if (n > 1) ck(hipMemcpyAsync(many, ps.data(), n * sizeof(RcGmresProb), hipMemcpyHostToDevice, ctx->stream));
+    ck(hipMemsetAsync(out, 0, ((size_t)8 * n + 8) * 8, ctx->stream));
+    if (nb > 1) ck(rc_launch_fill_empty(exch, n * eb, ctx->stream));
+    ck(rc_launch_gmres(nb, n, ps[0], many, reinterpret_cast<uint32_t*>(out + 8 * n),
+                       (long long)(10.0 * ctx->clock_mhz * 1e6), ctx->stream));
+    std::vector<double> o((size_t)8 * n);
+    ck(hipMemcpyAsync(o.data(), out, o.size() * 8, hipMemcpyDeviceToHost, ctx->stream));
+    ck(hipStreamSynchronize(ctx->stream));
+    res.resize(n);
+    for (int i = 0; i < n; ++i) {
+        const double* q = o.data() + 8 * i;
+        if (q[0] != 0) throw Fail{(int)q[0]};
+        res[i] = FusedResult{q[1] != 0, (int)q[2], q[3], q[4], q[5]};
+    }
+}
+
+// the same in the context's workspaces, in as many launches as it takes
+void fused_solve(rcmps_context* ctx, const rcmps_state* st0, std::vector<RcGmresProb>& ps, std::vector<FusedResult>& res) {
+    const int nb = st0->Dp / 16, cap = std::min(fused_capacity(ctx, st0), 256);
+    res.clear();
+    for (size_t i0 = 0; i0 < ps.size(); i0 += cap) {
+        std::vector<RcGmresProb> part(ps.begin() + i0, ps.begin() + std::min(ps.size(), i0 + cap));
+        const size_t n = part.size();
+        ck(ctx->gm_exch.ensure(n * rc_gmres_exch_bytes(nb)));
+        ck(ctx->gm_out.ensure((8 * n + 8) * 8));
+        ck(ctx->gm_prob.ensure(n * sizeof(RcGmresProb)));
+        std::vector<FusedResult> r;
+        fused_run(ctx, nb, part, ctx->gm_exch.d(), ctx->gm_out.d(),
+                  static_cast<RcGmresProb*>(ctx->gm_prob.p), r);
+        res.insert(res.end(), r.begin(), r.end());
+    }
+}
+
 void state_spectral(rcmps_context* ctx, rcmps_state* st) {
     const int D = st->D, Dp = st->Dp;
     Mat q = download(ctx, D, Dp, st->Q.d());
@@ -860,7 +954,7 @@ void rcmps_context_destroy(rcmps_context* ctx) {
                      &ctx->traj_points, &ctx->abort_word, &ctx->nodes_w, &ctx->nodes_j,
                      &ctx->tmpM, &ctx->partial, &ctx->scratch, &ctx->small, &ctx->kry_V, &ctx->kry_w,
                      &ctx->kry_t1, &ctx->kry_t2, &ctx->kry_x, &ctx->kry_b, &ctx->kry_z, &ctx->kry_h,
-                     &ctx->kry_tmp, &ctx->tune_buf};
+                     &ctx->kry_tmp, &ctx->tune_buf, &ctx->gm_exch, &ctx->gm_prob, &ctx->gm_out};
     for (auto* b : all) b->release();
     for (auto& b : ctx->tb) b->release();
     if (ctx->blas) (void)rocblas_destroy_handle(ctx->blas);
@@ -935,37 +1029,53 @@ int rcmps_state_create(rcmps_context* ctx, int D, const double* R, const double*
         } else {
             // (-L + |I><I|/D) x = I/D with the Sherman-Morrison right preconditioner built on the
             // no-jump inverse (gpu/src/rcmps_gpu/optimizer/runtime/numerics.py:74-100)
-            double* t1 = ctx->kry_t1.d();
-            double* t2 = ctx->kry_t2.d();
-            ck(ctx->kry_z.ensure(mb));
-            ck(ctx->kry_b.ensure(mb));
-            ck(ctx->kry_x.ensure(mb));
-            ck(ctx->scratch.ensure(4 * mb));
-            double* z = ctx->kry_z.d();
-            double* tmp = ctx->scratch.d();
-            double* tmp2 = tmp + (size_t)Dp * Dp * 2;
-            double* tr2 = ctx->small.d();
-            nojump_apply(dv, st, st->ident.d(), z, false, t1, t2);
-            dv.trace_prod(st->ident.d(), z, tr2);
-            cd den = 1.0 + dv.fetch2(tr2) / (double)D;
-            auto pre = [&](const double* y, double* xo) {
-                nojump_apply(dv, st, y, xo, false, t1, t2);
-                dv.trace_prod(st->ident.d(), xo, tr2);
-                dv.sub_scaled(tr2, (double)D * den, z, xo);
-            };
-            auto op = [&](const double* xin, double* yo) {
-                lindblad(dv, st, xin, yo, false, t1);
-                dv.trace_prod(st->ident.d(), xin, tr2);
-                dv.neg_add_identity(tr2, 1.0 / D, yo);
-            };
-            dv.axpby(cd(1.0 / D, 0), st->ident.d(), cd(0, 0), nullptr, ctx->kry_b.d());
             int mv = 0;
             double res = 0;
-            auto A = [&](const double* v, double* w) { pre(v, tmp2); op(tmp2, w); };
-            const int m = std::min(D * D, 40);
-            // the reference iterates its CPTP Arnoldi to tol / 10 (src/transfer.jl:103-105)
-            bool okg = gmres(dv, A, ctx->kry_b.d(), ctx->kry_x.d(), steady_tol / 10, m, 200, mv, res);
-            pre(ctx->kry_x.d(), st->rho.d());
+            bool okg = false;
+            ck(ctx->kry_b.ensure(mb));
+            dv.axpby(cd(1.0 / D, 0), st->ident.d(), cd(0, 0), nullptr, ctx->kry_b.d());
+            if (fused_capacity(ctx, st) > 0) {
+                std::vector<RcGmresProb> ps{fused_problem(st, false, 0.0)};
+                ps[0].psi = st->ident.d();
+                ps[0].c2 = ps[0].ds = 1.0 / D;
+                ps[0].pin = 1;
+                ps[0].tol = steady_tol / 10;
+                ps[0].a = ctx->kry_b.d();
+                ps[0].x = st->rho.d();
+                std::vector<FusedResult> fr;
+                fused_solve(ctx, st, ps, fr);
+                okg = fr[0].converged;
+                mv = fr[0].matvecs;
+                res = fr[0].resid;
+            } else {
+                double* t1 = ctx->kry_t1.d();
+                double* t2 = ctx->kry_t2.d();
+                ck(ctx->kry_z.ensure(mb));
+                ck(ctx->kry_x.ensure(mb));
+                ck(ctx->scratch.ensure(4 * mb));
+                double* z = ctx->kry_z.d();
+                double* tmp = ctx->scratch.d();
+                double* tmp2 = tmp + (size_t)Dp * Dp * 2;
+                double* tr2 = ctx->small.d();
+                nojump_apply(dv, st, st->ident.d(), z, false, t1, t2);
+                dv.trace_prod(st->ident.d(), z, tr2);
+                cd den = 1.0 + dv.fetch2(tr2) / (double)D;
+                auto pre = [&](const double* y, double* xo) {
+                    nojump_apply(dv, st, y, xo, false, t1, t2);
+                    dv.trace_prod(st->ident.d(), xo, tr2);
+                    dv.sub_scaled(tr2, (double)D * den, z, xo);
+                };
+                auto op = [&](const double* xin, double* yo) {
+                    lindblad(dv, st, xin, yo, false, t1);
+                    dv.trace_prod(st->ident.d(), xin, tr2);
+                    dv.neg_add_identity(tr2, 1.0 / D, yo);
+                };
+                auto A = [&](const double* v, double* w) { pre(v, tmp2); op(tmp2, w); };
+                const int m = std::min(D * D, 40);
+                // the reference iterates its CPTP Arnoldi to tol / 10 (src/transfer.jl:103-105)
+                okg = gmres(dv, A, ctx->kry_b.d(), ctx->kry_x.d(), steady_tol / 10, m, 200, mv, res);
+                pre(ctx->kry_x.d(), st->rho.d());
+            }
             if (stats) { stats->krylov_matvecs = mv; stats->krylov_residual = res; }
             // accepted at steady_tol when the tighter target stagnates (as the boundary solve)
             if (!okg && !(res <= steady_tol)) throw Fail{RCMPS_ERR_SOLVER};
@@ -1003,13 +1113,35 @@ namespace {
 struct BoundaryBufs {
     double *t1, *t2, *z, *b, *x, *tmp, *small;
     GmresBufs g;
+    double *fexch, *fout;   // of the fused solve, in the same memory
 };
+
+RcGmresProb boundary_problem(const rcmps_state* st, const double* a, double tol, double* h) {
+    RcGmresProb p = fused_problem(st, true, 0.0);
+    p.project_b = p.pin = 1;
+    p.tol = tol;
+    p.a = a;
+    p.x = h;
+    return p;
+}
+void boundary_result(const FusedResult& r, double tol, double accept_tol, rcmps_stats* stats) {
+    if (stats) { stats->krylov_matvecs = r.matvecs; stats->krylov_residual = r.true_res; }
+    if (!(r.true_res <= 20 * std::max(tol, accept_tol) * std::max(1.0, r.nb))) throw Fail{RCMPS_ERR_SOLVER};
+}
 
 void boundary_solve(rcmps_context* ctx, const rcmps_state* st, const double* a, double tol, double accept_tol,
                     double* h, rcmps_stats* stats, const BoundaryBufs* bb = nullptr) {
     const int D = st->D, Dp = st->Dp;
     const size_t mb = (size_t)Dp * Dp * 16;
     Dev dv{ctx, Dp, D};
+    if (D > 1 && fused_capacity(ctx, st) > 0) {
+        std::vector<RcGmresProb> ps{boundary_problem(st, a, tol, h)};
+        std::vector<FusedResult> fr;
+        if (bb) fused_run(ctx, Dp / 16, ps, bb->fexch, bb->fout, nullptr, fr);
+        else fused_solve(ctx, st, ps, fr);
+        boundary_result(fr[0], tol, accept_tol, stats);
+        return;
+    }
     double *t1, *t2, *z, *b, *x, *tmp;
     if (bb) {
         t1 = bb->t1; t2 = bb->t2; z = bb->z; b = bb->b; x = bb->x; tmp = bb->tmp;
@@ -1381,11 +1513,20 @@ const double* metric_inverse(rcmps_context* ctx, const rcmps_state* st, double m
 // Pullback over the Gauss nodes, boundary correction and gradients of one evaluation whose
 // trajectories are in tb (src/observables.jl:161-212).  With kin_cov/kin_env (device) the two
 // kinetic terms come from the infinite-line backend and only the :phi^4: trajectories are pulled back.
-void finish_state(rcmps_context* ctx, EvalReq& r, TrajBufs& tb, const rcmps_integrator* ip, double metric_reg,
-                  int flags, const double* kin_cov = nullptr, const double* kin_env = nullptr) {
+// The finishing of an evaluation in three parts: the pullback into tb.fin, the boundary solve of its
+// environment, the gradient.  tb.fin holds XR, XQ, env, cov and the boundary's solution, with
+// dE = 2 Re tr(XR dR) + 2 Re tr(XQ dQ) for any (dR, dQ) and covector = XR - XQ R^+ (+ the kinetic one).
+void covector(Dev& dv, const rcmps_state* st, const double* XR, const double* XQ, const double* kin_cov, double* cterm,
+              double* cov) {   // horizontal directions dQ = -R^+ W
+    dv.gemm(0, XQ, 0, st->Rh.d(), cterm);
+    dv.axpby(cd(1, 0), XR, cd(-1, 0), cterm, cov);
+    if (kin_cov) dv.axpby(cd(1, 0), cov, cd(1, 0), kin_cov, cov);
+}
+
+void finish_pullback(rcmps_context* ctx, EvalReq& r, TrajBufs& tb, const rcmps_integrator* ip,
+                     const double* kin_cov = nullptr, const double* kin_env = nullptr) {
     const rcmps_state* st = r.st;
-    rcmps_stats* S = r.S;
-    double *grad = r.grad, *raw_cov = r.raw_cov, *raw_env = r.raw_env, *grad_R = r.grad_R, *grad_K = r.grad_K;
+    double *raw_cov = r.raw_cov, *raw_env = r.raw_env;
     const int D = st->D, Dp = st->Dp;
     Dev dv{ctx, Dp, D};
     const size_t mb = (size_t)Dp * Dp * 16;
@@ -1399,22 +1540,21 @@ void finish_state(rcmps_context* ctx, EvalReq& r, TrajBufs& tb, const rcmps_inte
     ck(hipEventRecord(ctx->ev[2], ctx->stream));
     ck(ctx->tmpM.ensure((size_t)nn * mb));
     ck(ctx->scratch.ensure(12 * mb));
+    ck(tb.fin.ensure(5 * mb));
     double* M = ctx->tmpM.d();
-    double* cov = ctx->scratch.d();
-    double* env = cov + mcount;
-    double* T1 = cov + 2 * mcount;
-    double* T2 = cov + 3 * mcount;
-    double* U = cov + 4 * mcount;
-    double* X1 = cov + 5 * mcount;
-    double* X2 = cov + 6 * mcount;
-    double* cterm = cov + 7 * mcount;
-    double* tmp = cov + 8 * mcount;
-    double* tmp2 = cov + 9 * mcount;
-    // dE = 2 Re tr(XR dR) + 2 Re tr(XQ dQ) for any (dR, dQ); covector = XR - XQ R^+
-    double* XR = cov + 10 * mcount;
-    double* XQ = cov + 11 * mcount;
-    ck(hipMemsetAsync(env, 0, mb, ctx->stream));
-    ck(hipMemsetAsync(XR, 0, 2 * mb, ctx->stream));
+    double* T1 = ctx->scratch.d();
+    double* T2 = T1 + mcount;
+    double* U = T1 + 2 * mcount;
+    double* X1 = T1 + 3 * mcount;
+    double* X2 = T1 + 4 * mcount;
+    double* cterm = T1 + 5 * mcount;
+    double* tmp = T1 + 6 * mcount;
+    double* tmp2 = T1 + 7 * mcount;
+    double* XR = tb.fin.d();
+    double* XQ = XR + mcount;
+    double* env = XR + 2 * mcount;
+    double* cov = XR + 3 * mcount;
+    ck(hipMemsetAsync(XR, 0, 3 * mb, ctx->stream));
     const long long node = (long long)Dp * Dp;   // complex elements per matrix
     for (int term = kin_cov ? 2 : 0; term < 3; ++term) {
         const int sf = 2 * term, sa = sf + 1;
@@ -1505,32 +1645,37 @@ void finish_state(rcmps_context* ctx, EvalReq& r, TrajBufs& tb, const rcmps_inte
         dv.axpby(cd(1, 0), env, cd(c, 0), tmp, env);
     }
     if (kin_env) dv.axpby(cd(1, 0), env, cd(1, 0), kin_env, env);
-    auto covector = [&] {   // horizontal directions dQ = -R^+ W
-        dv.gemm(0, XQ, 0, st->Rh.d(), cterm);
-        dv.axpby(cd(1, 0), XR, cd(-1, 0), cterm, cov);
-        if (kin_cov) dv.axpby(cd(1, 0), cov, cd(1, 0), kin_cov, cov);
-    };
-    covector();
+    covector(dv, st, XR, XQ, kin_cov, cterm, cov);
     ck(hipEventRecord(ctx->ev[3], ctx->stream));
     if (raw_cov) pad_out(ctx, D, Dp, cov, raw_cov);
     if (raw_env) pad_out(ctx, D, Dp, env, raw_env);
+}
 
-    // ----------------------------------------------------------------------------------
-    // finish_gradient (src/observables.jl:201-212)
-    // ----------------------------------------------------------------------------------
-    if (grad || grad_R || grad_K) {
-        if (!(flags & RCMPS_FLAG_NO_BOUNDARY)) {
-            ck(ctx->tmpM.ensure(2 * mb));
-            double* hb = X1;
-            // aims two digits below the reference's 1e-11 and accepts at its bar
-            boundary_solve(ctx, st, env, 1e-13, 1e-11, hb, S);
-            // rho0 responds to dL(rho0) = dQ rho0 + rho0 dQ^+ + dR rho0 R^+ + R rho0 dR^+:
-            // XR += rho R^+ H, XQ += rho H  (covector += rho R^+ H - rho H R^+)
-            dv.gemm(0, st->rho.d(), 0, st->Rh.d(), tmp);
-            dv.gemm(0, tmp, 0, hb, XR, 1.0, 1.0);
-            dv.gemm(0, st->rho.d(), 0, hb, XQ, 1.0, 1.0);
-            covector();
-        }
+bool wants_gradient(const EvalReq& r) { return r.grad || r.grad_R || r.grad_K; }
+
+// finish_gradient (src/observables.jl:201-212) after the boundary solve (h in tb.fin; none: skipped)
+void finish_gradient_part(rcmps_context* ctx, EvalReq& r, TrajBufs& tb, double metric_reg, bool boundary,
+                          const double* kin_cov) {
+    const rcmps_state* st = r.st;
+    double *grad = r.grad, *grad_R = r.grad_R, *grad_K = r.grad_K;
+    const int D = st->D, Dp = st->Dp;
+    Dev dv{ctx, Dp, D};
+    const size_t mcount = (size_t)Dp * Dp * 2;
+    ck(ctx->scratch.ensure(12 * mcount * 8));
+    double* cterm = ctx->scratch.d();
+    double* tmp = cterm + mcount;
+    double* tmp2 = cterm + 2 * mcount;
+    double* XR = tb.fin.d();
+    double* XQ = XR + mcount;
+    double* cov = XR + 3 * mcount;
+    const double* hb = XR + 4 * mcount;
+    if (wants_gradient(r) && boundary) {
+        // rho0 responds to dL(rho0) = dQ rho0 + rho0 dQ^+ + dR rho0 R^+ + R rho0 dR^+:
+        // XR += rho R^+ H, XQ += rho H  (covector += rho R^+ H - rho H R^+)
+        dv.gemm(0, st->rho.d(), 0, st->Rh.d(), tmp);
+        dv.gemm(0, tmp, 0, hb, XR, 1.0, 1.0);
+        dv.gemm(0, st->rho.d(), 0, hb, XQ, 1.0, 1.0);
+        covector(dv, st, XR, XQ, kin_cov, cterm, cov);
     }
     if (grad_R || grad_K) {
         // Q = -iK - R^+R/2: dQ = -i dK - (dR^+ R + R^+ dR)/2, so
@@ -1554,13 +1699,25 @@ void finish_state(rcmps_context* ctx, EvalReq& r, TrajBufs& tb, const rcmps_inte
         dv.gemm(1, cov, 0, metric_inverse(ctx, st, metric_reg), tmp);
         pad_out(ctx, D, Dp, tmp, grad);
     }
+}
+
+// all three on one context
+void finish_state(rcmps_context* ctx, EvalReq& r, TrajBufs& tb, const rcmps_integrator* ip, double metric_reg,
+                  int flags, const double* kin_cov = nullptr, const double* kin_env = nullptr) {
+    const bool boundary = !(flags & RCMPS_FLAG_NO_BOUNDARY);
+    finish_pullback(ctx, r, tb, ip, kin_cov, kin_env);
+    // the boundary solve aims two digits below the reference's 1e-11 and accepts at its bar
+    const size_t mcount = (size_t)r.st->Dp * r.st->Dp * 2;
+    if (wants_gradient(r) && boundary)
+        boundary_solve(ctx, r.st, tb.fin.d() + 2 * mcount, 1e-13, 1e-11, tb.fin.d() + 4 * mcount, r.S);
+    finish_gradient_part(ctx, r, tb, metric_reg, boundary, kin_cov);
     ck(hipEventRecord(ctx->ev[4], ctx->stream));
     ck(hipStreamSynchronize(ctx->stream));
     float pms = 0, bms = 0;
     ck(hipEventElapsedTime(&pms, ctx->ev[2], ctx->ev[3]));
     ck(hipEventElapsedTime(&bms, ctx->ev[3], ctx->ev[4]));
-    S->pullback_ms = pms;
-    S->boundary_ms = bms;
+    r.S->pullback_ms = pms;
+    r.S->boundary_ms = bms;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2177,12 +2334,11 @@ bool valid_integrator(const rcmps_integrator* ip) {
 
 // A batch of evaluations: grouped by padded size, one persistent launch per group, then the
 // pullback of each evaluation.  Every request gets its stats; the first failure is returned.
-// The per-state pullback, boundary and metric solves of one class run on up to kFinishWorkers worker
-// contexts, each driven by its own host thread and stream, while the main stream integrates the
-// next class.  Each state is finished by one worker with the same kernels and tile choices as on the
-// main context (every tile variant gives the same bits), so the results equal the sequential ones
-// bit for bit.  Not for a single state or when a state appears twice (its cached metric inverse
-// would be shared between threads).
+// The per-state pullbacks of one class run on up to kFinishWorkers worker contexts, each driven by its
+// own host thread and stream, while the main stream integrates the next class; the boundary solves of
+// the class then run together on the main context, and the gradients.  The kernels and tile choices
+// are those of a single call (every tile variant gives the same bits), so the results equal the
+// sequential ones bit for bit.  Not for a single state or when a state appears twice.
 constexpr int kFinishWorkers = 4;
 
 bool can_finish_concurrently(const std::vector<int>& idx, const std::vector<EvalReq>& reqs) {
@@ -2193,11 +2349,11 @@ bool can_finish_concurrently(const std::vector<int>& idx, const std::vector<Eval
     return std::adjacent_find(seen.begin(), seen.end()) == seen.end();
 }
 
-// Finish the evaluations idx (trajectories in ctx->tb[tb0 + j]) on the worker contexts.  Only this
-// function touches ctx->workers; it may run on a host thread of its own while the main thread
+// The pullbacks of the evaluations idx (trajectories in ctx->tb[tb0 + j]) on the worker contexts.  Only
+// this function touches ctx->workers; it may run on a host thread of its own while the main thread
 // drives ctx->stream.
-void finish_concurrently(rcmps_context* ctx, const rcmps_integrator* ip, double metric_reg, int flags,
-                         const std::vector<int>& idx, size_t tb0, std::vector<EvalReq>& reqs) {
+void pull_back_concurrently(rcmps_context* ctx, const rcmps_integrator* ip, const std::vector<int>& idx, size_t tb0,
+                            std::vector<EvalReq>& reqs) {
     const int nw = std::min<int>(kFinishWorkers, (int)idx.size());
     while ((int)ctx->workers.size() < nw) {
         rcmps_context* w = nullptr;
@@ -2222,8 +2378,11 @@ void finish_concurrently(rcmps_context* ctx, const rcmps_integrator* ip, double 
             int code = RCMPS_OK;
             try {
                 code = guard([&] {
-                    finish_state(wc, r, *ctx->tb[tb0 + j], ip, metric_reg, flags);
+                    finish_pullback(wc, r, *ctx->tb[tb0 + j], ip);
                     ck(hipStreamSynchronize(wc->stream));
+                    float pms = 0;
+                    ck(hipEventElapsedTime(&pms, wc->ev[2], wc->ev[3]));
+                    r.S->pullback_ms = pms;
                 });
             } catch (...) {   // nothing may leave a worker thread
                 code = RCMPS_ERR_DEVICE;
@@ -2235,6 +2394,46 @@ void finish_concurrently(rcmps_context* ctx, const rcmps_integrator* ip, double 
     for (int w = 1; w < nw; ++w) threads.emplace_back(work, ctx->workers[w]);
     work(ctx->workers[0]);
     for (auto& t : threads) t.join();
+}
+
+// The rest of evaluations whose pullbacks are done, on the main context: the boundary solves of all of
+// them in one launch (per fused_capacity), then the gradients.
+void finish_pulled_back(rcmps_context* ctx, double metric_reg, int flags, const std::vector<int>& idx, size_t tb0,
+                        std::vector<EvalReq>& reqs) {
+    const bool boundary = !(flags & RCMPS_FLAG_NO_BOUNDARY);
+    const auto t0 = std::chrono::steady_clock::now();
+    std::vector<int> live, fused;   // positions in idx
+    std::vector<RcGmresProb> ps;
+    for (size_t j = 0; j < idx.size(); ++j) {
+        const EvalReq& r = reqs[idx[j]];
+        if (r.S->status != RCMPS_OK || !wants_gradient(r)) continue;
+        live.push_back((int)j);
+        double* fin = ctx->tb[tb0 + j]->fin.d();
+        const size_t mcount = (size_t)r.st->Dp * r.st->Dp * 2;
+        if (boundary && r.st->D > 1 && fused_capacity(ctx, r.st) > 0) {
+            fused.push_back((int)j);
+            ps.push_back(boundary_problem(r.st, fin + 2 * mcount, 1e-13, fin + 4 * mcount));
+        }
+    }
+    std::vector<FusedResult> fr;
+    if (!ps.empty()) fused_solve(ctx, reqs[idx[fused[0]]].st, ps, fr);
+    size_t f = 0;
+    for (int j : live) {
+        EvalReq& r = reqs[idx[j]];
+        TrajBufs& tb = *ctx->tb[tb0 + j];
+        const bool was_fused = f < fused.size() && fused[f] == j;
+        const int code = guard([&] {
+            const size_t mcount = (size_t)r.st->Dp * r.st->Dp * 2;
+            if (was_fused) boundary_result(fr[f], 1e-13, 1e-11, r.S);
+            else if (boundary) boundary_solve(ctx, r.st, tb.fin.d() + 2 * mcount, 1e-13, 1e-11, tb.fin.d() + 4 * mcount, r.S);
+            finish_gradient_part(ctx, r, tb, metric_reg, boundary, nullptr);
+        });
+        if (was_fused) ++f;
+        if (code != RCMPS_OK) r.S->status = code;
+    }
+    ck(hipStreamSynchronize(ctx->stream));
+    const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+    for (int j : live) reqs[idx[j]].S->boundary_ms = ms / live.size();
 }
 
 // The classes run smallest first: a class's finishing then runs under a longer launch, and only the
@@ -2287,23 +2486,34 @@ int fg_phi4_batch_impl(rcmps_context* ctx, std::vector<EvalReq>& reqs, const rcm
         const bool overlap = !krylov && classes.size() > 1;
         // sized before any class starts: a worker thread reads ctx->tb while the next class runs
         while (ctx->tb.size() < (overlap ? 2 : 1) * largest) ctx->tb.emplace_back(new TrajBufs());
+        int pulled = -1;   // the class whose pullbacks run on the workers
+        auto first_buf = [&](size_t c) { return overlap ? (c & 1) * largest : 0; };
+        // its rest on the main context, beside the next class's pullbacks
+        auto finish_rest = [&](int c) {
+            if (c >= 0) finish_pulled_back(ctx, metric_reg, flags, classes[c], first_buf(c), reqs);
+        };
         for (size_t c = 0; c < classes.size(); ++c) {
             const std::vector<int>& idx = classes[c];
             const int Dp = reqs[idx[0]].st->Dp;
-            const size_t tb0 = overlap ? (c & 1) * largest : 0;
+            const size_t tb0 = first_buf(c);
             run_class(ctx, Dp, (flags & RCMPS_FLAG_SPLIT) != 0, krylov, (flags & RCMPS_FLAG_PHASE_TIMERS) != 0,
                       (flags & RCMPS_FLAG_DENSE) == 0, ip, idx, tb0, reqs);
-            join_finisher();   // the previous class's finishing, overlapped with this class's launch
+            join_finisher();   // the previous class's pullbacks, overlapped with this class's launch
+            const int prev = pulled;
+            pulled = -1;
             if (!krylov && can_finish_concurrently(idx, reqs)) {
                 finisher = std::thread([&, c, tb0] {
                     try {
-                        finish_concurrently(ctx, ip, metric_reg, flags, classes[c], tb0, reqs);
+                        pull_back_concurrently(ctx, ip, classes[c], tb0, reqs);
                     } catch (...) {
                         finish_error = std::current_exception();
                     }
                 });
+                pulled = (int)c;
+                finish_rest(prev);
                 continue;
             }
+            finish_rest(prev);
             for (size_t j = 0; j < idx.size(); ++j) {
                 EvalReq& r = reqs[idx[j]];
                 if (r.S->status != RCMPS_OK) continue;
@@ -2329,6 +2539,7 @@ int fg_phi4_batch_impl(rcmps_context* ctx, std::vector<EvalReq>& reqs, const rcm
             }
         }
         join_finisher();
+        finish_rest(pulled);
         } catch (...) {
             if (finisher.joinable()) finisher.join();   // never leave a running thread behind
             throw;
@@ -2505,10 +2716,11 @@ int rcmps_trajectory_samples(rcmps_context* ctx, int system, double* dst, long l
 #define RC_NOALLOC_SCRATCH_BYTES ((size_t)4 << 20)
 #define RC_NOALLOC_MAX_DEVICES 64
 
-// Layout per call (mb = 16 Dp^2 bytes, m = min(D^2, 40) GMRES vectors): padded input and output
-// (2 mb), t1, t2, z, b, x (5 mb), tmp (2 mb), the basis V ((m + 1) mb), w (mb), the Hessenberg column
-// h, then 64 doubles of device scalars.  Everything a kernel reads is written earlier in the same
-// call (pad_in and GMRES clear what has to start at zero), so stale contents never matter.
+// Layout per call (mb = 16 Dp^2 bytes): padded input and output (2 mb), then the fused solve's
+// exchange area and results, or for a state in the Schur form t1, t2, z, b, x (5 mb), tmp
+// (2 mb), the basis V of m = min(D^2, 40) GMRES vectors ((m + 1) mb), w (mb), the Hessenberg column h
+// and 64 doubles of device scalars.  Everything a kernel reads is written earlier in the same call
+// (pad_in, GMRES and the exchange's fill clear what has to start so), so stale contents never matter.
 static __device__ __align__(256) double scratch[RC_NOALLOC_SCRATCH_BYTES / sizeof(double)];
 
 namespace {
@@ -2533,7 +2745,9 @@ size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 // bytes of scratch one boundary solve at padded size Dp with m GMRES vectors takes
 size_t noalloc_boundary_bytes(int Dp, int m) {
     const size_t mb = (size_t)Dp * Dp * 16;
-    return (size_t)(2 + 5 + 2 + (m + 1) + 1) * mb + align256(gmres_col(m) * 8 + 64) + 64 * 8;
+    const size_t schur = (size_t)(5 + 2 + (m + 1) + 1) * mb + align256(gmres_col(m) * 8 + 64) + 64 * 8;
+    const size_t fused = Dp > 64 ? 0 : rc_gmres_exch_bytes(Dp / 16) + 16 * 8;
+    return 2 * mb + std::max(schur, fused);
 }
 
 struct NoAllocScope {
@@ -2562,6 +2776,8 @@ extern "C" int rcmps_boundary_environment_noalloc(rcmps_context* ctx, const rcmp
         double* ap = p; p += md;
         double* hp = p; p += md;
         BoundaryBufs bb{};
+        bb.fexch = p;
+        if (Dp <= 64) bb.fout = p + rc_gmres_exch_bytes(Dp / 16) / 8;
         bb.t1 = p; p += md;
         bb.t2 = p; p += md;
         bb.z = p; p += md;

@@ -155,4 +155,17 @@ __device__ __forceinline__ double wave_sum(double v) {
     return ((read_lane(v, 0) + read_lane(v, 16)) + read_lane(v, 32)) + read_lane(v, 48);
 }
 
+// Record i of a read-only array through scalar loads, so that every field is known wave-uniform.
+template <typename T>
+__device__ __forceinline__ T load_scalar(const T* arr, int i) {
+    static_assert(sizeof(T) % 8 == 0, "records are copied in 8-byte words");
+    const __attribute__((address_space(4))) uint64_t* q =
+        (const __attribute__((address_space(4))) uint64_t*)(arr + __builtin_amdgcn_readfirstlane(i));
+    T t;
+    uint64_t* w = reinterpret_cast<uint64_t*>(&t);
+#pragma unroll
+    for (int k = 0; k < (int)(sizeof(T) / 8); ++k) w[k] = q[k];
+    return t;
+}
+
 }  // namespace

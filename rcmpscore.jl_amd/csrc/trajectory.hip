@@ -60,19 +60,6 @@ struct Lay {
     static constexpr int BYTES = NCPLX * 16 + NDOUBLE_SCRATCH * 8;
 };
 
-// Record i of a read-only array through scalar loads, so that every field is known wave-uniform.
-template <typename T>
-__device__ __forceinline__ T load_scalar(const T* arr, int i) {
-    static_assert(sizeof(T) % 8 == 0, "records are copied in 8-byte words");
-    const __attribute__((address_space(4))) uint64_t* q =
-        (const __attribute__((address_space(4))) uint64_t*)(arr + __builtin_amdgcn_readfirstlane(i));
-    T t;
-    uint64_t* w = reinterpret_cast<uint64_t*>(&t);
-#pragma unroll
-    for (int k = 0; k < (int)(sizeof(T) / 8); ++k) w[k] = q[k];
-    return t;
-}
-
 // ---------------------------------------------------------------------------------------
 // split precision: LDS layout, panel loads into digit planes, wave-split real products
 // ---------------------------------------------------------------------------------------
