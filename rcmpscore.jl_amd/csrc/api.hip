@@ -1257,11 +1257,11 @@ int system_tasks(int s, int NT, bool adjoint, bool quartic_only) {
     return (!adjoint && s % 2) || (quartic_only && s < 4) ? 0 : kLive[s] * NT + (s == 3 ? NT : 0);
 }
 
-// bytes of a system's exchange rings (stage inputs twice, level-1 tiles, E, error records) and of one
-// evaluation's
+// bytes of a system's exchange rings (stage inputs twice, level-1 tiles twice, E, error records) and
+// of one evaluation's
 size_t system_exchange_bytes(int Dp, int s, int ntasks) {
     const size_t mb = (size_t)Dp * Dp * 16;
-    return ntasks == 0 ? 0 : RC_RING * (3 * kLive[s] + (s == 3 ? 1 : 0)) * mb + (size_t)RC_REC_RING * ntasks * RC_REC * 8;
+    return ntasks == 0 ? 0 : RC_RING * (4 * kLive[s] + (s == 3 ? 1 : 0)) * mb + (size_t)RC_REC_RING * ntasks * RC_REC * 8;
 }
 size_t exchange_bytes(int Dp, bool adjoint, bool quartic_only) {
     const int NT = (Dp / 16) * (Dp / 16);
@@ -1376,6 +1376,59 @@ void build_state(rcmps_context* ctx, TrajBufs& tb, char* exch, double* out, cons
     }
 }
 
+// Task of each workgroup of a round over the given systems (at most `capacity` tasks).  Workgroups are
+// dealt to the device's eight XCDs in turn, and an exchange inside one XCD stays in its L2 (the kernel
+// looks where its workgroups really run; this is only where they should): a system goes to one XCD
+// if it fits, the largest first, else channel by channel to as few as possible (a commutator adjoint's E
+// tasks with the channel they read), and what fits no XCD as a whole is spread over the free places.
+void place_tasks(const std::vector<TrajSys>& sys, const std::vector<TrajTask>& tasks, std::vector<int> order,
+                 int capacity, std::vector<int>& out) {
+    constexpr int kXcds = 8;
+    int total = 0;
+    for (int q : order) total += sys[q].ntasks;
+    const int room = capacity / kXcds;
+    std::vector<std::vector<int>> bin(kXcds);
+    std::vector<int> rest;
+    auto place = [&](const std::vector<int>& ts, int prefer) -> int {   // the bin taken, -1: none
+        int best = -1;
+        for (int x = 0; x < kXcds; ++x) {
+            const int free = room - (int)bin[x].size();
+            if ((int)ts.size() > free) continue;
+            if (x == prefer) { best = x; break; }
+            if (best < 0 || free < room - (int)bin[best].size()) best = x;
+        }
+        if (best >= 0) bin[best].insert(bin[best].end(), ts.begin(), ts.end());
+        return best;
+    };
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return sys[a].ntasks > sys[b].ntasks; });
+    for (int q : order) {
+        std::vector<int> all(sys[q].ntasks);
+        for (int i = 0; i < sys[q].ntasks; ++i) all[i] = sys[q].first_task + i;
+        if (place(all, -1) >= 0) continue;
+        int last = -1;
+        for (int ch = sys[q].nlive - 1; ch >= 0; --ch) {
+            std::vector<int> part;
+            for (int i : all)
+                if (tasks[i].ch == ch) part.push_back(i);
+            const int x = place(part, last);
+            if (x < 0) rest.insert(rest.end(), part.begin(), part.end());
+            else last = x;
+        }
+    }
+    size_t deep = 0;
+    for (const auto& b : bin) deep = std::max(deep, b.size());
+    out.assign(std::max((size_t)total, kXcds * deep), -1);
+    for (int x = 0; x < kXcds; ++x)
+        for (size_t i = 0; i < bin[x].size(); ++i) out[kXcds * i + x] = bin[x][i];
+    for (size_t w = 0; !rest.empty(); ++w) {
+        if (w == out.size()) out.push_back(-1);
+        if (out[w] < 0) {
+            out[w] = rest.back();
+            rest.pop_back();
+        }
+    }
+}
+
 // Integrate every system of the given evaluations (all of one padded size Dp) in one persistent
 // launch; states are packed into rounds of at most the resident workgroup count.  Evaluation j
 // keeps its trajectories in ctx->tb[tb0 + j].
@@ -1408,17 +1461,32 @@ void run_class(rcmps_context* ctx, int Dp, bool split, bool quartic_only, bool t
     int capacity = 0;
     ck(rc_trajectory_capacity(NB, split ? 1 : 0, all_z2 ? 1 : 0, timers ? 1 : 0, &capacity));
     // gang schedule: a state's tasks share one round
-    std::vector<std::vector<int>> rounds;
-    int nblocks = 0;
+    std::vector<std::vector<int>> rounds;   // the states of each round
+    int load = 0;
     for (size_t j = 0; j < idx.size(); ++j) {
         if (state_ntasks[j] > capacity) throw Fail{RCMPS_ERR_UNSUPPORTED};
-        if (rounds.empty() || (int)rounds.back().size() + state_ntasks[j] > capacity) rounds.emplace_back();
-        for (int k = 0; k < state_ntasks[j]; ++k) rounds.back().push_back(state_first[j] + k);
-        nblocks = std::max(nblocks, (int)rounds.back().size());
+        if (rounds.empty() || load + state_ntasks[j] > capacity) {
+            rounds.emplace_back();
+            load = 0;
+        }
+        rounds.back().push_back((int)j);
+        load += state_ntasks[j];
     }
-    std::vector<int> sched((size_t)rounds.size() * nblocks, -1);
-    for (size_t r = 0; r < rounds.size(); ++r)
-        for (size_t w = 0; w < rounds[r].size(); ++w) sched[r * nblocks + w] = rounds[r][w];
+    std::vector<std::vector<int>> slots;    // task of each workgroup, by round
+    size_t nblocks = 0;
+    for (const auto& states : rounds) {
+        std::vector<int> order;             // the round's systems
+        for (size_t q = 0; q < sys.size(); ++q)
+            for (int j : states)
+                if (sys[q].ntasks > 0 && sys[q].first_task >= state_first[j] &&
+                    sys[q].first_task < state_first[j] + state_ntasks[j])
+                    order.push_back((int)q);
+        slots.emplace_back();
+        place_tasks(sys, tasks, order, capacity, slots.back());
+        nblocks = std::max(nblocks, slots.back().size());
+    }
+    std::vector<int> sched(rounds.size() * nblocks, -1);
+    for (size_t r = 0; r < rounds.size(); ++r) std::copy(slots[r].begin(), slots[r].end(), sched.begin() + r * nblocks);
 
     TrajParams P{};
     P.Dp = Dp;
@@ -1452,7 +1520,7 @@ void run_class(rcmps_context* ctx, int Dp, bool split, bool quartic_only, bool t
     ck(hipMemsetAsync(ctx->traj_out.p, 0, out_bytes, ctx->stream));
     ck(hipMemsetAsync(ctx->abort_word.p, 0, 256, ctx->stream));
     ck(hipEventRecord(ctx->ev[0], ctx->stream));
-    ck(rc_launch_trajectory(NB, split ? 1 : 0, all_z2 ? 1 : 0, timers ? 1 : 0, nblocks, static_cast<const TrajParams*>(ctx->traj_params.p),
+    ck(rc_launch_trajectory(NB, split ? 1 : 0, all_z2 ? 1 : 0, timers ? 1 : 0, (int)nblocks, static_cast<const TrajParams*>(ctx->traj_params.p),
                             ctx->stream));
     ck(hipEventRecord(ctx->ev[1], ctx->stream));
     std::vector<double> outs(idx.size() * RC_NSYS * RC_OUT_STRIDE);

@@ -76,6 +76,15 @@ __device__ __forceinline__ void st_coh_s(__amdgpu_buffer_rsrc_t r, uint32_t voff
     v.x = (uint32_t)a; v.y = (uint32_t)(a >> 32); v.z = (uint32_t)b; v.w = (uint32_t)(b >> 32);
     __builtin_amdgcn_raw_buffer_store_b128(v, r, voff, soff, RC_COHERENT_POLICY);
 }
+// the same, kept in the L2 of this workgroup's XCD: seen by the device-coherent loads of workgroups there
+__device__ __forceinline__ void st_xcd_s(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, cplx z) {
+    uint64_t a = __builtin_bit_cast(uint64_t, z.re), b = __builtin_bit_cast(uint64_t, z.im);
+    v4u v;
+    v.x = (uint32_t)a; v.y = (uint32_t)(a >> 32); v.z = (uint32_t)b; v.w = (uint32_t)(b >> 32);
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, voff, soff, 0);
+}
+// the XCD this workgroup runs on (hardware register XCC_ID, bits 0..3)
+__device__ __forceinline__ int xcd_id() { return (int)__builtin_amdgcn_s_getreg(20 | (3 << 11)); }
 
 __device__ __forceinline__ double ld_coh_f64(const double* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -6,9 +6,8 @@
 #define RC_MAX_LIVE 4
 #define RC_RING 32          // exchange slots: one per stage event, emptied again 16 events later
 #define RC_REC_RING 4       // slots of the error records: one per attempt
-// word of an empty exchange slot (in all four dwords of a complex): as the high half of a double a
-// quiet NaN with a payload of its own
-#define RC_EMPTY_WORD 0xfffac0deu
+// word of an empty exchange slot (all four dwords of a complex)
+#define RC_EMPTY_WORD 0xffffffffu
 #define RC_REC 16           // doubles per workgroup record: e5, e3, 12 trace partials, spare
 
 // status codes (shared with the C-ABI): 1-5 as the DOP853 controller of the reference GPU
@@ -45,8 +44,9 @@ struct TrajSys {
     int nlive, has_scalar, adj, first_task, ntasks, D;
     double n_elems;          // nlive * D^2 + has_scalar: denominator of the RMS norm
     const double *Q, *Qh, *R, *Rh, *C;   // the state's matrices, Dp x Dp
-    // exchange buffers: Y in two orders and P, each [RC_RING][nlive][Dp*Dp] complex, with has_E
-    // E [RC_RING][Dp*Dp], error records [RC_REC_RING][ntasks][RC_REC] doubles
+    // exchange buffers: Y in two orders, P and P again (for insertions on another XCD), each
+    // [RC_RING][nlive][Dp*Dp] complex, with has_E E [RC_RING][Dp*Dp], error records
+    // [RC_REC_RING][ntasks][RC_REC] doubles
     double* exch;
     uint32_t exch_bytes;
     int has_E;

@@ -23,13 +23,19 @@
 // with device-coherent loads straight into its MFMA fragments and repeats those that are still
 // empty.  An exchange is then one store and one load of device scope, with no wait for the store's
 // completion, no flag and no barrier of the workgroup; the products were a third of a stage and
-// these round trips most of the rest.  Ring of RC_RING events: the step-end all-gather of error
-// records meets at least every 15 events (slots 12..15 and 1..11 of a step), so at event e every
+// these round trips most of the rest.  Ring of RC_RING events: an attempt's error records are posted
+// after stage 11 and taken within the next event (the FSAL stage), so between two takes lie at most
+// 16 events from post to take (stages 12..15 and 1..11, and the FSAL stage again).  At event e every
 // reader is done with event e - 16, whose slot the producer empties again; the slot is used next at
-// event e + 16, and a gather lies between, before which the producer waited for its stores.
+// event e + 16, and a post lies between, before which the producer waited for its stores.
 // The gather is deterministic (every workgroup adds the same records in the same order), so every
 // workgroup of a system takes the same controller decision.  Every wait is bounded by a time
 // budget and watches an abort word.
+//
+// Places: the launch lays a system on one XCD where it fits, and a channel's tiles are then kept in
+// that XCD's L2 (rc_put).  At D = 64 that is 10% of a stage of a system of one or two channels; the
+// longest systems span two XCDs and gain 4%, at D = 32 to 48 it is within the noise, at D = 8 (only
+// insertions are exchanged) 9%.
 //
 // FP64 products read no LDS: each wave runs one k-step of every k-tile, so the operands of its
 // products are fragments it alone needs, loaded from the exchange buffers into registers (the
@@ -38,11 +44,14 @@
 // LDS (every wave needs every row of a panel's digits).  With one tile per channel (Dp = 16) the
 // stage input and P stay in LDS and only what another channel reads is exchanged.
 //
-// What bounds it: two exchanges of about 1.7 us and 2 us of products (64 MFMAs a wave) per stage at
-// D = 64.  Measured on MI355X, per right-hand side of the slowest system, against one flag per
-// tile, a wait for the store and LDS panels: D = 8 5.8 -> 3.0 us, D = 32 with Z2 blocks 7.3 -> 3.7,
-// D = 40 9.1 -> 4.7, D = 64 9.4 -> 5.4 (split 9.5 -> 6.6); six trajectories at D = 64, window 30,
-// 1e-13/1e-12: 62 -> 36 ms.
+// What bounds it: a chain of two exchanges, 1.7 us of matrix instructions (64 a wave, 64 cycles each) and
+// two sums of partial tiles per stage at D = 64, and the wave's own instructions: a check of the arrived
+// words by one running maximum instead of two compares an element is worth 5% of a stage, running sums
+// of the combinations ahead instead of a window of derivatives, the wide gather of records and the FSAL
+// stage ahead of the verdict another 5%.  Measured on MI355X, per right-hand side of the slowest system,
+// against one flag per tile, a wait for the store and LDS panels: D = 8 5.8 -> 2.7 us, D = 32 with Z2
+// blocks 7.3 -> 3.0, D = 40 9.1 -> 4.3, D = 64 9.4 -> 4.5 (split 9.5 -> 5.8); six trajectories at
+// D = 64, window 30, 1e-13/1e-12: 62 -> 30 ms.
 #include "device_common.h"
 #include "exchange.h"
 #include "split.h"
@@ -182,39 +191,99 @@ __device__ __forceinline__ cplx sum_partial_split(const double* red) {
     return cmake(red[t] - red[256 + t], red[512 + t] + red[768 + t]);
 }
 
-// Combinations that follow stage s, without their last term: rows of coefficients for the window of
-// stage derivatives before k_s enters it (k_j at position 16 - s + j, zero elsewhere).  Row s, s in
-// 1..14: the next stage input, A[s + 1]; row 11: the solution, B; 16 and 17: the error estimators E5
-// and E3 (after stage 11); 18..21: the dense output D (after stage 15).
-#define RC_NROWS 22
+// What the derivative of stage s adds to the combinations that still lie ahead of it.  Row s: the
+// coefficients of k_s in the next RC_AHEAD combinations after stage s + 1 (the input of stage s + 2 first;
+// the one after stage 11 is the solution, the FSAL stage's input), then in the error estimators E5 and
+// E3 and the dense output's four rows.
+#define RC_AHEAD 14
 struct RcRows {
-    double c[RC_NROWS][16];
+    double c[RC_NSTAGES_EXT][24];
 };
 constexpr RcRows rc_make_rows() {
     RcRows r{};
-    for (int s = 1; s < RC_NSTAGES_EXT - 1; ++s)
-        for (int j = 0; j < s; ++j) r.c[s][16 - s + j] = s == RC_NSTAGES - 1 ? RC_B[j] : RC_A[s + 1][j];
-    for (int j = 0; j < RC_NSTAGES - 1; ++j) {
-        r.c[16][16 - (RC_NSTAGES - 1) + j] = RC_E5[j];
-        r.c[17][16 - (RC_NSTAGES - 1) + j] = RC_E3[j];
+    for (int s = 0; s < RC_NSTAGES_EXT - 1; ++s) {
+        for (int i = 0; s + 2 + i < RC_NSTAGES_EXT; ++i)
+            r.c[s][i] = s + 2 + i == RC_NSTAGES ? (s < RC_NSTAGES ? RC_B[s] : 0.0) : RC_A[s + 2 + i][s];
+        if (s < RC_NSTAGES) {
+            r.c[s][RC_AHEAD] = RC_E5[s];
+            r.c[s][RC_AHEAD + 1] = RC_E3[s];
+        }
+        for (int q = 0; q < 4; ++q) r.c[s][RC_AHEAD + 2 + q] = RC_D[q][s];
     }
-    for (int q = 0; q < 4; ++q)
-        for (int j = 0; j < RC_NSTAGES_EXT - 1; ++j) r.c[18 + q][1 + j] = RC_D[q][j];
     return r;
 }
 __constant__ const RcRows rc_rows = rc_make_rows();
-
-// sum_q c[row][q] k[q], q increasing (row uniform: the coefficients come through the scalar cache).
-// One loop-free sum for every stage: the zero coefficients cost a few multiply-adds in the shadow of
-// an exchange and spare a branch tree over stages with its own code and constants for each.
-__device__ __forceinline__ cplx rc_row_sum(int row, const cplx* k) {
-    const __attribute__((address_space(4))) double* c =
-        (const __attribute__((address_space(4))) double*)&rc_rows.c[row][0];
-    cplx s = cmake(0, 0);
-#pragma unroll
-    for (int q = 0; q < RC_NSTAGES_EXT; ++q) s = cfma(c[q], k[q], s);
-    return s;
+// coefficients of the trace's derivatives k_j in the solution and the error estimators
+struct RcScalarRows {
+    double c[RC_NSTAGES][4];
+};
+constexpr RcScalarRows rc_make_scalar_rows() {
+    RcScalarRows r{};
+    for (int j = 0; j < RC_NSTAGES; ++j) {
+        r.c[j][0] = RC_B[j];
+        r.c[j][1] = RC_E5[j];
+        r.c[j][2] = RC_E3[j];
+    }
+    return r;
 }
+__constant__ const RcScalarRows rc_scalar_rows = rc_make_scalar_rows();
+
+// The combinations ahead, as running sums in stage order: add(s, k) adds k_s to each and moves them up by
+// one, so that a[0] is all but the last term of the combination after the next stage.  A sum's move is
+// the destination of its multiply-add: no register array is indexed at run time and nothing is shifted
+// (a window of the k_s themselves costs 60 moves a stage for the shift).  The coefficients come through the
+// scalar cache.
+struct RcAhead {
+    cplx a[RC_AHEAD + 1], e5, e3, d[4];
+    __device__ __forceinline__ void clear() {
+        e5 = e3 = cmake(0, 0);
+#pragma unroll
+        for (int i = 0; i <= RC_AHEAD; ++i) a[i] = cmake(0, 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) d[q] = cmake(0, 0);
+    }
+    __device__ __forceinline__ void add(int s, cplx k) {
+        const __attribute__((address_space(4))) double* c =
+            (const __attribute__((address_space(4))) double*)&rc_rows.c[s][0];
+#pragma unroll
+        for (int i = 0; i < RC_AHEAD; ++i) a[i] = cfma(c[i], k, a[i + 1]);
+        e5 = cfma(c[RC_AHEAD], k, e5);
+        e3 = cfma(c[RC_AHEAD + 1], k, e3);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) d[q] = cfma(c[RC_AHEAD + 2 + q], k, d[q]);
+    }
+};
+
+// One attempt's records of every workgroup of the system, for wave 0: lane 8 q + i takes pair q of the
+// records of tasks i, i + 8, .. (those beyond the last repeat it and count nothing).
+struct RcRecords {
+    uint32_t so, pair;
+    int part, ntasks;
+    cplx* v;
+    __device__ __forceinline__ void fetch(__amdgpu_buffer_rsrc_t r) const {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (8 * i < ntasks) v[i] = ld_coh_s(r, (uint32_t)(min(part + 8 * i, ntasks - 1) * RC_REC * 8) + pair, so);
+    }
+    __device__ __forceinline__ bool late() const {
+        uint32_t m = 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (8 * i < ntasks) m = rc_max_word(m, v[i]);
+        return __any(m == RC_EMPTY_WORD);
+    }
+    __device__ __forceinline__ void settle() const {}
+    // the pair's sums over the tasks, on each of the pair's eight lanes
+    __device__ __forceinline__ cplx sum() const {
+        cplx t = cmake(0, 0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (8 * i < ntasks && part + 8 * i < ntasks) t = cadd(t, v[i]);
+        t = cadd(t, cmake(dpp_move<0xB1>(t.re), dpp_move<0xB1>(t.im)));
+        t = cadd(t, cmake(dpp_move<0x4E>(t.re), dpp_move<0x4E>(t.im)));
+        return cadd(t, cmake(dpp_move<0x141>(t.re), dpp_move<0x141>(t.im)));
+    }
+};
 
 }  // namespace
 
@@ -242,7 +311,8 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
     double* scratch = SPLIT ? reinterpret_cast<double*>(smem_raw + LaySplit::SCR)
                             : reinterpret_cast<double*>(sm + L::NCPLX);
     __shared__ int s_bad;   // a wait of this attempt failed (read at the step's end only)
-    __shared__ double s_tot[17];
+    __shared__ int s_loc;   // which of this workgroup's stores stay on the XCD
+    __shared__ double s_verdict[4];   // an attempt's error, step factor, scalar solution; whether a wait failed
     __shared__ double s_err[8];
     __shared__ double s_trp[RC_NSTAGES_EXT][4], s_trs[RC_NSTAGES_EXT];   // trace: wave sums, coefficient
     __shared__ double s_src[2][RC_NSTAGES_EXT];                         // source values, by attempt parity
@@ -275,7 +345,7 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
     // the system's exchange buffers: rings of stage inputs Y (copies A and B), of level-1 tiles P and of
     // E tiles, then the error records
     const __amdgpu_buffer_rsrc_t rX = rc_rsrc(S.exch, S.exch_bytes);
-    const uint32_t oB = RC_RING * stage_stride, oP = 2 * oB, oE = 3 * oB, oR = oE + (S.has_E ? RC_RING * mat_bytes : 0);
+    const uint32_t oB = RC_RING * stage_stride, oP = 2 * oB, oP2 = 3 * oB, oE = 4 * oB, oR = oE + (S.has_E ? RC_RING * mat_bytes : 0);
     const uint32_t el_off = (uint32_t)((row * Dp + col) * 16);
     // The exchange buffers hold whole tiles (tile (r, c) at (r NB + c) TB), each in the order in which
     // its readers' waves take it, so that one load instruction of a wave reads one contiguous 1 KB
@@ -380,18 +450,14 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
     };
 
     // ------------------------------------------------------------------------------------
-    // integrator state.  The stage derivatives of the attempt are kept per element in a window kst
-    // that shifts by one as each arrives (the newest at kst[15]), so no register array is indexed at
-    // run time.  All of a combination (next stage input, solution, error estimators) but its last term
-    // is summed while the stage waits for its neighbours' P tiles, so one multiply-add stands between
-    // a stage's derivative and the next stage input.
+    // integrator state.  All of a combination (next stage input, solution, error estimators) but its last
+    // term is summed while the stages before it wait for their neighbours, so one multiply-add stands
+    // between a stage's derivative and the next stage input.
     // ------------------------------------------------------------------------------------
     const double a = p.a;
-    cplx kst[RC_NSTAGES_EXT];
-#pragma unroll
-    for (int q = 0; q < RC_NSTAGES_EXT; ++q) kst[q] = cmake(0, 0);
+    RcAhead ahead;
+    ahead.clear();
     cplx y = cmake(0, 0), ynew = cmake(0, 0), k0 = cmake(0, 0), k12 = cmake(0, 0);
-    cplx pre5 = cmake(0, 0), pre3 = cmake(0, 0);   // prefix sums of the error estimators
     double ysc = 0.0, ysc_new = 0.0;
     double t = -a, h = fmin(p.h0, 2.0 * a), t_new = t, endpoint = 0.0, factor = 1.0;
     uint32_t ev = 0;
@@ -401,6 +467,42 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
     const __amdgpu_buffer_rsrc_t rS = rc_rsrc(S.samples, (uint32_t)((size_t)p.npoints * S.nlive * mat_bytes));
     const int my_rank = task - S.first_task;
 
+    // Who shares an XCD: every workgroup posts the id of its own (the record of attempt 0) and looks at
+    // those of its partners, so the verdicts agree.  A channel's tiles stay in the L2 when all its tasks
+    // (with the E tasks that read it) run on one XCD; when its insertions' readers do not, they get a
+    // copy of P through memory.
+    if (tid == 0) s_loc = 0;
+    if (wave == 0) {
+        const uint32_t rec0 = (uint32_t)(lane * RC_REC * 8);
+        if (lane == 0) rc_put(rX, (uint32_t)(my_rank * RC_REC * 8), oR, cmake(xcd_id(), 0.0));
+        const bool in = lane < S.ntasks;
+        cplx v;
+        rc_fetch<1>(rX, rec0, oR, 16, &v, in);
+        const bool ok = rc_await<1>(ctl, rX, rec0, oR, 16, &v, in);
+        const int id = (int)v.re;
+        const TrajTask& t = p.tasks[S.first_task + (in ? lane : 0)];
+        const int t_ch = t.ch, t_src = t.edge_from_E || !in ? -1 : t.edge_src;
+        auto tiles = [&](int x) { return rc_same(__ballot(in && t_ch == x), id); };
+        auto inserts = [&](int x) { return rc_same(__ballot(in && (t_ch == x || t_src == x)), id); };
+        int f = 0;
+        if (tiles(ch)) f |= 1;
+        if (inserts(ch)) f |= 2;
+        if (tk.edge_src >= 0 && !tk.edge_from_E && tiles(tk.edge_src) && !inserts(tk.edge_src)) f |= 4;
+        if (rc_same(__ballot(in && (t.e_only || t.edge_from_E)), id)) f |= 8;
+        if (rc_same(__ballot(in), id)) f |= 16;
+        if (__ballot(in && t_src == ch) != 0) f |= 32;
+        if (lane == 0) {
+            s_loc = f;
+            if (!ok) s_bad = 1;
+        }
+    }
+    __syncthreads();
+    const int loc = uni(s_loc);
+    const bool loc_Y = loc & 1, loc_P = LOCAL ? (loc & 2) != 0 : (loc & 1) != 0;   // Dp = 16: P is for insertions only
+    const bool copy_P = !LOCAL && (loc & 35) == 33;           // tiles together, an insertion's reader elsewhere
+    const bool ins_copy = !LOCAL && (loc & 4);                // this task's insertion reads the copy
+    const bool loc_E = loc & 8, loc_R = loc & 16;
+
     // stage input of the next event
     auto publish_Y = [&](cplx v) {
         ++ev;
@@ -408,8 +510,8 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
         if constexpr (LOCAL) Yt[ei * 17 + ej] = v;
         const uint32_t so = (ev & (RC_RING - 1)) * stage_stride + (uint32_t)ch * mat_bytes;
         if (LOCAL ? tk.pub_y : do2) {
-            rc_put(rX, ya_off, so, v);
-            if constexpr (!LOCAL) rc_put(rX, yb_off, oB + so, v);
+            rc_put(rX, ya_off, so, v, loc_Y);
+            if constexpr (!LOCAL) rc_put(rX, yb_off, oB + so, v, loc_Y);
         }
     };
 
@@ -418,14 +520,54 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
         if (ev <= RC_RING / 2) return;
         const uint32_t old = (ev - RC_RING / 2) & (RC_RING - 1), so = old * stage_stride + (uint32_t)ch * mat_bytes;
         if (e_only) {
-            rc_reset(rX, yb_off, oE + old * mat_bytes);
+            rc_reset(rX, yb_off, oE + old * mat_bytes, loc_E);
             return;
         }
         if (LOCAL ? tk.pub_y : do2) {
-            rc_reset(rX, ya_off, so);
-            if constexpr (!LOCAL) rc_reset(rX, yb_off, oB + so);
+            rc_reset(rX, ya_off, so, loc_Y);
+            if constexpr (!LOCAL) rc_reset(rX, yb_off, oB + so, loc_Y);
         }
-        if (LOCAL ? tk.pub_p : do1) rc_reset(rX, pub_off, oP + so);
+        if (LOCAL ? tk.pub_p : do1) {
+            rc_reset(rX, pub_off, oP + so, loc_P);
+            if (copy_P) rc_reset(rX, pub_off, oP2 + so);
+        }
+    };
+
+    // wave 0: the current attempt's records, and from their sums the attempt's verdict (every workgroup adds
+    // the same records in the same order)
+    const uint32_t rec_bytes = (uint32_t)(S.ntasks * RC_REC * 8);
+    constexpr int NREC = (2 + RC_NSTAGES) / 2;   // pairs of a record: (e5, e3), the trace partials of k_0..k_11
+    auto records = [&](cplx* v) {
+        const int q = lane >> 3;
+        return RcRecords{oR + (attempts & (RC_REC_RING - 1)) * rec_bytes,
+                         (uint32_t)(16 * (q < (S.has_scalar ? NREC : 1) ? q : 0)), lane & 7, S.ntasks, v};
+    };
+    auto judge = [&](const RcRecords& recs) {
+        const bool ok = rc_await_all(ctl, rX, recs);
+        const cplx t = recs.sum();
+        double e5 = read_lane(t.re, 0), e3 = read_lane(t.im, 0), sc_new = ysc;
+        if (S.has_scalar) {
+            const int q = lane >> 3, j = min(max(2 * q - 2, 0), RC_NSTAGES - 2);
+            const double *c0 = rc_scalar_rows.c[j], *c1 = rc_scalar_rows.c[j + 1];
+            const bool on = (lane & 7) == 0 && q >= 1 && q < NREC;
+            const double sb = wave_sum(on ? fma(c0[0], t.re, c1[0] * t.im) : 0.0);
+            const double s5 = wave_sum(on ? fma(c0[1], t.re, c1[1] * t.im) : 0.0);
+            const double s3 = wave_sum(on ? fma(c0[2], t.re, c1[2] * t.im) : 0.0);
+            sc_new = fma(h, sb, ysc);
+            const double sc = 1.0 / (p.atol + p.rtol * fmax(fabs(ysc), fabs(sc_new)));
+            e5 = fma(s5 * sc, s5 * sc, e5);
+            e3 = fma(s3 * sc, s3 * sc, e3);
+        }
+        const double den = e5 + 0.01 * e3;
+        const double error = den > 0.0 ? h * e5 / sqrt(den * S.n_elems) : 0.0;
+        // 0.9 error^(-1/8)
+        const double grow = error > 0.0 ? fmin(10.0, 0.9 / sqrt(sqrt(sqrt(error)))) : 10.0;
+        if (lane == 0) {
+            s_verdict[0] = error;
+            s_verdict[1] = grow;
+            s_verdict[2] = sc_new;
+            s_verdict[3] = ok && !s_bad ? 0.0 : 1.0;
+        }
     };
 
     // ------------------------------------------------------------------------------------
@@ -468,9 +610,18 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
                     lds_barrier();
                     Ee = sum_partial(red);
                 }
-                rc_put(rX, yb_off, oE + ring * mat_bytes, Ee);
+                rc_put(rX, yb_off, oE + ring * mat_bytes, Ee, loc_E);
             }
             empty_old();
+            if (slot == RC_NSTAGES) {
+                if (wave == 0) {
+                    cplx rec[8];
+                    RcRecords recs = records(rec);
+                    recs.fetch(rX);
+                    judge(recs);
+                }
+                lds_barrier();
+            }
             k_out = comb_out = cmake(0, 0);
             if (chain) publish_Y(comb_out);
             lap(2);
@@ -524,7 +675,8 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
             lds_barrier();
             Pe = SPLIT ? sum_partial_split(redd1) : sum_partial(red1);
             if constexpr (LOCAL) Pt[ei * 17 + ej] = Pe;
-            if (!LOCAL || tk.pub_p) rc_put(rX, pub_off, oP + so, Pe);
+            if (!LOCAL || tk.pub_p) rc_put(rX, pub_off, oP + so, Pe, loc_P);
+            if (copy_P) rc_put(rX, pub_off, oP2 + so, Pe);
         } else {
             lds_barrier();   // two level-2 sums in a row need a barrier between them
         }
@@ -549,13 +701,13 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
         cplx vp[NF], s1 = cmake(0, 0), s2 = cmake(0, 0);
         const bool insert = do2 && tk.edge_src >= 0;
         const uint32_t so_i = tk.edge_from_E ? oE + ring * mat_bytes
-                                             : oP + ring * stage_stride + (uint32_t)tk.edge_src * mat_bytes;
+                                             : (ins_copy ? oP2 : oP) + ring * stage_stride + (uint32_t)tk.edge_src * mat_bytes;
         if (!LOCAL && do2) rc_fetch<NF>(rX, p_off, oP + so, p_step, vp, use_p);
         if (insert) {
             s1 = ld_coh_s(rX, ins_off, so_i);
             s2 = ld_coh_s(rX, ins_off_t, so_i);
         }
-        // while they arrive: the trace of this stage and the prefix sums
+        // while they arrive: the trace of this stage, the records of the attempt at its FSAL stage
         if (tk.trace_kind) {
             double trv = 0.0;
             if (tk.trace_kind == 2 && b == c && ei == ej && real_el) trv = Pe.re;
@@ -563,13 +715,11 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
             trv = wave_sum(trv);
             if (lane == 0) s_trp[slot][wave] = trv;
         }
-        const cplx pre = rc_row_sum(slot, kst);
-        if (slot == RC_NSTAGES - 1) {
-            pre5 = rc_row_sum(16, kst);
-            pre3 = rc_row_sum(17, kst);
-        }
         const double src = slot == 0 ? rc_source(ts, s_cheb) : unid(s_src[attempts & 1][slot]);
         if (tk.trace_kind && tid == 0) s_trs[slot] = tk.trace_coef * src;
+        cplx rec[8];
+        RcRecords recs = records(rec);
+        if (slot == RC_NSTAGES && wave == 0) recs.fetch(rX);
         lap(3);
         cplx Le = cmake(0, 0);
         if (do2) {
@@ -594,27 +744,28 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
                     const int s2[4] = {sc, sc, sc, sc};
                     rc_split_product(part, pKp, spa, pPb, spb, s2, lane);
                 }
-                put_partial_split(part, redd2, wave, lane);
             } else {
                 if (!adj) frag_product<KT>(acc, vp, Kp);
                 else frag_product<KT>(acc, Kp, vp);
-                put_partial(acc, red2, wave, lane);
             }
+        }
+        if (slot == RC_NSTAGES && wave == 0) judge(recs);   // in the shadow of the products
+        if (do2) {
+            if constexpr (SPLIT) put_partial_split(part, redd2, wave, lane);
+            else put_partial(acc, red2, wave, lane);
             if (insert) {
                 ok = rc_await_all(ctl, rX, RcWant<1>{ins_off, so_i, 0, &s1, true, true},
                                   RcWant<1>{ins_off_t, so_i, 0, &s2, true, true}) && ok;
             }
-            lds_barrier();
-            Le = SPLIT ? sum_partial_split(redd2) : sum_partial(red2);
-        } else {
-            lds_barrier();   // two level-1 sums in a row likewise
         }
+        lds_barrier();   // without level 2: two level-1 sums in a row likewise
+        if (do2) Le = SPLIT ? sum_partial_split(redd2) : sum_partial(red2);
         if (!ok) s_bad = 1;
         const cplx ins = cfma(insert ? tk.edge_coef : 0.0, cadd(s1, cconj(s2)), fixed_e);
         cplx k = cfma(jac, Le, cscale(src, ins));
         if (!real_el) k = cmake(0, 0);
         k_out = k;
-        comb_out = cfma(h, cfma(al, k, pre), y);
+        comb_out = cfma(h, cfma(al, k, ahead.a[0]), y);
         lap(6);
         if (chain) publish_Y(comb_out);
         lap(10);
@@ -631,9 +782,8 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
     while (true) {
         cplx kn, comb;
         ++rhs;
-        // stages 1..10 and, when a quadrature node lies in the step, 12..14 chain to the next one
-        const bool node_due = slot >= RC_NSTAGES && next_point < p.npoints && ld_const(p.points, next_point) <= t_new;
-        const bool chain = slot < RC_NSTAGES - 1 ? slot > 0 : node_due && slot < RC_NSTAGES_EXT - 1;
+        // stages 1..10 chain to the next one, and 13..14 of the dense output's
+        const bool chain = (slot > 0 && slot < RC_NSTAGES - 1) || (slot > RC_NSTAGES && slot < RC_NSTAGES_EXT - 1);
         stage(slot, ts, Yin, s_alast[slot], chain, kn, comb);
         int next = -1;       // -1: start a new step attempt
         bool published = chain, interpolate = false;
@@ -646,12 +796,12 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
         } else if (slot == RC_NSTAGES - 1) {
             lap(7);
             ynew = comb;
-            const cplx acc5 = cfma(RC_E5[RC_NSTAGES - 1], kn, pre5);
-            const cplx acc3 = cfma(RC_E3[RC_NSTAGES - 1], kn, pre3);
+            const cplx acc5 = cfma(RC_E5[RC_NSTAGES - 1], kn, ahead.e5);
+            const cplx acc3 = cfma(RC_E3[RC_NSTAGES - 1], kn, ahead.e3);
             double e5p = 0.0, e3p = 0.0;
             if (real_el) {
-                double sc = p.atol + p.rtol * fmax(cabsd(y), cabsd(ynew));
-                const cplx r5 = cmake(acc5.re / sc, acc5.im / sc), r3 = cmake(acc3.re / sc, acc3.im / sc);
+                const double sc = 1.0 / (p.atol + p.rtol * fmax(cabsd(y), cabsd(ynew)));
+                const cplx r5 = cscale(sc, acc5), r3 = cscale(sc, acc3);
                 e5p = fma(r5.re, r5.re, r5.im * r5.im);
                 e3p = fma(r3.re, r3.re, r3.im * r3.im);
             }
@@ -661,13 +811,11 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
                 s_err[wave] = e5p;
                 s_err[4 + wave] = e3p;
             }
-            // every emptied slot is empty at device scope before the record can be seen
+            // every emptied slot is empty at its scope before the record can be seen
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             lds_barrier();
-            // record for the all-gather: (e5, e3), then the trace partials of k_0..k_11 in pairs
-            const uint32_t rec_bytes = (uint32_t)(S.ntasks * RC_REC * 8);
-            const uint32_t so_rec = oR + (attempts & (RC_REC_RING - 1)) * rec_bytes;
-            constexpr int NREC = (2 + RC_NSTAGES) / 2;
+            // the record, and behind it the FSAL stage on the solution, ahead of the verdict: the records
+            // arrive during that stage (a rejected step's is not counted and its derivative not used)
             if (wave == 0 && lane < (S.has_scalar ? NREC : 1)) {
                 cplx v;
                 if (lane == 0) {
@@ -680,82 +828,32 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
                                       : cmake(0, 0);
                 }
                 const uint32_t off = (uint32_t)(my_rank * RC_REC * 8 + 16 * lane);
-                rc_put(rX, off, so_rec, v);
+                rc_put(rX, off, oR + (attempts & (RC_REC_RING - 1)) * rec_bytes, v, loc_R);
                 // the record of attempt - 2: every workgroup published that of attempt - 1, so all read it
-                rc_reset(rX, off, oR + ((attempts + 2) & (RC_REC_RING - 1)) * rec_bytes);
+                rc_reset(rX, off, oR + ((attempts + 2) & (RC_REC_RING - 1)) * rec_bytes, loc_R);
             }
-            // the FSAL stage's input, published ahead of the verdict (a rejected step's is never read)
-            publish_Y(ynew);
-            if (wave == 0) {
-                // every record in flight at once, then one deterministic reduction per entry
-                cplx v[NREC];
-                const uint32_t off = (uint32_t)(lane * RC_REC * 8);
-                bool ok;
-                if (S.has_scalar) {
-                    rc_fetch<NREC>(rX, off, so_rec, 16, v, lane < S.ntasks);
-                    ok = rc_await<NREC>(ctl, rX, off, so_rec, 16, v, lane < S.ntasks);
-                } else {
-                    rc_fetch<1>(rX, off, so_rec, 16, v, lane < S.ntasks);
-                    ok = rc_await<1>(ctl, rX, off, so_rec, 16, v, lane < S.ntasks);
-                }
-                if (lane == 0) s_tot[16] = ok && !s_bad ? 0.0 : 1.0;
-#pragma unroll
-                for (int q = 0; q < NREC; ++q) {
-                    if (q > 0 && !S.has_scalar) break;
-                    double x = v[q].re, z = v[q].im;
-#pragma unroll
-                    for (int off = 32; off > 0; off >>= 1) {
-                        x += __shfl_xor(x, off);
-                        z += __shfl_xor(z, off);
-                    }
-                    if (lane == 0) {
-                        s_tot[2 * q] = x;
-                        s_tot[2 * q + 1] = z;
-                    }
-                }
-            }
-            lds_barrier();
-            if (!(alive = unid(s_tot[16]) == 0.0)) break;
-            double e5 = unid(s_tot[0]), e3 = unid(s_tot[1]);
-            ysc_new = ysc;
-            if (S.has_scalar) {
-                double sb = 0.0, s5 = 0.0, s3 = 0.0;
-#pragma unroll
-                for (int j = 0; j < RC_NSTAGES; ++j) {
-                    const double kj = unid(s_tot[2 + j]);
-                    sb += RC_B[j] * kj;
-                    s5 += RC_E5[j] * kj;
-                    s3 += RC_E3[j] * kj;
-                }
-                ysc_new = ysc + h * sb;
-                double sc = p.atol + p.rtol * fmax(fabs(ysc), fabs(ysc_new));
-                e5 += (s5 / sc) * (s5 / sc);
-                e3 += (s3 / sc) * (s3 / sc);
-            }
-            const double den = e5 + 0.01 * e3;
-            const double error = den > 0.0 ? h * e5 / sqrt(den * S.n_elems) : 0.0;
             lap(8);
-            if (!isfinite(error)) { status = RC_ST_NONFINITE; break; }
-            factor = error > 0.0 ? fmin(10.0, 0.9 * pow(error, -1.0 / 8.0)) : 10.0;
+            next = RC_NSTAGES;
+        } else if (slot == RC_NSTAGES) {
+            if (!(alive = unid(s_verdict[3]) == 0.0)) break;
+            const double error = unid(s_verdict[0]);
+            factor = unid(s_verdict[1]);
+            ysc_new = unid(s_verdict[2]);
+            if (!isfinite(error)) { --rhs; status = RC_ST_NONFINITE; break; }
             if (error > 1.0) {
+                --rhs;
                 ++rejected;
                 rej = 1;
                 h *= fmax(0.2, factor);
-                empty_old();   // the FSAL event published above is skipped
-                next = -1;
             } else {
                 ++accepted;
                 t_new = (h == endpoint - t) ? endpoint : t + h;
-                next = RC_NSTAGES;   // FSAL stage
-                published = true;
-            }
-        } else if (slot == RC_NSTAGES) {
-            k12 = kn;
-            if (node_due) {
-                ++dense;
-                next = RC_NSTAGES + 1;
-            } else {
-                next = -2;   // finish the accepted step
+                k12 = kn;
+                next = -2;   // finish the accepted step, unless a quadrature node lies in it
+                if (next_point < p.npoints && ld_const(p.points, next_point) <= t_new) {
+                    ++dense;
+                    next = RC_NSTAGES + 1;
+                }
             }
         } else if (slot < RC_NSTAGES_EXT - 1) {
             next = slot + 1;
@@ -806,14 +904,14 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
             if (!published) publish_Y(Yin);
         }
         // behind the publish: the source values of the attempt's stages (one lane each), the dense
-        // output, the window
+        // output, the combinations ahead
         if (next == 1 && !done && tid >= 1 && tid < RC_NSTAGES_EXT)
             s_src[attempts & 1][tid] = rc_source(t + s_cnode[tid] * h, s_cheb);
         if (interpolate) {
             cplx dd[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q)
-                dd[q] = cscale(h_old, cfma(RC_D[q][RC_NSTAGES_EXT - 1], kn, rc_row_sum(18 + q, kst)));
+                dd[q] = cscale(h_old, cfma(RC_D[q][RC_NSTAGES_EXT - 1], kn, ahead.d[q]));
             const cplx d0 = csub(ynew, y_old);
             const cplx d1 = cfma(h_old, k0_old, cmake(-d0.re, -d0.im));
             const cplx d2 = cfma(-h_old, cadd(k12, k0_old), cscale(2.0, d0));
@@ -838,15 +936,8 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
             next_point = uni(next_point);
         }
         if (done) break;
-        if (next == 1) {   // k_0 of a new attempt enters an empty window
-#pragma unroll
-            for (int q = 0; q < RC_NSTAGES_EXT - 1; ++q) kst[q] = cmake(0, 0);
-            kst[RC_NSTAGES_EXT - 1] = k0;
-        } else {
-#pragma unroll
-            for (int q = 0; q < RC_NSTAGES_EXT - 1; ++q) kst[q] = kst[q + 1];
-            kst[RC_NSTAGES_EXT - 1] = kn;
-        }
+        if (next == 1) ahead.clear();
+        ahead.add(next - 1, next == 1 ? k0 : kn);
         slot = uni(next);
     }
     // an attempt cut short by a wait that failed anywhere may end in a nonfinite error norm first

@@ -11,7 +11,9 @@ Against plain numpy in double precision:
   (src/excitation_environments.jl:75-85);
 - the launch sequence on the same state (the Schur form forced) agrees to the sum of the two residuals
   times the inverse's norm, taken as 1e-9 relative (as the existing route test does);
-- evaluations of one batch, whose boundary solves share a launch, equal single calls bit for bit.
+- evaluations of one batch, whose boundary solves share a launch and whose trajectories lie on other
+  XCDs than a single call's (several systems to an XCD, some on two, some spread), equal single calls
+  bit for bit.
 """
 import numpy as np
 import pytest
@@ -101,7 +103,7 @@ def test_excitation_poisson_equations(rg, d):
     s.close()
 
 
-@pytest.mark.parametrize("d", [5, 16, 17, 33])
+@pytest.mark.parametrize("d", [5, 16, 17, 33, 48, 64])
 def test_batched_boundary_solves_equal_single_ones(rg, d):
     note(f"case: batch of 3 at D={d}")
     states = [rg.State(*rg.random_state_arrays(d, scaling=0.2, seed=i)) for i in range(3)]
