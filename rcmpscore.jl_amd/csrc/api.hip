@@ -28,6 +28,7 @@
 
 int rc_trajectory_smem_bytes(int nb, int split);
 hipError_t rc_trajectory_capacity(int nb, int split, int z2, int timed, int* blocks);
+#include "arnoldi.h"
 #include "gmres.h"
 
 hipError_t rc_launch_fill_empty(void* dst, size_t bytes, hipStream_t stream);
@@ -192,6 +193,10 @@ struct rcmps_context {
     // per launch by tiles per side (-1: not asked yet)
     DevBuf gm_exch, gm_prob, gm_out;
     int gm_cap[5] = {-1, -1, -1, -1, -1};
+    // persistent Arnoldi steps (rc_arnoldi): exchange areas, descriptors behind the abort word; bases
+    // per launch by blocks and tiles per side
+    DevBuf arn_exch, arn_prob;
+    int arn_cap[2][5] = {{-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}};
     // GMRES read-back: two pinned slots of one Hessenberg column each, and their completion events
     double* kry_pinned = nullptr;
     size_t kry_pinned_doubles = 0;
@@ -770,6 +775,37 @@ void fused_solve(rcmps_context* ctx, const rcmps_state* st0, std::vector<RcGmres
     }
 }
 
+// Arnoldi steps of every given basis in one launch (or as many as the device holds bases for); false,
+// with nothing done, where rc_arnoldi does not serve them: Dp > 64, or a basis beyond its sum records
+// (the launch sequence then).
+bool arnoldi_steps(rcmps_context* ctx, int Dp, int blocks, std::vector<RcArnProb>& ps) {
+    const int nb = Dp / 16;
+    if (nb > 4) return false;
+    for (const RcArnProb& p : ps)
+        if (p.k1 > RC_ARN_MAX_K) return false;
+    int& cap = ctx->arn_cap[blocks - 1][nb];
+    if (cap < 0) ck(rc_arn_capacity(nb, blocks, &cap));
+    if (cap == 0) return false;
+    const size_t eb = rc_arn_exch_bytes(nb, blocks);
+    for (size_t i0 = 0; i0 < ps.size(); i0 += cap) {
+        const size_t n = std::min(ps.size() - i0, (size_t)cap);
+        ck(ctx->arn_exch.ensure(n * eb));
+        ck(ctx->arn_prob.ensure(256 + n * sizeof(RcArnProb)));
+        char* base = static_cast<char*>(ctx->arn_prob.p);
+        for (size_t i = 0; i < n; ++i) ps[i0 + i].exch = ctx->arn_exch.d() + i * (eb / 8);
+        ck(hipMemsetAsync(base, 0, 256, ctx->stream));
+        ck(hipMemcpyAsync(base + 256, &ps[i0], n * sizeof(RcArnProb), hipMemcpyHostToDevice, ctx->stream));
+        ck(rc_launch_fill_empty(ctx->arn_exch.p, n * eb, ctx->stream));
+        ck(rc_launch_arnoldi(nb, blocks, (int)n, reinterpret_cast<const RcArnProb*>(base + 256),
+                             reinterpret_cast<uint32_t*>(base), (long long)(10.0 * ctx->clock_mhz * 1e6), ctx->stream));
+        uint32_t abort = 0;
+        ck(hipMemcpyAsync(&abort, base, 4, hipMemcpyDeviceToHost, ctx->stream));
+        ck(hipStreamSynchronize(ctx->stream));
+        if (abort) throw Fail{RC_ST_WAIT_LIMIT};
+    }
+    return true;
+}
+
 void state_spectral(rcmps_context* ctx, rcmps_state* st) {
     const int D = st->D, Dp = st->Dp;
     Mat q = download(ctx, D, Dp, st->Q.d());
@@ -954,7 +990,8 @@ void rcmps_context_destroy(rcmps_context* ctx) {
                      &ctx->traj_points, &ctx->abort_word, &ctx->nodes_w, &ctx->nodes_j,
                      &ctx->tmpM, &ctx->partial, &ctx->scratch, &ctx->small, &ctx->kry_V, &ctx->kry_w,
                      &ctx->kry_t1, &ctx->kry_t2, &ctx->kry_x, &ctx->kry_b, &ctx->kry_z, &ctx->kry_h,
-                     &ctx->kry_tmp, &ctx->tune_buf, &ctx->gm_exch, &ctx->gm_prob, &ctx->gm_out};
+                     &ctx->kry_tmp, &ctx->tune_buf, &ctx->gm_exch, &ctx->gm_prob, &ctx->gm_out,
+                     &ctx->arn_exch, &ctx->arn_prob};
     for (auto* b : all) b->release();
     for (auto& b : ctx->tb) b->release();
     if (ctx->blas) (void)rocblas_destroy_handle(ctx->blas);
@@ -1887,8 +1924,24 @@ void basis_extend_multi(rcmps_context* ctx, const rcmps_state* st, Dev& dv, Kryl
     }
     if (maxsteps == 0) return;
     ck(kw.hd4.ensure(total * 16));
-    ck(kw.w4.ensure((size_t)nb * n * 16));
-    for (int s = 0; s < maxsteps; ++s) {
+    std::vector<RcArnProb> ps(nb);
+    for (int i = 0; i < nb; ++i) {
+        RcArnProb& p = ps[i];
+        p = RcArnProb{};
+        p.Q = st->Q.d(); p.Qh = st->Qh.d(); p.R = st->R.d(); p.Rh = st->Rh.d();
+        p.V = bs[i]->V.d();
+        p.hw = kw.hd4.d() + 2 * off[i];
+        p.h1 = p.hw + 2;
+        p.h2 = p.h1 + 2 * (bs[i]->cap + 1);
+        p.hn = p.h2 + 2 * (bs[i]->cap + 1);
+        p.hstride = 2 * (long long)stride[i];
+        p.adj = adj[i] ? 1 : 0;
+        p.k0 = k0[i];
+        p.k1 = k0[i] + nsteps[i];
+    }
+    const bool fused = arnoldi_steps(ctx, dv.Dp, 1, ps);
+    if (!fused) ck(kw.w4.ensure((size_t)nb * n * 16));
+    for (int s = 0; s < maxsteps && !fused; ++s) {
         RcArnBatch B{};
         RcLindbladMulti L{};
         B.n = n;

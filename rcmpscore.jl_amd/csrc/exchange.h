@@ -167,6 +167,47 @@ __device__ __forceinline__ double wave_sum(double v) {
     return ((read_lane(v, 0) + read_lane(v, 16)) + read_lane(v, 32)) + read_lane(v, 48);
 }
 
+// sum over each row of 16 lanes (every lane of the row holds it)
+__device__ __forceinline__ double row_sum(double v) {
+    v += dpp_move<0xB1>(v);
+    v += dpp_move<0x4E>(v);
+    v += dpp_move<0x141>(v);
+    v += dpp_move<0x140>(v);
+    return v;
+}
+
+// The sums of sixteen values over each row of 16 lanes: lane l of the row gets the sum of v[l].  Each
+// step halves the values a lane still carries (it keeps those whose index shares its own next bit and
+// hands over the others), 15 additions and exchanges instead of the 64 of sixteen separate sums.
+template <int CTRL>
+__device__ __forceinline__ double xchg(double x) {   // the value of the lane across the step
+    if constexpr (CTRL == 4) {   // lane ^ 4: rotations of the row by 4 and by 12, by banks of four lanes
+        int lo = __double2loint(x), hi = __double2hiint(x);
+        int l4 = __builtin_amdgcn_update_dpp(0, lo, 0x124, 0xF, 0xA, false);
+        int h4 = __builtin_amdgcn_update_dpp(0, hi, 0x124, 0xF, 0xA, false);
+        l4 = __builtin_amdgcn_update_dpp(l4, lo, 0x12C, 0xF, 0x5, false);
+        h4 = __builtin_amdgcn_update_dpp(h4, hi, 0x12C, 0xF, 0x5, false);
+        return __hiloint2double(h4, l4);
+    } else {
+        return dpp_move<CTRL == 1 ? 0xB1 : CTRL == 2 ? 0x4E : 0x128>(x);
+    }
+}
+template <int CTRL, int N>
+__device__ __forceinline__ void halve(double* v, bool up) {
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+        const double keep = up ? v[2 * i + 1] : v[2 * i], give = up ? v[2 * i] : v[2 * i + 1];
+        v[i] = keep + xchg<CTRL>(give);
+    }
+}
+__device__ __forceinline__ double row_sums16(double* v, int lane) {
+    halve<1, 16>(v, lane & 1);
+    halve<2, 8>(v, lane & 2);
+    halve<4, 4>(v, lane & 4);
+    halve<8, 2>(v, lane & 8);
+    return v[0];
+}
+
 // Record i of a read-only array through scalar loads, so that every field is known wave-uniform.
 template <typename T>
 __device__ __forceinline__ T load_scalar(const T* arr, int i) {
