@@ -79,13 +79,13 @@ struct KrylovBasis {
 // workspace of the infinite-line kinetic backend
 struct KineticWork {
     KrylovBasis basis[4];     // (op R, op [Q,R]) x (forward, adjoint)
-    DevBuf X, A, X2, A2, rhs2, w4, hd4, LX, T, Yd, zd, wd, wzd, res, hd, tmp;
+    DevBuf X, A, X2, A2, rhs2, w4, hd4, LX, T, Yd, zd, wd, wzd, res, hd, tmp, proj;
     int actions = 0;
     double max_res = 0.0;
     double ms[4] = {0.0, 0.0, 0.0, 0.0};   // Arnoldi, projected solves, solutions + residuals, total
     void release() {
         for (auto& b : basis) { b.V.release(); b = KrylovBasis(); }
-        DevBuf* all[] = {&X, &A, &X2, &A2, &rhs2, &w4, &hd4, &LX, &T, &Yd, &zd, &wd, &wzd, &res, &hd, &tmp};
+        DevBuf* all[] = {&X, &A, &X2, &A2, &rhs2, &w4, &hd4, &LX, &T, &Yd, &zd, &wd, &wzd, &res, &hd, &tmp, &proj};
         for (auto* d : all) d->release();
     }
 };
@@ -2072,6 +2072,57 @@ bool projected_solutions(const KrylovBasis& b, const std::vector<double>& z, std
     return true;
 }
 
+// The projected solves of several bases at every node on the device (rc_projected): y of node i of basis b
+// at Y + (first[b] + i ld[b]) complex, the estimates est[b nz + i].  False, with nothing done, when a
+// basis is larger than the kernel's (then on host threads).
+struct ProjJob {
+    const std::vector<cd>* H;   // (cap + 1) x cap, row-major
+    int cap, k, ld;             // k = 0: zeros
+    double beta;
+    long long first;
+};
+bool projected_device(rcmps_context* ctx, const std::vector<ProjJob>& jobs, int nz, double* Y, std::vector<double>& est) {
+    KineticWork& kw = ctx->kin;
+    const int n = (int)jobs.size();
+    int maxk = 0;
+    size_t total = 0;
+    for (const ProjJob& j : jobs) {
+        maxk = std::max(maxk, j.k);
+        total += (size_t)j.k * (j.k + 3) / 2;
+    }
+    if (maxk > RC_PROJ_MAX_K) return false;
+    est.assign((size_t)n * nz, 0.0);
+    const size_t hb = std::max<size_t>(total, 1) * 16, pb = (size_t)n * sizeof(RcProjProb);
+    ck(kw.proj.ensure(hb + pb + est.size() * 8));
+    double* dH = kw.proj.d();
+    RcProjProb* dp = reinterpret_cast<RcProjProb*>(dH + hb / 8);
+    double* de = reinterpret_cast<double*>(dp + n);
+    std::vector<char> host(hb + pb);
+    cd* h = reinterpret_cast<cd*>(host.data());
+    RcProjProb* p = reinterpret_cast<RcProjProb*>(host.data() + hb);
+    size_t off = 0;
+    for (int b = 0; b < n; ++b) {
+        const ProjJob& j = jobs[b];
+        p[b] = RcProjProb{dH + 2 * off, Y + 2 * j.first, de + (size_t)b * nz, j.beta, j.k, j.ld};
+        for (int c = 0; c < j.k; ++c)
+            for (int r = 0; r <= c + 1; ++r) h[off++] = (*j.H)[(size_t)r * j.cap + c];
+    }
+    ck(hipMemcpyAsync(dH, host.data(), host.size(), hipMemcpyHostToDevice, ctx->stream));
+    ck(rc_launch_projected(n, maxk, dp, nz, kw.zd.d(), ctx->stream));
+    ck(hipMemcpyAsync(est.data(), de, est.size() * 8, hipMemcpyDeviceToHost, ctx->stream));
+    ck(hipStreamSynchronize(ctx->stream));
+    return true;
+}
+// the largest of a basis's estimates; false if one is not finite (a singular or nonfinite solve)
+bool worst_estimate(const double* e, int nz, double& est) {
+    est = 0.0;
+    for (int i = 0; i < nz; ++i) {
+        if (!std::isfinite(e[i])) return false;
+        est = std::max(est, e[i]);
+    }
+    return true;
+}
+
 // Shifted solutions X_i = (I - z_i L)^{-1} rhs (or L*) for all nodes, each accepted on its true
 // relative residual (kinetic_krylov.jl:114-155).  X: nz matrices at stride Dp^2.  Every job (one
 // basis, its right-hand side and direction) runs its own sequence of tests; the extensions the
@@ -2088,38 +2139,52 @@ struct KinJob {
     bool done;
     bool form = false;       // the projected solves passed: form and check the node solutions
     bool terminal = false;
-    std::vector<cd> Y;       // projected solutions, k per node
+    double* Yd = nullptr;    // projected solutions on the device, k per node
+    std::vector<cd> Y;       // or on the host
 };
 
-// The host part of one pass of a job's tests (kinetic_krylov.jl:114-155): the projected solves.  It
-// leaves the job asking for a larger basis, or with projected solutions to form (form), or failed
-// (neither: a terminal basis whose projected solves did not pass).
-void kinetic_project(const rcmps_kinetic_options& o, int maxdim, int initdim, KinJob& jb,
-                     const std::vector<double>& z, const std::vector<double>& zone) {
-    KrylovBasis& b = *jb.b;
-    jb.want = 0;
-    jb.form = false;
-    if (b.k == 0) {
-        jb.want = initdim;
-        return;
+// One pass of a job's tests (kinetic_krylov.jl:114-155) on its projected solves: it leaves the job asking
+// for a larger basis, or with projected solutions to form (form), or failed (neither: a terminal
+// basis whose projected solves did not pass).
+void kinetic_judge(const rcmps_kinetic_options& o, int maxdim, KinJob& jb, bool ok, double est) {
+    jb.form = ok && (est <= o.tolerance || jb.terminal);
+    jb.want = !jb.form && !jb.terminal ? std::min(2 * jb.b->k, maxdim) : 0;
+}
+void kinetic_project(rcmps_context* ctx, const rcmps_kinetic_options& o, int maxdim, int initdim,
+                     std::vector<KinJob*>& pending, const std::vector<double>& z) {
+    KineticWork& kw = ctx->kin;
+    const int nz = (int)z.size();
+    std::vector<KinJob*> js;
+    std::vector<ProjJob> pj;
+    long long first = 0;
+    for (KinJob* jb : pending) {
+        const KrylovBasis& b = *jb->b;
+        jb->form = false;
+        jb->want = initdim;
+        if (b.k == 0) continue;
+        jb->terminal = b.exhausted || b.k >= maxdim;
+        js.push_back(jb);
+        pj.push_back(ProjJob{&b.H, b.cap, b.k, b.k, b.beta, first});
+        first += (long long)b.k * nz;
     }
-    const int k = b.k;
-    jb.terminal = b.exhausted || k >= maxdim;
-    double est = 0;
-    // the node of largest z alone first: when its projected residual (one term of the full test)
-    // misses the tolerance on a basis that can grow, the basis extends without the other nodes' solves
-    if (!jb.terminal && z.size() > 1) {
-        if (!projected_solutions(b, zone, jb.Y, est, 1) || est > o.tolerance) {
-            jb.want = std::min(2 * k, maxdim);
-            return;
+    if (js.empty()) return;
+    ck(kw.Yd.ensure((size_t)first * 16));
+    std::vector<double> est;
+    if (projected_device(ctx, pj, nz, kw.Yd.d(), est)) {
+        for (size_t q = 0; q < js.size(); ++q) {
+            double e = 0;
+            const bool ok = worst_estimate(est.data() + q * nz, nz, e);
+            js[q]->Yd = kw.Yd.d() + 2 * pj[q].first;
+            kinetic_judge(o, maxdim, *js[q], ok, e);
         }
-    }
-    const bool ok = projected_solutions(b, z, jb.Y, est, kProjectedThreads);
-    if (ok && (est <= o.tolerance || jb.terminal)) {
-        jb.form = true;
         return;
     }
-    if (!jb.terminal) jb.want = std::min(2 * k, maxdim);
+    for (KinJob* jb : js) {
+        double e = 0;
+        const bool ok = projected_solutions(*jb->b, z, jb->Y, e, kProjectedThreads);
+        jb->Yd = nullptr;
+        kinetic_judge(o, maxdim, *jb, ok, e);
+    }
 }
 
 // The device part: form the node solutions of a job whose projected solves passed and accept them on
@@ -2130,10 +2195,9 @@ void kinetic_form(rcmps_context* ctx, const rcmps_state* st, Dev& dv, KinJob& jb
     const rcmps_kinetic_options& o = ctx->kopt;
     KrylovBasis& b = *jb.b;
     const int n = dv.n(), k = b.k;
-    ck(kw.Yd.ensure(jb.Y.size() * 16));
-    ck(hipMemcpyAsync(kw.Yd.p, jb.Y.data(), jb.Y.size() * 16, hipMemcpyHostToDevice, ctx->stream));
+    if (!jb.Yd) ck(hipMemcpyAsync(kw.Yd.p, jb.Y.data(), jb.Y.size() * 16, hipMemcpyHostToDevice, ctx->stream));
     hipLaunchKernelGGL(rc_basis_combine, dim3(ceil_div(n, 256), ceil_div(nz, 8)), dim3(256), 0, ctx->stream, b.V.d(),
-                       (long long)n, k, kw.Yd.d(), nz, n, jb.X);
+                       (long long)n, k, jb.Yd ? jb.Yd : kw.Yd.d(), nz, n, jb.X);
     ck(hipGetLastError());
     lindblad_batched(dv, st, jb.X, kw.LX.d(), kw.T.d(), nz, jb.adj);
     hipLaunchKernelGGL(rc_shifted_residual, dim3(nz), dim3(256), 0, ctx->stream, jb.X, kw.LX.d(), jb.rhs, kw.zd.d(), n,
@@ -2154,7 +2218,7 @@ void kinetic_form(rcmps_context* ctx, const rcmps_state* st, Dev& dv, KinJob& jb
     jb.want = std::min(2 * k, maxdim);
 }
 
-// Every round: the projected solves of all pending jobs at once (one host thread per job), then their
+// Every round: the projected solves of all pending jobs at once, then their
 // node solutions on the device one job after the other, then the extensions they ask for together.
 void kinetic_solutions(rcmps_context* ctx, const rcmps_state* st, Dev& dv, std::vector<KinJob>& jobs,
                        const std::vector<double>& z) {
@@ -2176,10 +2240,6 @@ void kinetic_solutions(rcmps_context* ctx, const rcmps_state* st, Dev& dv, std::
     ck(kw.zd.ensure((size_t)nz * 8));
     ck(kw.res.ensure((size_t)nz * 8));
     ck(hipMemcpyAsync(kw.zd.d(), z.data(), (size_t)nz * 8, hipMemcpyHostToDevice, ctx->stream));
-    int zhard = 0;
-    for (int i = 1; i < nz; ++i)
-        if (std::fabs(z[i]) > std::fabs(z[zhard])) zhard = i;
-    const std::vector<double> zone(1, z[zhard]);
     using clock = std::chrono::steady_clock;
     auto since = [](clock::time_point t0) { return std::chrono::duration<double, std::milli>(clock::now() - t0).count(); };
     for (;;) {
@@ -2188,23 +2248,7 @@ void kinetic_solutions(rcmps_context* ctx, const rcmps_state* st, Dev& dv, std::
             if (!jb.done) pending.push_back(&jb);
         if (pending.empty()) return;
         auto t0 = clock::now();
-        if (pending.size() == 1) {
-            kinetic_project(o, maxdim, initdim, *pending[0], z, zone);
-        } else {
-            std::vector<std::thread> threads;
-            std::vector<std::exception_ptr> errs(pending.size());
-            for (size_t q = 0; q < pending.size(); ++q)
-                threads.emplace_back([&, q] {
-                    try {
-                        kinetic_project(o, maxdim, initdim, *pending[q], z, zone);
-                    } catch (...) {   // nothing may leave a host thread
-                        errs[q] = std::current_exception();
-                    }
-                });
-            for (auto& t : threads) t.join();
-            for (auto& e : errs)
-                if (e) std::rethrow_exception(e);
-        }
+        kinetic_project(ctx, o, maxdim, initdim, pending, z);
         kw.ms[1] += since(t0);
         KrylovBasis* bs[4];
         bool adj[4];

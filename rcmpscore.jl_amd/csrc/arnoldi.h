@@ -32,3 +32,18 @@ __host__ __device__ inline size_t rc_arn_exch_bytes(int nb, int blocks) {
 hipError_t rc_arn_capacity(int nb, int blocks, int* bases);
 hipError_t rc_launch_arnoldi(int nb, int blocks, int n, const RcArnProb* probs, uint32_t* abort_flag,
                              long long wait_ticks, hipStream_t stream);
+
+#define RC_PROJ_MAX_K 512
+
+// Projected solves (I - z_i H_k) y_i = beta e_1 of one basis: H upper Hessenberg with its row k, column c
+// (rows 0 .. c + 1) at complex offset c (c + 3) / 2; y_i at Y + i ldy complex, zero from k on; est[i]
+// the Arnoldi residual estimate |z_i h_{k+1,k} y_i[k-1]| / beta, not finite when the solve is singular
+struct RcProjProb {
+    const double* H;
+    double* Y;
+    double* est;
+    double beta;
+    int k, ldy;   // k <= RC_PROJ_MAX_K; 0: zeros
+};
+// every basis at every node z_i, i < nz; maxk: the largest k among them
+hipError_t rc_launch_projected(int n, int maxk, const RcProjProb* probs, int nz, const double* z, hipStream_t stream);

@@ -3,7 +3,8 @@
 - kinetic1/kinetic2 (one-block bases of L and L*) from a basis grown in one call (up to 40 vectors in
   registers, later ones in memory) against one grown by doubling from 3, and against 300 steps asked for
   at once, which is beyond the kernel's sum records and takes the launch sequence; D = 65 takes that
-  anyway.  Every solve is accepted at a true residual of 1e-12: values to 1e-11, gradients to 1e-8 of
+  anyway.  The projected solves (rc_projected) meet one to eight rows a lane that way, and 600 vectors
+  (D = 33) their host route.  Every solve is accepted at a true residual of 1e-12: values to 1e-11, gradients to 1e-8 of
   their largest entry (the bars of the route's oracle tests).
 - the excitation action's kinetic part (two-block bases) against the dense resolvents of the same state,
   to 1e-8 of |F| with solves accepted at 1e-11 (as the route's batch test).
@@ -32,8 +33,8 @@ def test_basis_sizes_agree(rg, d):
     r, k = rg.random_state_arrays(d, scaling=0.2, seed=11)
     s = rg.State(r, k, steady_tol=1e-12)
     out = []
-    for initial in (3, min(100, d * d), min(300, d * d)):
-        o = rg.KineticKrylovOptions(initialdim=initial)
+    for initial in (3, min(100, d * d), min(300, d * d)) + ((600,) if d == 33 else ()):
+        o = rg.KineticKrylovOptions(initialdim=initial, maxdim=max(512, initial))
         (v1, g1), st = rg.kinetic1(s, krylov_options=o, return_stats=True)
         v2, g2 = rg.kinetic2(s, krylov_options=o)
         note(f"  initial {initial}: basis {st['kinetic_basis']}, residual {st['kinetic_residual']:.2e}")
