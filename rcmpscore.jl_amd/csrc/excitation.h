@@ -174,3 +174,5 @@ __global__ void rc_trace_axpy(int n, int nj, int nodes, const double* tr, const 
                               const double* Z, double* X);
 __global__ void rc_trace_axpy_n(int n, int nj, int nodes, const double* tr, const double* wz, double scale,
                                 const double* Z, long long sz, double* X, long long sx);
+__global__ void rc_parity_flags(int D, int Dp, const double* w, const double* v, long long ts, int* flags);
+__global__ void rc_parity_project(int D, int Dp, int parity, double* x, long long ts);

@@ -1297,3 +1297,33 @@ __global__ void __launch_bounds__(256) rc_pair_rhs(RcPairArgs g) {
         g.partial[2 * slot + 1] = s3[0];
     }
 }
+
+// Which parity blocks (halves of the basis) of the tangents' matrices hold a nonzero: bit 0 of
+// flags[i] an even block of W, bit 1 an odd one, bits 2 and 3 the same of v.  Matrix i at + i ts complex.
+__global__ void __launch_bounds__(256) rc_parity_flags(int D, int Dp, const double* w, const double* v, long long ts,
+                                                       int* flags) {
+    __shared__ int s;
+    if (threadIdx.x == 0) s = 0;
+    __syncthreads();
+    const long long off = (long long)blockIdx.x * ts;
+    const cplx* a = reinterpret_cast<const cplx*>(w) + off;
+    const cplx* b = reinterpret_cast<const cplx*>(v) + off;
+    int f = 0;
+    for (int e = threadIdx.x; e < D * D; e += 256) {
+        const int i = e / D, j = e % D, odd = (i < D / 2) != (j < D / 2) ? 1 : 0;
+        const cplx x = a[(long long)i * Dp + j], y = b[(long long)i * Dp + j];
+        if (x.re != 0.0 || x.im != 0.0) f |= 1 << odd;
+        if (y.re != 0.0 || y.im != 0.0) f |= 4 << odd;
+    }
+    atomicOr(&s, f);
+    __syncthreads();
+    if (threadIdx.x == 0) flags[blockIdx.x] = s;
+}
+// X_i: the blocks of the other parity set to zero
+__global__ void __launch_bounds__(256) rc_parity_project(int D, int Dp, int parity, double* x, long long ts) {
+    cplx* a = reinterpret_cast<cplx*>(x) + (long long)blockIdx.y * ts;
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= D * D) return;
+    const int i = e / D, j = e % D, odd = (i < D / 2) != (j < D / 2) ? 1 : 0;
+    if (odd != parity) a[(long long)i * Dp + j] = cmake(0, 0);
+}
