@@ -1413,61 +1413,128 @@ void build_state(rcmps_context* ctx, TrajBufs& tb, char* exch, double* out, cons
     }
 }
 
-// Task of each workgroup of a round over the given systems (at most `capacity` tasks).  Workgroups are
-// dealt to the device's eight XCDs in turn, and an exchange inside one XCD stays in its L2 (the kernel
-// looks where its workgroups really run; this is only where they should): a system goes to one XCD
-// if it fits, the largest first, else channel by channel to as few as possible (a commutator adjoint's E
-// tasks with the channel they read), and what fits no XCD as a whole is spread over the free places.
-void place_tasks(const std::vector<TrajSys>& sys, const std::vector<TrajTask>& tasks, std::vector<int> order,
-                 int capacity, std::vector<int>& out) {
+// The tasks of each workgroup, in the order it runs them: list scheduling of the launch's systems on at
+// most `capacity` workgroups, the longest first, each where it can end first.  All workgroups' lists
+// follow one order of the systems, so the first unfinished system always has all of its workgroups.
+// Lengths are unknown before the launch; kLength holds the systems' right-hand sides relative to the
+// longest's, as measured over D = 8 to 64 (0.50 to 0.75, 0.78 to 0.89, ...).  Against one state
+// after the other, a round as long as its longest system, 48 states of D = 8 to 64 take 231 -> 194 ms.
+//
+// Workgroups are dealt to the device's eight XCDs in turn, and an exchange inside one XCD stays in its
+// L2 (the kernel looks where its workgroups really run; this is only where they should): a system goes
+// to one XCD, or channel by channel to several (a commutator adjoint's E tasks with the channel they
+// read), or anywhere, taken as 5% and 10% slower than the first.
+bool schedule_tasks(const std::vector<TrajSys>& sys, const std::vector<TrajTask>& tasks, int capacity,
+                    std::vector<std::vector<int>>& lists) {
     constexpr int kXcds = 8;
-    int total = 0;
-    for (int q : order) total += sys[q].ntasks;
+    static const double kLength[RC_NSYS] = {0.6, 0.82, 0.72, 1.0, 0.6, 0.94};
     const int room = capacity / kXcds;
-    std::vector<std::vector<int>> bin(kXcds);
-    std::vector<int> rest;
-    auto place = [&](const std::vector<int>& ts, int prefer) -> int {   // the bin taken, -1: none
-        int best = -1;
-        for (int x = 0; x < kXcds; ++x) {
-            const int free = room - (int)bin[x].size();
-            if ((int)ts.size() > free) continue;
-            if (x == prefer) { best = x; break; }
-            if (best < 0 || free < room - (int)bin[best].size()) best = x;
-        }
-        if (best >= 0) bin[best].insert(bin[best].end(), ts.begin(), ts.end());
-        return best;
+    struct Place {
+        int x, w;   // XCD and workgroup within it; without whole XCDs: one of `capacity` single ones
     };
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return sys[a].ntasks > sys[b].ntasks; });
+    using Free = std::vector<std::vector<double>>;   // when each workgroup is free
+    Free free_at(kXcds, std::vector<double>(room, 0.0));
+    if (room == 0) free_at.assign(1, std::vector<double>(capacity, 0.0));
+    const int nx = (int)free_at.size();
+    lists.assign((size_t)nx * free_at[0].size(), {});
+    std::vector<int> order;
+    for (size_t q = 0; q < sys.size(); ++q)
+        if (sys[q].ntasks > 0) order.push_back((int)q);
+    auto length = [&](int q) { return kLength[q % RC_NSYS]; };
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return length(a) > length(b); });
+    // n workgroups of the candidates by the earliest start, among those the latest free; the start
+    auto take = [](std::vector<std::pair<double, Place>> c, int n, std::vector<Place>& out) -> double {
+        auto by_time = [](const std::pair<double, Place>& a, const std::pair<double, Place>& b) { return a.first < b.first; };
+        std::stable_sort(c.begin(), c.end(), by_time);
+        const double start = c[n - 1].first;
+        size_t last = n;
+        while (last < c.size() && c[last].first <= start) ++last;
+        for (size_t i = last - n; i < last; ++i) out.push_back(c[i].second);
+        return start;
+    };
+    auto of_xcd = [&](const Free& f, int x) {
+        std::vector<std::pair<double, Place>> c;
+        for (int w = 0; w < (int)f[x].size(); ++w) c.push_back({f[x][w], Place{x, w}});
+        return c;
+    };
+    // the XCD where n workgroups are free first (then: `prefer`, then the busiest); its start, -1: none has n
+    auto best_xcd = [&](const Free& f, int n, int prefer, std::vector<Place>& out, int& at) -> double {
+        at = -1;
+        double start = 0.0, busy = 0.0;
+        std::vector<Place> pick;
+        for (int x = 0; x < nx && n <= room; ++x) {
+            std::vector<Place> p;
+            const double t = take(of_xcd(f, x), n, p);
+            double b = 0.0;
+            for (double v : f[x]) b += v > t ? 1.0 : 0.0;
+            if (at < 0 || t < start || (t == start && at != prefer && (x == prefer || b > busy))) {
+                at = x;
+                start = t;
+                busy = b;
+                pick = p;
+            }
+        }
+        if (at < 0) return -1.0;
+        out.insert(out.end(), pick.begin(), pick.end());
+        return start;
+    };
+    const double never = 1e300;
     for (int q : order) {
-        std::vector<int> all(sys[q].ntasks);
-        for (int i = 0; i < sys[q].ntasks; ++i) all[i] = sys[q].first_task + i;
-        if (place(all, -1) >= 0) continue;
+        const int n = sys[q].ntasks;
+        std::vector<int> all(n);
+        for (int i = 0; i < n; ++i) all[i] = sys[q].first_task + i;
+        // on one XCD
+        std::vector<Place> one, many, spread;
+        std::vector<int> many_tasks;
+        int at;
+        double t1 = best_xcd(free_at, n, -1, one, at);
+        if (t1 < 0) t1 = never;
+        // channel by channel
+        double t2 = 0.0;
+        Free f = free_at;
         int last = -1;
-        for (int ch = sys[q].nlive - 1; ch >= 0; --ch) {
+        for (int ch = sys[q].nlive - 1; ch >= 0 && t2 < never; --ch) {
             std::vector<int> part;
             for (int i : all)
                 if (tasks[i].ch == ch) part.push_back(i);
-            const int x = place(part, last);
-            if (x < 0) rest.insert(rest.end(), part.begin(), part.end());
-            else last = x;
+            std::vector<Place> p;
+            const double t = best_xcd(f, (int)part.size(), last, p, at);
+            if (t < 0) {
+                t2 = never;
+                break;
+            }
+            t2 = std::max(t2, t);
+            last = at;
+            for (size_t i = 0; i < part.size(); ++i) {
+                f[p[i].x][p[i].w] = never;
+                many.push_back(p[i]);
+                many_tasks.push_back(part[i]);
+            }
+        }
+        if (t2 >= never) t2 = never;
+        // anywhere
+        std::vector<std::pair<double, Place>> c;
+        for (int x = 0; x < nx; ++x) {
+            auto cx = of_xcd(free_at, x);
+            c.insert(c.end(), cx.begin(), cx.end());
+        }
+        const double t3 = n <= (int)c.size() ? take(c, n, spread) : never;
+        const double len = length(q), e1 = t1 + len, e2 = t2 + 1.05 * len, e3 = t3 + 1.1 * len;
+        if (std::min(t1, std::min(t2, t3)) >= never) return false;   // more tasks than workgroups
+        const bool use1 = e1 <= e2 && e1 <= e3, use2 = !use1 && e2 <= e3;
+        const std::vector<Place>& p = use1 ? one : use2 ? many : spread;
+        const std::vector<int>& ts = use2 ? many_tasks : all;
+        const double end = use1 ? e1 : use2 ? e2 : e3;
+        for (int i = 0; i < n; ++i) {
+            lists[(size_t)nx * p[i].w + p[i].x].push_back(ts[i]);
+            free_at[p[i].x][p[i].w] = end;
         }
     }
-    size_t deep = 0;
-    for (const auto& b : bin) deep = std::max(deep, b.size());
-    out.assign(std::max((size_t)total, kXcds * deep), -1);
-    for (int x = 0; x < kXcds; ++x)
-        for (size_t i = 0; i < bin[x].size(); ++i) out[kXcds * i + x] = bin[x][i];
-    for (size_t w = 0; !rest.empty(); ++w) {
-        if (w == out.size()) out.push_back(-1);
-        if (out[w] < 0) {
-            out[w] = rest.back();
-            rest.pop_back();
-        }
-    }
+    return true;
 }
 
 // Integrate every system of the given evaluations (all of one padded size Dp) in one persistent
-// launch; states are packed into rounds of at most the resident workgroup count.  Evaluation j
+// launch of at most the resident workgroup count.  Evaluation j
 // keeps its trajectories in ctx->tb[tb0 + j].
 void run_class(rcmps_context* ctx, int Dp, bool split, bool quartic_only, bool timers, bool z2,
                const rcmps_integrator* ip, const std::vector<int>& idx, size_t tb0, std::vector<EvalReq>& reqs) {
@@ -1479,7 +1546,6 @@ void run_class(rcmps_context* ctx, int Dp, bool split, bool quartic_only, bool t
     // k-tile: the same bits)
     bool all_z2 = z2;
     for (int i : idx) all_z2 = all_z2 && reqs[i].st->z2_tiles > 0;
-    std::vector<int> state_first, state_ntasks;
     size_t exch_bytes = 0;
     for (int i : idx) exch_bytes += exchange_bytes(Dp, reqs[i].adjoint(), quartic_only);
     const size_t out_bytes = idx.size() * RC_NSYS * RC_OUT_STRIDE * 8;
@@ -1487,48 +1553,27 @@ void run_class(rcmps_context* ctx, int Dp, bool split, bool quartic_only, bool t
     ck(ctx->traj_out.ensure(out_bytes));
     char* exch = static_cast<char*>(ctx->traj_exch.p);
     for (size_t j = 0; j < idx.size(); ++j) {
-        const int first = (int)tasks.size();
         const EvalReq& r = reqs[idx[j]];
         build_state(ctx, *ctx->tb[tb0 + j], exch, ctx->traj_out.d() + j * RC_NSYS * RC_OUT_STRIDE, r.st, r.adjoint(),
                     quartic_only, all_z2, npts, sys, tasks);
         exch += exchange_bytes(Dp, r.adjoint(), quartic_only);
-        state_first.push_back(first);
-        state_ntasks.push_back((int)tasks.size() - first);
     }
     int capacity = 0;
     ck(rc_trajectory_capacity(NB, split ? 1 : 0, all_z2 ? 1 : 0, timers ? 1 : 0, &capacity));
-    // gang schedule: a state's tasks share one round
-    std::vector<std::vector<int>> rounds;   // the states of each round
-    int load = 0;
-    for (size_t j = 0; j < idx.size(); ++j) {
-        if (state_ntasks[j] > capacity) throw Fail{RCMPS_ERR_UNSUPPORTED};
-        if (rounds.empty() || load + state_ntasks[j] > capacity) {
-            rounds.emplace_back();
-            load = 0;
-        }
-        rounds.back().push_back((int)j);
-        load += state_ntasks[j];
-    }
-    std::vector<std::vector<int>> slots;    // task of each workgroup, by round
-    size_t nblocks = 0;
-    for (const auto& states : rounds) {
-        std::vector<int> order;             // the round's systems
-        for (size_t q = 0; q < sys.size(); ++q)
-            for (int j : states)
-                if (sys[q].ntasks > 0 && sys[q].first_task >= state_first[j] &&
-                    sys[q].first_task < state_first[j] + state_ntasks[j])
-                    order.push_back((int)q);
-        slots.emplace_back();
-        place_tasks(sys, tasks, order, capacity, slots.back());
-        nblocks = std::max(nblocks, slots.back().size());
-    }
-    std::vector<int> sched(rounds.size() * nblocks, -1);
-    for (size_t r = 0; r < rounds.size(); ++r) std::copy(slots[r].begin(), slots[r].end(), sched.begin() + r * nblocks);
+    std::vector<std::vector<int>> lists;
+    if (!schedule_tasks(sys, tasks, capacity, lists)) throw Fail{RCMPS_ERR_UNSUPPORTED};
+    while (!lists.empty() && lists.back().empty()) lists.pop_back();
+    const size_t nblocks = lists.size();
+    size_t nrounds = 0;
+    for (const auto& l : lists) nrounds = std::max(nrounds, l.size());
+    std::vector<int> sched(nrounds * nblocks, -1);
+    for (size_t w = 0; w < nblocks; ++w)
+        for (size_t r = 0; r < lists[w].size(); ++r) sched[r * nblocks + w] = lists[w][r];
 
     TrajParams P{};
     P.Dp = Dp;
     P.npoints = npts;
-    P.nrounds = (int)rounds.size();
+    P.nrounds = (int)nrounds;
     P.a = std::sqrt(ip->max_point);
     P.atol = ip->atol;
     P.rtol = ip->rtol;

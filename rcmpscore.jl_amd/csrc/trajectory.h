@@ -54,9 +54,10 @@ struct TrajSys {
     double* out;             // [32]: status/counters, then phase timers of workgroup 0
 };
 
-// One launch integrates the systems of one or more states of the same padded size Dp.  Tasks
-// are gang-scheduled in rounds: workgroup w runs task schedule[r * nblocks + w] (or idles, -1)
-// in round r, and all tasks of a system share a round, so every wait is on a running partner.
+// One launch integrates the systems of one or more states of the same padded size Dp.  Workgroup w
+// runs tasks schedule[r * nblocks + w], r = 0, 1, .. (-1: none), one after the other; the lists of all
+// workgroups follow one order of the systems, so a wait is on a partner that is running, or will be
+// once systems earlier in that order have ended.
 struct TrajParams {
     int Dp, npoints, nrounds, pad;
     double a, atol, rtol, h0;
