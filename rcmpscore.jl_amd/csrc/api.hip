@@ -30,6 +30,7 @@ int rc_trajectory_smem_bytes(int nb, int split);
 hipError_t rc_trajectory_capacity(int nb, int split, int z2, int timed, int* blocks);
 #include "arnoldi.h"
 #include "gmres.h"
+#include "pullback.h"
 
 hipError_t rc_launch_fill_empty(void* dst, size_t bytes, hipStream_t stream);
 hipError_t rc_launch_trajectory(int nb, int split, int z2, int timed, int nblocks, const TrajParams* dparams, hipStream_t stream);
@@ -1688,111 +1689,90 @@ void finish_pullback(rcmps_context* ctx, EvalReq& r, TrajBufs& tb, const rcmps_i
     // pullback (src/observables.jl:161-199) in reduced channels
     // ----------------------------------------------------------------------------------
     ck(hipEventRecord(ctx->ev[2], ctx->stream));
-    ck(ctx->tmpM.ensure((size_t)nn * mb));
+    const int NB = Dp / 16, streams = rc_pull_streams(NB);
     ck(ctx->scratch.ensure(12 * mb));
     ck(tb.fin.ensure(5 * mb));
-    double* M = ctx->tmpM.d();
-    double* T1 = ctx->scratch.d();
-    double* T2 = T1 + mcount;
-    double* U = T1 + 2 * mcount;
-    double* X1 = T1 + 3 * mcount;
-    double* X2 = T1 + 4 * mcount;
-    double* cterm = T1 + 5 * mcount;
-    double* tmp = T1 + 6 * mcount;
-    double* tmp2 = T1 + 7 * mcount;
+    double* S1 = ctx->scratch.d();
+    double* Z = S1 + mcount;
+    double* W = S1 + 2 * mcount;
+    double* S2 = S1 + 3 * mcount;
+    double* U = S1 + 4 * mcount;
+    double* cterm = S1 + 5 * mcount;
     double* XR = tb.fin.d();
     double* XQ = XR + mcount;
     double* env = XR + 2 * mcount;
     double* cov = XR + 3 * mcount;
-    ck(hipMemsetAsync(XR, 0, 3 * mb, ctx->stream));
     const long long node = (long long)Dp * Dp;   // complex elements per matrix
-    for (int term = kin_cov ? 2 : 0; term < 3; ++term) {
+    // With F_1 = rho, A_5 = I (and for the kinetic terms F_2^+, A_2^+ as the third channel):
+    //   XQ = rho S1 + sum c T2,   XR = rho (R^+ S1 + Z) + W + sum c T1,
+    // T1 and T2 the sums over the channels that have samples on both sides (rc_pullback), S1 = sum c w A_1,
+    // and the edges' halves with a constant matrix: Z = j A_2 beside rho, W = j F beside I.  A kinetic
+    // term's edge operator has the coefficient u = sqrt2 (rho sum j A2 + (sum j F2)^+): op = R adds u
+    // to XR; op = C = QR - RQ, dC = dQ R + Q dR - dR Q - R dQ, adds (u Q - Q u, R u - u R).
+    RcPullArgs pa{};
+    RcLinArgs la{};
+    auto lin = [&](int o, const double* X, long long s, double c, int kind, int conj) {
+        la.src[o][la.nsrc[o]++] = RcLinSource{X, s, c, kind, conj};
+    };
+    double* louts[RC_LIN_OUTS] = {S1, Z, W, env, S2, U};
+    la.nouts = kin_cov ? 4 : 6;
+    int ne = 0, nt = 0, work[RC_PULL_TERMS] = {0, 0, 0}, total = 0;
+    for (int term = kin_cov ? 2 : 0; term < 3; ++term, ++nt) {
         const int sf = 2 * term, sa = sf + 1;
-        const int lf = kLive[sf], la = kLive[sa];
+        const int lf = kLive[sf], lad = kLive[sa];
         const double* Fs = tb.samples[sf].d();
         const double* As = tb.samples[sa].d();
-        const long long fstride = lf * node, astride = la * node;
+        const long long fstride = lf * node, astride = lad * node;
         // adjoint sample of node i is at index nn-1-i: base at nn-1, negative stride
         auto Aptr = [&](int ch) { return As + 2 * ((long long)(nn - 1) * astride + ch * node); };
         auto Fptr = [&](int ch) { return Fs + 2 * (ch * node); };
-        ck(hipMemsetAsync(T1, 0, 3 * mb, ctx->stream));   // T1, T2, U
+        auto entry = [&](const double* F, const double* A, const double* Dm, double jk, int conj) {
+            pa.e[ne++] = RcPullEntry{F, A, Dm, fstride, -astride, jk, conj, 0};
+            ++work[nt];
+            ++total;
+        };
+        const double c = coef[term];
+        pa.first[nt] = ne;
+        pa.c[nt] = c;
+        lin(0, Aptr(0), -astride, c, 0, 0);
         if (term < 2) {
-            // k = 1 (F1 = rho):  T1 += rho R^+ (sum w A1), T2 += rho (sum w A1)
-            hipLaunchKernelGGL(rc_lincomb, dim3(ceil_div(dv.n(), 64)), dim3(64), 0, ctx->stream, Aptr(0), -astride,
-                               ctx->nodes_w.d(), nn, dv.n(), 0.0, X1);
-            hipLaunchKernelGGL(rc_lincomb, dim3(ceil_div(dv.n(), 64)), dim3(64), 0, ctx->stream, Aptr(1), -astride,
-                               ctx->nodes_j.d(), nn, dv.n(), 0.0, X2);           // sum j A2
-            hipLaunchKernelGGL(rc_lincomb, dim3(ceil_div(dv.n(), 64)), dim3(64), 0, ctx->stream, Fptr(0), fstride,
-                               ctx->nodes_j.d(), nn, dv.n(), 0.0, tmp2);         // sum j F2
-            ck(hipGetLastError());
-            dv.gemm(0, st->Rh.d(), 0, X1, tmp);
-            dv.gemm(0, st->rho.d(), 0, tmp, T1);
-            dv.gemm(0, st->rho.d(), 0, X1, T2);
-            // k = 2: F2 (w R^+ A2), w F2 A2 ; k = 3: F2^+ (w R^+ A2^+), w F2^+ A2^+
-            for (int k3 = 0; k3 < 2; ++k3) {
-                GemmArgs gb{};
-                gb.opA = 0; gb.A = st->Rh.d(); gb.strideA = 0;
-                gb.opB = k3; gb.B = Aptr(1); gb.strideB = -astride;
-                gb.C = M; gb.strideC = node;
-                gb.alpha = ctx->nodes_w.d(); gb.alpha_stride = 1;
-                dv.batched(gb, nn);
-                GemmArgs gr{};
-                gr.opA = k3; gr.A = Fptr(0); gr.strideA = fstride;
-                gr.opB = 0; gr.B = M; gr.strideB = node;
-                dv.reduce(gr, nn, T1, 1.0, 1.0);
-                GemmArgs g2{};
-                g2.opA = k3; g2.A = Fptr(0); g2.strideA = fstride;
-                g2.opB = k3; g2.B = Aptr(1); g2.strideB = -astride;
-                g2.alpha = ctx->nodes_w.d(); g2.alpha_stride = 1;
-                dv.reduce(g2, nn, T2, 1.0, 1.0);
-            }
-            // u = sqrt2 (rho sum j A2 + (sum j F2)^+), the coefficient of the edge operator
-            dv.gemm(0, st->rho.d(), 0, X2, U, s2);
-            dv.herm(1, s2, tmp2, tmp);
-            dv.axpby(cd(1, 0), U, cd(1, 0), tmp, U);
-            if (term == 0) {
-                dv.axpby(cd(1, 0), T1, cd(1, 0), U, T1);           // op = R
-            } else {
-                // op = C = QR - RQ: dC = dQ R + Q dR - dR Q - R dQ
-                dv.gemm(0, U, 0, st->Q.d(), T1, 1.0, 1.0);
-                dv.gemm(0, st->Q.d(), 0, U, T1, -1.0, 1.0);
-                dv.gemm(0, st->R.d(), 0, U, T2, 1.0, 1.0);
-                dv.gemm(0, U, 0, st->R.d(), T2, -1.0, 1.0);
-            }
+            entry(Fptr(0), Aptr(1), nullptr, 0.0, 0);
+            entry(Fptr(0), Aptr(1), nullptr, 0.0, 1);
+            lin(term == 0 ? 1 : 4, Aptr(1), -astride, s2 * c, 1, 0);
+            lin(term == 0 ? 2 : 5, Fptr(0), fstride, s2 * c, 1, 1);
         } else {
-            // phi^4: sum_k F_k (w R^+ A_k + j k A_{k+1}) - (sum_k w F_k A_k) R^+,  F_1 = rho, A_5 = I
-            for (int k = 1; k <= 4; ++k) {
-                GemmArgs gb{};
-                gb.opA = 0; gb.A = st->Rh.d(); gb.strideA = 0;
-                gb.opB = 0; gb.B = Aptr(k - 1); gb.strideB = -astride;
-                gb.C = M; gb.strideC = node;
-                gb.alpha = ctx->nodes_w.d(); gb.alpha_stride = 1;
-                gb.dalpha = ctx->nodes_j.d(); gb.dscale = k;
-                if (k < 4) { gb.addD = Aptr(k); gb.strideD = -astride; }
-                else gb.add_identity = 4.0;
-                dv.batched(gb, nn);
-                GemmArgs gr{};
-                gr.opA = 0;
-                gr.A = k == 1 ? st->rho.d() : Fptr(k - 2);
-                gr.strideA = k == 1 ? 0 : fstride;
-                gr.opB = 0; gr.B = M; gr.strideB = node;
-                dv.reduce(gr, nn, T1, 1.0, 1.0);
-                GemmArgs g2{};
-                g2.opA = 0;
-                g2.A = k == 1 ? st->rho.d() : Fptr(k - 2);
-                g2.strideA = k == 1 ? 0 : fstride;
-                g2.opB = 0; g2.B = Aptr(k - 1); g2.strideB = -astride;
-                g2.alpha = ctx->nodes_w.d(); g2.alpha_stride = 1;
-                dv.reduce(g2, nn, T2, 1.0, 1.0);
-            }
+            for (int k = 2; k <= 4; ++k) entry(Fptr(k - 2), Aptr(k - 1), k < 4 ? Aptr(k) : nullptr, k, 0);
+            lin(1, Aptr(1), -astride, c, 1, 0);
+            lin(2, Fptr(2), fstride, 4 * c, 1, 0);
         }
         // environment: hermitised adjoint channel 1 at the endpoint
         const double* aend = As + 2 * ((long long)nn * astride);
-        dv.herm(0, 1.0, aend, tmp);
-        const double c = coef[term];
-        dv.axpby(cd(1, 0), XR, cd(c, 0), T1, XR);
-        dv.axpby(cd(1, 0), XQ, cd(c, 0), T2, XQ);
-        dv.axpby(cd(1, 0), env, cd(c, 0), tmp, env);
+        lin(3, aend, 0, 0.5 * c, 2, 0);
+        lin(3, aend, 0, 0.5 * c, 2, 1);
+    }
+    pa.first[nt] = ne;
+    pa.nterms = nt;
+    // about a workgroup per CU, the terms' shares by their pairs; no more streams than nodes
+    for (int t = 0; t < nt; ++t)
+        pa.wg0[t + 1] = pa.wg0[t] + std::max(1, std::min(ceil_div(nn, streams), 256 * work[t] / total));
+    pa.Rh = st->Rh.d();
+    pa.wn = la.wn = ctx->nodes_w.d();
+    pa.jn = la.jn = ctx->nodes_j.d();
+    pa.nn = la.nn = nn;
+    ck(ctx->partial.ensure((size_t)pa.wg0[nt] * streams * 2 * mb));
+    pa.partial = ctx->partial.d();
+    for (int o = 0; o < RC_LIN_OUTS; ++o) la.out[o] = louts[o];
+    ck(rc_launch_lin(Dp, la, ctx->stream));
+    ck(rc_launch_pullback(NB, pa, W, XR, XQ, ctx->stream));
+    dv.gemm(0, st->Rh.d(), 0, S1, Z, 1.0, 1.0);
+    dv.gemm(0, st->rho.d(), 0, Z, XR, 1.0, 1.0);
+    dv.gemm(0, st->rho.d(), 0, S1, XQ, 1.0, 1.0);
+    if (!kin_cov) {
+        dv.gemm(0, st->rho.d(), 0, S2, U, 1.0, 1.0);
+        dv.gemm(0, U, 0, st->Q.d(), XR, 1.0, 1.0);
+        dv.gemm(0, st->Q.d(), 0, U, XR, -1.0, 1.0);
+        dv.gemm(0, st->R.d(), 0, U, XQ, 1.0, 1.0);
+        dv.gemm(0, U, 0, st->R.d(), XQ, -1.0, 1.0);
     }
     if (kin_env) dv.axpby(cd(1, 0), env, cd(1, 0), kin_env, env);
     covector(dv, st, XR, XQ, kin_cov, cterm, cov);
