@@ -243,6 +243,7 @@ struct rcmps_state {
     // Z2 symmetry under diag(1, .., 1, -1, .., -1) (D/2 each): R odd, K and rho0 even, exactly.  When
     // the parity blocks are whole 16 x 16 tiles, z2_tiles = D / 32 (tiles per parity block), else 0.
     int z2_tiles = 0;
+    double opnorm_sum = 0.0;   // 2 |Q| + |R|^2 (spectral norms)
     DevBuf R, K, Q, Qh, Rh, C, Ch, rho, V, Vinv, lam, ident;
     DevBuf VH, VinvH;   // V^+ and V^-+ for the fused two-sided products of the eigenbasis form
     // eigendecomposition L = W diag(mu) W^-1 of the transfer superoperator on the padded Dp^2 space
@@ -834,6 +835,7 @@ void state_spectral(rcmps_context* ctx, rcmps_state* st) {
         rc::matmul(D, Winv, rc::adjoint(D, Z), Vinv);
     }
     double nq = rc::opnorm2(D, q), nr = rc::opnorm2(D, r);
+    st->opnorm_sum = 2 * nq + nr * nr;
     double scale = std::max(1.0, std::max(nq, nr * nr));
     double maxre = -INFINITY;
     std::vector<double> lam((size_t)Dp * 2, 0.0);
@@ -858,7 +860,8 @@ void state_spectral(rcmps_context* ctx, rcmps_state* st) {
 }
 
 // checked_density (src/transfer.jl:33-47) on the host copy; returns the normalised density
-bool checked_density(int D, const Mat& q, const Mat& r, Mat& rho, double tol) {
+// (opnorm_sum: 2 |Q| + |R|^2)
+bool checked_density(int D, const Mat& q, const Mat& r, double opnorm_sum, Mat& rho, double tol) {
     for (auto& z : rho)
         if (!std::isfinite(z.real()) || !std::isfinite(z.imag())) return false;
     cd z = 0;
@@ -882,12 +885,12 @@ bool checked_density(int D, const Mat& q, const Mat& r, Mat& rho, double tol) {
     rc::matmul(D, r, rho, t3);
     rc::matmul(D, t3, rc::adjoint(D, r), t4);
     for (size_t i = 0; i < l.size(); ++i) l[i] = t1[i] + t2[i] + t4[i];
-    double scale = std::max(1.0, 2 * rc::opnorm2(D, q) + std::pow(rc::opnorm2(D, r), 2));
+    double scale = std::max(1.0, opnorm_sum);
     if (!(fro(l) <= tol * scale)) return false;
-    Mat T = rho, Z;
-    if (!rc::schur(D, T, Z)) return false;
+    std::vector<cd> lam;
+    if (!rc::eigenvalues(D, rho, lam)) return false;
     double mn = INFINITY;
-    for (int i = 0; i < D; ++i) mn = std::min(mn, T[(size_t)i * D + i].real());
+    for (const cd& x : lam) mn = std::min(mn, x.real());
     return mn >= -10 * tol;
 }
 
@@ -1119,7 +1122,7 @@ int rcmps_state_create(rcmps_context* ctx, int D, const double* R, const double*
             if (!okg && !(res <= steady_tol)) throw Fail{RCMPS_ERR_SOLVER};
             rho_h = download(ctx, D, Dp, st->rho.d());
         }
-        if (!checked_density(D, qh, rh, rho_h, steady_tol)) throw Fail{RCMPS_ERR_SOLVER};
+        if (!checked_density(D, qh, rh, st->opnorm_sum, rho_h, steady_tol)) throw Fail{RCMPS_ERR_SOLVER};
         upload(ctx, D, Dp, rho_h, st->rho.d());
         st->rho_host = rho_h;
         st->z2_tiles = z2_tiles_of(D, rh, kh, rho_h);

@@ -6,7 +6,24 @@
 
 namespace rc {
 
-static inline cd at(const Mat& A, int n, int i, int j) { return A[(size_t)i * n + j]; }
+// Products written out: std::complex's operator* checks every product for NaN and calls the runtime, which
+// keeps the loops scalar (a Schur form at D = 64 took twice as long).
+static inline cd mul(cd a, cd b) {
+    return cd(a.real() * b.real() - a.imag() * b.imag(), a.real() * b.imag() + a.imag() * b.real());
+}
+// conj(a) b
+static inline cd cmul(cd a, cd b) {
+    return cd(a.real() * b.real() + a.imag() * b.imag(), a.real() * b.imag() - a.imag() * b.real());
+}
+// (x, y) <- (c x + s y, -conj(s) x + c y) over n elements
+static inline void rotate(cd* x, cd* y, int n, double c, cd s) {
+    const double sr = s.real(), si = s.imag();
+    for (int j = 0; j < n; ++j) {
+        const double xr = x[j].real(), xi = x[j].imag(), yr = y[j].real(), yi = y[j].imag();
+        x[j] = cd(c * xr + (sr * yr - si * yi), c * xi + (sr * yi + si * yr));
+        y[j] = cd(c * yr - (sr * xr + si * xi), c * yi - (sr * xi - si * xr));
+    }
+}
 
 void matmul(int n, const Mat& A, const Mat& B, Mat& C) {
     C.assign((size_t)n * n, cd(0, 0));
@@ -14,7 +31,7 @@ void matmul(int n, const Mat& A, const Mat& B, Mat& C) {
         for (int k = 0; k < n; ++k) {
             cd a = A[(size_t)i * n + k];
             if (a == cd(0, 0)) continue;
-            for (int j = 0; j < n; ++j) C[(size_t)i * n + j] += a * B[(size_t)k * n + j];
+            for (int j = 0; j < n; ++j) C[(size_t)i * n + j] += mul(a, B[(size_t)k * n + j]);
         }
 }
 
@@ -35,10 +52,15 @@ static void rotation(cd x, cd y, double& c, cd& s) {
     s = (x / ax) * std::conj(y) / r;
 }
 
-bool schur(int n, Mat& A, Mat& Z) {
-    Z.assign((size_t)n * n, cd(0, 0));
-    for (int i = 0; i < n; ++i) Z[(size_t)i * n + i] = 1;
-    std::vector<cd> v(n);
+// QR iteration on A; ZT: the transposed unitary factor (its columns are rows here, so that a rotation of
+// two of them is a contiguous loop), or null: then A's diagonal holds the eigenvalues and the rest
+// of it is not meaningful (only the window at hand is rotated).
+static bool schur_impl(int n, Mat& A, Mat* ZT) {
+    if (ZT) {
+        ZT->assign((size_t)n * n, cd(0, 0));
+        for (int i = 0; i < n; ++i) (*ZT)[(size_t)i * n + i] = 1;
+    }
+    std::vector<cd> v(n), w(n);
     // Householder reduction to upper Hessenberg form
     for (int k = 0; k + 2 < n; ++k) {
         double alpha = 0;
@@ -54,23 +76,26 @@ bool schur(int n, Mat& A, Mat& Z) {
         for (int i = k + 1; i < n; ++i) vn += std::norm(v[i]);
         if (vn == 0) continue;
         const double f = 2.0 / vn;
-        for (int j = 0; j < n; ++j) {
-            cd s = 0;
-            for (int i = k + 1; i < n; ++i) s += std::conj(v[i]) * A[(size_t)i * n + j];
-            s *= f;
-            for (int i = k + 1; i < n; ++i) A[(size_t)i * n + j] -= v[i] * s;
-        }
+        // A -= v (f v^H A), row by row
+        std::fill(w.begin(), w.end(), cd(0, 0));
+        for (int i = k + 1; i < n; ++i)
+            for (int j = 0; j < n; ++j) w[j] += cmul(v[i], A[(size_t)i * n + j]);
+        for (int j = 0; j < n; ++j) w[j] *= f;
+        for (int i = k + 1; i < n; ++i)
+            for (int j = 0; j < n; ++j) A[(size_t)i * n + j] -= mul(v[i], w[j]);
         for (int i = 0; i < n; ++i) {
             cd s = 0;
-            for (int j = k + 1; j < n; ++j) s += A[(size_t)i * n + j] * v[j];
+            for (int j = k + 1; j < n; ++j) s += mul(A[(size_t)i * n + j], v[j]);
             s *= f;
-            for (int j = k + 1; j < n; ++j) A[(size_t)i * n + j] -= s * std::conj(v[j]);
+            for (int j = k + 1; j < n; ++j) A[(size_t)i * n + j] -= cmul(v[j], s);
         }
-        for (int i = 0; i < n; ++i) {
-            cd s = 0;
-            for (int j = k + 1; j < n; ++j) s += Z[(size_t)i * n + j] * v[j];
-            s *= f;
-            for (int j = k + 1; j < n; ++j) Z[(size_t)i * n + j] -= s * std::conj(v[j]);
+        if (ZT) {   // Z -= (f Z v) v^H: ZT's rows are Z's columns
+            std::fill(w.begin(), w.end(), cd(0, 0));
+            for (int j = k + 1; j < n; ++j)
+                for (int i = 0; i < n; ++i) w[i] += mul((*ZT)[(size_t)j * n + i], v[j]);
+            for (int i = 0; i < n; ++i) w[i] *= f;
+            for (int j = k + 1; j < n; ++j)
+                for (int i = 0; i < n; ++i) (*ZT)[(size_t)j * n + i] -= cmul(v[j], w[i]);
         }
         for (int i = k + 2; i < n; ++i) A[(size_t)i * n + k] = 0;
     }
@@ -96,31 +121,38 @@ bool schur(int n, Mat& A, Mat& Z) {
         cd mu = std::abs(m1 - d) < std::abs(m2 - d) ? m1 : m2;
         if (iter % 11 == 10) mu = d + std::abs(A[(size_t)hi * n + hi - 1]) * 1.5;
         cd x = A[(size_t)lo * n + lo] - mu, y = A[(size_t)(lo + 1) * n + lo];
+        const int jend = ZT ? n : hi + 1, ibegin = ZT ? 0 : lo;
         for (int k = lo; k < hi; ++k) {
             if (k > lo) { x = A[(size_t)k * n + k - 1]; y = A[(size_t)(k + 1) * n + k - 1]; }
             double cg; cd sg;
             rotation(x, y, cg, sg);
-            for (int j = (k > lo ? k - 1 : lo); j < n; ++j) {
-                cd t1 = A[(size_t)k * n + j], t2 = A[(size_t)(k + 1) * n + j];
-                A[(size_t)k * n + j] = cg * t1 + sg * t2;
-                A[(size_t)(k + 1) * n + j] = -std::conj(sg) * t1 + cg * t2;
-            }
-            int imax = std::min(k + 2, hi);
-            for (int i = 0; i <= imax; ++i) {
-                cd t1 = A[(size_t)i * n + k], t2 = A[(size_t)i * n + k + 1];
-                A[(size_t)i * n + k] = cg * t1 + std::conj(sg) * t2;
-                A[(size_t)i * n + k + 1] = -sg * t1 + cg * t2;
-            }
-            for (int i = 0; i < n; ++i) {
-                cd t1 = Z[(size_t)i * n + k], t2 = Z[(size_t)i * n + k + 1];
-                Z[(size_t)i * n + k] = cg * t1 + std::conj(sg) * t2;
-                Z[(size_t)i * n + k + 1] = -sg * t1 + cg * t2;
-            }
+            const int j0 = k > lo ? k - 1 : lo;
+            rotate(&A[(size_t)k * n + j0], &A[(size_t)(k + 1) * n + j0], jend - j0, cg, sg);
+            const int imax = std::min(k + 2, hi);
+            for (int i = ibegin; i <= imax; ++i) rotate(&A[(size_t)i * n + k], &A[(size_t)i * n + k + 1], 1, cg, std::conj(sg));
+            if (ZT) rotate(&(*ZT)[(size_t)k * n], &(*ZT)[(size_t)(k + 1) * n], n, cg, std::conj(sg));
             if (k > lo) A[(size_t)(k + 1) * n + k - 1] = 0;
         }
     }
     for (int i = 0; i < n; ++i)
         for (int j = 0; j < i; ++j) A[(size_t)i * n + j] = 0;
+    return true;
+}
+
+bool schur(int n, Mat& A, Mat& Z) {
+    Mat ZT;
+    if (!schur_impl(n, A, &ZT)) return false;
+    Z.resize((size_t)n * n);
+    for (int i = 0; i < n; ++i)
+        for (int j = 0; j < n; ++j) Z[(size_t)i * n + j] = ZT[(size_t)j * n + i];
+    return true;
+}
+
+bool eigenvalues(int n, const Mat& A, std::vector<cd>& lam) {
+    Mat T = A;
+    if (!schur_impl(n, T, nullptr)) return false;
+    lam.resize(n);
+    for (int i = 0; i < n; ++i) lam[i] = T[(size_t)i * n + i];
     return true;
 }
 
@@ -192,28 +224,44 @@ bool inverse(int n, const Mat& A_in, Mat& X) {
 }
 
 double opnorm2(int n, const Mat& A) {
-    std::vector<cd> x(n), y(n);
+    // power iteration on A^H A, 300 steps: all but the last three eight at a time on its eighth power (three
+    // squarings cost what a hundred steps on A do, and 37 steps replace 296)
+    Mat B, C;
+    matmul(n, adjoint(n, A), A, B);
+    for (int p = 0; p < 4; ++p) {
+        double f = 0;
+        for (auto& v : B) f += std::norm(v);
+        f = std::sqrt(f);
+        if (!(f > 0)) return f;
+        for (auto& v : B) v /= f;
+        if (p == 3) break;
+        matmul(n, B, B, C);
+        B.swap(C);
+    }
+    std::vector<cd> x(n), z(n);
     for (int i = 0; i < n; ++i) x[i] = 1.0 + 0.1 * i;
     double lam = 0;
-    for (int it = 0; it < 300; ++it) {
-        for (int i = 0; i < n; ++i) {
-            cd s = 0;
-            for (int k = 0; k < n; ++k) s += A[(size_t)i * n + k] * x[k];
-            y[i] = s;
+    for (int it = 0; it < 40; ++it) {
+        const bool last = it >= 37;
+        std::fill(z.begin(), z.end(), cd(0, 0));
+        if (!last) {   // B is Hermitian: z = B x = sum_i conj(B_i)^T x_i, row by row
+            for (int i = 0; i < n; ++i)
+                for (int k = 0; k < n; ++k) z[k] += cmul(B[(size_t)i * n + k], x[i]);
+        } else {
+            for (int i = 0; i < n; ++i) {   // z += conj(A_i) (A_i x)
+                const cd* row = &A[(size_t)i * n];
+                cd y = 0;
+                for (int k = 0; k < n; ++k) y += mul(row[k], x[k]);
+                for (int k = 0; k < n; ++k) z[k] += cmul(row[k], y);
+            }
         }
-        for (int k = 0; k < n; ++k) {
-            cd s = 0;
-            for (int i = 0; i < n; ++i) s += std::conj(A[(size_t)i * n + k]) * y[i];
-            x[k] = s;
-        }
+        x.swap(z);
         double nx = 0;
-        for (auto& z : x) nx += std::norm(z);
+        for (auto& v : x) nx += std::norm(v);
         nx = std::sqrt(nx);
         if (nx == 0) break;
-        double prev = lam;
-        lam = std::sqrt(nx);
-        for (auto& z : x) z /= nx;
-        if (it > 10 && std::fabs(lam - prev) <= 1e-14 * lam) break;
+        if (last) lam = std::sqrt(nx);
+        for (auto& v : x) v /= nx;
     }
     return lam;
 }

@@ -12,6 +12,8 @@ using Mat = std::vector<cd>;   // row-major n x n
 
 // A = Z T Z^H with T upper triangular.  Returns false if QR iteration did not converge.
 bool schur(int n, Mat& A_to_T, Mat& Z);
+// The eigenvalues of A alone.  Returns false if QR iteration did not converge.
+bool eigenvalues(int n, const Mat& A, std::vector<cd>& lam);
 // Eigenvectors of upper-triangular T (columns of W, unit diagonal, W upper triangular).
 void triangular_eigenvectors(int n, const Mat& T, Mat& W);
 // Inverse of an upper-triangular matrix.
