@@ -41,3 +41,27 @@ def test_routes_give_the_same_bits(rg, d, z2, ntan):
         for x, y in zip(out[p], out[False]):
             assert np.isfinite(x).all()
             assert np.array_equal(x, y)
+
+
+def test_z2_samples_of_the_other_parity_are_zero(rg):
+    """A Z2 state's tiles of the other parity have no workgroup in the persistent launch; their samples
+    must be zero whatever the memory held, here the samples of a general state of the same size."""
+    from rcmps_gpu.excitation import action_batch
+    d = 32
+    out = {}
+    for persistent in (True, False):
+        for z2 in (False, True):
+            make = rg.random_state_z2_arrays if z2 else rg.random_state_arrays
+            s = rg.State(*make(d, scaling=0.2, seed=d))
+            s.integrator_param = rg.IntegratorParameters(n_quad=12, max_point=20.0, atol=1e-11, rtol=1e-10)
+            w = np.random.default_rng(1).standard_normal((d, d)).astype(complex)
+            if z2:
+                w[:d // 2, :d // 2] = 0
+                w[d // 2:, d // 2:] = 0
+            ctx = rg.ExcitationContext(s, 0.3, dense_transfer=False)
+            (f,) = action_batch(ctx, [w], rg.ExcitationModel("phi4", 1.5), 8, parts=2, persistent=persistent)
+            out[persistent, z2] = f
+            ctx.close()
+            s.close()
+    assert np.array_equal(out[True, True], out[False, True])
+    assert np.array_equal(out[True, False], out[False, False])
