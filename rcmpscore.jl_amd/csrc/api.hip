@@ -197,6 +197,7 @@ struct rcmps_context {
     // persistent Arnoldi steps (rc_arnoldi): exchange areas, descriptors behind the abort word; bases
     // per launch by blocks and tiles per side
     DevBuf arn_exch, arn_prob;
+    DevBuf pull_list;   // a pullback's entries and terms
     int arn_cap[2][5] = {{-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}};
     // GMRES read-back: two pinned slots of one Hessenberg column each, and their completion events
     double* kry_pinned = nullptr;
@@ -995,7 +996,7 @@ void rcmps_context_destroy(rcmps_context* ctx) {
                      &ctx->tmpM, &ctx->partial, &ctx->scratch, &ctx->small, &ctx->kry_V, &ctx->kry_w,
                      &ctx->kry_t1, &ctx->kry_t2, &ctx->kry_x, &ctx->kry_b, &ctx->kry_z, &ctx->kry_h,
                      &ctx->kry_tmp, &ctx->tune_buf, &ctx->gm_exch, &ctx->gm_prob, &ctx->gm_out,
-                     &ctx->arn_exch, &ctx->arn_prob};
+                     &ctx->arn_exch, &ctx->arn_prob, &ctx->pull_list};
     for (auto* b : all) b->release();
     for (auto& b : ctx->tb) b->release();
     if (ctx->blas) (void)rocblas_destroy_handle(ctx->blas);
@@ -1667,6 +1668,19 @@ const double* metric_inverse(rcmps_context* ctx, const rcmps_state* st, double m
 // Pullback over the Gauss nodes, boundary correction and gradients of one evaluation whose
 // trajectories are in tb (src/observables.jl:161-212).  With kin_cov/kin_env (device) the two
 // kinetic terms come from the infinite-line backend and only the :phi^4: trajectories are pulled back.
+// the lists of a pullback's sums on the device
+void pull_lists(rcmps_context* ctx, const std::vector<RcPullEntry>& en, const std::vector<RcPullTerm>& tm, RcPullArgs& pa) {
+    const size_t eb = en.size() * sizeof(RcPullEntry), tb = tm.size() * sizeof(RcPullTerm);
+    std::vector<char> h(eb + tb);
+    std::memcpy(h.data(), en.data(), eb);
+    std::memcpy(h.data() + eb, tm.data(), tb);
+    ck(ctx->pull_list.ensure(h.size()));
+    ck(hipMemcpyAsync(ctx->pull_list.p, h.data(), h.size(), hipMemcpyHostToDevice, ctx->stream));
+    pa.e = static_cast<const RcPullEntry*>(ctx->pull_list.p);
+    pa.t = reinterpret_cast<const RcPullTerm*>(static_cast<char*>(ctx->pull_list.p) + eb);
+    pa.nterms = (int)tm.size();
+}
+
 // The finishing of an evaluation in three parts: the pullback into tb.fin, the boundary solve of its
 // environment, the gradient.  tb.fin holds XR, XQ, env, cov and the boundary's solution, with
 // dE = 2 Re tr(XR dR) + 2 Re tr(XQ dQ) for any (dR, dQ) and covector = XR - XQ R^+ (+ the kinetic one).
@@ -1719,8 +1733,9 @@ void finish_pullback(rcmps_context* ctx, EvalReq& r, TrajBufs& tb, const rcmps_i
     };
     double* louts[RC_LIN_OUTS] = {S1, Z, W, env, S2, U};
     la.nouts = kin_cov ? 4 : 6;
-    int ne = 0, nt = 0, work[RC_PULL_TERMS] = {0, 0, 0}, total = 0;
-    for (int term = kin_cov ? 2 : 0; term < 3; ++term, ++nt) {
+    std::vector<RcPullEntry> en;
+    std::vector<RcPullTerm> tm;
+    for (int term = kin_cov ? 2 : 0; term < 3; ++term) {
         const int sf = 2 * term, sa = sf + 1;
         const int lf = kLive[sf], lad = kLive[sa];
         const double* Fs = tb.samples[sf].d();
@@ -1730,13 +1745,10 @@ void finish_pullback(rcmps_context* ctx, EvalReq& r, TrajBufs& tb, const rcmps_i
         auto Aptr = [&](int ch) { return As + 2 * ((long long)(nn - 1) * astride + ch * node); };
         auto Fptr = [&](int ch) { return Fs + 2 * (ch * node); };
         auto entry = [&](const double* F, const double* A, const double* Dm, double jk, int conj) {
-            pa.e[ne++] = RcPullEntry{F, A, Dm, fstride, -astride, jk, conj, 0};
-            ++work[nt];
-            ++total;
+            en.push_back(RcPullEntry{F, A, Dm, fstride, -astride, jk, conj, 0});
         };
         const double c = coef[term];
-        pa.first[nt] = ne;
-        pa.c[nt] = c;
+        tm.push_back(RcPullTerm{st->Rh.d(), c, (int)en.size(), 0, 0, 0});
         lin(0, Aptr(0), -astride, c, 0, 0);
         if (term < 2) {
             entry(Fptr(0), Aptr(1), nullptr, 0.0, 0);
@@ -1752,17 +1764,19 @@ void finish_pullback(rcmps_context* ctx, EvalReq& r, TrajBufs& tb, const rcmps_i
         const double* aend = As + 2 * ((long long)nn * astride);
         lin(3, aend, 0, 0.5 * c, 2, 0);
         lin(3, aend, 0, 0.5 * c, 2, 1);
+        tm.back().last = (int)en.size();
     }
-    pa.first[nt] = ne;
-    pa.nterms = nt;
     // about a workgroup per CU, the terms' shares by their pairs; no more streams than nodes
-    for (int t = 0; t < nt; ++t)
-        pa.wg0[t + 1] = pa.wg0[t] + std::max(1, std::min(ceil_div(nn, streams), 256 * work[t] / total));
-    pa.Rh = st->Rh.d();
+    for (RcPullTerm& t : tm) {
+        t.wg0 = pa.nwg;
+        t.nwg = std::max(1, std::min(ceil_div(nn, streams), 256 * (t.last - t.first) / (int)en.size()));
+        pa.nwg += t.nwg;
+    }
+    pull_lists(ctx, en, tm, pa);
     pa.wn = la.wn = ctx->nodes_w.d();
     pa.jn = la.jn = ctx->nodes_j.d();
     pa.nn = la.nn = nn;
-    ck(ctx->partial.ensure((size_t)pa.wg0[nt] * streams * 2 * mb));
+    ck(ctx->partial.ensure((size_t)pa.nwg * streams * 2 * mb));
     pa.partial = ctx->partial.d();
     for (int o = 0; o < RC_LIN_OUTS; ++o) la.out[o] = louts[o];
     ck(rc_launch_lin(Dp, la, ctx->stream));

@@ -3,13 +3,11 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#define RC_PULL_ENTRIES 7
-#define RC_PULL_TERMS 3
 #define RC_LIN_OUTS 6
 #define RC_LIN_SRCS 6
 
 // The contribution of one pair of channels to a term's sums over the nodes i < nn:
-//   T1 += op(F_i) M_i,  M_i = w_i R^+ op(A_i) + jk j_i D_i;   T2 += w_i op(F_i) op(A_i)
+//   T1 += op(F_i) M_i,  M_i = w_i B op(A_i) + jk j_i D_i;   T2 += w_i op(F_i) op(A_i)
 // (op: identity, or the conjugate transpose; F_i = F + i sF complex, A_i, D_i likewise at i sA)
 struct RcPullEntry {
     const double *F, *A, *D;   // D null: no second summand
@@ -17,14 +15,18 @@ struct RcPullEntry {
     double jk;
     int conj, pad;
 };
+// one pair of sums: entries first .. last - 1 on workgroups wg0 .. wg0 + nwg - 1, B their constant matrix
+struct RcPullTerm {
+    const double* B;
+    double c;                  // weight of the term where terms are summed
+    int first, last, wg0, nwg;
+};
 struct RcPullArgs {
-    RcPullEntry e[RC_PULL_ENTRIES];
-    int first[RC_PULL_TERMS + 1];   // entries of term t: first[t] .. first[t + 1] - 1
-    int wg0[RC_PULL_TERMS + 1];     // workgroups of term t
-    double c[RC_PULL_TERMS];        // weight of term t in the sums over the terms
-    const double *Rh, *wn, *jn;     // R^+, node weights w and j
-    int nn, nterms;
-    double* partial;                // two Dp x Dp matrices per stream of nodes
+    const RcPullEntry* e;        // device arrays
+    const RcPullTerm* t;
+    const double *wn, *jn;       // node weights w and j
+    int nn, nterms, nwg, pad;
+    double* partial;             // two Dp x Dp matrices per stream of nodes
 };
 // streams of nodes of one workgroup (each forms whole partial matrices)
 __host__ __device__ inline int rc_pull_streams(int nb) { return nb == 1 ? 4 : nb == 2 ? 2 : 1; }
@@ -47,3 +49,8 @@ struct RcLinArgs {
 hipError_t rc_launch_lin(int Dp, const RcLinArgs& a, hipStream_t stream);
 // the partial sums, then XR = W + sum_t c_t T1_t, XQ = sum_t c_t T2_t
 hipError_t rc_launch_pullback(int nb, const RcPullArgs& a, const double* W, double* XR, double* XQ, hipStream_t stream);
+// the partial sums, then every term's T1 and T2 by itself: sums + 2 t Dp^2 complex, T2 behind T1
+hipError_t rc_launch_pullback_terms(int nb, const RcPullArgs& a, double* sums, hipStream_t stream);
+// out_a += g (T1 of terms 2 a and 2 a + 1) - g tr(T2 of term 2 a + 1) wrho_a, a < na (out, wrho at complex stride ts)
+hipError_t rc_launch_action_pull(int Dp, int na, const double* sums, double g, const double* wrho, double* out,
+                                 long long ts, hipStream_t stream);

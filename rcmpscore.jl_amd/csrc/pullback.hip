@@ -18,6 +18,18 @@
 
 namespace {
 
+// a record through scalar loads (the address is uniform)
+template <class T>
+__device__ __forceinline__ T load_uniform(const T* p) {
+    static_assert(sizeof(T) % 8 == 0, "records are copied in 8-byte words");
+    const __attribute__((address_space(4))) uint64_t* q =
+        (const __attribute__((address_space(4))) uint64_t*)uni64(reinterpret_cast<uint64_t>(p));
+    T t;
+    uint64_t* w = reinterpret_cast<uint64_t*>(&t);
+#pragma unroll
+    for (int k = 0; k < (int)(sizeof(T) / 8); ++k) w[k] = q[k];
+    return t;
+}
 // two accumulators a tile: re += a.re b.re - a.im b.im, im += a.re b.im + a.im b.re
 struct Acc2 {
     v4d re, im;
@@ -44,8 +56,9 @@ __global__ void __launch_bounds__(NB == 3 ? 192 : 256, 1) rc_pullback(const RcPu
     const int lane = threadIdx.x & 63, wave = uni(threadIdx.x >> 6), bj = wave % NB;
     const int fi = lane & 15, fk = lane >> 4;
     int term = 0;
-    while (term + 1 < g.nterms && (int)blockIdx.x >= g.wg0[term + 1]) ++term;
-    const int stream = ((int)blockIdx.x - g.wg0[term]) * G + wave / NB, nstreams = (g.wg0[term + 1] - g.wg0[term]) * G;
+    RcPullTerm tm = load_uniform(g.t);
+    while ((int)blockIdx.x >= tm.wg0 + tm.nwg) tm = load_uniform(g.t + ++term);
+    const int stream = ((int)blockIdx.x - tm.wg0) * G + wave / NB, nstreams = tm.nwg * G;
     // left-hand fragments of op(F)(b, :): row 16 b + fi, column 4 s + fk
     auto left = [&](cplx* f, const cplx* F, int b, bool conj) {
         if (!conj) {
@@ -66,7 +79,7 @@ __global__ void __launch_bounds__(NB == 3 ? 192 : 256, 1) rc_pullback(const RcPu
             for (int s = 0; s < NF; ++s) f[s] = cconj(A[(16 * bj + fi) * Dp + 4 * s + fk]);
         }
     };
-    const cplx* rh = reinterpret_cast<const cplx*>(g.Rh);
+    const cplx* rh = reinterpret_cast<const cplx*>(tm.B);
     cplx rf[SHARED ? 1 : NB][NF];
     if constexpr (SHARED) {
         cplx f[NF];
@@ -86,17 +99,17 @@ __global__ void __launch_bounds__(NB == 3 ? 192 : 256, 1) rc_pullback(const RcPu
     }
     // the stream's units: pair q of node i, one after the other; the next one's A (and the share of its F)
     // is loaded ahead
-    const int q0 = g.first[term], q1 = g.first[term + 1];
+    const int q0 = tm.first, q1 = tm.last;
     int i = stream, q = q0;
     cplx af[NF], na[NF], nf[SHARED ? NF : 1];
     auto load = [&](int i, int q) {
-        const RcPullEntry& e = g.e[q];
+        const RcPullEntry e = load_uniform(g.e + q);
         right(na, reinterpret_cast<const cplx*>(e.A) + (long long)i * e.sA, e.conj);
         if constexpr (SHARED) left(nf, reinterpret_cast<const cplx*>(e.F) + (long long)i * e.sF, bj, e.conj);
     };
     if (i < g.nn) load(i, q);
     while (i < g.nn) {
-        const RcPullEntry& e = g.e[q];
+        const RcPullEntry e = load_uniform(g.e + q);
         const double wi = ld_const(g.wn, i), ji = ld_const(g.jn, i);
         cplx mf[NF];
 #pragma unroll
@@ -174,6 +187,15 @@ __device__ __forceinline__ cplx quarters(cplx v, cplx* red) {
     return cadd(cadd(cadd(red[l], red[64 + l]), red[128 + l]), red[192 + l]);
 }
 
+// quarter q of the sum over matrices s0 .. s0 + ns - 1 (two matrices of n elements apart)
+__device__ __forceinline__ cplx quarter_sum(const cplx* p, int s0, int ns, int q, int n) {
+    const int a = s0 + ns * q / 4, b = s0 + ns * (q + 1) / 4;
+    cplx s = cmake(0, 0);
+#pragma unroll 8
+    for (int i = a; i < b; ++i) s = cadd(s, p[(long long)i * 2 * n]);
+    return s;
+}
+
 // blockIdx.y = 0: XR = W + sum_t c_t T1_t; 1: XQ = sum_t c_t T2_t, over the terms' partial matrices
 __global__ void __launch_bounds__(256) rc_pull_sum(const RcPullArgs g, int n, int streams, const double* W, double* XR,
                                                    double* XQ) {
@@ -182,17 +204,39 @@ __global__ void __launch_bounds__(256) rc_pull_sum(const RcPullArgs g, int n, in
     const cplx* p = reinterpret_cast<const cplx*>(g.partial) + (long long)y * n + e;
     cplx v = cmake(0, 0);
     for (int t = 0; t < g.nterms; ++t) {
-        const int s0 = g.wg0[t] * streams, ns = (g.wg0[t + 1] - g.wg0[t]) * streams;
-        const int a = s0 + ns * q / 4, b = s0 + ns * (q + 1) / 4;
-        cplx s = cmake(0, 0);
-#pragma unroll 8
-        for (int i = a; i < b; ++i) s = cadd(s, p[(long long)i * 2 * n]);
-        v = cadd(v, cscale(g.c[t], s));
+        const RcPullTerm tm = load_uniform(g.t + t);
+        v = cadd(v, cscale(tm.c, quarter_sum(p, tm.wg0 * streams, tm.nwg * streams, q, n)));
     }
     v = quarters(v, red);
     if (q) return;
     if (y == 0 && W) v = cadd(v, reinterpret_cast<const cplx*>(W)[e]);
     reinterpret_cast<cplx*>(y ? XQ : XR)[e] = v;
+}
+
+// sum blockIdx.y & 1 of term blockIdx.y >> 1, into sums
+__global__ void __launch_bounds__(256) rc_pull_sum_terms(const RcPullArgs g, int n, int streams, double* sums) {
+    __shared__ cplx red[256];
+    const int e = blockIdx.x * 64 + (threadIdx.x & 63), q = threadIdx.x >> 6, y = blockIdx.y & 1;
+    const RcPullTerm tm = load_uniform(g.t + (blockIdx.y >> 1));
+    const cplx* p = reinterpret_cast<const cplx*>(g.partial) + (long long)y * n + e;
+    const cplx v = quarters(quarter_sum(p, tm.wg0 * streams, tm.nwg * streams, q, n), red);
+    if (q == 0) reinterpret_cast<cplx*>(sums)[(long long)blockIdx.y * n + e] = v;
+}
+
+__global__ void __launch_bounds__(256) rc_action_pull(int Dp, const double* sums, double g, const double* wrho,
+                                                      double* out, long long ts) {
+    __shared__ cplx red[256];
+    const int n = Dp * Dp, l = threadIdx.x, a = blockIdx.y;
+    const cplx* s = reinterpret_cast<const cplx*>(sums) + (long long)4 * a * n;   // T1, T2 of term 2 a, then of 2 a + 1
+    red[l] = l < Dp ? s[3 * n + l * Dp + l] : cmake(0, 0);
+    __syncthreads();
+    cplx tr = cmake(0, 0);
+    for (int i = 0; i < Dp; ++i) tr = cadd(tr, red[i]);
+    const int e = blockIdx.x * 256 + l;
+    if (e >= n) return;
+    cplx* o = reinterpret_cast<cplx*>(out) + (long long)a * ts + e;
+    const cplx w = reinterpret_cast<const cplx*>(wrho)[(long long)a * ts + e];
+    *o = cadd(*o, cscale(g, csub(cadd(s[e], s[2 * n + e]), cmul(tr, w))));
 }
 
 // blockIdx.y: output
@@ -228,9 +272,9 @@ hipError_t rc_launch_lin(int Dp, const RcLinArgs& a, hipStream_t stream) {
     return hipGetLastError();
 }
 
-hipError_t rc_launch_pullback(int nb, const RcPullArgs& a, const double* W, double* XR, double* XQ, hipStream_t stream) {
-    const dim3 grid(a.wg0[a.nterms]);
-    const int lds = nb > 2 ? 2 * nb * 4 * nb * 1024 : 0;   // R^+ and F
+static hipError_t launch_partial(int nb, const RcPullArgs& a, hipStream_t stream) {
+    const dim3 grid(a.nwg);
+    const int lds = nb > 2 ? 2 * nb * 4 * nb * 1024 : 0;   // B and F
     hipError_t e = hipSuccess;
     switch (nb) {
         case 1: hipLaunchKernelGGL(rc_pullback<1>, grid, dim3(256), 0, stream, a); break;
@@ -245,10 +289,27 @@ hipError_t rc_launch_pullback(int nb, const RcPullArgs& a, const double* W, doub
             break;
         default: return hipErrorInvalidValue;
     }
-    if (e != hipSuccess) return e;
-    e = hipGetLastError();
+    return e != hipSuccess ? e : hipGetLastError();
+}
+
+hipError_t rc_launch_pullback(int nb, const RcPullArgs& a, const double* W, double* XR, double* XQ, hipStream_t stream) {
+    const hipError_t e = launch_partial(nb, a, stream);
     if (e != hipSuccess) return e;
     const int n = 256 * nb * nb;
     hipLaunchKernelGGL(rc_pull_sum, dim3(n / 64, 2), dim3(256), 0, stream, a, n, rc_pull_streams(nb), W, XR, XQ);
+    return hipGetLastError();
+}
+
+hipError_t rc_launch_pullback_terms(int nb, const RcPullArgs& a, double* sums, hipStream_t stream) {
+    const hipError_t e = launch_partial(nb, a, stream);
+    if (e != hipSuccess) return e;
+    const int n = 256 * nb * nb;
+    hipLaunchKernelGGL(rc_pull_sum_terms, dim3(n / 64, 2 * a.nterms), dim3(256), 0, stream, a, n, rc_pull_streams(nb), sums);
+    return hipGetLastError();
+}
+
+hipError_t rc_launch_action_pull(int Dp, int na, const double* sums, double g, const double* wrho, double* out,
+                                 long long ts, hipStream_t stream) {
+    hipLaunchKernelGGL(rc_action_pull, dim3((Dp * Dp + 255) / 256, na), dim3(256), 0, stream, Dp, sums, g, wrho, out, ts);
     return hipGetLastError();
 }
