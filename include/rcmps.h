@@ -78,7 +78,7 @@ typedef struct rcmps_excitation rcmps_excitation;
 #define RCMPS_EXC_GRAPH 8         /* with either: step the action ODE by replayed launch graphs */
 #define RCMPS_EXC_PERSISTENT 16   /* with either: integrate it in one persistent launch wherever every
                                      tile's workgroup fits on the device at once (neither flag: the
-                                     faster of the two for the size; all three give the same bits) */
+                                     same; all three give the same bits) */
 
 /* IntegratorParameters (src/state.jl:4-10) plus the DOP853 initial step. */
 typedef struct {
@@ -150,9 +150,9 @@ int rcmps_fg_phi4(rcmps_context* ctx, const rcmps_state* st, double g, const rcm
 /* fg_phi4 over n independent states (any mix of bond dimensions and couplings g[i]) with one
    integrator: energies[i] (host) and, where grads and grads[i] are non-null, the Riemannian
    gradient into the device buffer grads[i] (D_i x D_i).  States of the same padded size share a
-   persistent launch in which their trajectories are gang-scheduled in rounds of resident
-   workgroups (the largest size in two launches); each launch's pullback, boundary and metric
-   solves run on worker streams while the next launch integrates.  stats may be null or an array
+   persistent launch in which every workgroup runs a list of their trajectories' tasks (the largest
+   size in two launches); each launch's pullbacks run on worker streams beside the next launch, its
+   boundary solves together and the metric solves behind them.  stats may be null or an array
    of n.  Returns the first failure (each stats[i]
    holds its own status); the evaluations that succeeded are complete.  Replaces a loop of
    fg_phi4(s_i, g_i) calls (src/observables.jl:257); the reference has no batched form. */
