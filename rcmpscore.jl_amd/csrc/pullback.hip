@@ -12,7 +12,7 @@
 //
 // Bound by the matrix cores at D = 64 (3 products a node and pair: 0.28 ms at the peak rate for 512
 // nodes), by the latency of a node's chain of loads and products below.  Measured on MI355X, the
-// whole pullback: D = 8 0.55 -> 0.10 ms, D = 32 0.65 -> 0.24, D = 64 1.61 -> 0.74 (256 node pairs, window 20).
+// whole pullback: D = 8 0.55 -> 0.07 ms, D = 32 0.65 -> 0.18, D = 64 1.61 -> 0.69 (256 node pairs, window 20).
 #include "device_common.h"
 #include "pullback.h"
 
@@ -239,10 +239,12 @@ __global__ void __launch_bounds__(256) rc_action_pull(int Dp, const double* sums
     *o = cadd(*o, cscale(g, csub(cadd(s[e], s[2 * n + e]), cmul(tr, w))));
 }
 
-// blockIdx.y: output
-__global__ void __launch_bounds__(256) rc_lin(const RcLinArgs g, int Dp) {
-    __shared__ cplx red[256];
-    const int e = blockIdx.x * 64 + (threadIdx.x & 63), q = threadIdx.x >> 6, o = blockIdx.y;
+// blockIdx.y: output; sixteen waves share the nodes of 64 elements (four took 199 us at D = 64 with 512
+// nodes, a chain of 128 loads' latency in eights)
+__global__ void __launch_bounds__(1024) rc_lin(const RcLinArgs g, int Dp) {
+    constexpr int P = 16;
+    __shared__ cplx red[64 * P];
+    const int l = threadIdx.x & 63, e = blockIdx.x * 64 + l, q = threadIdx.x >> 6, o = blockIdx.y;
     const int et = (e % Dp) * Dp + e / Dp;
     cplx v = cmake(0, 0);
     for (int k = 0; k < g.nsrc[o]; ++k) {
@@ -253,8 +255,8 @@ __global__ void __launch_bounds__(256) rc_lin(const RcLinArgs g, int Dp) {
             if (q == 0) t = x[0];
         } else {
             const double* w = s.kind ? g.jn : g.wn;
-            const int a = g.nn * q / 4, b = g.nn * (q + 1) / 4;
-#pragma unroll 16
+            const int a = g.nn * q / P, b = g.nn * (q + 1) / P;
+#pragma unroll 8
             for (int i = a; i < b; ++i) {
                 const double c = w[i];
                 const cplx y = x[(long long)i * s.s];
@@ -263,12 +265,15 @@ __global__ void __launch_bounds__(256) rc_lin(const RcLinArgs g, int Dp) {
         }
         v = cadd(v, cscale(s.c, s.conj ? cconj(t) : t));
     }
-    v = quarters(v, red);
-    if (q == 0) reinterpret_cast<cplx*>(g.out[o])[e] = v;
+    red[threadIdx.x] = v;
+    __syncthreads();
+    if (q) return;
+    for (int p = 1; p < P; ++p) v = cadd(v, red[64 * p + l]);
+    reinterpret_cast<cplx*>(g.out[o])[e] = v;
 }
 
 hipError_t rc_launch_lin(int Dp, const RcLinArgs& a, hipStream_t stream) {
-    hipLaunchKernelGGL(rc_lin, dim3(Dp * Dp / 64, a.nouts), dim3(256), 0, stream, a, Dp);
+    hipLaunchKernelGGL(rc_lin, dim3(Dp * Dp / 64, a.nouts), dim3(1024), 0, stream, a, Dp);
     return hipGetLastError();
 }
 
