@@ -132,6 +132,7 @@ struct RcOdeRun {
     double* exch;
     uint32_t exch_bytes;
     int nslots;                // tiles of every matrix
+    int spread, pad;           // every eighth workgroup of the launch works (all on one XCD)
     double* Sf;                // samples, as OdeWork
     double* Sa;
     long long N, half;
@@ -149,7 +150,7 @@ struct RcOdeRun {
 };
 // z2: only the tiles of the parity blocks that can be nonzero have a workgroup (g.zt > 0)
 hipError_t rc_quartic_ode_capacity(int nb, int z2, int nslots, int ntrack, int* blocks);
-hipError_t rc_launch_quartic_ode(int nb, int z2, int nwg, int nslots, int ntrack, const RcOdeRun* dparams,
+hipError_t rc_launch_quartic_ode(int nb, int z2, int nwg, int spread, int nslots, int ntrack, const RcOdeRun* dparams,
                                  hipStream_t stream);
 __global__ void rc_ode_step(RcOdeCtl* c, int finish, const double* partial, const int* ranges, int nranges,
                             int ntrack, double cnt, const double* stops, const int* stop_node, const double* cheb,

@@ -182,7 +182,7 @@ __device__ __forceinline__ void ode_step_body(RcOdeCtl* c, int finish, const dou
                     c->si += 1;
                     moved = 1;
                 }
-                double factor = err == 0 ? 10.0 : fmin(10.0, 0.9 * pow(err, -1.0 / 8));
+                double factor = err == 0 ? 10.0 : fmin(10.0, 0.9 / sqrt(sqrt(sqrt(err))));   // 0.9 err^(-1/8)
                 if (c->last_rejected) factor = fmin(1.0, factor);
                 const double hn = he * factor;
                 c->h = c->clipped ? fmax(hn, c->h) : hn;
@@ -193,7 +193,7 @@ __device__ __forceinline__ void ode_step_body(RcOdeCtl* c, int finish, const dou
                 }
             } else {
                 c->rejected += 1;
-                c->h = he * fmax(0.2, 0.9 * pow(err, -1.0 / 8));
+                c->h = he * fmax(0.2, 0.9 / sqrt(sqrt(sqrt(err))));
                 c->last_rejected = 1;
             }
         }
@@ -764,34 +764,48 @@ __global__ void __launch_bounds__(256) rc_quartic_rhs(RcQuarticArgs g) {
 // time: a workgroup that outlasts the budget sets the abort word and every workgroup leaves with
 // RC_ST_WAIT_LIMIT.
 //
+// Up to 32 workgroups (D <= 16 with one tangent) are laid on one XCD and exchange through its L2.  With
+// that and running sums of the combinations instead of a window of derivatives a right-hand side
+// takes 3.1 us at D = 16 (3.35 before), 4.7 at D = 64 with parity blocks (4.9), 3.4 at D = 32 (3.4).
+//
 // What bounds it: the two exchanges (about 1.2 us each) around up to eight products of a tile.
 // ---------------------------------------------------------------------------------------------
-// Combinations after stage s of the action ODE without their last term, over a window of 13 (k_j at
-// 13 - s + j before k_s enters): rows 1..10 the next stage input, 11 the step end, 12 and 13 the
-// error estimators after stage 12.
+// What the derivative of stage s adds to the combinations still ahead of it: row s, the coefficients of
+// k_s in the inputs of stages s + 2, s + 3, .. (stage 12's is the step end), then in E5 and E3.
+#define RC_ODE_AHEAD 11
 struct RcOdeRows {
-    double c[14][13];
+    double c[12][RC_ODE_AHEAD + 3];
 };
 constexpr RcOdeRows rc_make_ode_rows() {
     RcOdeRows r{};
-    for (int s = 1; s < 12; ++s)
-        for (int j = 0; j < s; ++j) r.c[s][13 - s + j] = s == 11 ? RC_B[j] : RC_A[s + 1][j];
-    for (int j = 0; j < 12; ++j) {
-        r.c[12][1 + j] = RC_E5[j];
-        r.c[13][1 + j] = RC_E3[j];
+    for (int s = 0; s < 12; ++s) {
+        for (int i = 0; s + 2 + i <= 12; ++i) r.c[s][i] = s + 2 + i == 12 ? RC_B[s] : RC_A[s + 2 + i][s];
+        r.c[s][RC_ODE_AHEAD] = RC_E5[s];
+        r.c[s][RC_ODE_AHEAD + 1] = RC_E3[s];
     }
     return r;
 }
 __constant__ const RcOdeRows rc_ode_rows = rc_make_ode_rows();
 
-__device__ __forceinline__ cplx ode_row_sum(int row, const cplx* k) {
-    const __attribute__((address_space(4))) double* c =
-        (const __attribute__((address_space(4))) double*)&rc_ode_rows.c[row][0];
-    cplx s = cmake(0, 0);
+// Running sums of the combinations ahead, in stage order: each moves up by one as its multiply-add's
+// destination, so a[0] is all but the last term of the input after the next stage (the sums of a window
+// of derivatives, in the same order: the graph route's bits)
+struct RcOdeAhead {
+    cplx a[RC_ODE_AHEAD + 1], e5, e3;
+    __device__ __forceinline__ void clear() {
+        e5 = e3 = cmake(0, 0);
 #pragma unroll
-    for (int q = 0; q < 13; ++q) s = cfma(c[q], k[q], s);
-    return s;
-}
+        for (int i = 0; i <= RC_ODE_AHEAD; ++i) a[i] = cmake(0, 0);
+    }
+    __device__ __forceinline__ void add(int s, cplx k) {
+        const __attribute__((address_space(4))) double* c =
+            (const __attribute__((address_space(4))) double*)&rc_ode_rows.c[s][0];
+#pragma unroll
+        for (int i = 0; i < RC_ODE_AHEAD; ++i) a[i] = cfma(c[i], k, a[i + 1]);
+        e5 = cfma(c[RC_ODE_AHEAD], k, e5);
+        e3 = cfma(c[RC_ODE_AHEAD + 1], k, e3);
+    }
+};
 
 // dynamic LDS: two levels of partial tiles, every tile's error sums, the trajectories' slot ranges (two
 // of two ints each)
@@ -818,7 +832,9 @@ __global__ void __launch_bounds__(256, KT <= 2 ? 2 : 1) rc_quartic_ode(const RcO
     const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
     const int ei = tid >> 4, ej = tid & 15, fi = lane & 15, fk = 4 * wave + (lane >> 4);
     const int nb = g.na * RC_QCH, nmat = rc_qmats(nb);
-    const int wg = blockIdx.x, mi = wg / (NB * KT), bi = wg / KT % NB, jj = wg % KT;
+    // spread: only every eighth workgroup works, so that all share an XCD
+    if (p.spread && (blockIdx.x & 7)) return;
+    const int wg = p.spread ? blockIdx.x >> 3 : blockIdx.x, mi = wg / (NB * KT), bi = wg / KT % NB, jj = wg % KT;
     int blk, a, k;
     qmat_of(mi, nb, blk, a, k);
     // parities (all k-tiles when KT = NB): as quartic_tile
@@ -878,20 +894,35 @@ __global__ void __launch_bounds__(256, KT <= 2 ? 2 : 1) rc_quartic_ode(const RcO
     const Ctl ctl{p.abort_flag, p.wait_ticks};
     const long long e = (long long)mi * m + (16 * bi + ei) * Dp + 16 * bj + ej;
 
+    // Whether all workgroups share an XCD (they post its id as the record of attempt 0): then nothing needs
+    // to leave its L2.  Only asked when they were laid out for it.
+    bool loc = false;
+    if (p.spread) {
+        __shared__ int s_far;
+        if (tid == 0) s_far = 0;
+        __syncthreads();
+        if (tid < (KT < NB ? 2 : 1))
+            rc_put(rX, (uint32_t)(mi * NT + bi * NB + (tid ? bjp : bj)) * 16, oR, cmake(xcd_id(), 0.0));
+        for (int q0 = 0; q0 < p.nslots; q0 += 256) {
+            const bool use = q0 + tid < p.nslots;
+            cplx v;
+            rc_fetch<1>(rX, (uint32_t)(q0 + tid) * 16, oR, 0, &v, use);
+            if (!rc_await<1>(ctl, rX, (uint32_t)(q0 + tid) * 16, oR, 0, &v, use) || (use && (int)v.re != xcd_id())) s_far = 1;
+        }
+        __syncthreads();
+        loc = uni(s_far) == 0;
+    }
     uint32_t ev = 0;
     auto put = [&](cplx v) {
         ++ev;
         const uint32_t so = (ev & (RC_RING - 1)) * ring_bytes + sx;
-        rc_put(rX, a_el, so, v);
-        rc_put(rX, b_el, oB + so, v);
+        rc_put(rX, a_el, so, v, loc);
+        rc_put(rX, b_el, oB + so, v, loc);
     };
-    cplx kst[13];   // window of stage derivatives, the newest last
-#pragma unroll
-    for (int q = 0; q < 13; ++q) kst[q] = cmake(0, 0);
-    cplx pre = cmake(0, 0), pre3 = cmake(0, 0);
-    // right-hand side on the stage input of event ev; row: the combinations to sum meanwhile (after
-    // stage `row`), -1 none
-    auto rhs = [&](double jac, double jt, int row) -> cplx {
+    RcOdeAhead ahead;
+    ahead.clear();
+    // right-hand side on the stage input of event ev
+    auto rhs = [&](double jac, double jt) -> cplx {
         const uint32_t ring = (ev & (RC_RING - 1)) * ring_bytes;
         const double c = c_nbr * jt;
         cplx r1[KT], r2[KT], c1[KT], c2[KT], c3[KT], c4[KT], q1[KT], q2[KT], ins = cmake(0, 0);
@@ -912,12 +943,12 @@ __global__ void __launch_bounds__(256, KT <= 2 ? 2 : 1) rc_quartic_ode(const RcO
         if (blk == 2) frag_product<KT>(acc, r2, cW);
         put_partial(acc, red1, wave, lane);
         lds_barrier();
-        rc_put(rX, p_el, oP + ring + sx, sum_partial(red1));
+        rc_put(rX, p_el, oP + ring + sx, sum_partial(red1), loc);
         if (ev > RC_RING / 2) {   // empty the slots of event ev - 16
             const uint32_t old = ((ev - RC_RING / 2) & (RC_RING - 1)) * ring_bytes + sx;
-            rc_reset(rX, a_el, old);
-            rc_reset(rX, b_el, oB + old);
-            rc_reset(rX, p_el, oP + old);
+            rc_reset(rX, a_el, old, loc);
+            rc_reset(rX, b_el, oB + old, loc);
+            rc_reset(rX, p_el, oP + old, loc);
         }
         // one-sided products
         cacc_zero(acc);
@@ -937,8 +968,6 @@ __global__ void __launch_bounds__(256, KT <= 2 ? 2 : 1) rc_quartic_ode(const RcO
         p1.fetch(rX);
         p2.fetch(rX);
         p3.fetch(rX);
-        if (row >= 0) pre = ode_row_sum(row, kst);
-        if (row == 12) pre3 = ode_row_sum(13, kst);
         ok = rc_await_all(ctl, rX, p1, p2, p3) && ok;
         scaled(jac, cR, q1);
         if (blk == 1) scaled(jac, cW, q2);
@@ -970,33 +999,30 @@ __global__ void __launch_bounds__(256, KT <= 2 ? 2 : 1) rc_quartic_ode(const RcO
     if (tid < 13) s_al[tid] = tid == 11 ? RC_B[11] : tid < 11 ? RC_A[tid + 1][tid] : 0.0;
     __syncthreads();
     put(yv);
-    k0 = rhs(p.jac0, p.jt0, -1);   // the first right-hand side (first same as last)
+    k0 = rhs(p.jac0, p.jt0);   // the first right-hand side (first same as last)
     ode_step_body<true>(&sc, 0, s_slots, s_ranges, p.nranges, p.ntrack, p.cnt, s_stops, &s_node, s_cheb, s_cf);
     lds_barrier();
     while (sc.active && !s_stop) {
         const double he = s_cf[26];
         put(cfma(he, cscale(RC_A[1][0], k0), yv));
-#pragma unroll
-        for (int q = 0; q < 12; ++q) kst[q] = cmake(0, 0);
-        kst[12] = k0;
+        ahead.clear();
+        ahead.add(0, k0);
         cplx ynew = cmake(0, 0), F = cmake(0, 0);
         lap(t_ctl);
         // the stops the verdict of this attempt may need, behind its first publish
         if (tid < 2) s_stops[tid] = sc.si + tid < sc.nstops ? p.stops[sc.si + tid] : 0.0;
         if (tid == 2) s_node = p.stop_node[sc.si];
         for (int st = 1; st < 13; ++st) {
-            F = rhs(s_cf[2 * st], s_cf[2 * st + 1], st);
+            F = rhs(s_cf[2 * st], s_cf[2 * st + 1]);
             if (st == 12) break;
-            const cplx u = cfma(he, cfma(s_al[st], F, pre), yv);
+            const cplx u = cfma(he, cfma(s_al[st], F, ahead.a[0]), yv);
             put(u);
             ynew = u;   // stage 11's is the step end
-#pragma unroll
-            for (int q = 0; q < 12; ++q) kst[q] = kst[q + 1];
-            kst[12] = F;
+            ahead.add(st, F);
         }
         lap(t_rhs);
         // error sums of this tile, and of every other
-        tile_error_put(cfma(RC_E5[12], F, pre), cfma(RC_E3[12], F, pre3), p.atol + p.rtol * fmax(cabsd(yv), cabsd(ynew)),
+        tile_error_put(cfma(RC_E5[12], F, ahead.e5), cfma(RC_E3[12], F, ahead.e3), p.atol + p.rtol * fmax(cabsd(yv), cabsd(ynew)),
                        s_err, wave, lane);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every emptied slot is empty before the record is seen
         lds_barrier();
@@ -1005,8 +1031,8 @@ __global__ void __launch_bounds__(256, KT <= 2 ? 2 : 1) rc_quartic_ode(const RcO
         const uint32_t so_old = oR + ((att + 2) & (RC_REC_RING - 1)) * rec_bytes;
         if (tid < (KT < NB ? 2 : 1)) {   // Z2: the tile of the other parity block, exactly zero, has no workgroup
             const uint32_t off = (uint32_t)(mi * NT + bi * NB + (tid ? bjp : bj)) * 16;
-            rc_put(rX, off, so_rec, tid ? cmake(0, 0) : tile_error_sum(s_err));
-            rc_reset(rX, off, so_old);   // attempt - 2: all published attempt - 1 after reading it
+            rc_put(rX, off, so_rec, tid ? cmake(0, 0) : tile_error_sum(s_err), loc);
+            rc_reset(rX, off, so_old, loc);   // attempt - 2: all published attempt - 1 after reading it
         }
         bool ok = true;
         for (int q0 = 0; q0 < p.nslots; q0 += 256) {
@@ -1078,7 +1104,7 @@ hipError_t rc_quartic_ode_capacity(int nb, int z2, int nslots, int ntrack, int* 
     return hipSuccess;
 }
 
-hipError_t rc_launch_quartic_ode(int nb, int z2, int nwg, int nslots, int ntrack, const RcOdeRun* dparams,
+hipError_t rc_launch_quartic_ode(int nb, int z2, int nwg, int spread, int nslots, int ntrack, const RcOdeRun* dparams,
                                  hipStream_t stream) {
     void* args[] = {(void*)&dparams};
     const void* fn = quartic_ode_fn(nb, z2);
@@ -1090,6 +1116,7 @@ hipError_t rc_launch_quartic_ode(int nb, int z2, int nwg, int nslots, int ntrack
     // a workgroup per CU where there are CUs for all: more LDS than half a CU's keeps two from sharing one
     // (and its matrix cores) while others idle
     const int lds = RC_ODE_LDS(nslots, ntrack);
+    if (spread) nwg *= 8;
     return hipLaunchCooperativeKernel(fn, dim3(nwg), dim3(256), args, nwg <= cus ? std::max(lds, RC_ODE_LDS_ALONE) : lds,
                                       stream);
 }
