@@ -47,14 +47,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rc_rsrc(const void* base, uint
     return __builtin_amdgcn_make_buffer_rsrc(b, 0, (int)__builtin_amdgcn_readfirstlane(bytes), RC_BUF_DWORD3);
 }
 
-__device__ __forceinline__ cplx ld_coh(__amdgpu_buffer_rsrc_t r, uint32_t byte_offset) {
-    v4u v = __builtin_amdgcn_raw_buffer_load_b128(r, byte_offset, 0, RC_COHERENT_POLICY);
-    cplx z;
-    z.re = __builtin_bit_cast(double, (uint64_t)v.x | ((uint64_t)v.y << 32));
-    z.im = __builtin_bit_cast(double, (uint64_t)v.z | ((uint64_t)v.w << 32));
-    return z;
-}
-
 __device__ __forceinline__ void st_coh(__amdgpu_buffer_rsrc_t r, uint32_t byte_offset, cplx z) {
     uint64_t a = __builtin_bit_cast(uint64_t, z.re), b = __builtin_bit_cast(uint64_t, z.im);
     v4u v;
@@ -86,12 +78,6 @@ __device__ __forceinline__ void st_xcd_s(__amdgpu_buffer_rsrc_t r, uint32_t voff
 // the XCD this workgroup runs on (hardware register XCC_ID, bits 0..3)
 __device__ __forceinline__ int xcd_id() { return (int)__builtin_amdgcn_s_getreg(20 | (3 << 11)); }
 
-__device__ __forceinline__ double ld_coh_f64(const double* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_coh_f64(double* p, double v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 // read-only data written before the launch, read at a wave-uniform index: through the scalar cache
 __device__ __forceinline__ double ld_const(const double* p, int i) {
     return ((const __attribute__((address_space(4))) double*)p)[__builtin_amdgcn_readfirstlane(i)];

@@ -108,8 +108,6 @@ __global__ void rc_msubtract(const double* V, long long sb, long long sv, int nk
                              double* W, long long sw);
 __global__ void rc_mnormalize(int n, const double* W, long long sw, const double* nrm2, int ldn, double* out,
                               long long so);
-__global__ void rc_stage(long long N, const double* y, const double* K, long long sk, RcStageCoef c, double h,
-                         const double* hp, double* out, const int* active);
 
 // Device-resident DOP853 step controller of the action ODE.  One attempt is rc_ode_stage (which
 // first commits the previous attempt when it was accepted: y <- y_new, K_0 <- K_12, the sample of a

@@ -90,20 +90,6 @@ __global__ void rc_mnormalize(int n, const double* W, long long sw, const double
         cscale(s, reinterpret_cast<const cplx*>(W)[(long long)b * sw + i]);
 }
 
-// out = y + h sum_{j < c.nk} c.a[j] K_j  (N complex, K_j at K + j sk); h from hp when non-null
-__global__ void rc_stage(long long N, const double* y, const double* K, long long sk, RcStageCoef c, double h,
-                         const double* hp, double* out, const int* active) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N || (active && !*active)) return;
-    if (hp) h = hp[0];
-    const cplx* kk = reinterpret_cast<const cplx*>(K);
-    cplx s = cmake(0, 0);
-    for (int j = 0; j < c.nk; ++j)
-        if (c.a[j] != 0.0) s = cadd(s, cscale(c.a[j], kk[(long long)j * sk + i]));
-    const cplx yy = reinterpret_cast<const cplx*>(y)[i];
-    reinterpret_cast<cplx*>(out)[i] = cadd(yy, cscale(h, s));
-}
-
 // ---------------------------------------------------------------------------------------------
 // The action ODE's step controller on the device (the host loop it replaces: SciPy's DOP853
 // controller as the reference's action integration uses it, src/excitation_action.jl:56-123).
