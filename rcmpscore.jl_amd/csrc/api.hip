@@ -1629,7 +1629,7 @@ void run_class(rcmps_context* ctx, int Dp, bool split, bool quartic_only, bool t
             S->dense_steps[s] = (long long)o[RC_OUT_DENSE];
             S->rhs_calls[s] = (long long)o[RC_OUT_RHS];
             for (int q = 0; q < RC_NTIMERS; ++q) S->phase_us[s][q] = o[RC_OUT_TIMERS + q] / ctx->clock_mhz;
-            const int stt = (int)o[RC_OUT_STATUS];
+            const int stt = rc_system_status(o);
             if (stt != RC_ST_OK && S->status == RCMPS_OK) { S->status = stt; S->failed_system = s; }
         }
         if (S->status == RCMPS_OK) {

@@ -72,6 +72,13 @@ struct TrajParams {
 
 // out[] layout per system
 enum { RC_OUT_STATUS = 0, RC_OUT_ATTEMPTS, RC_OUT_ACCEPTED, RC_OUT_REJECTED, RC_OUT_DENSE,
-       RC_OUT_RHS, RC_OUT_SCALAR, RC_OUT_T, RC_OUT_NEXTPOINT, RC_OUT_TIMERS = 16 };
+       RC_OUT_RHS, RC_OUT_SCALAR, RC_OUT_T, RC_OUT_NEXTPOINT, RC_OUT_WAIT_FAILED, RC_OUT_TIMERS = 16 };
 #define RC_OUT_STRIDE 32
 #define RC_NTIMERS 12
+
+// A system's status.  The controller's own comes from its first workgroup and knows of the waits up to
+// the last verdict; a wait that failed in any workgroup, also in the dense output's stages after that
+// verdict, leaves RC_OUT_WAIT_FAILED nonzero, and then neither samples nor counters can be trusted.
+inline int rc_system_status(const double* out) {
+    return out[RC_OUT_WAIT_FAILED] != 0.0 ? RC_ST_WAIT_LIMIT : (int)out[RC_OUT_STATUS];
+}

@@ -940,8 +940,10 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
         ahead.add(next - 1, next == 1 ? k0 : kn);
         slot = uni(next);
     }
-    // an attempt cut short by a wait that failed anywhere may end in a nonfinite error norm first
-    if (!alive || (status == RC_ST_NONFINITE && uni((int)ld_flag(ctl.abort_flag)))) status = RC_ST_WAIT_LIMIT;
+    // every workgroup reports a wait of its own that failed, in whatever stage (rc_system_status)
+    lds_barrier();
+    if (tid == 0 && (s_bad || !alive))
+        __hip_atomic_store(&S.out[RC_OUT_WAIT_FAILED], 1.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (status == RC_ST_OK && next_point != p.npoints) status = RC_ST_MISSING_SAMPLES;
     __builtin_amdgcn_s_waitcnt(0);
     if (my_rank == 0 && tid == 0) {

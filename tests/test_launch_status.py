@@ -1,0 +1,42 @@
+"""What the host makes of a persistent launch's results when a bounded wait failed (CPU: the rules of the
+launch headers, compiled with the host compiler).
+
+A wait that fails marks the results of its launch whatever the controller's status says: the controller may
+have taken its last verdict before (the dense output's stages of the last step), and only one workgroup
+writes its status."""
+import subprocess
+
+import pytest
+
+from conftest import PACKAGE_DIR
+
+CSRC = PACKAGE_DIR / "csrc"
+
+
+def run(tmp_path, body, *includes):
+    """Compile and run a host program over the launch headers; its output's words."""
+    src, exe = tmp_path / "t.cpp", tmp_path / "t"
+    head = "".join(f'#include "{h}"\n' for h in includes)
+    src.write_text(f"#include <stdio.h>\n{head}int main() {{\n{body}\nreturn 0; }}\n")
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", f"-I{CSRC}", "-o", str(exe),
+                    str(src)], check=True)
+    return subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split()
+
+
+@pytest.mark.parametrize("status", ["RC_ST_OK", "RC_ST_MAX_STEPS", "RC_ST_NONFINITE"])
+def test_trajectory_system_with_a_failed_wait(tmp_path, status):
+    out = run(tmp_path, f"""
+        double out[RC_OUT_STRIDE] = {{0}};
+        out[RC_OUT_STATUS] = {status};
+        const int without = rc_system_status(out);
+        out[RC_OUT_WAIT_FAILED] = 1.0;   // by any workgroup, also after the last verdict
+        printf("%d %d\\n", without == {status}, rc_system_status(out) == RC_ST_WAIT_LIMIT);""", "trajectory.h")
+    assert out == ["1", "1"]
+
+
+def test_trajectory_results_have_a_place_each(tmp_path):
+    """The mark lies between the counters and the phase timers."""
+    out = run(tmp_path, """
+        printf("%d %d\\n", RC_OUT_WAIT_FAILED > RC_OUT_NEXTPOINT && RC_OUT_WAIT_FAILED < RC_OUT_TIMERS,
+               RC_OUT_TIMERS + RC_NTIMERS <= RC_OUT_STRIDE);""", "trajectory.h")
+    assert out == ["1", "1"]
