@@ -428,7 +428,10 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
         // coefficient of the newest derivative k_s in the stage input after stage s
         s_alast[tid] = tid == RC_NSTAGES - 1 ? RC_B[tid] : tid + 1 < RC_NSTAGES_EXT ? RC_A[tid + 1][tid] : 0.0;
     }
-    if (tid == 0) s_bad = 0;
+    if (tid == 0) {
+        s_bad = 0;
+        s_verdict[3] = 0.0;
+    }
     __syncthreads();
 
     // phase timers (constant-rate clock ticks): wait for the stage input, (split) slice it, level 1 +
@@ -463,7 +466,6 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
     uint32_t ev = 0;
     uint32_t attempts = 0, accepted = 0, rejected = 0, dense = 0, rhs = 0;
     int next_point = 0, rej = 0, status = RC_ST_OK;
-    bool alive = true;
     const __amdgpu_buffer_rsrc_t rS = rc_rsrc(S.samples, (uint32_t)((size_t)p.npoints * S.nlive * mat_bytes));
     const int my_rank = task - S.first_task;
 
@@ -835,7 +837,7 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
             lap(8);
             next = RC_NSTAGES;
         } else if (slot == RC_NSTAGES) {
-            if (!(alive = unid(s_verdict[3]) == 0.0)) break;
+            if (unid(s_verdict[3]) != 0.0) break;
             const double error = unid(s_verdict[0]);
             factor = unid(s_verdict[1]);
             ysc_new = unid(s_verdict[2]);
@@ -942,7 +944,7 @@ __device__ void run_task(const TrajParams& p, int task, unsigned char* smem_raw)
     }
     // every workgroup reports a wait of its own that failed, in whatever stage (rc_system_status)
     lds_barrier();
-    if (tid == 0 && (s_bad || !alive))
+    if (tid == 0 && (s_bad || s_verdict[3] != 0.0))
         __hip_atomic_store(&S.out[RC_OUT_WAIT_FAILED], 1.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (status == RC_ST_OK && next_point != p.npoints) status = RC_ST_MISSING_SAMPLES;
     __builtin_amdgcn_s_waitcnt(0);
