@@ -747,8 +747,8 @@ __global__ void __launch_bounds__(256) rc_quartic_rhs(RcQuarticArgs g) {
 // Step controller: every workgroup reads all tiles' error sums and runs ode_step_body on them, so
 // all take the same decision.  Ring: 12 events between two gathers, so at event e every reader is
 // done with event e - 16, which is emptied then and next used at e + 16.  Waits are bounded in wall
-// time: a workgroup that outlasts the budget sets the abort word and every workgroup leaves with
-// RC_ST_WAIT_LIMIT.
+// time: a workgroup that outlasts the budget sets the abort word and every workgroup leaves; the host
+// then reports RC_ST_WAIT_LIMIT.
 //
 // Up to 32 workgroups (D <= 16 with one tangent) are laid on one XCD and exchange through its L2.  With
 // that and running sums of the combinations instead of a window of derivatives a right-hand side
@@ -1049,8 +1049,7 @@ __global__ void __launch_bounds__(256, KT <= 2 ? 2 : 1) rc_quartic_ode(const RcO
     }
     reinterpret_cast<cplx*>(p.ybuf)[e] = yv;
     if (wg == 0 && tid == 0) {
-        const bool cut = s_stop || (sc.status == RC_ST_NONFINITE && ld_flag(p.abort_flag));
-        p.out[0] = cut ? (double)RC_ST_WAIT_LIMIT : (double)sc.status;
+        p.out[0] = (double)sc.status;   // the host looks at the abort word first (rc_launch_status)
         p.out[1] = (double)sc.attempts;
         p.out[2] = (double)sc.accepted;
         p.out[3] = (double)sc.rejected;

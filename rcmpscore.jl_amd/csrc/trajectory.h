@@ -82,3 +82,8 @@ enum { RC_OUT_STATUS = 0, RC_OUT_ATTEMPTS, RC_OUT_ACCEPTED, RC_OUT_REJECTED, RC_
 inline int rc_system_status(const double* out) {
     return out[RC_OUT_WAIT_FAILED] != 0.0 ? RC_ST_WAIT_LIMIT : (int)out[RC_OUT_STATUS];
 }
+// The same for a launch that is one integration (rc_quartic_ode): its abort word is set by the first wait that
+// fails, in any workgroup, whatever the status of the workgroup that reports
+inline int rc_launch_status(double status, uint32_t abort_word) {
+    return abort_word ? RC_ST_WAIT_LIMIT : (int)status;
+}

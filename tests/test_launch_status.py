@@ -40,3 +40,11 @@ def test_trajectory_results_have_a_place_each(tmp_path):
         printf("%d %d\\n", RC_OUT_WAIT_FAILED > RC_OUT_NEXTPOINT && RC_OUT_WAIT_FAILED < RC_OUT_TIMERS,
                RC_OUT_TIMERS + RC_NTIMERS <= RC_OUT_STRIDE);""", "trajectory.h")
     assert out == ["1", "1"]
+
+
+def test_integration_launch_with_its_abort_word_set(tmp_path):
+    """The action ODE's launch: another workgroup than the one that reports may have left early."""
+    out = run(tmp_path, """
+        printf("%d %d %d\\n", rc_launch_status(RC_ST_OK, 0) == RC_ST_OK, rc_launch_status(RC_ST_OK, 1) == RC_ST_WAIT_LIMIT,
+               rc_launch_status(RC_ST_NONFINITE, 0) == RC_ST_NONFINITE);""", "trajectory.h")
+    assert out == ["1", "1", "1"]
