@@ -704,12 +704,6 @@ int fused_capacity(rcmps_context* ctx, const rcmps_state* st) {
     return ctx->gm_cap[nb];
 }
 
-struct FusedResult {
-    bool converged;
-    int matvecs;
-    double resid, nb, true_res;
-};
-
 // the operator's part of an equation: direction, momentum shift and the rank-one pin phi, psi
 RcGmresProb fused_problem(const rcmps_state* st, bool adj, double sigma) {
     RcGmresProb p{};
@@ -734,11 +728,12 @@ RcGmresProb fused_problem(const rcmps_state* st, bool adj, double sigma) {
     return p;
 }
 
-// Solve the equations (one padded size, at most fused_capacity of them) and read the results.  The
+// Solve the equations (one padded size, at most fused_capacity of them) and read the results; an equation
+// that failed says so in its own, and its launch's others stand.  The
 // workspaces are given (per equation exch and 8 doubles of out, and an abort word behind those), so
 // that a caller with fixed memory allocates nothing.
 void fused_run(rcmps_context* ctx, int nb, std::vector<RcGmresProb>& ps, double* exch, double* out,
-               RcGmresProb* many, std::vector<FusedResult>& res) {
+               RcGmresProb* many, std::vector<RcGmresResult>& res) {
     const int n = (int)ps.size();
     const size_t eb = rc_gmres_exch_bytes(nb);
     for (int i = 0; i < n; ++i) {
@@ -754,15 +749,11 @@ void fused_run(rcmps_context* ctx, int nb, std::vector<RcGmresProb>& ps, double*
     ck(hipMemcpyAsync(o.data(), out, o.size() * 8, hipMemcpyDeviceToHost, ctx->stream));
     ck(hipStreamSynchronize(ctx->stream));
     res.resize(n);
-    for (int i = 0; i < n; ++i) {
-        const double* q = o.data() + 8 * i;
-        if (q[0] != 0) throw Fail{(int)q[0]};
-        res[i] = FusedResult{q[1] != 0, (int)q[2], q[3], q[4], q[5]};
-    }
+    for (int i = 0; i < n; ++i) res[i] = rc_gmres_result(o.data() + 8 * i);
 }
 
 // the same in the context's workspaces, in as many launches as it takes
-void fused_solve(rcmps_context* ctx, const rcmps_state* st0, std::vector<RcGmresProb>& ps, std::vector<FusedResult>& res) {
+void fused_solve(rcmps_context* ctx, const rcmps_state* st0, std::vector<RcGmresProb>& ps, std::vector<RcGmresResult>& res) {
     const int nb = st0->Dp / 16, cap = std::min(fused_capacity(ctx, st0), 256);
     res.clear();
     for (size_t i0 = 0; i0 < ps.size(); i0 += cap) {
@@ -771,7 +762,7 @@ void fused_solve(rcmps_context* ctx, const rcmps_state* st0, std::vector<RcGmres
         ck(ctx->gm_exch.ensure(n * rc_gmres_exch_bytes(nb)));
         ck(ctx->gm_out.ensure((8 * n + 8) * 8));
         ck(ctx->gm_prob.ensure(n * sizeof(RcGmresProb)));
-        std::vector<FusedResult> r;
+        std::vector<RcGmresResult> r;
         fused_run(ctx, nb, part, ctx->gm_exch.d(), ctx->gm_out.d(),
                   static_cast<RcGmresProb*>(ctx->gm_prob.p), r);
         res.insert(res.end(), r.begin(), r.end());
@@ -1084,8 +1075,9 @@ int rcmps_state_create(rcmps_context* ctx, int D, const double* R, const double*
                 ps[0].tol = steady_tol / 10;
                 ps[0].a = ctx->kry_b.d();
                 ps[0].x = st->rho.d();
-                std::vector<FusedResult> fr;
+                std::vector<RcGmresResult> fr;
                 fused_solve(ctx, st, ps, fr);
+                if (fr[0].status) throw Fail{fr[0].status};
                 okg = fr[0].converged;
                 mv = fr[0].matvecs;
                 res = fr[0].resid;
@@ -1166,9 +1158,10 @@ RcGmresProb boundary_problem(const rcmps_state* st, const double* a, double tol,
     p.x = h;
     return p;
 }
-void boundary_result(const FusedResult& r, double tol, double accept_tol, rcmps_stats* stats) {
+void boundary_result(const RcGmresResult& r, double tol, double accept_tol, rcmps_stats* stats) {
     if (stats) { stats->krylov_matvecs = r.matvecs; stats->krylov_residual = r.true_res; }
-    if (!(r.true_res <= 20 * std::max(tol, accept_tol) * std::max(1.0, r.nb))) throw Fail{RCMPS_ERR_SOLVER};
+    const int code = rc_gmres_code(r, 20 * std::max(tol, accept_tol), RCMPS_ERR_SOLVER);
+    if (code) throw Fail{code};
 }
 
 void boundary_solve(rcmps_context* ctx, const rcmps_state* st, const double* a, double tol, double accept_tol,
@@ -1178,7 +1171,7 @@ void boundary_solve(rcmps_context* ctx, const rcmps_state* st, const double* a, 
     Dev dv{ctx, Dp, D};
     if (D > 1 && fused_capacity(ctx, st) > 0) {
         std::vector<RcGmresProb> ps{boundary_problem(st, a, tol, h)};
-        std::vector<FusedResult> fr;
+        std::vector<RcGmresResult> fr;
         if (bb) fused_run(ctx, Dp / 16, ps, bb->fexch, bb->fout, nullptr, fr);
         else fused_solve(ctx, st, ps, fr);
         boundary_result(fr[0], tol, accept_tol, stats);
@@ -2622,8 +2615,9 @@ void finish_pulled_back(rcmps_context* ctx, double metric_reg, int flags, const 
             ps.push_back(boundary_problem(r.st, fin + 2 * mcount, 1e-13, fin + 4 * mcount));
         }
     }
-    std::vector<FusedResult> fr;
-    if (!ps.empty()) fused_solve(ctx, reqs[idx[fused[0]]].st, ps, fr);
+    // a launch that cannot be made fails the evaluations it was for, not the batch
+    std::vector<RcGmresResult> fr;
+    const int launched = ps.empty() ? RCMPS_OK : guard([&] { fused_solve(ctx, reqs[idx[fused[0]]].st, ps, fr); });
     size_t f = 0;
     for (int j : live) {
         EvalReq& r = reqs[idx[j]];
@@ -2631,6 +2625,7 @@ void finish_pulled_back(rcmps_context* ctx, double metric_reg, int flags, const 
         const bool was_fused = f < fused.size() && fused[f] == j;
         const int code = guard([&] {
             const size_t mcount = (size_t)r.st->Dp * r.st->Dp * 2;
+            if (was_fused && f >= fr.size()) throw Fail{launched};
             if (was_fused) boundary_result(fr[f], 1e-13, 1e-11, r.S);
             else if (boundary) boundary_solve(ctx, r.st, tb.fin.d() + 2 * mcount, 1e-13, 1e-11, tb.fin.d() + 4 * mcount, r.S);
             finish_gradient_part(ctx, r, tb, metric_reg, boundary, nullptr);

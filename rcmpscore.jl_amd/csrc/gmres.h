@@ -23,6 +23,23 @@ struct RcGmresProb {
     double s_re, s_im, sig, c2, ds;
     double tol;              // the GMRES residual aims at tol max(1, |b|)
 };
+// an equation's results as the host reads them from out
+struct RcGmresResult {
+    int status;   // not 0: a wait failed, and the rest means nothing
+    bool converged;
+    int matvecs;
+    double resid, nb, true_res;
+};
+inline RcGmresResult rc_gmres_result(const double* q) {
+    return RcGmresResult{(int)q[0], q[1] != 0, (int)q[2], q[3], q[4], q[5]};
+}
+// what becomes of the equation, whatever became of the launch's others: 0 when its solution is accepted, its
+// status, or `refused` when the residual of the physical equation is above bar max(1, |b|)
+inline int rc_gmres_code(const RcGmresResult& r, double bar, int refused) {
+    if (r.status != 0) return r.status;
+    return r.true_res <= bar * (r.nb > 1.0 ? r.nb : 1.0) ? 0 : refused;
+}
+
 // bytes of the exchange area of one equation at Dp = 16 nb
 __host__ __device__ inline size_t rc_gmres_exch_bytes(int nb) {
     return nb == 1 ? 16 : (size_t)RC_GMRES_RING * nb * nb * 4096 + (size_t)4 * nb * nb * RC_GMRES_REC * 16;

@@ -48,3 +48,16 @@ def test_integration_launch_with_its_abort_word_set(tmp_path):
         printf("%d %d %d\\n", rc_launch_status(RC_ST_OK, 0) == RC_ST_OK, rc_launch_status(RC_ST_OK, 1) == RC_ST_WAIT_LIMIT,
                rc_launch_status(RC_ST_NONFINITE, 0) == RC_ST_NONFINITE);""", "trajectory.h")
     assert out == ["1", "1", "1"]
+
+
+def test_each_equation_of_a_fused_launch_has_its_own_outcome(tmp_path):
+    """Three equations of one launch: accepted, a wait that failed, a residual above the bar (and NaN).  Only
+    the failed ones carry a code, so the evaluations beside them in a batch are complete."""
+    out = run(tmp_path, """
+        const double q[4][8] = {{0, 1, 17, 1e-14, 2.0, 1e-13, 0, 0}, {7, 0, 3, 0, 0, 0, 0, 0},
+                                {0, 0, 200, 1e-3, 0.5, 1e-3, 0, 0}, {0, 0, 2, __builtin_nan(""), 1.0, __builtin_nan(""), 0, 0}};
+        for (const double* o : q) printf("%d ", rc_gmres_code(rc_gmres_result(o), 2e-10, 10));
+        const RcGmresResult r = rc_gmres_result(q[0]);
+        printf("%d %d\\n", r.converged && r.matvecs == 17 && r.resid == 1e-14 && r.nb == 2.0 && r.true_res == 1e-13,
+               rc_gmres_code({0, true, 1, 0.0, 2.0, 3e-10}, 2e-10, 10));""", "gmres.h")
+    assert out == ["0", "7", "10", "10", "1", "0"]
