@@ -51,7 +51,10 @@ struct RcQuarticArgs {
     const int* active;    // device flag: the launch does nothing when it reads 0 (null: always runs)
 };
 
+// WIDE: Dp > 64 (more than four k-tiles)
+template <bool WIDE>
 __global__ void rc_quartic_p(RcQuarticArgs g);
+template <bool WIDE>
 __global__ void rc_quartic_rhs(RcQuarticArgs g);
 
 // arguments of rc_pair_rhs: pair p's state at U + p ustride (matrix (channel c, block k) at (4 c + k)

@@ -470,6 +470,28 @@ __device__ __forceinline__ void qprod(cacc& acc, const cplx* A, const cplx* B, i
         if (i < nk && ((kmask >> i) & 1)) cmfma(acc, cscale(scale, a[i]), b[i]);
 }
 
+// The same beyond Dp = 64, over k-tiles first .. first + count - 1, four at a time in the k order.  (One
+// function for both, with the loop, costs a right-hand side at D = 16 to 64 1 to 3%.)
+struct KTiles {
+    int first, count;
+};
+__device__ __forceinline__ void qprod_wide(cacc& acc, const cplx* A, const cplx* B, int Dp, int bi, int bj, int wave,
+                                           int lane, double scale, KTiles kt) {
+    for (int g = 0; g < kt.count; g += 4) {
+        cplx a[4], b[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (g + i < kt.count) {
+                const int kk = 16 * (kt.first + g + i) + 4 * wave + (lane >> 4);
+                a[i] = A[(16 * bi + (lane & 15)) * Dp + kk];
+                b[i] = B[kk * Dp + 16 * bj + (lane & 15)];
+            }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (g + i < kt.count) cmfma(acc, cscale(scale, a[i]), b[i]);
+    }
+}
+
 // A[tile rows, :] T with T a Dp x 16 block in LDS
 __device__ __forceinline__ void qprod_t(cacc& acc, const cplx* A, const cplx* T, int Dp, int bi, int wave, int lane,
                                         double scale, int kmask = 15) {
@@ -486,9 +508,16 @@ __device__ __forceinline__ void qprod_t(cacc& acc, const cplx* A, const cplx* T,
         }
 }
 
-// k-tile mask of A(b, :) B(:, c) for operands of parities pa, pb under parity blocks of zt tiles (zt = 0:
-// every k-tile): zero unless the output tile's blocks have parity pa ^ pb, then the k-tiles of block
+// k-tiles of A(b, :) B(:, c) for operands of parities pa, pb under parity blocks of zt tiles (zt = 0:
+// every k-tile): none unless the output tile's blocks have parity pa ^ pb, then the k-tiles of block
 // blk(b) ^ pa.  The skipped k-steps multiply exact zeros, so the sums keep their bits.
+__device__ __forceinline__ KTiles zrange(int zt, int nk, int b, int c, int pa, int pb) {
+    if (zt == 0) return KTiles{0, nk};
+    const int bb = b / zt, bc = c / zt;
+    if ((bb ^ bc) != (pa ^ pb)) return KTiles{0, 0};
+    return KTiles{(bb ^ pa) * zt, zt};
+}
+// the same as a mask, up to four k-tiles
 __device__ __forceinline__ int zmask(int zt, int nk, int b, int c, int pa, int pb) {
     if (zt == 0) return 15;
     const int bb = b / zt, bc = c / zt;
@@ -564,10 +593,11 @@ __device__ __forceinline__ void qmat_of(int mi, int nb, int& blk, int& a, int& k
 
 // Operands of tile (bi, bj) of matrix mi: the constant matrices, the tangent's, the stage input's and the
 // level-1 matrices' of this channel and of its neighbour, whose insertion it takes; Z2 parities and
-// k-tile masks (see RcQuarticArgs).  Parities for g.zt > 0: Q, Q^+ and the shifted ones even, R, R^+
+// their k-tiles (see RcQuarticArgs).  Parities for g.zt > 0: Q, Q^+ and the shifted ones even, R, R^+
 // odd, w = W of parity pw, v = -R^+ W of parity pw ^ 1; channels x_k and a1_k of parity k & 1 (x_0 =
 // rho, a1 of the last channel = I), y_k and a0_k of parity (k + 1 + pw) & 1 (y_0 = R W, a0 driven by
 // a1 w and a1 v).
+template <bool WIDE>
 struct QTile {
     int Dp, bi, bj, blk, a, k, nb, zt, nk, pw, px, py, lane, wave;
     long long m;
@@ -600,7 +630,8 @@ struct QTile {
     }
     // acc += scale A(bi, :) B(:, bj), operands of parities pa, pb
     __device__ __forceinline__ void add(cacc& acc, double scale, const cplx* A, int pa, const cplx* B, int pb) const {
-        qprod(acc, A, B, Dp, bi, bj, wave, lane, scale, zmask(zt, nk, bi, bj, pa, pb));
+        if constexpr (WIDE) qprod_wide(acc, A, B, Dp, bi, bj, wave, lane, scale, zrange(zt, nk, bi, bj, pa, pb));
+        else qprod(acc, A, B, Dp, bi, bj, wave, lane, scale, zmask(zt, nk, bi, bj, pa, pb));
     }
     __device__ __forceinline__ long long element() const {
         return (long long)blockIdx.y * m + (16 * bi + (threadIdx.x >> 4)) * Dp + 16 * bj + (threadIdx.x & 15);
@@ -608,10 +639,11 @@ struct QTile {
 };
 
 // Level 1 of a right-hand side: the tiles of P (x R^+, y R^+, a0 R + a1 w, a1 R).
+template <bool WIDE>
 __global__ void __launch_bounds__(256) rc_quartic_p(RcQuarticArgs g) {
     __shared__ cplx red[1024];
     if (g.active && !*g.active) return;
-    const QTile q(g);
+    const QTile<WIDE> q(g);
     const cplx* U = reinterpret_cast<const cplx*>(g.U);
     cacc acc;
     cacc_zero(acc);
@@ -626,7 +658,8 @@ __global__ void __launch_bounds__(256) rc_quartic_p(RcQuarticArgs g) {
 
 // Level 2: the one-sided products, then R P (and w P^x), then the insertion's P tile; thread t receives
 // element (t/16, t%16).  The order of the sums is rc_quartic_ode's.
-__device__ __forceinline__ cplx quartic_tile(const RcQuarticArgs& g, const QTile& q, double jac, double jt, cplx* red) {
+template <bool WIDE>
+__device__ __forceinline__ cplx quartic_tile(const RcQuarticArgs& g, const QTile<WIDE>& q, double jac, double jt, cplx* red) {
     const cplx* U = reinterpret_cast<const cplx*>(g.U);
     const cplx* P = reinterpret_cast<const cplx*>(g.P);
     const int blk = q.blk, k = q.k, px = q.px, py = q.py, pw = q.pw;
@@ -686,11 +719,12 @@ __device__ __forceinline__ cplx tile_error_sum(const double* s) {
     return cmake(((s[0] + s[1]) + s[2]) + s[3], ((s[4] + s[5]) + s[6]) + s[7]);
 }
 
+template <bool WIDE>
 __global__ void __launch_bounds__(256) rc_quartic_rhs(RcQuarticArgs g) {
     __shared__ cplx red[1024];
     if (g.active && !*g.active) return;
     const int tid = threadIdx.x;
-    const QTile q(g);
+    const QTile<WIDE> q(g);
     const int nbt = q.nk, mi = blockIdx.y;
     const cplx* U = reinterpret_cast<const cplx*>(g.U);
     const double jac = g.coef ? g.coef[0] : g.jac;
@@ -727,6 +761,10 @@ __global__ void __launch_bounds__(256) rc_quartic_rhs(RcQuarticArgs g) {
         g.partial[2 * slot + 1] = es.im;
     }
 }
+template __global__ void rc_quartic_p<false>(RcQuarticArgs g);
+template __global__ void rc_quartic_p<true>(RcQuarticArgs g);
+template __global__ void rc_quartic_rhs<false>(RcQuarticArgs g);
+template __global__ void rc_quartic_rhs<true>(RcQuarticArgs g);
 
 // ---------------------------------------------------------------------------------------------
 // The whole :phi^4: action ODE integration in one persistent launch (cooperative: every workgroup
