@@ -290,7 +290,8 @@ int rcmps_excitation_action_multi(rcmps_context* ctx, int n, rcmps_excitation* c
 /* Connected matrix elements <Phi_p(U_i)|H - E0|Phi_p(W_i)> per 2 pi delta(0) of n tangent pairs (each with
    its context; one state): the pair environments, the four-block :phi^4: transfer ODE and the kinetic
    resolvent sum on kinetic_nodes theta nodes (excitation_element, src/excitations.jl:98-113, with
-   ExcitationPair src/excitation_environments.jl:105-127).  out (host): 2n doubles, the complex values.
+   ExcitationPair src/excitation_environments.jl:105-127).  D <= 272 (RCMPS_ERR_UNSUPPORTED above).  out
+   (host): 2n doubles, the complex values.
    The route the reference's validation calls "bilinear" (src/excitation_eigsolve.jl:273-279). */
 int rcmps_excitation_element(rcmps_context* ctx, int n, rcmps_excitation* const* exs, const double* const* U,
                              const double* const* W, double g, const double* kinetic_coef, const rcmps_integrator* ip,

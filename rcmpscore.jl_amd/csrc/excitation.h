@@ -85,6 +85,10 @@ struct RcPairArgs {
     const int* active;    // as RcQuarticArgs::active
 };
 
+// WIDE: Dp > 64, with RC_PAIR_LDS(Dp) bytes of dynamic LDS, at most RC_PAIR_LDS_MAX (beside the kernel's own 16 KB)
+#define RC_PAIR_LDS(Dp) ((size_t)2 * (Dp) * 256)
+#define RC_PAIR_LDS_MAX ((size_t)143 * 1024)
+template <bool WIDE>
 __global__ void rc_pair_rhs(RcPairArgs g);
 __global__ void rc_res_scale(long long N, int nz, int per_basis, int adjoint, const double* Y, const double* mu,
                              const double* z, const double* s, double* out);

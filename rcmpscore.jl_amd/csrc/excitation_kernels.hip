@@ -508,6 +508,22 @@ __device__ __forceinline__ void qprod_t(cacc& acc, const cplx* A, const cplx* T,
         }
 }
 
+// the same beyond Dp = 64
+__device__ __forceinline__ void qprod_t_wide(cacc& acc, const cplx* A, const cplx* T, int Dp, int bi, int wave,
+                                             int lane, double scale) {
+    const int nk = Dp / 16;
+    for (int g = 0; g < nk; g += 4) {
+        cplx a[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (g + i < nk) a[i] = A[(16 * bi + (lane & 15)) * Dp + 16 * (g + i) + 4 * wave + (lane >> 4)];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (g + i < nk)
+                cmfma(acc, cscale(scale, a[i]), T[(16 * (g + i) + 4 * wave + (lane >> 4)) * 16 + (lane & 15)]);
+    }
+}
+
 // k-tiles of A(b, :) B(:, c) for operands of parities pa, pb under parity blocks of zt tiles (zt = 0:
 // every k-tile): none unless the output tile's blocks have parity pa ^ pb, then the k-tiles of block
 // blk(b) ^ pa.  The skipped k-steps multiply exact zeros, so the sums keep their bits.
@@ -1242,10 +1258,14 @@ __global__ void __launch_bounds__(256) rc_two_sided(int Dp, int D, const double*
 // jt = 0 this is the transfer alone (the Krylov operator of the kinetic resolvent).  grid
 // ((Dp/16)^2, npair * nch * 4).
 // ---------------------------------------------------------------------------------------------
+template <bool WIDE>
 __global__ void __launch_bounds__(256) rc_pair_rhs(RcPairArgs g) {
     __shared__ cplx red[1024];
-    __shared__ cplx T1[64 * 16];
-    __shared__ cplx T2[64 * 16];
+    // the column blocks T1 and T2, Dp x 16 each: for WIDE in dynamic LDS
+    __shared__ cplx columns[WIDE ? 1 : 2 * 64 * 16];
+    extern __shared__ __align__(16) unsigned char pair_lds[];
+    cplx* T1 = WIDE ? reinterpret_cast<cplx*>(pair_lds) : columns;
+    cplx* T2 = T1 + (WIDE ? g.Dp * 16 : 64 * 16);
     if (g.active && !*g.active) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int Dp = g.Dp, nbt = Dp / 16, bi = blockIdx.x / nbt, bj = blockIdx.x % nbt;
@@ -1269,40 +1289,49 @@ __global__ void __launch_bounds__(256) rc_pair_rhs(RcPairArgs g) {
     const double cj = c * jt;
     cacc acc;
     cacc_zero(acc);
+    // acc += scale A(bi, :) B(:, bj); with T in LDS, of its columns
+    auto mul = [&](const cplx* A, const cplx* B, double scale) {
+        if constexpr (WIDE) qprod_wide(acc, A, B, Dp, bi, bj, wave, lane, scale, KTiles{0, nbt});
+        else qprod(acc, A, B, Dp, bi, bj, wave, lane, scale);
+    };
+    auto mul_t = [&](const cplx* A, const cplx* T) {
+        if constexpr (WIDE) qprod_t_wide(acc, A, T, Dp, bi, wave, lane, jac);
+        else qprod_t(acc, A, T, Dp, bi, wave, lane, jac);
+    };
     if (jac != 0.0) {
         const cplx* xk = x(c, k);
-        qprod(acc, k == 1 ? Qs : k == 2 ? Qb : Q, xk, Dp, bi, bj, wave, lane, jac);
-        qprod(acc, xk, Qh, Dp, bi, bj, wave, lane, jac);
+        mul(k == 1 ? Qs : k == 2 ? Qb : Q, xk, jac);
+        mul(xk, Qh, jac);
         if (k == 0) {
             qcolumns(T1, QTerm{xk, Rh}, QTerm{}, nullptr, QTerm{}, QTerm{}, Dp, bj, wave, lane);
-            qprod_t(acc, R, T1, Dp, bi, wave, lane, jac);
+            mul_t(R, T1);
         } else if (k == 1) {
-            qprod(acc, v, x(c, 0), Dp, bi, bj, wave, lane, jac);
+            mul(v, x(c, 0), jac);
             qcolumns(T1, QTerm{xk, Rh}, QTerm{}, T2, QTerm{x(c, 0), Rh}, QTerm{}, Dp, bj, wave, lane);
-            qprod_t(acc, R, T1, Dp, bi, wave, lane, jac);
-            qprod_t(acc, w, T2, Dp, bi, wave, lane, jac);
+            mul_t(R, T1);
+            mul_t(w, T2);
         } else if (k == 2) {
-            qprod(acc, x(c, 0), vbh, Dp, bi, bj, wave, lane, jac);
+            mul(x(c, 0), vbh, jac);
             qcolumns(T1, QTerm{xk, Rh}, QTerm{x(c, 0), uh}, nullptr, QTerm{}, QTerm{}, Dp, bj, wave, lane);
-            qprod_t(acc, R, T1, Dp, bi, wave, lane, jac);
+            mul_t(R, T1);
         } else {
-            qprod(acc, v, x(c, 2), Dp, bi, bj, wave, lane, jac);
-            qprod(acc, x(c, 1), vbh, Dp, bi, bj, wave, lane, jac);
+            mul(v, x(c, 2), jac);
+            mul(x(c, 1), vbh, jac);
             qcolumns(T1, QTerm{xk, Rh}, QTerm{x(c, 1), uh}, T2, QTerm{x(c, 2), Rh},
                      QTerm{x(c, 0), uh}, Dp, bj, wave, lane);
-            qprod_t(acc, R, T1, Dp, bi, wave, lane, jac);
-            qprod_t(acc, w, T2, Dp, bi, wave, lane, jac);
+            mul_t(R, T1);
+            mul_t(w, T2);
         }
     }
     if (c >= 1 && cj != 0.0) {
         const cplx* xp = x(c - 1, k);
-        qprod(acc, R, xp, Dp, bi, bj, wave, lane, cj);
-        qprod(acc, xp, Rh, Dp, bi, bj, wave, lane, cj);
-        if (k == 1) qprod(acc, w, x(c - 1, 0), Dp, bi, bj, wave, lane, cj);
-        if (k == 2) qprod(acc, x(c - 1, 0), uh, Dp, bi, bj, wave, lane, cj);
+        mul(R, xp, cj);
+        mul(xp, Rh, cj);
+        if (k == 1) mul(w, x(c - 1, 0), cj);
+        if (k == 2) mul(x(c - 1, 0), uh, cj);
         if (k == 3) {
-            qprod(acc, w, x(c - 1, 2), Dp, bi, bj, wave, lane, cj);
-            qprod(acc, x(c - 1, 1), uh, Dp, bi, bj, wave, lane, cj);
+            mul(w, x(c - 1, 2), cj);
+            mul(x(c - 1, 1), uh, cj);
         }
     }
     cplx val = qreduce(acc, red, wave, lane);
@@ -1347,6 +1376,8 @@ __global__ void __launch_bounds__(256) rc_pair_rhs(RcPairArgs g) {
         g.partial[2 * slot + 1] = s3[0];
     }
 }
+template __global__ void rc_pair_rhs<false>(RcPairArgs g);
+template __global__ void rc_pair_rhs<true>(RcPairArgs g);
 
 // Which parity blocks (halves of the basis) of the tangents' matrices hold a nonzero: bit 0 of
 // flags[i] an even block of W, bit 1 an odd one, bits 2 and 3 the same of v.  Matrix i at + i ts complex.

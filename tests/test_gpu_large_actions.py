@@ -4,6 +4,9 @@ sums serve them and a product has more than four k-tiles.
 - D = 65: the :phi^4: part of F(W) against the oracle's (dense Poisson factors, SciPy's DOP853), both
   integrated to 1e-11 over a short window: within 1e-8 of |F|, the existing action test's 1e-9 at 1e-12
   scaled with the tolerance.
+- D = 65: the connected element's kinetic part against <u, F(w)>, whose products are other kernels (2e-8, as
+  the existing element test), its :phi^4: part against the oracle's (1e-8, as above; <u, F(w)> has the
+  quadrature error of its few nodes there, the element none).
 - D = 96: a Z2 state's parity blocks (three tiles each) skip only zeros, so the bits are those of every
   k-tile.
 """
@@ -32,13 +35,17 @@ def short_window(rg, tol=1e-11):
     return rg.IntegratorParameters(n_quad=8, max_point=2.0, atol=tol, rtol=tol)
 
 
-def oracle_context(s, ip, p):
-    """The oracle's context with the two Poisson factors an action needs (no Schur form of the transfer)."""
+def oracle_context(s, ip, p, bra=False):
+    """The oracle's context with the Poisson factors an action needs, an element's third on request (no Schur
+    form of the transfer)."""
     xs = X.XState(s.R, s.Q, s.rho, n_quad=ip.n_quad, max_point=ip.max_point, atol=ip.atol, rtol=ip.rtol)
     a = np.outer(s.rho.ravel(), np.eye(s.D).ravel()) - X.transfer_matrix(s.Q, s.R)
-    poisson = sla.lu_factor(a)
-    a[np.diag_indices(len(a))] += 1j * p
-    return X.Context(xs, p, None, None, None, poisson, sla.lu_factor(a, overwrite_a=True), None, 1e-10)
+    factors = []
+    for shift in (0.0, 1.0, -1.0) if bra else (0.0, 1.0):
+        b = a.copy()
+        b[np.diag_indices(len(b))] += 1j * shift * p
+        factors.append(sla.lu_factor(b, overwrite_a=True))
+    return X.Context(xs, p, None, None, None, factors[0], factors[1], factors[2] if bra else None, 1e-10)
 
 
 def test_phi4_action_matches_oracle(rg):
@@ -73,5 +80,24 @@ def test_z2_blocks_of_three_tiles_give_the_same_bits(rg):
     a, b = (action_batch(ctx, [w], ExcitationModel("phi4", 1.5), 8, parts=2, z2_blocks=z2)[0] for z2 in (True, False))
     assert np.isfinite(a).all() and np.abs(a).max() > 0
     assert np.array_equal(a, b)
+    ctx.close()
+    s.close()
+
+
+def test_connected_element(rg):
+    d, p, g = 65, 0.3, 1.5
+    note(f"case: connected element D={d} p={p}")
+    from rcmps_gpu.excitation import ExcitationContext, ExcitationModel, action_batch, excitation_element
+    s = rg.State(*rg.random_state_arrays(d, scaling=0.1, seed=3), steady_tol=1e-12)
+    s.integrator_param = short_window(rg)
+    rng = np.random.default_rng(1)
+    u, w = rng.standard_normal((2, d, d)) + 1j * rng.standard_normal((2, d, d))
+    ctx, model = ExcitationContext(s, p, dense_transfer=False), ExcitationModel("phi4", g)
+    (f,) = action_batch(ctx, [w], model, 32, parts=1)
+    kin, pot = (excitation_element(ctx, [u], [w], model=model, kinetic_nodes=32, parts=parts)[0] for parts in (1, 2))
+    ref = g * X.excitation_observable(X.pair(oracle_context(s, s.integrator_param, p, bra=True), u, w), X.monomial_spec(4))
+    note(f"  kinetic {kin} vs {np.vdot(u, f)}; potential {pot} vs {ref}")
+    assert abs(np.vdot(u, f) - kin) <= 2e-8 * max(1.0, abs(kin))
+    assert abs(pot - ref) <= 1e-8 * max(1.0, abs(ref))
     ctx.close()
     s.close()
