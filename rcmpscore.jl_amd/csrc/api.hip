@@ -2638,6 +2638,12 @@ void finish_pulled_back(rcmps_context* ctx, double metric_reg, int flags, const 
     for (int j : live) reqs[idx[j]].S->boundary_ms = ms / live.size();
 }
 
+// A launch's evaluations each have exchange rings of their own (122 MiB at Dp = 64).  A class whose rings would
+// take more than this runs in several launches, so that the memory of a batch of hundreds is that of its
+// samples (110 evaluations at D = 64: 12.6 -> 8.2 GiB).  67 evaluations at Dp = 64 fill the chip 67 times over, so
+// that one more launch costs nothing: 128 of them took 1367 ms in one launch and take 1363 in two.
+constexpr size_t kRingBytes = (size_t)8 << 30;
+
 // The classes run smallest first: a class's finishing then runs under a longer launch, and only the
 // last class's is left.  That one is cut in two launches, the second of about an eighth of its
 // states, so that the first part finishes under the second launch.  Results do not depend on
@@ -2674,7 +2680,11 @@ int fg_phi4_batch_impl(rcmps_context* ctx, std::vector<EvalReq>& reqs, const rcm
             std::vector<int> idx;
             for (size_t i = 0; i < reqs.size(); ++i)
                 if (reqs[i].st->Dp == Dp) idx.push_back((int)i);
-            if (!idx.empty()) classes.push_back(std::move(idx));
+            if (idx.empty()) continue;
+            const size_t fit = std::max<size_t>(1, kRingBytes / exchange_bytes(Dp, true, krylov));
+            const size_t parts = (idx.size() + fit - 1) / fit, n = idx.size();
+            for (size_t p = 0; p < parts; ++p)
+                classes.emplace_back(idx.begin() + n * p / parts, idx.begin() + n * (p + 1) / parts);
         }
         if (!krylov && !classes.empty() && classes.back().size() >= 8) {
             std::vector<int>& last = classes.back();
