@@ -232,7 +232,7 @@ double opnorm2(int n, const Mat& A) {
         double f = 0;
         for (auto& v : B) f += std::norm(v);
         f = std::sqrt(f);
-        if (!(f > 0)) return f;
+        if (!(f > 0) || !std::isfinite(f)) return f;   // zero, or |A|^4 overflows: the power iteration has no step
         for (auto& v : B) v /= f;
         if (p == 3) break;
         matmul(n, B, B, C);
