@@ -1,5 +1,5 @@
 """Excitation actions and elements beyond 64 (Dp = 80 and 96), where no persistent launch and no fused node
-sums serve them and a product has more than four k-tiles.
+sums serve them and a product has more than four k-tiles, and more Arnoldi bases than fit one launch.
 
 - D = 65: the :phi^4: part of F(W) against the oracle's (dense Poisson factors, SciPy's DOP853), both
   integrated to 1e-11 over a short window: within 1e-8 of |F|, the existing action test's 1e-9 at 1e-12
@@ -7,6 +7,9 @@ sums serve them and a product has more than four k-tiles.
 - D = 65: the connected element's kinetic part against <u, F(w)>, whose products are other kernels (2e-8, as
   the existing element test), its :phi^4: part against the oracle's (1e-8, as above; <u, F(w)> has the
   quadrature error of its few nodes there, the element none).
+- D = 64, five tangents: ten two-block bases, of which eight fit a launch of the persistent Arnoldi steps.
+  The kinetic part of each against the tangent alone, 1e-8 of |F| with solves accepted at 1e-11 (as the
+  existing batch test: a set's bases grow together, so alone they may be smaller).
 - D = 96: a Z2 state's parity blocks (three tiles each) skip only zeros, so the bits are those of every
   k-tile.
 """
@@ -100,4 +103,24 @@ def test_connected_element(rg):
     assert abs(np.vdot(u, f) - kin) <= 2e-8 * max(1.0, abs(kin))
     assert abs(pot - ref) <= 1e-8 * max(1.0, abs(ref))
     ctx.close()
+    s.close()
+
+
+def test_more_bases_than_a_launch_holds(rg):
+    d, n = 64, 5
+    note(f"case: kinetic action D={d}, {n} tangents")
+    from rcmps_gpu.excitation import ExcitationContext, ExcitationModel, action_batch
+    s = rg.State(*rg.random_state_arrays(d, scaling=0.2, seed=7), steady_tol=1e-12)
+    rng = np.random.default_rng(d)
+    ws = [rng.standard_normal((d, d)) + 1j * rng.standard_normal((d, d)) for _ in range(n)]
+    ctxs = [ExcitationContext(s, 0.1 + 0.2 * i, dense_transfer=False) for i in range(n)]
+    tight = rg.KineticKrylovOptions(tolerance=1e-11, fallback_tolerance=1e-11)
+    model = ExcitationModel("phi4", 2.0)
+    together = action_batch(ctxs, ws, model, 32, parts=1, krylov_options=tight)
+    for c, w, f in zip(ctxs, ws, together):
+        (alone,) = action_batch(c, [w], model, 32, parts=1, krylov_options=tight)
+        note(f"  |together - alone| / |F| = {np.abs(f - alone).max() / np.abs(alone).max():.2e}")
+        assert np.abs(f - alone).max() <= 1e-8 * np.abs(alone).max()
+    for c in ctxs:
+        c.close()
     s.close()
