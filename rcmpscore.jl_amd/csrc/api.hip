@@ -310,7 +310,7 @@ int gemm_variant(rcmps_context* ctx, int Dp, int nbatch) {
     double* buf = ctx->tune_buf.d();
     ck(hipMemsetAsync(buf, 0, 3 * (size_t)nb_t * mat * 8, ctx->stream));
     GemmArgs g{};
-    g.Dp = Dp; g.D = Dp; g.nbatch = nb_t;
+    g.Dp = Dp; g.nbatch = nb_t;
     g.A = buf; g.B = buf + nb_t * mat; g.C = buf + 2 * nb_t * mat;
     g.strideA = g.strideB = g.strideC = (long long)Dp * Dp;
     hipEvent_t e0, e1;
@@ -362,19 +362,19 @@ struct Dev {
     void gemm(int opA, const double* A, int opB, const double* B, double* C, double alpha = 1.0,
               double beta = 0.0) {
         GemmArgs g{};
-        g.Dp = Dp; g.D = D; g.nbatch = 1; g.opA = opA; g.opB = opB;
+        g.Dp = Dp; g.nbatch = 1; g.opA = opA; g.opB = opB;
         g.A = A; g.B = B; g.C = C;
         g.beta = beta;
         g.alpha_scale = alpha;
         launch_zgemm(ctx, g, 1);
     }
     void batched(GemmArgs g, int nbatch) {
-        g.Dp = Dp; g.D = D; g.nbatch = nbatch;
+        g.Dp = Dp; g.nbatch = nbatch;
         launch_zgemm(ctx, g, nbatch);
     }
     // C = beta C + scale * sum_b alpha_b op(A_b) op(B_b)
     void reduce(GemmArgs g, int nbatch, double* C, double scale, double beta) {
-        g.Dp = Dp; g.D = D; g.nbatch = nbatch;
+        g.Dp = Dp; g.nbatch = nbatch;
         const int nt = (Dp / 16) * (Dp / 16);
         int chunks = std::max(1, std::min(nbatch, 256 / nt * 2));
         int chunk = ceil_div(nbatch, chunks);

@@ -494,15 +494,15 @@ __device__ __forceinline__ void qprod_wide(cacc& acc, const cplx* A, const cplx*
 
 // A[tile rows, :] T with T a Dp x 16 block in LDS
 __device__ __forceinline__ void qprod_t(cacc& acc, const cplx* A, const cplx* T, int Dp, int bi, int wave, int lane,
-                                        double scale, int kmask = 15) {
+                                        double scale) {
     const int nk = Dp / 16;
     cplx a[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-        if (i < nk && ((kmask >> i) & 1)) a[i] = A[(16 * bi + (lane & 15)) * Dp + 4 * (wave + 4 * i) + (lane >> 4)];
+        if (i < nk) a[i] = A[(16 * bi + (lane & 15)) * Dp + 4 * (wave + 4 * i) + (lane >> 4)];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-        if (i < nk && ((kmask >> i) & 1)) {
+        if (i < nk) {
             const int kk = 4 * (wave + 4 * i) + (lane >> 4);
             cmfma(acc, cscale(scale, a[i]), T[kk * 16 + (lane & 15)]);
         }

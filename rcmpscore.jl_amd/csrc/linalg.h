@@ -3,18 +3,14 @@
 #include <hip/hip_runtime.h>
 
 struct GemmArgs {
-    int Dp, D, nbatch, opA, opB, alpha_stride;
-    long long strideA, strideB, strideC, strideD;   // in complex elements
+    int Dp, nbatch, opA, opB, alpha_stride;
+    long long strideA, strideB, strideC;   // in complex elements
     const double* A;
     const double* B;
     double* C;
     const double* alpha;    // per-batch real weight (index batch*alpha_stride) or null
     double beta;
     double alpha_scale;     // scalar factor on the product; 0 means 1
-    const double* addD;     // optional: C += dscale * dalpha_b * D_b
-    const double* dalpha;
-    double dscale;
-    double add_identity;    // optional: C += add_identity * dalpha_b * I (on the D x D block)
 };
 
 __global__ void rc_zgemm_batched(GemmArgs g);
