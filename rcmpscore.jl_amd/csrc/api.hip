@@ -197,7 +197,8 @@ struct rcmps_context {
     // persistent Arnoldi steps (rc_arnoldi): exchange areas, descriptors behind the abort word; bases
     // per launch by blocks and tiles per side
     DevBuf arn_exch, arn_prob;
-    DevBuf pull_list;   // a pullback's entries and terms
+    DevBuf pull_list;   // a pullback's entries and terms, and the host's copy, which lives until the copy has run
+    std::vector<char> pull_host;
     int arn_cap[2][5] = {{-1, -1, -1, -1, -1}, {-1, -1, -1, -1, -1}};
     // GMRES read-back: two pinned slots of one Hessenberg column each, and their completion events
     double* kry_pinned = nullptr;
@@ -1658,13 +1659,12 @@ const double* metric_inverse(rcmps_context* ctx, const rcmps_state* st, double m
     return st->Minv.d();
 }
 
-// Pullback over the Gauss nodes, boundary correction and gradients of one evaluation whose
-// trajectories are in tb (src/observables.jl:161-212).  With kin_cov/kin_env (device) the two
-// kinetic terms come from the infinite-line backend and only the :phi^4: trajectories are pulled back.
 // the lists of a pullback's sums on the device
 void pull_lists(rcmps_context* ctx, const std::vector<RcPullEntry>& en, const std::vector<RcPullTerm>& tm, RcPullArgs& pa) {
     const size_t eb = en.size() * sizeof(RcPullEntry), tb = tm.size() * sizeof(RcPullTerm);
-    std::vector<char> h(eb + tb);
+    // every caller waits for its stream before the next pullback on this context
+    std::vector<char>& h = ctx->pull_host;
+    h.resize(eb + tb);
     std::memcpy(h.data(), en.data(), eb);
     std::memcpy(h.data() + eb, tm.data(), tb);
     ck(ctx->pull_list.ensure(h.size()));
