@@ -1532,9 +1532,8 @@ bool schedule_tasks(const std::vector<TrajSys>& sys, const std::vector<TrajTask>
     return true;
 }
 
-// Integrate every system of the given evaluations (all of one padded size Dp) in one persistent
-// launch of at most the resident workgroup count.  Evaluation j
-// keeps its trajectories in ctx->tb[tb0 + j].
+// Integrate every system of the given evaluations (all of one padded size Dp) in one persistent launch of at
+// most the resident workgroup count.  Evaluation j keeps its trajectories in ctx->tb[tb0 + j].
 void run_class(rcmps_context* ctx, int Dp, bool split, bool quartic_only, bool timers, bool z2,
                const rcmps_integrator* ip, const std::vector<int>& idx, size_t tb0, std::vector<EvalReq>& reqs) {
     const int NB = Dp / 16, npts = 2 * ip->n_quad + 1;
@@ -1674,9 +1673,11 @@ void pull_lists(rcmps_context* ctx, const std::vector<RcPullEntry>& en, const st
     pa.nterms = (int)tm.size();
 }
 
-// The finishing of an evaluation in three parts: the pullback into tb.fin, the boundary solve of its
-// environment, the gradient.  tb.fin holds XR, XQ, env, cov and the boundary's solution, with
-// dE = 2 Re tr(XR dR) + 2 Re tr(XQ dQ) for any (dR, dQ) and covector = XR - XQ R^+ (+ the kinetic one).
+// The finishing of an evaluation whose trajectories are in tb (src/observables.jl:161-212), in three parts: the
+// pullback over the Gauss nodes into tb.fin, the boundary solve of its environment, the gradient.  tb.fin
+// holds XR, XQ, env, cov and the boundary's solution, with dE = 2 Re tr(XR dR) + 2 Re tr(XQ dQ) for any
+// (dR, dQ) and covector = XR - XQ R^+ (+ the kinetic one).  With kin_cov/kin_env (device) the two kinetic
+// terms come from the infinite-line backend and only the :phi^4: trajectories are pulled back.
 void covector(Dev& dv, const rcmps_state* st, const double* XR, const double* XQ, const double* kin_cov, double* cterm,
               double* cov) {   // horizontal directions dQ = -R^+ W
     dv.gemm(0, XQ, 0, st->Rh.d(), cterm);
@@ -2532,8 +2533,8 @@ bool valid_integrator(const rcmps_integrator* ip) {
     return ip && ip->n_quad >= 8 && ip->max_point > 0 && ip->atol > 0 && ip->rtol > 0 && ip->maxiters >= 1;
 }
 
-// A batch of evaluations: grouped by padded size, one persistent launch per group, then the
-// pullback of each evaluation.  Every request gets its stats; the first failure is returned.
+// A batch of evaluations: grouped by padded size, one persistent launch per group (several for a group of
+// hundreds, kRingBytes), then the pullback of each evaluation.  Every request gets its stats; the first failure is returned.
 // The per-state pullbacks of one class run on up to kFinishWorkers worker contexts, each driven by its
 // own host thread and stream, while the main stream integrates the next class; the boundary solves of
 // the class then run together on the main context, and the gradients.  The kernels and tile choices
@@ -2638,9 +2639,9 @@ void finish_pulled_back(rcmps_context* ctx, double metric_reg, int flags, const 
     for (int j : live) reqs[idx[j]].S->boundary_ms = ms / live.size();
 }
 
-// A launch's evaluations each have exchange rings of their own (122 MiB at Dp = 64).  A class whose rings would
+// A launch's evaluations each have exchange rings of their own (106 MiB at Dp = 64).  A class whose rings would
 // take more than this runs in several launches, so that the memory of a batch of hundreds is that of its
-// samples (110 evaluations at D = 64: 12.6 -> 8.2 GiB).  67 evaluations at Dp = 64 fill the chip 67 times over, so
+// samples (110 evaluations at D = 64: 12.6 -> 8.2 GiB).  77 evaluations at Dp = 64 fill the chip 77 times over, so
 // that one more launch costs nothing: 128 of them took 1367 ms in one launch and take 1363 in two.
 constexpr size_t kRingBytes = (size_t)8 << 30;
 

@@ -26,9 +26,9 @@ __device__ __forceinline__ double cabsd(cplx a) { return hypot(a.re, a.im); }
 
 // ---------------------------------------------------------------------------------------
 // Agent-coherent (sc1) accesses through buffer resources.  Stores write through the
-// workgroup's L2, loads are served coherently, so data produced by a workgroup on another
-// XCD is seen once its flag is seen.  num_records bounds every access: an access outside
-// [0, bytes) reads zero / is dropped instead of faulting.
+// workgroup's L2, loads are served coherently: a load repeated on an exchange slot sees what a
+// workgroup on another XCD stored there, each aligned 8 bytes whole (exchange.h).  num_records bounds
+// every access: an access outside [0, bytes) reads zero / is dropped instead of faulting.
 // ---------------------------------------------------------------------------------------
 #define RC_COHERENT_POLICY 16  // CPol::SC1
 #define RC_BUF_DWORD3 0x00020000

@@ -55,9 +55,9 @@ __device__ __forceinline__ bool rc_same(uint64_t mask, int id) {
 
 // Elements voff + soff + t stride, t < N, of the lanes that `use` them: the loads alone; rc_await then
 // repeats them until every element of the wave has arrived.  False when the abort word is set or
-// the wait outlasts its time budget (then the abort word is set).  The budget is wall-clock time: a
-// workgroup that starts a later round of a batched launch early may wait a whole round for
-// partners that are still running.
+// the wait outlasts its time budget (then the abort word is set).  The budget is wall-clock time: in
+// a batched launch every workgroup runs a list of tasks, and one that starts a system early waits while its
+// partners still run the systems before it in theirs.
 template <int N>
 __device__ __forceinline__ void rc_fetch(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, uint32_t stride,
                                          cplx* v, bool use = true) {

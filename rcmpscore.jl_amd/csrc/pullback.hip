@@ -4,10 +4,11 @@
 //
 // As batched products and reductions per channel the pullback was 85 launches: 0.55 ms at D = 8, all of it
 // launches, and 1.6 ms at D = 64, where the products' intermediates made two more passes over memory.
-// Here a wave takes one column block of a stream of nodes and keeps everything in registers: the
+// Here a wave takes one column block of a stream of nodes and keeps its products in registers: the
 // accumulator of M = w R^+ A + .. (lane: rows 4 q + lane / 16, column lane % 16) is, quad by quad, the
 // right-hand fragment of k-step q, so M feeds the next product without a move.  The waves of a
-// workgroup hold the column blocks of the same nodes, whose F they read together.  Every stream of nodes
+// workgroup hold the column blocks of the same nodes, whose F they read together.  From three column blocks
+// on R^+ and F are in LDS, and still 208 bytes a lane (NB = 3; 272 at NB = 4) are kept in scratch.  Every stream of nodes
 // leaves whole partial matrices, summed in order by a second kernel.
 //
 // Bound by the matrix cores at D = 64 (3 products a node and pair: 0.28 ms at the peak rate for 512
@@ -239,8 +240,8 @@ __global__ void __launch_bounds__(256) rc_action_pull(int Dp, const double* sums
     *o = cadd(*o, cscale(g, csub(cadd(s[e], s[2 * n + e]), cmul(tr, w))));
 }
 
-// blockIdx.y: output; sixteen waves share the nodes of 64 elements (four took 199 us at D = 64 with 512
-// nodes, a chain of 128 loads' latency in eights)
+// blockIdx.y: output; sixteen waves share the nodes of 64 elements (133 us at D = 64 with 512 nodes; four took
+// 199, a chain of 128 loads' latency in eights)
 __global__ void __launch_bounds__(1024) rc_lin(const RcLinArgs g, int Dp) {
     constexpr int P = 16;
     __shared__ cplx red[64 * P];

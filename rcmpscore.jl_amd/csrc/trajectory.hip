@@ -19,7 +19,7 @@
 //
 // Exchange between workgroups: the data are their own arrival flags.  Every stage input Y, level-1
 // tile P, E tile and error record goes into a ring of slots whose words hold a NaN pattern no
-// computation produces (rc_empty) until the value is stored; a consumer loads the elements it needs
+// computation produces (RC_EMPTY_WORD) until the value is stored; a consumer loads the elements it needs
 // with device-coherent loads straight into its MFMA fragments and repeats those that are still
 // empty.  An exchange is then one store and one load of device scope, with no wait for the store's
 // completion, no flag and no barrier of the workgroup; the products were a third of a stage and
@@ -30,7 +30,8 @@
 // event e + 16, and a post lies between, before which the producer waited for its stores.
 // The gather is deterministic (every workgroup adds the same records in the same order), so every
 // workgroup of a system takes the same controller decision.  Every wait is bounded by a time
-// budget and watches an abort word.
+// budget and watches an abort word; a workgroup whose wait failed leaves a mark in its system's results
+// (rc_system_status), which the host takes before the status.
 //
 // Places: the launch lays a system on one XCD where it fits, and a channel's tiles are then kept in
 // that XCD's L2 (rc_put).  At D = 64 that is 10% of a stage of a system of one or two channels; the
@@ -48,10 +49,10 @@
 // two sums of partial tiles per stage at D = 64, and the wave's own instructions: a check of the arrived
 // words by one running maximum instead of two compares an element is worth 5% of a stage, running sums
 // of the combinations ahead instead of a window of derivatives, the wide gather of records and the FSAL
-// stage ahead of the verdict another 5%.  Measured on MI355X, per right-hand side of the slowest system,
-// against one flag per tile, a wait for the store and LDS panels: D = 8 5.8 -> 2.7 us, D = 32 with Z2
-// blocks 7.3 -> 3.0, D = 40 9.1 -> 4.3, D = 64 9.4 -> 4.5 (split 9.5 -> 5.8); six trajectories at
-// D = 64, window 30, 1e-13/1e-12: 62 -> 30 ms.
+// stage ahead of the verdict another 5%.  Measured on MI355X, the launch's time over the right-hand sides of the
+// system that has most of them, against one flag per tile, a wait for the store and LDS panels, in one run:
+// D = 8 6.1 -> 2.7 us, D = 32 with Z2 blocks 7.1 -> 3.0, D = 40 9.0 -> 4.2, D = 64 9.2 -> 4.5 (split 9.3 ->
+// 5.8); six trajectories at D = 64, window 30, 1e-13/1e-12: 60.6 -> 29.8 ms.
 #include "device_common.h"
 #include "exchange.h"
 #include "split.h"

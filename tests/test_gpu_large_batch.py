@@ -1,4 +1,4 @@
-"""A batch of more evaluations than one launch's exchange rings are kept for (8 GiB, 67 of them at D = 64): its
+"""A batch of more evaluations than one launch's exchange rings are kept for (8 GiB, 77 of them at D = 64): its
 device memory is bounded, and the results are the single calls' bits, also where the boundary solves of a launch
 need several launches of their own (more than 16 of them at D = 64)."""
 import numpy as np
@@ -25,7 +25,7 @@ def test_rings_of_a_large_batch_are_bounded(rg):
     free = torch.cuda.mem_get_info()[0]
     energies, gradients = rg.fg_phi4_batch(states, gs)
     taken = free - torch.cuda.mem_get_info()[0]
-    samples = 17 * 15 * d * d * 16 * n          # one evaluation's 15 channels at 17 points
+    samples = 17 * 13 * d * d * 16 * n          # one evaluation's 13 channels at 17 points
     print(f"  taken {taken / 2**30:.2f} GiB, samples {samples / 2**30:.2f} GiB", flush=True)
     assert taken <= (8 << 30) + samples + (1 << 30)   # rings, samples, workspaces; with rings of all 12.6 GiB
     for i in (0, 20, 54, 55, n - 1):
